@@ -68,7 +68,7 @@ struct hgpm_ctx {
     void* boxes = nullptr;   // half-tile cell boxes of the last windows pass
     bool boxes_valid = false; // ... and the positions have not changed since
     int nslots = HGPM_DEP_SLOTS;
-    float2 *twf = nullptr, *twr = nullptr, *twf_ic = nullptr;
+    float2 *twf = nullptr, *twr = nullptr, *twf_ic = nullptr, *twr_ic = nullptr; // _ic: length np, shared when np = ng
     float* hs = nullptr; // sin^2(pi m/ng), the Green's function's per-axis terms
     // FP64 plain path
     double *pos64 = nullptr, *vel64 = nullptr, *grad64 = nullptr;
@@ -540,8 +540,11 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
         }
         if ((rc = upload_twiddles<float2>(c, c->fft, &c->twf, &c->twr))) return bail(rc);
         if (c->np != c->ng) {
-            if ((rc = upload_twiddles<float2>(c, c->fftic, &c->twf_ic, nullptr))) return bail(rc);
-        } else c->twf_ic = c->twf;
+            if ((rc = upload_twiddles<float2>(c, c->fftic, &c->twf_ic, &c->twr_ic))) return bail(rc);
+        } else {
+            c->twf_ic = c->twf;
+            c->twr_ic = c->twr;
+        }
         // per-axis Green's function table sin^2(pi m/ng)
         std::vector<float> hs(p->ng);
         for (int m = 0; m < p->ng; m++) {
@@ -603,6 +606,7 @@ int hgpm_destroy(hgpm_ctx* c) {
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     if (c->twf_ic && c->twf_ic != c->twf) (void)hipFree(c->twf_ic);
+    if (c->twr_ic && c->twr_ic != c->twr) (void)hipFree(c->twr_ic);
     if (c->tw64_ic && c->tw64_ic != c->tw64) (void)hipFree(c->tw64_ic);
     for (auto& pe : c->pending) { (void)hipEventDestroy(pe.a); (void)hipEventDestroy(pe.b); }
     for (auto e : c->evpool) (void)hipEventDestroy(e);
@@ -914,23 +918,58 @@ int generate_ic_from(hgpm_ctx* c, const double* d_ipk, int ipk_bins, double ipk_
         // reference float rounding of the velocity factor (place_particles_initializer.cu:200-205)
         float velA = (float)(a - (deltaT * 0.5f));
         float velMul = (float)((double)(velA * velA) * dot_delta * fscal);
-        launch_ic_noise<float2>(c->A, np, seed, c->st);
-        if ((rc = fft3d_f32(c, c->fftic, c->A, c->twf_ic, -1))) return rc;
-        launch_ic_scale<float2>(c->A, np, d_ipk, ipk_bins, ipk_k_delta, c->p.rl, c->st);
-        for (int d = 0; d < 3; d++) {
-            launch_ic_displacement<float2>(c->A, c->B, np, d, delta, c->p.rl, c->st);
-            if ((rc = fft3d_f32(c, c->fftic, c->B, c->twf_ic, +1))) return rc;
-            launch_ic_place_split(c->B, c->pos, c->vel, np, c->ng, d, delta, velMul, c->st);
+        // Half spectra throughout (the noise and the displacements are real): noise ->
+        // modes -> phi^ (k_x_ic) -> the three displacement components, in the arena
+        // (24 bytes per grid cell: one half spectrum and four real grids of np^3), which
+        // holds nothing between deposits.
+        const FftOps* f = c->fftic;
+        const size_t n3 = (size_t)np * np * np;
+        float2* h3 = (float2*)c->arena;
+        float* real = (float*)(c->arena + 2 * n3);
+        float *sx = real, *sy = real + n3, *sz = real + 2 * n3;
+        const int v = f == c->fft ? c->var_cols : 2;
+        IcSpectrum sp;
+        sp.tab = d_ipk;
+        sp.nbins = ipk_bins;
+        sp.k_delta = ipk_k_delta;
+        sp.dk = (2 * HGPM_PI_D) / c->p.rl;
+        sp.amp = sqrt((double)n3 / (c->p.rl * c->p.rl * c->p.rl)) / delta;
+        // the bins a mode can fall into (ic_check bounds them by the table, one more for the
+        // FP32 rounding of k), as lines beside the noise: sy and sz are free until then
+        const int reach = (int)(sqrt(3.0) * (np / 2) * sp.dk / ipk_k_delta) + 2;
+        const bool room = (size_t)reach * sizeof(double2) <= 2 * sizeof(float) * n3 && sp.amp > 0.0;
+        sp.line = room ? (const double2*)sy : nullptr;
+        sp.nline = reach;
+        {
+            Timed t(c, "ic_noise");
+            if (room) launch_ic_lines(d_ipk, ipk_bins, ipk_k_delta, sp.amp, (double2*)sy, reach, c->st);
+            launch_ic_noise_f32(sx, np, seed, c->st);
         }
+        {
+            Timed t(c, "ic_forward");
+            f->fwd_z_r2c_real(sx, c->A, c->twf_ic, c->st);
+            f->pass_half(c->A, 1, -1, c->twf_ic, v, 1, c->st);
+        }
+        {
+            Timed t(c, "ic_inverse");
+            f->ic_x(c->A, c->B, c->twf_ic, c->twr_ic, sp, c->st);
+            f->pass_half(c->A, 1, +1, c->twf_ic, v, 1, c->st);
+            f->ic_y(c->B, h3, c->twf_ic, sp.dk, c->st);
+            f->inv_z_c2r_real(c->A, sx, c->twf_ic, 1, c->st);
+            f->inv_z_c2r_real(h3, sy, c->twf_ic, 1, c->st);
+            f->ic_z(c->B, sz, c->twf_ic, sp.dk, c->st);
+        }
+        Timed t(c, "ic_place");
+        launch_ic_place_split(sx, sy, sz, c->pos, c->vel, np, c->ng, delta, velMul, c->st);
     } else {
         double velA = a - deltaT * 0.5;
         double velMul = velA * velA * dot_delta * fscal;
         double2* amp = (double2*)c->grad64;
-        launch_ic_noise<double2>(amp, np, seed, c->st);
+        launch_ic_noise_f64(amp, np, seed, c->st);
         if ((rc = fft3d_f64(c, c->fftic, amp, c->tw64_ic, -1))) return rc;
-        launch_ic_scale<double2>(amp, np, d_ipk, ipk_bins, ipk_k_delta, c->p.rl, c->st);
+        launch_ic_scale_f64(amp, np, d_ipk, ipk_bins, ipk_k_delta, c->p.rl, c->st);
         for (int d = 0; d < 3; d++) {
-            launch_ic_displacement<double2>(amp, c->grid64, np, d, delta, c->p.rl, c->st);
+            launch_ic_displacement_f64(amp, c->grid64, np, d, delta, c->p.rl, c->st);
             if ((rc = fft3d_f64(c, c->fftic, c->grid64, c->tw64_ic, +1))) return rc;
             launch_ic_place_f64(c->grid64, c->pos64, c->vel64, np, c->ng, d, delta, velMul, c->st);
         }

@@ -103,8 +103,14 @@ __host__ __device__ __forceinline__ PosSplit unpack(const PosPack& q) {
 // Fixed-point coordinate of the grid-unit position x (FP64): rint(x 2^22) mod ng 2^22.
 __host__ __device__ __forceinline__ unsigned fx_from_double(double x, int ng) {
     const long long span = (long long)ng << HGPM_FRAC_BITS;
-    long long s = (long long)rint(x * (double)(1u << HGPM_FRAC_BITS)) % span;
+    long long s = (long long)rint(x * (double)(1u << HGPM_FRAC_BITS));
+    // one box out at most, mostly: a 64-bit remainder costs far more than the test
     if (s < 0) s += span;
+    else if (s >= span) s -= span;
+    if ((unsigned long long)s >= (unsigned long long)span) {
+        s %= span;
+        if (s < 0) s += span;
+    }
     return (unsigned)s;
 }
 // Drift of one coordinate (UpdatePosKernel, update_positions_pm.cu:3-20, in fixed point):

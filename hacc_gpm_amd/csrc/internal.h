@@ -6,6 +6,17 @@
 
 namespace hgpm {
 
+// Spectrum of the initial conditions, for the x pass that applies it (k_fft.hip ic_factor).
+struct IcSpectrum {
+    const double2* line; // (A, B) per bin of the .ipk table: a mode's factor is exp(A + B log k^2)
+    int nline;           // bins a mode of the grid can fall into
+    const double* tab;   // the .ipk table itself, where the lines found no room (line null)
+    int nbins;
+    double k_delta;      // bin width of the table
+    double dk;           // 2 pi / rl
+    double amp;          // sqrt(np^3 / rl^3) / delta
+};
+
 // Transform-length-specific operations, one table per supported length.
 struct FftOps {
     int n;
@@ -31,6 +42,14 @@ struct FftOps {
                   hipStream_t s);
     // real rows from their half spectra (after the inverse x, y passes)
     void (*inv_z_c2r_real)(const float2* hz, float* out, const float2* tw, int nbox, hipStream_t s);
+    // initial conditions, one box on half spectra: half spectra of a real grid; the x pass
+    // (noise -> modes of the x displacement in h1, shared modes in h2), the y pass of the
+    // shared modes (h2 in place, the y displacement's to h3), and the real rows of the z
+    // displacement's modes
+    void (*fwd_z_r2c_real)(const float* in, float2* out, const float2* tw, hipStream_t s);
+    void (*ic_x)(float2* h1, float2* h2, const float2* twf, const float2* twr, const IcSpectrum& sp, hipStream_t s);
+    void (*ic_y)(float2* h2, float2* h3, const float2* tw, double dk, hipStream_t s);
+    void (*ic_z)(const float2* hz, float* out, const float2* tw, double dk, hipStream_t s);
 };
 
 #define HGPM_FFT_SIZES(X) X(32) X(64) X(96) X(128) X(192) X(256) X(384) X(512) X(768) X(1024)
@@ -165,14 +184,20 @@ void launch_power_bins(const V* spec, int ng, double rl_fold, double minK, doubl
 int power_partial_blocks(int ng);
 
 // ---- IC (k_ic.hip) ----
-template <typename V>
-void launch_ic_noise(V* grid, int np, uint32_t seed, hipStream_t s);
-template <typename V>
-void launch_ic_scale(V* grid, int np, const double* ipk, int ipk_bins, double k_delta, double rl, hipStream_t s);
-template <typename V>
-void launch_ic_displacement(const V* amp, V* out, int np, int dim, double delta, double rl, hipStream_t s);
-void launch_ic_place_split(const float2* s_grid, PosPackH* pos, float* vel, int np, int ng, int dim,
-                           double delta, float vel_mul, hipStream_t s);
+// FP32: the white noise as a real grid; the first n lines of the .ipk table as IcSpectrum
+// wants them; every particle from the three displacement components (real grids in the
+// reference's order, unnormalised).
+void launch_ic_noise_f32(float* grid, int np, uint32_t seed, hipStream_t s);
+void launch_ic_lines(const double* ipk, int ipk_bins, double k_delta, double amp, double2* line, int n,
+                     hipStream_t s);
+void launch_ic_place_split(const float* sx, const float* sy, const float* sz, PosPackH* pos, float* vel, int np,
+                           int ng, double delta, float vel_mul, hipStream_t s);
+// FP64 plain path: complex grids, one axis per call
+void launch_ic_noise_f64(double2* grid, int np, uint32_t seed, hipStream_t s);
+void launch_ic_scale_f64(double2* grid, int np, const double* ipk, int ipk_bins, double k_delta, double rl,
+                         hipStream_t s);
+void launch_ic_displacement_f64(const double2* amp, double2* out, int np, int dim, double delta, double rl,
+                                hipStream_t s);
 void launch_ic_place_f64(const double2* s_grid, double* pos, double* vel, int np, int ng, int dim,
                          double delta, double vel_mul, hipStream_t s);
 // Device address of the fixed .ipk staging array (HGPM_IC_STATIC_BINS doubles) on

@@ -19,12 +19,16 @@
 //           x transform, in place;
 //   c2r   : phi rows in pairs as one complex transform of the Hermitian extension of
 //           phi^_a + i phi^_b.
+// The initial conditions use the same passes: the noise is real and so is each
+// displacement component (k_x_ic, k_y_ic, k_rows_c2r_real<KZ>).
 // The reference's gradient, F_d^ = -i sin(k_d) G rho^ with G = -g, is F_d^ = i sin(k_d)
 // psi^ with psi = IFFT(g rho^): the central difference F_d[n] = (psi[n + e_d] -
 // psi[n - e_d]) / 2 = phi[n + e_d] - phi[n - e_d] of the real field phi = psi / 2, which
 // the force gather forms (one inverse transform, not three).
 #include "fft.h"
 #include "internal.h"
+
+using hgpm::IcSpectrum;
 
 #ifndef HGPM_FFT_N
 #error "compile with -DHGPM_FFT_N=<transform length>"
@@ -106,7 +110,8 @@ __global__ __launch_bounds__(NTC) void k_cols_c2c(V* __restrict d, const V* __re
 // once; A[k] = (C[k] + conj C[N-k]) / 2 and B[k] = (C[k] - conj C[N-k]) / 2i give the
 // half spectra, k = 0..N/2, written with pitch HZ (padding written as zero).
 // rhof: see fwd_z_r2c (the owner pass wrote the same FP32 values when no tile was deferred).
-template <int RC>
+// REAL: the rows are those of the FP32 grid rhof (initial conditions' noise).
+template <int RC, bool REAL>
 __global__ __launch_bounds__(NT) void k_rows_r2c_density(const long long* __restrict rho,
                                                          const float* __restrict rhof,
                                                          const unsigned long long* __restrict ctl,
@@ -116,9 +121,9 @@ __global__ __launch_bounds__(NT) void k_rows_r2c_density(const long long* __rest
     __shared__ float2 lds[lds_elems<N, PC>()];
     float2* spec = lds; // the last stage has read all its inputs before the first output
     const size_t row0 = (size_t)blockIdx.x * RC;
-    const bool f32 = rhof != nullptr && ctl[1] == 0ull;
+    const bool f32 = REAL || (rhof != nullptr && ctl[1] == 0ull);
     // total of this row's box: a batch holds several boxes of the same shape
-    const double mean = (double)(long long)total[row0 / ((size_t)N * N)] / ((double)N * N * N);
+    const double mean = REAL ? 0.0 : (double)(long long)total[row0 / ((size_t)N * N)] / ((double)N * N * N);
     fft_tile<float2, N, PC, NT, -1, false, true>(
         [&](int, int, int n, int c) {
             if (f32) return make_float2(rhof[(row0 + 2 * c) * N + n], rhof[(row0 + 2 * c + 1) * N + n]);
@@ -179,6 +184,96 @@ __global__ __launch_bounds__(NTC) void k_x_psi(float2* __restrict h1, const floa
         [&](int, int, int n, int c, float2 v) { h1[base + n * NP + c] = v; }, lds, twr);
 }
 
+// ------------------------------------------------- initial conditions ----
+// k of mode index n along one axis (the reference's get_kmode in FP32: n, or n - N from
+// N/2 on, times dk = 2 pi / rl), and -i k v.
+__device__ __forceinline__ float mode_k(int n, double dk) { return (float)((double)(n > N / 2 - 1 ? n - N : n) * dk); }
+__device__ __forceinline__ float2 minus_ik(float2 v, float k) { return make_float2(v.y * k, -v.x * k); }
+
+// sqrt(P) amp / k^2 of a mode, in FP64: the .ipk log-log interpolation
+// (do_pk_interpolation, src/initial_conditions/cuda/interpolation_initializer.cu:3-30,
+// on k from the FP32 sum of squares), ScaleAmplitudes and the 1 / k^2 of
+// transformDensityField: one logarithm and one exponential on the bin's line, or
+// written out where a bin has none (an empty bin; a table with so many bins below the
+// grid's largest k that the lines found no room).
+__device__ __forceinline__ double ic_factor(float kx, float ky, float kz, const IcSpectrum& sp) {
+#pragma clang fp contract(off)
+    float s = kx * kx;
+    s = s + ky * ky;
+    s = s + kz * kz;
+    if (s == 0.0f) return 0.0;
+    const double k = sqrt((double)s), ls = log((double)s);
+    if (sp.line) {
+        const double2 ab = sp.line[min((int)(k / sp.k_delta), sp.nline - 1)];
+        if (ab.x == ab.x) return exp(ab.x + ab.y * ls);
+    }
+    const int l = min((int)(k / sp.k_delta), sp.nbins - 2);
+    double y = log(sp.tab[1]);
+    if (l > 0) {
+        const double x1 = log(sp.k_delta * (double)l), x2 = log(sp.k_delta * (double)(l + 1)), y1 = log(sp.tab[l]);
+        y = y1 + (log(sp.tab[l + 1]) - y1) / (x2 - x1) * (0.5 * ls - x1);
+    }
+    return exp(0.5 * y - ls) * sp.amp;
+}
+
+// x pass of the initial conditions.  In: h1 = the noise after the z and y forward passes.
+// Forward x transform, phi^ = amplitude * sqrt(P) / (delta k^2), and two inverse x
+// transforms: of -i k_x phi^ (to h1: the x displacement's modes) and of phi^ itself (to
+// h2: -i k_y and -i k_z act on the other axes, so the y and z displacements share this
+// transform and take their factors in the passes along y and z).  The reference
+// transforms complex grids and keeps the real part; a mode at N/2 of axis d is its own
+// mirror there with the same sign of k_d, so its -i k_d part is imaginary: dropped here.
+// Bound by the FP64 work of the factor (a logarithm, an exponential, a root and a
+// quotient per mode) and its three transforms: 8.3 ms at 1024^3 for 13 GB.  8 columns x
+// 1024 threads there: with 16 columns the modes kept between the transforms do not fit
+// the registers (85 spilled, 9.5 ms).  The whole of the initial conditions at 1024^3 went
+// from 131 ms on complex grids (four transforms, three displacement passes, the spectrum
+// with five logarithms per mode) to 38 ms.
+template <int CC, int NTC>
+__global__ __launch_bounds__(NTC) void k_x_ic(float2* __restrict h1, float2* __restrict h2,
+                                              const float2* __restrict twf, const float2* __restrict twr,
+                                              IcSpectrum sp) {
+    __shared__ float2 lds[lds_elems<N, CC>()];
+    const int tile = (int)xcd_remap(blockIdx.x, gridDim.x);
+    const int y = tile / (HZ / CC), zc = tile % (HZ / CC);
+    const size_t base = (size_t)y * HZ + (size_t)zc * CC;
+    typedef LastShape<N, CC, NTC> LS;
+    float2 R[LS::NB][LS::R];
+    const float ky = mode_k(y, sp.dk), kz = mode_k(zc * CC + (int)threadIdx.x % CC, sp.dk);
+    fft_tile<float2, N, CC, NTC, -1, false, false>(
+        [&](int, int, int n, int c) { return h1[base + n * NPH + c]; },
+        [&](int b, int r, int n, int, float2 v) {
+            const double f = ic_factor(mode_k(n, sp.dk), ky, kz, sp);
+            R[b][r] = make_float2((float)((double)v.x * f), (float)((double)v.y * f));
+        },
+        lds, twf);
+    fft_tile<float2, N, CC, NTC, +1, true, false>(
+        [&](int b, int r, int n, int) { return minus_ik(R[b][r], n == N / 2 ? 0.0f : mode_k(n, sp.dk)); },
+        [&](int, int, int n, int c, float2 v) { h1[base + n * NPH + c] = v; }, lds, twr);
+    fft_tile<float2, N, CC, NTC, +1, true, false>(
+        [&](int b, int r, int, int) { return R[b][r]; },
+        [&](int, int, int n, int c, float2 v) { h2[base + n * NPH + c] = v; }, lds, twr);
+}
+
+// y pass of the initial conditions: inverse y transforms of phi^ (h2, in place: the z
+// displacement's, its factor taken by the z pass) and of -i k_y phi^ (to h3), from one
+// read of the tile (3.5 ms at 1024^3, two passes over memory and one more of writing).
+template <int CC, int NTC>
+__global__ __launch_bounds__(NTC) void k_y_ic(float2* __restrict h2, float2* __restrict h3,
+                                              const float2* __restrict tw, double dk) {
+    __shared__ float2 lds[lds_elems<N, CC>()];
+    const int tile = (int)xcd_remap(blockIdx.x, gridDim.x);
+    const size_t base = (size_t)(tile / (HZ / CC)) * NPH + (size_t)(tile % (HZ / CC)) * CC;
+    typedef StageShape<N, CC, NTC, Plan<N>::R(0)> SS;
+    float2 X[SS::NB][Plan<N>::R(0)];
+    fft_tile<float2, N, CC, NTC, +1, false, false>(
+        [&](int b, int r, int n, int c) { return X[b][r] = h2[base + (size_t)n * HZ + c]; },
+        [&](int, int, int n, int c, float2 v) { h2[base + (size_t)n * HZ + c] = v; }, lds, tw);
+    fft_tile<float2, N, CC, NTC, +1, false, false>(
+        [&](int b, int r, int n, int) { return minus_ik(X[b][r], n == N / 2 ? 0.0f : mode_k(n, dk)); },
+        [&](int, int, int n, int c, float2 v) { h3[base + (size_t)n * HZ + c] = v; }, lds, tw);
+}
+
 // Element n of the Hermitian extension of a half-spectrum row: h[n] for n <= N/2,
 // conj h[N-n] above.
 __device__ __forceinline__ float2 herm(const float2* __restrict row, int n) {
@@ -193,15 +288,22 @@ __device__ __forceinline__ float2 herm(const float2* __restrict row, int n) {
 // than a wave (N / R_last < 64: lengths with a radix-3 or radix-16 first stage, and
 // N <= 256) its direct stores would scatter each wave over several rows in short
 // pieces; the rows then go through LDS and are stored whole, lane after lane.
-template <int RC>
+// KZ: the half spectra are multiplied by -i k_z first (k_z = m dk; zero at N/2, see k_x_ic).
+template <int RC, bool KZ>
 __global__ __launch_bounds__(NT) void k_rows_c2r_real(const float2* __restrict hz, float* __restrict out,
-                                                      const float2* __restrict tw) {
+                                                      const float2* __restrict tw, double dk) {
     constexpr int PC = RC / 2;
     constexpr bool STAGED = N / Plan<N>::R(Plan<N>::S - 1) < 64;
     __shared__ float2 lds[lds_elems<N, PC>()];
     const size_t row0 = (size_t)blockIdx.x * RC;
     auto ld = [&](int, int, int n, int c) {
-        const float2 a = herm(hz + hrow(row0 + 2 * c), n), b = herm(hz + hrow(row0 + 2 * c + 1), n);
+        float2 a = herm(hz + hrow(row0 + 2 * c), n), b = herm(hz + hrow(row0 + 2 * c + 1), n);
+        if constexpr (KZ) {
+            // conj(-i k v) = -i (-k) conj(v): the mirrored half takes its own (negative) k_z
+            const float k = n == N / 2 ? 0.0f : mode_k(n, dk);
+            a = minus_ik(a, k);
+            b = minus_ik(b, k);
+        }
         return make_float2(a.x - b.y, a.y + b.x);
     };
     if constexpr (!STAGED) {
@@ -296,12 +398,30 @@ void fwd_z_r2c(const long long* rho, const float* rhof, const unsigned long long
                const unsigned long long* totals, float2* out, const float2* tw, int nbox, hipStream_t s) {
     constexpr int RC = 2 * rc32();
     unsigned nb = (unsigned)((size_t)nbox * N * N / RC);
-    k_rows_r2c_density<RC><<<nb, NT, 0, s>>>(rho, rhof, ctl, totals, out, tw);
+    k_rows_r2c_density<RC, false><<<nb, NT, 0, s>>>(rho, rhof, ctl, totals, out, tw);
+}
+void fwd_z_r2c_real(const float* in, float2* out, const float2* tw, hipStream_t s) {
+    constexpr int RC = 2 * rc32();
+    k_rows_r2c_density<RC, true><<<(unsigned)((size_t)N * N / RC), NT, 0, s>>>(nullptr, in, nullptr, nullptr, out, tw);
 }
 void inv_z_c2r_real(const float2* hz, float* out, const float2* tw, int nbox, hipStream_t s) {
     constexpr int RC = 2 * rc32();
     unsigned nb = (unsigned)((size_t)nbox * N * N / RC);
-    k_rows_c2r_real<RC><<<nb, NT, 0, s>>>(hz, out, tw);
+    k_rows_c2r_real<RC, false><<<nb, NT, 0, s>>>(hz, out, tw, 0.0);
+}
+// The initial conditions' passes, one box: 16 columns (128-byte rows), 1024 threads where
+// such a tile leaves one workgroup per CU; the x pass then 8 columns (k_x_ic).
+constexpr int NT_IC = N >= 512 ? 1024 : 512;
+void ic_x(float2* h1, float2* h2, const float2* twf, const float2* twr, const IcSpectrum& sp, hipStream_t s) {
+    constexpr int CC = N >= 512 ? 8 : 16;
+    k_x_ic<CC, NT_IC><<<N * (HZ / CC), NT_IC, 0, s>>>(h1, h2, twf, twr, sp);
+}
+void ic_y(float2* h2, float2* h3, const float2* tw, double dk, hipStream_t s) {
+    k_y_ic<16, NT_IC><<<N * (HZ / 16), NT_IC, 0, s>>>(h2, h3, tw, dk);
+}
+void ic_z(const float2* hz, float* out, const float2* tw, double dk, hipStream_t s) {
+    constexpr int RC = 2 * rc32();
+    k_rows_c2r_real<RC, true><<<(unsigned)((size_t)N * N / RC), NT, 0, s>>>(hz, out, tw, dk);
 }
 template <int CC, int NTC>
 void x_psi_launch(float2* h1, const float2* twf, const float2* twr, const float* hs, int nbox, hipStream_t s) {
@@ -332,7 +452,7 @@ extern const FftOps HGPM_CAT(HGPM_CAT(fft_ops_, HGPM_FFT_N), _alt) = {
 extern const FftOps HGPM_CAT(fft_ops_, HGPM_FFT_N) = {
 #endif
     N, Plan<N>::S, NVAR, variant_mask(), twiddles, pass_f32, pass_f64, fwd_z_density,
-    HZ, pass_half, fwd_z_r2c, x_psi, inv_z_c2r_real,
+    HZ, pass_half, fwd_z_r2c, x_psi, inv_z_c2r_real, fwd_z_r2c_real, ic_x, ic_y, ic_z,
 };
 } // namespace hgpm
 #endif

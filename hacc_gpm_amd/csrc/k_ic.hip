@@ -11,6 +11,8 @@
 //                  psi_d^ = -i k_d / k^2 * amp / delta.
 //   place        : placeParticles (place_particles_initializer.cu:49-65) after the
 //                  inverse transform and the 1/np^3 ScaleFFT.
+// The FP32 path runs scale and displacement inside its transform passes (k_fft.hip,
+// k_x_ic); the kernels here for them are the FP64 plain path's.
 #include "common.h"
 #include "internal.h"
 #include "../../include/hgpm.h"
@@ -98,14 +100,32 @@ __device__ double normal_at(uint32_t seed, uint64_t idx) {
     return r * det_cos2pi(u2);
 }
 
-template <typename V> __global__ void k_noise(V* __restrict g, int64_t n, uint32_t seed) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void k_noise_f32(float* __restrict g, int64_t n, uint32_t seed) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) g[i] = (float)normal_at(seed, (uint64_t)i);
+}
+__global__ void k_noise_f64(double2* __restrict g, int64_t n, uint32_t seed) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) g[i] = make_double2(normal_at(seed, (uint64_t)i), 0.0);
+}
+
+// The .ipk table as the FP32 path's x pass interpolates it (IcSpectrum::line): log P is
+// linear in log k between bins, so the factor sqrt(P) amp / k^2 of a mode of squared
+// wavenumber s is exp(A + B log s) with one (A, B) per bin.
+__global__ void k_ic_lines(const double* __restrict in, double2* __restrict line, int n, int nbins, double k_delta,
+                           double amp) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    typedef decltype(V().x) T;
-    V v;
-    v.x = (T)normal_at(seed, (uint64_t)i);
-    v.y = (T)0;
-    g[i] = v;
+    const int l = min(i, nbins - 2);
+    double m = 0.0, y = log(in[1]); // the first interval is constant
+    if (l > 0) {
+        const double x1 = log(k_delta * (double)l), y1 = log(in[l]);
+        m = (log(in[l + 1]) - y1) / (log(k_delta * (double)(l + 1)) - x1);
+        y = y1 - m * x1; // log P = y + m log k
+    }
+    const double A = 0.5 * y + log(amp), B = 0.25 * m - 1.0;
+    // an empty bin (log 0) has no line: NaN sends its modes to the formula itself
+    line[i] = isfinite(A) && isfinite(B) ? make_double2(A, B) : make_double2(__builtin_nan(""), 0.0);
 }
 
 __device__ __forceinline__ float kmode(int idx, int ng, double d) {
@@ -115,8 +135,7 @@ __device__ __forceinline__ float kmode(int idx, int ng, double d) {
 }
 
 // do_pk_interpolation (interpolation_initializer.cu:3-30) then ScaleAmplitudes.
-template <typename V>
-__global__ void k_scale(V* __restrict g, int np, const double* __restrict in, int nbins, double k_delta, double rl) {
+__global__ void k_scale_f64(double2* __restrict g, int np, const double* __restrict in, int nbins, double k_delta, double rl) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     int64_t G = (int64_t)np * np * np;
     if (i >= G) return;
@@ -146,35 +165,13 @@ __global__ void k_scale(V* __restrict g, int np, const double* __restrict in, in
         }
     }
     double f = sqrt(y);
-    V v = g[i];
-    typedef decltype(V().x) T;
-    v.x = (T)((double)v.x * f);
-    v.y = (T)((double)v.y * f);
+    double2 v = g[i];
+    v.x *= f;
+    v.y *= f;
     g[i] = v;
 }
 
-// transformDensityField for one axis.  FP32: the reference's float k and float data;
-// FP64: all double.
-__global__ void k_disp_f32(const float2* __restrict amp, float2* __restrict out, int np, int dim, double delta,
-                           double rl) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t G = (int64_t)np * np * np;
-    if (i >= G) return;
-    int ix = (int)(i / ((int64_t)np * np)), iy = (int)((i / np) % np), iz = (int)(i % np);
-    double d = (2 * HGPM_PI) / rl;
-    float kx = kmode(ix, np, d), ky = kmode(iy, np, d), kz = kmode(iz, np, d);
-    float s = kx * kx;
-    s = s + ky * ky;
-    s = s + kz * kz;
-    double k2 = (double)s;
-    double k2mul = k2 == 0 ? 0.0 : 1.0 / k2;
-    double mul = (1.0 / delta) * k2mul;
-    float2 c = amp[i];
-    c.x = (float)((double)c.x * mul);
-    c.y = (float)((double)c.y * mul);
-    float kd = dim == 0 ? kx : (dim == 1 ? ky : kz);
-    out[i] = make_float2(c.y * kd, -c.x * kd);
-}
+// transformDensityField for one axis.
 __global__ void k_disp_f64(const double2* __restrict amp, double2* __restrict out, int np, int dim, double delta,
                            double rl) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -193,25 +190,42 @@ __global__ void k_disp_f64(const double2* __restrict amp, double2* __restrict ou
     out[i] = make_double2(ci * kd, -cr * kd);
 }
 
-// placeParticles for one axis: x = q ng/np + delta psi (FP64, then fixed point:
-// rint(x 2^22) mod ng 2^22), v = velMul psi.
-__global__ void k_place_split(const float2* __restrict sg, PosPack* __restrict pos, float* __restrict vel, int np,
-                              int ng, int dim, double delta, float vel_mul) {
-    const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; // internal (tile) order
-    const int64_t G = (int64_t)np * np * np;
-    if (j >= G) return;
-    int qx, qy, qz;
-    const int64_t i = ref_index(j, np, &qx, &qy, &qz);
-    const int q = dim == 0 ? qx : (dim == 1 ? qy : qz);
-    float s = (float)((double)sg[i].x * (1.0 / (double)G));
-    double x = (double)q * ((double)ng / (double)np) + delta * (double)s;
-    const unsigned X = fx_from_double(x, ng);
-    // one axis per call: the others keep what the earlier calls placed (x, y, z order)
-    if (dim == 0) pos[j].x = X;
-    else if (dim == 1) pos[j].y = X;
-    else pos[j].z = X;
-    vel[3 * j + dim] = vel_mul * s;
+// placeParticles: x = q ng/np + delta psi (FP64, then fixed point: rint(x 2^22) mod
+// ng 2^22), v = velMul psi, the three axes of a particle together: one 12-byte store each
+// of position and velocity.  A workgroup places 16 rows of 16 lattice points of one
+// Lagrangian tile, so the tile's place is found by scalar divisions and a lane's by its
+// bits.  Bound by memory: three 4-byte grids read in 64-byte pieces (neighbouring tiles
+// share the 128-byte lines, on one XCD), 24 bytes written per particle: 7.6 ms at 1024^3,
+// 5.1 TB/s (36.5 ms one axis at a time from complex grids, with 4-byte stores 12 bytes
+// apart; 11.5 ms with 64-bit divisions per lane for the lattice place and the wrap).
+static_assert(BS == HGPM_TL * HGPM_TL, "one x plane of a tile per workgroup");
+__global__ __launch_bounds__(BS) void k_place_split(const float* __restrict sx, const float* __restrict sy,
+                                                    const float* __restrict sz, PosPack* __restrict pos,
+                                                    float* __restrict vel, int np, int ng, double delta,
+                                                    float vel_mul) {
+    const unsigned w = (unsigned)xcd_remap(blockIdx.x, gridDim.x); // tile, x plane of the tile
+    const unsigned t = w / HGPM_TL, nt = (unsigned)np / HGPM_TL, tyx = t / nt;
+    const unsigned l = threadIdx.x;
+    const unsigned q[3] = {tyx / nt * HGPM_TL + w % HGPM_TL, tyx % nt * HGPM_TL + l / HGPM_TL,
+                           t % nt * HGPM_TL + l % HGPM_TL};
+    const unsigned i = (q[0] * np + q[1]) * np + q[2]; // < 2^30
+    const float g[3] = {sx[i], sy[i], sz[i]};
+    const double inv = 1.0 / ((double)np * np * np), step = (double)ng / (double)np;
+    unsigned X[3];
+    float v[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const float s = (float)((double)g[d] * inv);
+        X[d] = fx_from_double((double)q[d] * step + delta * (double)s, ng);
+        v[d] = vel_mul * s;
+    }
+    const int64_t j = (int64_t)w * BS + l; // internal (tile) order
+    pos[j] = PosPack{X[0], X[1], X[2]};
+#pragma unroll
+    for (int d = 0; d < 3; d++) vel[3 * j + d] = v[d];
 }
+
+// ... FP64, one axis per call
 __global__ void k_place_f64(const double2* __restrict sg, double* __restrict pos, double* __restrict vel, int np,
                             int ng, int dim, double delta, double vel_mul) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -231,32 +245,29 @@ inline unsigned nblk(int64_t n) { return (unsigned)((n + BS - 1) / BS); }
 } // namespace
 
 namespace hgpm {
-template <typename V> void launch_ic_noise(V* g, int np, uint32_t seed, hipStream_t s) {
-    int64_t n = (int64_t)np * np * np;
-    k_noise<V><<<nblk(n), BS, 0, s>>>(g, n, seed);
+void launch_ic_noise_f32(float* g, int np, uint32_t seed, hipStream_t s) {
+    const int64_t n = (int64_t)np * np * np;
+    k_noise_f32<<<nblk(n), BS, 0, s>>>(g, n, seed);
 }
-template void launch_ic_noise<float2>(float2*, int, uint32_t, hipStream_t);
-template void launch_ic_noise<double2>(double2*, int, uint32_t, hipStream_t);
-
-template <typename V>
-void launch_ic_scale(V* g, int np, const double* ipk, int ipk_bins, double k_delta, double rl, hipStream_t s) {
-    int64_t n = (int64_t)np * np * np;
-    k_scale<V><<<nblk(n), BS, 0, s>>>(g, np, ipk, ipk_bins, k_delta, rl);
+void launch_ic_noise_f64(double2* g, int np, uint32_t seed, hipStream_t s) {
+    const int64_t n = (int64_t)np * np * np;
+    k_noise_f64<<<nblk(n), BS, 0, s>>>(g, n, seed);
 }
-template void launch_ic_scale<float2>(float2*, int, const double*, int, double, double, hipStream_t);
-template void launch_ic_scale<double2>(double2*, int, const double*, int, double, double, hipStream_t);
-
-template <> void launch_ic_displacement<float2>(const float2* amp, float2* out, int np, int dim, double delta,
-                                                double rl, hipStream_t s) {
-    k_disp_f32<<<nblk((int64_t)np * np * np), BS, 0, s>>>(amp, out, np, dim, delta, rl);
+void launch_ic_lines(const double* ipk, int ipk_bins, double k_delta, double amp, double2* line, int n,
+                     hipStream_t s) {
+    k_ic_lines<<<nblk(n), BS, 0, s>>>(ipk, line, n, ipk_bins, k_delta, amp);
 }
-template <> void launch_ic_displacement<double2>(const double2* amp, double2* out, int np, int dim, double delta,
-                                                 double rl, hipStream_t s) {
+void launch_ic_scale_f64(double2* g, int np, const double* ipk, int ipk_bins, double k_delta, double rl,
+                         hipStream_t s) {
+    k_scale_f64<<<nblk((int64_t)np * np * np), BS, 0, s>>>(g, np, ipk, ipk_bins, k_delta, rl);
+}
+void launch_ic_displacement_f64(const double2* amp, double2* out, int np, int dim, double delta, double rl,
+                                hipStream_t s) {
     k_disp_f64<<<nblk((int64_t)np * np * np), BS, 0, s>>>(amp, out, np, dim, delta, rl);
 }
-void launch_ic_place_split(const float2* sg, PosPackH* pos, float* vel, int np, int ng, int dim, double delta,
-                           float vel_mul, hipStream_t s) {
-    k_place_split<<<nblk((int64_t)np * np * np), BS, 0, s>>>(sg, (PosPack*)pos, vel, np, ng, dim, delta, vel_mul);
+void launch_ic_place_split(const float* sx, const float* sy, const float* sz, PosPackH* pos, float* vel, int np,
+                           int ng, double delta, float vel_mul, hipStream_t s) {
+    k_place_split<<<nblk((int64_t)np * np * np), BS, 0, s>>>(sx, sy, sz, (PosPack*)pos, vel, np, ng, delta, vel_mul);
 }
 void launch_ic_place_f64(const double2* sg, double* pos, double* vel, int np, int ng, int dim, double delta,
                          double vel_mul, hipStream_t s) {

@@ -621,6 +621,44 @@ def test_fp64_kick_drift(hg, orc):
         np.testing.assert_allclose(p2, orc.drift_f64(ng, pos, v, pf), rtol=0, atol=1e-11)
 
 
+@pytest.mark.parametrize("ng,np_,rl", [(32, 32, 64.0), (32, 32, 8.0), (96, 96, 50.0), (192, 32, 700.0),
+                                       (256, 128, 100.0), (256, 256, 512.0)])
+def test_initial_conditions_half_spectra(hg, ng, np_, rl, tmp_path):
+    """The FP32 initial conditions (real transforms on half spectra, the spectrum applied in
+    the x pass) against the FP64 plain path's complex ones, which keep the real part: the
+    padded and the unpadded half-spectrum pitch, a radix-3 length, np < ng, a box whose low
+    modes fall into the table's first, constant interval, and a table with more bins than
+    the lines have room for (rl 8).  Each FP32 transform is good
+    to 2e-6 in relative L2 (test_fft_fp32) and two follow one another; positions are
+    rounded to 2^-22 cells besides."""
+    case(f"ic half spectra ng={ng} np={np_}")
+    out = []
+    for prec in (0, 1):
+        p = hg.make_params(ng, np_, rl, 50.0, 0.0, 100, seed=77, precision=prec)
+        hdr, vals = ipk_for(hg, p, str(tmp_path))
+        if rl == 700.0:  # 2 pi / rl = 0.009: bins of 0.02 put the lowest modes in bin 0
+            vals, hdr = vals[::20].copy(), hdr.copy()
+            hdr[3] *= 20
+        ts = hg.Timestepper(p)
+        ts.setInitialZ(p.z_ini)
+        ts.reverseHalfStep()
+        with hg.MemoryManager(p) as m:
+            hg.GenerateDisplacementIC(m, p, ts, hdr, vals)
+            if prec:
+                out.append(m.get_particles_f64())
+            else:
+                c, o, v = m.get_particles_split()
+                out.append((c + o.astype(np.float64), v))
+    (x, v), (xo, vo) = out
+    half = ng / 2
+    q = np.indices((np_,) * 3).reshape(3, -1).T * (ng / np_)
+    d, disp = (x - xo + half) % ng - half, (xo - q + half) % ng - half
+    rms = lambda a: np.sqrt((a ** 2).mean(axis=0))  # noqa: E731  per axis
+    print(f"[result] rel dx {rms(d) / rms(disp)} rel dv {rms(v - vo) / rms(vo)}")
+    assert (rms(d) <= 4e-6 * rms(disp) + 2.0 ** -23).all()
+    assert (rms(v - vo) <= 4e-6 * rms(vo)).all()
+
+
 # ------------------------------------------------------------------ P(k) ----
 @pytest.mark.parametrize("ng,folds", [(32, 0), (64, 0), (64, 2)])
 def test_power_spectrum(hg, orc, ng, folds):
