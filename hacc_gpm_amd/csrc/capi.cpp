@@ -76,7 +76,7 @@ struct hgpm_ctx {
     double2 *tw64 = nullptr, *tw64_ic = nullptr;
     // P(k)
     double *pk_partial = nullptr, *pk_sums = nullptr, *pk_win = nullptr;
-    long long* pk_counts = nullptr;
+    long long* pk_counts = nullptr; // behind pk_sums
     int pk_blocks = 0;
     int* flag = nullptr;
     // state
@@ -259,7 +259,7 @@ float ref_mass(const hgpm_ctx* c) {
 }
 
 // ------------------------------------------------------------ FP32 ops ----
-DepositBuffers dep_buffers(hgpm_ctx* c) {
+DepositBuffers dep_buffers(hgpm_ctx* c, int fold) {
     DepositBuffers b;
     b.arena = c->arena;
     b.cap = c->arena_cap;
@@ -275,9 +275,10 @@ DepositBuffers dep_buffers(hgpm_ctx* c) {
     b.boxes = c->boxes;
     b.nbox = c->nbox;
     b.totals = c->total;
-    b.ppt = c->dep_ppt;
+    b.ppt = fold ? 8 : c->dep_ppt;
+    b.fold = fold;
     // about 256 tiles per sub-arena, at most HGPM_DEP_NSUB sub-arenas
-    const int64_t nt = c->N * c->nbox / (512 * c->dep_ppt);
+    const int64_t nt = c->N * c->nbox / (512 * b.ppt);
     b.nsub = (int)std::max<int64_t>(1, std::min<int64_t>(HGPM_DEP_NSUB, nt / 256));
     return b;
 }
@@ -286,21 +287,25 @@ DepositBuffers dep_buffers(hgpm_ctx* c) {
 // deferred tiles.  The density is the int64 grid B (every cell written); with fused
 // (a step whose solve follows at once) the owner pass writes it as the FP32 grid the
 // forward z transform takes, into psi's buffer, when no tile was deferred (decided on
-// the device).
-int f32_deposit(hgpm_ctx* c, bool fused = false) {
-    const DepositBuffers b = dep_buffers(c);
+// the device).  fold: the positions folded that many times (P(k) of one box).
+int f32_deposit(hgpm_ctx* c, bool fused = false, int fold = 0) {
+    const DepositBuffers b = dep_buffers(c, fold);
     Timed t(c, "deposit");
     launch_deposit_begin(c->ctl, (unsigned long long)(c->ng / 16) * (c->ng / 16) * (c->ng / 16) * c->nbox, c->st);
-    {
-        Timed t1(c, "deposit_windows");
-        launch_deposit_windows(c->pos, c->N * c->nbox, c->ng, ref_mass(c), b, c->st);
-        c->boxes_valid = true;
-    }
-    if (fused) {
-        Timed t2(c, "deposit_totals");
-        launch_deposit_totals(c->N * c->nbox, b, c->st);
-    }
-    {
+    if (fold) {
+        Timed t1(c, "deposit_binned");
+        launch_deposit_binned(c->pos, c->N, c->ng, ref_mass(c), (long long*)c->B, fused ? c->psi : nullptr, b, c->st);
+        c->boxes_valid = false;
+    } else {
+        {
+            Timed t1(c, "deposit_windows");
+            launch_deposit_windows(c->pos, c->N * c->nbox, c->ng, ref_mass(c), b, c->st);
+            c->boxes_valid = true;
+        }
+        if (fused) {
+            Timed t2(c, "deposit_totals");
+            launch_deposit_totals(c->N * c->nbox, b, c->st);
+        }
         Timed t2(c, "deposit_owner");
         launch_deposit_owner(c->ng, (long long*)c->B, fused ? c->psi : nullptr, b, c->st);
     }
@@ -403,18 +408,20 @@ int pk_bin_spectrum(hgpm_ctx* c, int fold, double* k, double* pk, int64_t* count
     {
         Timed t(c, "power_bins");
         if (c->prec == HGPM_FP32)
-            launch_power_bins<float2>(c->A, c->ng, rl_fold, minK, bd, nb, c->pk_win, scale, c->pk_partial,
-                                      c->pk_counts, c->pk_blocks, c->pk_sums, c->st);
+            launch_power_bins<float2, true>(c->A, c->ng, c->fft->hz, c->fft->plane, rl_fold, minK, bd, nb, c->pk_win,
+                                            scale, c->pk_partial, c->pk_blocks, c->pk_sums, c->pk_counts, c->st);
         else
-            launch_power_bins<double2>(c->grid64, c->ng, rl_fold, minK, bd, nb, c->pk_win, scale, c->pk_partial,
-                                       c->pk_counts, c->pk_blocks, c->pk_sums, c->st);
+            launch_power_bins<double2, false>(c->grid64, c->ng, c->ng, (size_t)c->ng * c->ng, rl_fold, minK, bd, nb,
+                                              c->pk_win, scale, c->pk_partial, c->pk_blocks, c->pk_sums,
+                                              c->pk_counts, c->st);
         LAUNCHCHK(c);
     }
-    std::vector<double> sums(nb);
-    std::vector<long long> cnt(nb);
-    HIPCHK(c, hipMemcpyAsync(sums.data(), c->pk_sums, sizeof(double) * nb, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipMemcpyAsync(cnt.data(), c->pk_counts, sizeof(long long) * nb, hipMemcpyDeviceToHost, c->st));
+    // sums and counts are one allocation: one copy
+    std::vector<double> sums(2 * (size_t)nb);
+    HIPCHK(c, hipMemcpyAsync(sums.data(), c->pk_sums, 2 * sizeof(double) * nb, hipMemcpyDeviceToHost, c->st));
     HIPCHK(c, hipStreamSynchronize(c->st));
+    std::vector<long long> cnt(nb);
+    memcpy(cnt.data(), sums.data() + nb, sizeof(long long) * nb);
     for (int i = 0; i < nb; i++) {
         if (k) k[i] = kb[i];
         if (count) count[i] = cnt[i];
@@ -580,12 +587,13 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
             win[m] = r * r * r * r;
         }
     }
-    if ((rc = dalloc(c, &c->pk_partial, sizeof(double) * (size_t)c->pk_blocks * p->pk_bins, "pk partial")) ||
-        (rc = dalloc(c, &c->pk_sums, sizeof(double) * p->pk_bins, "pk sums")) ||
-        (rc = dalloc(c, &c->pk_counts, sizeof(long long) * p->pk_bins, "pk counts")) ||
+    static_assert(sizeof(long long) == sizeof(double), "counts behind the sums");
+    if ((rc = dalloc(c, &c->pk_partial, 2 * sizeof(double) * (size_t)c->pk_blocks * p->pk_bins, "pk partial")) ||
+        (rc = dalloc(c, &c->pk_sums, 2 * sizeof(double) * p->pk_bins, "pk sums and counts")) ||
         (rc = dalloc(c, &c->pk_win, sizeof(double) * p->ng, "pk window")) ||
         (rc = dalloc(c, &c->flag, sizeof(int), "flag")))
         return bail(rc);
+    c->pk_counts = (long long*)(c->pk_sums + p->pk_bins);
     if (hipMemcpy(c->pk_win, win.data(), sizeof(double) * p->ng, hipMemcpyHostToDevice) != hipSuccess) {
         c->err = "window upload failed";
         return bail(HGPM_ERR_HIP);
@@ -602,7 +610,7 @@ int hgpm_destroy(hgpm_ctx* c) {
     if (c->st) (void)hipStreamSynchronize(c->st);
     void* ptrs[] = {c->pos, c->vel, c->A, c->B, c->psi, c->ctl, c->totals, c->arena, c->dslots, c->dcount, c->deferred, c->wide, c->wide_slots, c->tile_total, c->boxes, c->twf, c->twr, c->hs,
                     c->pos64, c->vel64, c->grid64, c->grad64, c->tw64, c->pk_partial, c->pk_sums,
-                    c->pk_counts, c->pk_win, c->flag};
+                    c->pk_win, c->flag};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     if (c->twf_ic && c->twf_ic != c->twf) (void)hipFree(c->twf_ic);
@@ -1255,13 +1263,15 @@ int hgpm_power_spectrum_grid(hgpm_ctx* c, int fold, double* k, double* pk, int64
     int rc;
     if (c->prec == HGPM_FP32) {
         {
+            // half spectra, as the solve's: the density is real
             Timed t(c, "pk_fwd_z_density");
-            c->fft->fwd_z_density((const long long*)c->B, c->total, c->A, c->twf, c->st);
+            c->fft->fwd_z_r2c((const long long*)c->B, c->dens_f32 ? c->psi : nullptr, c->ctl, c->total, c->A, c->twf, 1,
+                              c->st);
         }
         {
             Timed t(c, "pk_fwd_yx");
-            c->fft->pass_f32(c->A, 1, -1, c->twf, c->var_cols, c->st);
-            c->fft->pass_f32(c->A, 0, -1, c->twf, c->var_cols, c->st);
+            c->fft->pass_half(c->A, 1, -1, c->twf, c->var_cols, 1, c->st);
+            c->fft->pass_half(c->A, 0, -1, c->twf, c->var_cols, 1, c->st);
         }
         LAUNCHCHK(c);
     } else {
@@ -1278,25 +1288,8 @@ int hgpm_power_spectrum(hgpm_ctx* c, int fold, double* k, double* pk, int64_t* c
     if (rc) return rc;
     if (fold < 0 || fold > c->p.pk_folds) return fail(c, HGPM_ERR_ARG, "fold out of range");
     if (c->prec == HGPM_FP32) {
-        if (fold == 0) {
-            if ((rc = f32_deposit(c))) return rc;
-        } else {
-            // fold a copy of the positions (x -> 2^fold x mod ng, exact in the split
-            // layout) held in a temporary buffer
-            PosPackH* tmp = nullptr;
-            if ((rc = dalloc(c, &tmp, sizeof(PosPackH) * c->N, "fold copy"))) return rc;
-            c->bytes -= sizeof(PosPackH) * c->N;
-            HIPCHK(c, hipMemcpyAsync(tmp, c->pos, sizeof(PosPackH) * c->N, hipMemcpyDeviceToDevice, c->st));
-            for (int f = 0; f < fold; f++) launch_fold_split(tmp, c->N, c->ng, c->st);
-            PosPackH* keep = c->pos;
-            c->pos = tmp;
-            rc = f32_deposit(c);
-            c->pos = keep;
-            c->boxes_valid = false; // the boxes are those of the folded copy
-            HIPCHK(c, hipStreamSynchronize(c->st));
-            (void)hipFree(tmp);
-            if (rc) return rc;
-        }
+        // the transform follows at once: the FP32 density of a step serves
+        if ((rc = f32_deposit(c, true, fold))) return rc;
     } else {
         double* src = c->pos64;
         double* tmp = nullptr;

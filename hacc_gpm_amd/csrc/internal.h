@@ -27,11 +27,10 @@ struct FftOps {
     // axis 2 = rows (z), 1 = y, 0 = x; variant selects the column-pass shape
     void (*pass_f32)(float2* d, int axis, int dir, const float2* tw, int variant, hipStream_t s);
     void (*pass_f64)(double2* d, int axis, int dir, const double2* tw, hipStream_t s);
-    void (*fwd_z_density)(const long long* rho, const unsigned long long* total, float2* out,
-                          const float2* tw, hipStream_t s);
     // half-spectrum solve (rows of hz = n/2 + 16 complex, k_z = 0..n/2) on nbox grids of
     // the same shape stored back to back; totals[b] is box b's deposited mass
     int hz;
+    size_t plane; // elements from one x plane of half spectra to the next
     void (*pass_half)(float2* d, int axis, int dir, const float2* tw, int variant, int nbox, hipStream_t s);
     // rhof non-null: the density is the FP32 grid rhof when ctl[1] == 0 (no deferred
     // tiles, see launch_deposit_owner), else the int64 grid rho
@@ -122,7 +121,8 @@ struct DepositBuffers {
     void* boxes; // 32 B per half tile: the cell box the gather stages (written by the windows pass)
     int nbox;    // boxes of the same shape stored back to back (particles, grids, owner blocks)
     unsigned long long* totals; // deposited mass per box
-    int ppt;                    // particles per thread of a deposit tile: 8 or 4
+    int ppt;                    // particles per thread of a deposit tile: 8 or 4 (8 when folded)
+    int fold;                   // folds of the positions (P(k)), 0 = none
 };
 // The windows pass with 32-bit cells, then the 64-bit pass over the tiles it listed (a
 // cell over 2^32 - 1 mass units).  ctl must be cleared and the chunk counts zero.
@@ -142,6 +142,11 @@ void launch_deposit_owner(int ng, long long* rho, float* rhof, const DepositBuff
 void launch_deposit_totals(int64_t np3, const DepositBuffers& b, hipStream_t s);
 void launch_deposit_deferred(const PosPackH* pos, int64_t np3, int ng, float mass, long long* rho,
                              const DepositBuffers& b, hipStream_t s);
+// The deposit of one box's folded positions (b.fold > 0), between launch_deposit_begin and
+// launch_deposit_deferred in place of the windows, totals and owner passes: rho / rhof as
+// launch_deposit_owner writes them.
+void launch_deposit_binned(const PosPackH* pos, int64_t np3, int ng, float mass, long long* rho, float* rhof,
+                           const DepositBuffers& b, hipStream_t s);
 // variant 0: 512-thread workgroups on half tiles; 1: 256-thread workgroups on quarter tiles
 // boxes: the half-tile boxes of the last deposit when the positions have not changed
 // since, else nullptr (the gather reduces them itself); psi: the potential of the solve
@@ -158,7 +163,6 @@ void launch_to_internal(const PosPackH* src, const float* vsrc, PosPackH* dst, f
                         hipStream_t s);
 void launch_to_reference(const PosPackH* src, const float* vsrc, PosPackH* dst, float* vdst, int64_t np3, int np,
                          hipStream_t s);
-void launch_fold_split(PosPackH* pos, int64_t np3, int ng, hipStream_t s);
 // forces (3 floats per cell) of one box from its potential, as the gather forms them
 void launch_force_from_psi(const float* psi, float* out, int ng, hipStream_t s);
 void launch_scan_nonfinite(const float* v, int64_t n, int* flag, hipStream_t s);
@@ -176,11 +180,13 @@ void launch_compare(const PosPackH* pa, const float* va, const double* pa64, con
                     double* partial, hipStream_t s);
 
 // ---- P(k) (k_power.hip) ----
-// bins of a complex spectrum (ng^3) with FP64 deterministic sums.
-template <typename V>
-void launch_power_bins(const V* spec, int ng, double rl_fold, double minK, double binDelta, int nbins,
-                       const double* win, double scale, double* partial_sums, long long* counts,
-                       int nblocks, double* sums_out, hipStream_t s);
+// Shell bins of a spectrum with ordered FP64 sums: full grids, or (HALF) half spectra of a
+// real field, rows of `pitch` and x planes of `plane` elements.  partial holds
+// 2 nbins power_partial_blocks(ng) doubles; sums and counts receive nbins entries each.
+template <typename V, bool HALF>
+void launch_power_bins(const V* spec, int ng, int pitch, size_t plane, double rl_fold, double minK, double binDelta,
+                       int nbins, const double* win, double scale, double* partial, int nblocks, double* sums,
+                       long long* counts, hipStream_t s);
 int power_partial_blocks(int ng);
 
 // ---- IC (k_ic.hip) ----

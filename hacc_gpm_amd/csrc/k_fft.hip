@@ -65,23 +65,6 @@ __global__ __launch_bounds__(NT) void k_rows_c2c(V* __restrict d, const V* __res
         [&](int, int, int n, int c, V v) { d[(row0 + c) * N + n] = v; }, lds, tw);
 }
 
-// Forward transform along z of the int64 fixed-point density, mean removed in FP64
-// (the k = 0 normalisation) before the FP32 rounding.
-template <int RC>
-__global__ __launch_bounds__(NT) void k_rows_density(const long long* __restrict rho,
-                                                     const unsigned long long* __restrict total,
-                                                     float2* __restrict out, const float2* __restrict tw) {
-    __shared__ float2 lds[lds_elems<N, RC>()];
-    const size_t row0 = (size_t)blockIdx.x * RC;
-    const double mean = (double)(long long)(*total) / ((double)N * N * N);
-    fft_tile<float2, N, RC, NT, -1, false, true>(
-        [&](int, int, int n, int c) {
-            double q = (double)rho[(row0 + c) * N + n];
-            return make_float2((float)((q - mean) * (1.0 / 16777216.0)), 0.0f);
-        },
-        [&](int, int, int n, int c, float2 v) { out[(row0 + c) * N + n] = v; }, lds, tw);
-}
-
 // ------------------------------------------------------------- cols ----
 // axis 1 (y): tile = (x, z-chunk), element (n=y, c) at x N^2 + n N + z0 + c
 // axis 0 (x): tile = (y, z-chunk), element (n=x, c) at n N^2 + y N + z0 + c
@@ -105,8 +88,8 @@ __global__ __launch_bounds__(NTC) void k_cols_c2c(V* __restrict d, const V* __re
 }
 
 // ------------------------------------------------- half-spectrum solve ----
-// Forward z transform of the int64 density (mean removed in FP64, as k_rows_density)
-// for RC real rows: rows 2c and 2c+1 form the complex column c = a + i b, transformed
+// Forward z transform of the int64 density, mean removed in FP64 (the k = 0 normalisation)
+// before the FP32 rounding, for RC real rows: rows 2c and 2c+1 form the complex column c = a + i b, transformed
 // once; A[k] = (C[k] + conj C[N-k]) / 2 and B[k] = (C[k] - conj C[N-k]) / 2i give the
 // half spectra, k = 0..N/2, written with pitch HZ (padding written as zero).
 // rhof: see fwd_z_r2c (the owner pass wrote the same FP32 values when no tile was deferred).
@@ -388,11 +371,6 @@ void pass_f64(double2* d, int axis, int dir, const double2* tw, hipStream_t s) {
     if (axis == 2) rows_launch<double2, rc64()>(d, dir, tw, s);
     else cols_launch<double2, cc64(), 512>(d, axis, dir, tw, N, (size_t)N * N, s);
 }
-void fwd_z_density(const long long* rho, const unsigned long long* total, float2* out, const float2* tw,
-                   hipStream_t s) {
-    unsigned nb = (unsigned)((size_t)N * N / rc32());
-    k_rows_density<rc32()><<<nb, NT, 0, s>>>(rho, total, out, tw);
-}
 // nbox grids of the same shape back to back (rows of every box in one launch)
 void fwd_z_r2c(const long long* rho, const float* rhof, const unsigned long long* ctl,
                const unsigned long long* totals, float2* out, const float2* tw, int nbox, hipStream_t s) {
@@ -451,8 +429,8 @@ extern const FftOps HGPM_CAT(HGPM_CAT(fft_ops_, HGPM_FFT_N), _alt) = {
 #else
 extern const FftOps HGPM_CAT(fft_ops_, HGPM_FFT_N) = {
 #endif
-    N, Plan<N>::S, NVAR, variant_mask(), twiddles, pass_f32, pass_f64, fwd_z_density,
-    HZ, pass_half, fwd_z_r2c, x_psi, inv_z_c2r_real, fwd_z_r2c_real, ic_x, ic_y, ic_z,
+    N, Plan<N>::S, NVAR, variant_mask(), twiddles, pass_f32, pass_f64,
+    HZ, NPH, pass_half, fwd_z_r2c, x_psi, inv_z_c2r_real, fwd_z_r2c_real, ic_x, ic_y, ic_z,
 };
 } // namespace hgpm
 #endif

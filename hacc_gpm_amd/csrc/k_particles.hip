@@ -125,12 +125,33 @@ template <int PPT> struct DepRegs {
 };
 __device__ __forceinline__ float fx_off_units(unsigned X) { return (float)(X & HGPM_FRAC_MASK); }
 
+// Positions of a deposit: as stored, or (P(k) of the box folded f times) x -> 2 (x mod
+// ng/2) f times, exact in fixed point: X -> 2 (X mod ng 2^21) (foldParticles,
+// src/power_spectrum/cuda/fold_particles_power.cu:3-27).
+__device__ __forceinline__ unsigned fold_coord(unsigned X, int f, unsigned half) {
+    for (int i = 0; i < f; i++) X = 2u * (X >= half ? X - half : X);
+    return X;
+}
+__device__ __forceinline__ PosPack fold_pos(const PosPack& q, int f, int ng) {
+    const unsigned half = (unsigned)ng << (HGPM_FRAC_BITS - 1);
+    return PosPack{fold_coord(q.x, f, half), fold_coord(q.y, f, half), fold_coord(q.z, f, half)};
+}
+struct StoredPos {
+    const PosPack* __restrict p;
+    __device__ __forceinline__ PosPack operator[](int64_t j) const { return p[j]; }
+};
+struct FoldedPos {
+    const PosPack* __restrict p;
+    int f, ng;
+    __device__ __forceinline__ PosPack operator[](int64_t j) const { return fold_pos(p[j], f, ng); }
+};
+
 // Loads the tile starting at p0 and reduces the box of its cells: lo = minimum
 // relative cell, e = extent + 1 (the upper CIC neighbour).  The two halves of the tile
 // (particles k < PPT/2 and k >= PPT/2 of every thread: the gather's tiles when PPT = 8)
 // get their own boxes too: hb[h] = {lo[3], base cells per axis[3]}.
-template <int PPT>
-__device__ __forceinline__ void dep_load_box(const PosPack* __restrict pos, int64_t p0, int ng,
+template <int PPT, typename POS>
+__device__ __forceinline__ void dep_load_box(const POS& pos, int64_t p0, int ng,
                                              const PosSplit& r0, DepRegs<PPT>& R, int (*red)[DEP_NT / 64], int lo[3],
                                              int e[3], int (*hb)[6] = nullptr) {
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -526,7 +547,7 @@ __device__ __forceinline__ void dep_windows_tile(int tile, unsigned q, const Dep
     if (tid == 0) { sh.over = 0; sh.full = 0; } // ordered by the barrier in dep_load_box
     DepRegs<PPT> R;
     int lo[3], e[3], hb[2][6];
-    dep_load_box(g.pos, p0, ng, r0, R, sh.red, lo, e, hb);
+    dep_load_box(StoredPos{g.pos}, p0, ng, r0, R, sh.red, lo, e, hb);
     if (!WIDE && tid == 0) {
         // the gather of these positions stages its potential window from these boxes (one
         // per half Lagrangian tile, the gather's workgroup: both halves of a whole tile,
@@ -952,8 +973,8 @@ __global__ __launch_bounds__(OWN_NT) void k_deposit_owner64(OwnerArgs g) {
 }
 
 // Tiles listed by k_deposit_windows as deferred, after k_deposit_owner: int64 atomics.
-template <bool SMALL, int PPT>
-__global__ __launch_bounds__(DEP_NT) void k_deposit_deferred(const PosPack* __restrict pos, int64_t n, int ng,
+template <bool SMALL, int PPT, typename POS>
+__global__ __launch_bounds__(DEP_NT) void k_deposit_deferred(POS pos, int64_t n, int ng,
                                                              float mass, unsigned long long* __restrict rho,
                                                              const unsigned long long* __restrict ctl,
                                                              const unsigned* __restrict deferred,
@@ -991,6 +1012,201 @@ __global__ __launch_bounds__(256) void k_deposit_total(const unsigned long long*
     if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = t;
     __syncthreads();
     if (threadIdx.x == 0) atomicAdd(&totals[box], s[0] + s[1] + s[2] + s[3]);
+}
+
+// ----------------------------------------------------------------------------------
+// Binned deposit, for positions folded f times (P(k) of the folded box).  A tile's window
+// over folded positions is 2^f times as wide per axis and nearly empty: the windows
+// overflow the arena and every tile takes the atomic route.  Instead the particles are
+// sorted to the owner blocks whose cells they touch (one block, or two per axis where the
+// upper CIC corner lies in the next one: 1.2 entries per particle on average):
+//   k_bin_pass<false> : entries per block, counted per workgroup of 4096 particles in an
+//                       LDS hash table, one global atomic per block it touches; the
+//                       tiles' deposited mass;
+//   k_bin_scan        : where each block's entries start in the arena;
+//   k_bin_pass<true>  : the folded positions written there;
+//   k_bin_owner       : a workgroup per block adds its entries' weights in int64 LDS cells
+//                       and writes every cell once.
+// The sums are whole numbers, so the bits are those of every other route.  Entries beyond
+// the arena send the deposit to the atomic route (all tiles listed as deferred).  Bound by
+// the LDS table (an insertion or lookup per entry in both passes) more than by the 60
+// bytes a particle it moves.  Measured on evolved boxes with one fold: 0.66 ms at 256^3,
+// 4.9 ms at 512^3, 35 ms at 1024^3; through windows, nearly all of them deferred, a
+// fold's deposit took 5 ms at 256^3.
+constexpr int BIN_HASH = 8192;  // blocks a workgroup can count in LDS (64 KB with the keys)
+constexpr int BIN_PROBES = 64;  // slots tried before a block is counted in memory directly
+constexpr unsigned BIN_EMPTY = 0xFFFFFFFFu;
+struct BinArgs {
+    const PosPack* __restrict pos;
+    int ng, fold;
+    float mass;
+    PosPack* __restrict entries; // the arena
+    unsigned long long cap;      // entries it holds
+    unsigned* __restrict count;  // per block, zero between deposits
+    unsigned* __restrict start;  // per block: first entry ...
+    unsigned* __restrict cursor; // ... and the next free one (k_bin_pass<true>)
+    unsigned long long* __restrict ctl;
+    unsigned* __restrict deferred;
+    unsigned long long* __restrict tile_total;
+    unsigned long long* __restrict rho;
+    float* __restrict rhof; // see OwnerArgs
+    const unsigned long long* __restrict totals;
+    int nblk, nt;
+    int64_t gcells;
+};
+__device__ __forceinline__ unsigned bin_slot(unsigned* key, unsigned blk) {
+    unsigned h = (blk * 2654435761u) >> 19;
+    static_assert(BIN_HASH == 1 << 13, "13 hash bits");
+    for (int i = 0; i < BIN_PROBES; i++) {
+        const unsigned old = atomicCAS(&key[h], BIN_EMPTY, blk);
+        if (old == BIN_EMPTY || old == blk) return h;
+        h = (h + 1) & (BIN_HASH - 1);
+    }
+    return BIN_EMPTY;
+}
+// body(block) for every owner block the particle's corners lie in.
+template <typename F> __device__ __forceinline__ void bin_blocks(const PosPack& q, int ng, F&& body) {
+    const int nb = ng / OB;
+    const unsigned X[3] = {q.x, q.y, q.z};
+    int b[3][2];
+    bool two[3];
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        const int c = fx_cell(X[d]);
+        b[d][0] = c / OB;
+        two[d] = c % OB == OB - 1;
+        b[d][1] = c + 1 == ng ? 0 : c / OB + 1;
+    }
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+        const int ix = i >> 2, iy = (i >> 1) & 1, iz = i & 1;
+        if ((ix && !two[0]) || (iy && !two[1]) || (iz && !two[2])) continue;
+        body((unsigned)((b[0][ix] * nb + b[1][iy]) * nb + b[2][iz]));
+    }
+}
+template <bool SMALL, bool FILL> __global__ __launch_bounds__(DEP_NT) void k_bin_pass(BinArgs g) {
+    __shared__ unsigned key[BIN_HASH], num[BIN_HASH];
+    __shared__ long long s_tot[DEP_NT / 64];
+    if (FILL && g.ctl[1]) return; // the entries do not fit: the atomic route
+    const int tid = threadIdx.x;
+    const int tile = (int)xcd_remap(blockIdx.x, gridDim.x);
+    for (int i = tid; i < BIN_HASH; i += DEP_NT) {
+        key[i] = BIN_EMPTY;
+        num[i] = 0u;
+    }
+    const PosPack* __restrict at = g.pos + (int64_t)tile * DEP_TILE + tid; // tiles are full
+    __syncthreads();
+    long long dep = 0;
+#pragma unroll 1
+    for (int k = 0; k < DEP_PPT; k++) {
+        const PosPack q = fold_pos(at[k * DEP_NT], g.fold, g.ng);
+        bin_blocks(q, g.ng, [&](unsigned blk) {
+            const unsigned s = bin_slot(key, blk);
+            if (s != BIN_EMPTY) atomicAdd(&num[s], 1u);
+            else if (!FILL) atomicAdd(&g.count[blk], 1u);
+        });
+        if constexpr (!FILL) {
+            constexpr float ONE = (float)(1u << HGPM_FRAC_BITS);
+            const float fx = fx_off_units(q.x), fy = fx_off_units(q.y), fz = fx_off_units(q.z);
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                dep += fixed_weight<SMALL>(i & 4 ? fx : ONE - fx, i & 2 ? fy : ONE - fy, i & 1 ? fz : ONE - fz, g.mass);
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < BIN_HASH; i += DEP_NT) {
+        const unsigned blk = key[i];
+        if (blk == BIN_EMPTY) continue;
+        if constexpr (FILL) num[i] = atomicAdd(&g.cursor[blk], num[i]);
+        else atomicAdd(&g.count[blk], num[i]);
+    }
+    if constexpr (FILL) {
+        __syncthreads();
+#pragma unroll 1
+        for (int k = 0; k < DEP_PPT; k++) {
+            const PosPack q = fold_pos(at[k * DEP_NT], g.fold, g.ng);
+            bin_blocks(q, g.ng, [&](unsigned blk) {
+                const unsigned s = bin_slot(key, blk);
+                g.entries[s != BIN_EMPTY ? atomicAdd(&num[s], 1u) : atomicAdd(&g.cursor[blk], 1u)] = q;
+            });
+        }
+    } else {
+        dep_tile_total(dep, s_tot, &g.tile_total[tile]);
+    }
+}
+constexpr int BIN_SCAN = 1024;
+__global__ __launch_bounds__(BIN_SCAN) void k_bin_scan(BinArgs g) {
+    __shared__ unsigned long long s[BIN_SCAN];
+    const int tid = threadIdx.x;
+    const int per = (g.nblk + BIN_SCAN - 1) / BIN_SCAN, b0 = min(tid * per, g.nblk), b1 = min(b0 + per, g.nblk);
+    unsigned long long t = 0;
+    for (int b = b0; b < b1; b++) t += g.count[b];
+    s[tid] = t;
+    __syncthreads();
+    for (int off = 1; off < BIN_SCAN; off <<= 1) {
+        const unsigned long long v = tid >= off ? s[tid - off] : 0ull;
+        __syncthreads();
+        s[tid] += v;
+        __syncthreads();
+    }
+    const unsigned long long all = s[BIN_SCAN - 1];
+    if (all > g.cap) { // no entries: every block is written empty, every tile is deferred
+        for (int b = b0; b < b1; b++) g.count[b] = 0u;
+        for (int i = tid; i < g.nt; i += BIN_SCAN) g.deferred[i] = (unsigned)i;
+        if (tid == 0) g.ctl[1] = (unsigned long long)g.nt;
+        return;
+    }
+    t = s[tid] - t;
+    for (int b = b0; b < b1; b++) {
+        const unsigned n = g.count[b];
+        g.start[b] = (unsigned)t;
+        g.cursor[b] = (unsigned)t;
+        t += n;
+    }
+}
+template <bool SMALL> __global__ __launch_bounds__(OWN_NT) void k_bin_owner(BinArgs g) {
+    __shared__ unsigned long long acc[OB * OB * OB];
+    __shared__ unsigned s_n, s_at;
+    const int tid = threadIdx.x, ng = g.ng, nb = ng / OB;
+    const int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
+    const int b[3] = {blk / (nb * nb) * OB, blk / nb % nb * OB, blk % nb * OB};
+    if (tid == 0) {
+        s_n = g.count[blk];
+        s_at = g.start[blk]; // not read when the block has no entries
+        g.count[blk] = 0u;
+    }
+    for (int i = tid; i < OB * OB * OB; i += OWN_NT) acc[i] = 0ull;
+    __syncthreads();
+    const unsigned n = s_n;
+    const PosPack* __restrict e = g.entries + s_at;
+    for (unsigned i = tid; i < n; i += OWN_NT) {
+        const PosPack q = e[i];
+        const unsigned X[3] = {q.x, q.y, q.z};
+        int c[3];
+        float w[3][2];
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            c[d] = fx_cell(X[d]) - b[d]; // in [0, OB), or one cell below the block (periodic)
+            if (c[d] >= OB) c[d] -= ng;
+            w[d][1] = fx_off_units(X[d]);
+            w[d][0] = (float)(1u << HGPM_FRAC_BITS) - w[d][1];
+        }
+#pragma unroll
+        for (int k = 0; k < 8; k++) {
+            const int x = c[0] + (k >> 2), y = c[1] + ((k >> 1) & 1), z = c[2] + (k & 1);
+            if ((unsigned)x < (unsigned)OB && (unsigned)y < (unsigned)OB && (unsigned)z < (unsigned)OB)
+                atomicAdd(&acc[(x * OB + y) * OB + z], (unsigned long long)fixed_weight<SMALL>(
+                                                           w[0][k >> 2], w[1][(k >> 1) & 1], w[2][k & 1], g.mass));
+        }
+    }
+    __syncthreads();
+    const bool f32 = g.rhof != nullptr && g.ctl[1] == 0ull;
+    const double mean = (double)(long long)g.totals[0] / (double)g.gcells;
+    for (int i = tid; i < OB * OB * OB; i += OWN_NT) {
+        const int64_t at = gidx(ng, b[0] + i / (OB * OB), b[1] + i / OB % OB, b[2] + i % OB);
+        if (f32) g.rhof[at] = (float)(((double)(long long)acc[i] - mean) * (1.0 / 16777216.0));
+        else g.rho[at] = acc[i];
+    }
 }
 
 // Force of a cell from the stored field phi = psi / 2 (half the potential, so that no
@@ -1474,19 +1690,6 @@ __global__ __launch_bounds__(CMP_NT) void k_compare(ParticleView a, ParticleView
     if (threadIdx.x < 4) partial[4 * blockIdx.x + threadIdx.x] = red[threadIdx.x][0];
 }
 
-// foldParticles (src/power_spectrum/cuda/fold_particles_power.cu:3-27): x -> 2 (x mod ng/2),
-// exact in fixed point: X -> 2 (X mod ng 2^21).
-__global__ void k_fold_split(PosPack* __restrict pos, int64_t n, int ng) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const unsigned half = (unsigned)ng << (HGPM_FRAC_BITS - 1);
-    PosPack q = pos[i];
-    q.x = 2u * (q.x % half);
-    q.y = 2u * (q.y % half);
-    q.z = 2u * (q.z % half);
-    pos[i] = q;
-}
-
 // Force of every cell (x, y, z order, 3 floats per cell) from the stored half potential of one box.
 __global__ void k_force_from_psi(const float* __restrict psi, float* __restrict out, int ng) {
     const int64_t g3 = (int64_t)ng * ng * ng;
@@ -1614,20 +1817,53 @@ void launch_deposit_deferred(const PosPackH* pos, int64_t n, int ng, float mass,
     const int ntb = (int)(nt / b.nbox);
     const int64_t gc = (int64_t)ng * ng * ng;
     const unsigned grid = (unsigned)(nt < 512 ? nt : 512);
-    auto run = [&](auto pc) {
+    auto run = [&](auto pc, auto p) {
         constexpr int PPT = decltype(pc)::value;
         if (mass < 128.0f)
-            k_deposit_deferred<true, PPT><<<grid, DEP_NT, 0, s>>>((const PosPack*)pos, n, ng, mass,
-                                                                  (unsigned long long*)rho, b.ctl, b.deferred,
-                                                                  b.tile_total, ntb, gc);
+            k_deposit_deferred<true, PPT><<<grid, DEP_NT, 0, s>>>(p, n, ng, mass, (unsigned long long*)rho, b.ctl,
+                                                                  b.deferred, b.tile_total, ntb, gc);
         else
-            k_deposit_deferred<false, PPT><<<grid, DEP_NT, 0, s>>>((const PosPack*)pos, n, ng, mass,
-                                                                   (unsigned long long*)rho, b.ctl, b.deferred,
-                                                                   b.tile_total, ntb, gc);
+            k_deposit_deferred<false, PPT><<<grid, DEP_NT, 0, s>>>(p, n, ng, mass, (unsigned long long*)rho, b.ctl,
+                                                                   b.deferred, b.tile_total, ntb, gc);
     };
-    if (b.ppt == 4) run(std::integral_constant<int, 4>{});
-    else run(std::integral_constant<int, 8>{});
+    const StoredPos sp{(const PosPack*)pos};
+    if (b.fold) run(std::integral_constant<int, 8>{}, FoldedPos{(const PosPack*)pos, b.fold, ng});
+    else if (b.ppt == 4) run(std::integral_constant<int, 4>{}, sp);
+    else run(std::integral_constant<int, 8>{}, sp);
     launch_deposit_totals(n, b, s);
+}
+void launch_deposit_binned(const PosPackH* pos, int64_t n, int ng, float mass, long long* rho, float* rhof,
+                           const DepositBuffers& b, hipStream_t s) {
+    BinArgs g;
+    g.pos = (const PosPack*)pos;
+    g.ng = ng;
+    g.fold = b.fold;
+    g.mass = mass;
+    g.entries = (PosPack*)b.arena;
+    g.cap = b.cap / 3; // 12-byte entries in 32-bit arena cells
+    g.count = b.count;
+    g.nblk = (ng / OB) * (ng / OB) * (ng / OB);
+    // the blocks' slot lists (1 KB a block) are free: no chunk is listed here
+    g.start = (unsigned*)b.slots;
+    g.cursor = g.start + g.nblk;
+    g.ctl = b.ctl;
+    g.deferred = b.deferred;
+    g.tile_total = b.tile_total;
+    g.rho = (unsigned long long*)rho;
+    g.rhof = rhof;
+    g.totals = b.totals;
+    g.nt = (int)(n / DEP_TILE);
+    g.gcells = (int64_t)ng * ng * ng;
+    auto run = [&](auto sc) {
+        constexpr bool SMALL = decltype(sc)::value;
+        k_bin_pass<SMALL, false><<<(unsigned)g.nt, DEP_NT, 0, s>>>(g);
+        k_bin_scan<<<1, BIN_SCAN, 0, s>>>(g);
+        launch_deposit_totals(n, b, s);
+        k_bin_pass<SMALL, true><<<(unsigned)g.nt, DEP_NT, 0, s>>>(g);
+        k_bin_owner<SMALL><<<(unsigned)g.nblk, OWN_NT, 0, s>>>(g);
+    };
+    if (mass < 128.0f) run(std::true_type{});
+    else run(std::false_type{});
 }
 template <int NT>
 void gather_launch(PosPackH* pos, float* vel, int64_t n, int ng, const float* psi, double deltaT, double fscal,
@@ -1676,10 +1912,6 @@ void launch_to_reference(const PosPackH* src, const float* vsrc, PosPackH* dst, 
                          hipStream_t s) {
     if (!n) return;
     k_to_reference<<<grid_blocks(n, BS), BS, 0, s>>>((const PosPack*)src, vsrc, (PosPack*)dst, vdst, n, np);
-}
-void launch_fold_split(PosPackH* pos, int64_t n, int ng, hipStream_t s) {
-    if (!n) return;
-    k_fold_split<<<grid_blocks(n, BS), BS, 0, s>>>((PosPack*)pos, n, ng);
 }
 void launch_force_from_psi(const float* psi, float* out, int ng, hipStream_t s) {
     const int64_t g3 = (int64_t)ng * ng * ng;

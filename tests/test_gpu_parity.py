@@ -684,6 +684,37 @@ def test_power_spectrum(hg, orc, ng, folds):
         assert np.array_equal(pk2, pk) and np.array_equal(cnt2, cnt)
 
 
+@pytest.mark.parametrize("ng,np_,folds,nb,sigma", [(32, 32, 6, 64, 0.7), (96, 96, 3, 65, 3.0), (128, 64, 2, 256, 0.7),
+                                                   (192, 32, 1, 1, 0.7), (64, 64, 3, 221, 3.0)])
+def test_power_spectrum_folded_lattice(hg, orc, ng, np_, folds, nb, sigma):
+    """The binned deposit of folded positions: a displaced lattice at every fold, a radix-3
+    length, particle masses 8 and 216 (weights over 31 bits), both accumulator widths of the
+    bins (up to 64 and above) and their extremes: counts equal and values as in
+    test_power_spectrum.  With an arena too small for the entries the fold takes the atomic
+    route, with the same bits."""
+    case(f"power folded ng={ng} np={np_} folds={folds} bins={nb}")
+    rng = np.random.default_rng(ng + nb)
+    with mk(hg, ng, np_, pk_bins=nb, pk_folds=folds) as m:
+        cell, off = lattice_split(rng, np_, ng, sigma)
+        m.set_particles_split(cell, off, np.zeros((m.N, 3), np.float32))
+        c, o = cell, off
+        for f in range(folds + 1):
+            k, pk, cnt = m.power_spectrum(f)
+            assert f == 0 or m.get_tunable("deposit_deferred") == 0, f
+            q = orc.cic_split(ng, c, o, float((np.float32(ng) / np.float32(np_)) ** 3))
+            ko, pko, cnto = orc.power_grid(ng, 2.0 * ng, folds, f, nb, q * 2.0 ** -24)
+            assert np.array_equal(cnt, cnto), f
+            np.testing.assert_array_equal(k, ko)
+            nz = cnto > 0
+            assert np.abs(pk[nz] / pko[nz] - 1).max(initial=0.0) < 1e-4, f  # low folds of many have no bins
+            if f:
+                m.set_tunable("deposit_arena", 1000)
+                assert np.array_equal(m.power_spectrum(f)[1], pk), f
+                assert m.get_tunable("deposit_deferred") == m.N // 4096
+                m.set_tunable("deposit_arena", -1)
+            c, o = orc.fold_split(ng, c, o)
+
+
 def test_power_spectrum_fp64(hg, orc):
     case("power fp64 ng=32")
     ng, nb = 32, 16
