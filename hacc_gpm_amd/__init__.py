@@ -335,8 +335,8 @@ class MemoryManager:
         self._c(lib().hgpm_set_particles(self.h, _ptr(pos), _ptr(vel)))
 
     def get_particles(self):
-        pos = np.zeros((self.N, 3), np.float32)
-        vel = np.zeros((self.N, 3), np.float32)
+        pos = np.empty((self.N, 3), np.float32)
+        vel = np.empty((self.N, 3), np.float32)
         self._c(lib().hgpm_get_particles(self.h, _ptr(pos), _ptr(vel)))
         return pos, vel
 
@@ -348,9 +348,9 @@ class MemoryManager:
         self._c(lib().hgpm_set_particles_split(self.h, _ptr(cell), _ptr(off), _ptr(vel)))
 
     def get_particles_split(self):
-        cell = np.zeros((self.N, 3), np.int32)
-        off = np.zeros((self.N, 3), np.float32)
-        vel = np.zeros((self.N, 3), np.float32)
+        cell = np.empty((self.N, 3), np.int32)
+        off = np.empty((self.N, 3), np.float32)
+        vel = np.empty((self.N, 3), np.float32)
         self._c(lib().hgpm_get_particles_split(self.h, _ptr(cell), _ptr(off), _ptr(vel)))
         return cell, off, vel
 
@@ -361,8 +361,8 @@ class MemoryManager:
         self._c(lib().hgpm_set_particles_f64(self.h, _ptr(pos), _ptr(vel)))
 
     def get_particles_f64(self):
-        pos = np.zeros((self.N, 3), np.float64)
-        vel = np.zeros((self.N, 3), np.float64)
+        pos = np.empty((self.N, 3), np.float64)
+        vel = np.empty((self.N, 3), np.float64)
         self._c(lib().hgpm_get_particles_f64(self.h, _ptr(pos), _ptr(vel)))
         return pos, vel
 
@@ -370,7 +370,7 @@ class MemoryManager:
         """The array serial::PyAnalysis hands to the analysis module
         (src/analysis/cuda/py_analysis.cu:3-26): (np^3, 7) float32 rows of
         (index, x, y, z, vx, vy, vz) in the reference's particle order."""
-        out = np.zeros((self.N, 7), np.float32)
+        out = np.empty((self.N, 7), np.float32)
         self._c(lib().hgpm_analysis_particles(self.h, _ptr(out)))
         return out
 
@@ -408,12 +408,12 @@ class MemoryManager:
         self._c(lib().hgpm_cic(self.h))
 
     def get_density(self):
-        r = np.zeros(self.G, np.int64)
+        r = np.empty(self.G, np.int64)
         self._c(lib().hgpm_get_density(self.h, _ptr(r)))
         return r.reshape(self.ng, self.ng, self.ng)
 
     def get_density_f64(self):
-        r = np.zeros(self.G, np.float64)
+        r = np.empty(self.G, np.float64)
         self._c(lib().hgpm_get_density_f64(self.h, _ptr(r)))
         return r.reshape(self.ng, self.ng, self.ng)
 
@@ -432,10 +432,10 @@ class MemoryManager:
 
     def get_force(self):
         if self.precision == FP64:
-            f = np.zeros((self.G, 3), np.float64)
+            f = np.empty((self.G, 3), np.float64)
             self._c(lib().hgpm_get_force_f64(self.h, _ptr(f)))
         else:
-            f = np.zeros((self.G, 3), np.float32)
+            f = np.empty((self.G, 3), np.float32)
             self._c(lib().hgpm_get_force(self.h, _ptr(f)))
         return f
 
@@ -591,8 +591,8 @@ class Ensemble:
 
     def get_particles(self, box):
         n = self.params[box].np ** 3
-        pos = np.zeros((n, 3), np.float32)
-        vel = np.zeros((n, 3), np.float32)
+        pos = np.empty((n, 3), np.float32)
+        vel = np.empty((n, 3), np.float32)
         self._c(lib().hgpm_ensemble_get_particles(self.h, int(box), _ptr(pos), _ptr(vel)))
         return pos, vel
 

@@ -40,7 +40,7 @@ def _jobs():
     # the alternative radix order of the 1024-point transforms
     jobs.append((os.path.join(CSRC, "k_fft.hip"), os.path.join(OBJ, "k_fft_1024_alt.o"),
                  ["-DHGPM_FFT_N=1024", "-DHGPM_FFT_PLAN_ALT"]))
-    for name in ["k_particles.hip", "k_power.hip", "k_ic.hip", "k_fp64.hip", "capi.cpp", "host.cpp", "ensemble.cpp"]:
+    for name in ["k_particles.hip", "k_power.hip", "k_ic.hip", "k_fp64.hip", "capi.cpp", "host.cpp", "hostcopy.cpp"]:
         src = os.path.join(CSRC, name)
         if os.path.exists(src):
             base = os.path.splitext(name)[0]
@@ -64,7 +64,7 @@ def build(verbose=False, jobs=None):
             if verbose and out.strip():
                 print(out)
     objs = [o for _, o, _ in todo]
-    _run([HIPCC, "-shared", "-fPIC", f"--offload-arch={ARCH}", "-o", LIB] + objs)
+    _run([HIPCC, "-shared", "-fPIC", "-pthread", f"--offload-arch={ARCH}", "-o", LIB] + objs)
     _run([HIPCC, "-std=c++17", "-O2", "-I" + os.path.join(ROOT, "include"),
           os.path.join(CSRC, "driver_pm.cpp"), "-o", BIN, "-L" + HERE, "-lhgpm",
           "-Wl,-rpath,$ORIGIN/.."])

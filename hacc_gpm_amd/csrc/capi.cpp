@@ -3,6 +3,7 @@
 // asynchronous on it and host calls synchronise only where data crosses to the host.
 #include "../../include/hgpm.h"
 #include "host.h"
+#include "hostcopy.h"
 #include "internal.h"
 
 #include <hip/hip_runtime.h>
@@ -124,6 +125,16 @@ template <typename T> int dalloc(hgpm_ctx* c, T** p, size_t bytes, const char* w
                                            " B) failed: " + hipGetErrorString(e));
     }
     c->bytes += bytes;
+    return HGPM_OK;
+}
+
+// Host arrays to and from the device on the context's stream; both wait for the data.
+int to_host(hgpm_ctx* c, std::initializer_list<HostSeg> s) {
+    HIPCHK(c, copy_to_host(s.begin(), (int)s.size(), c->st));
+    return HGPM_OK;
+}
+int to_device(hgpm_ctx* c, std::initializer_list<HostSeg> s, int* bad = nullptr) {
+    HIPCHK(c, copy_to_device(s.begin(), (int)s.size(), c->st, bad));
     return HGPM_OK;
 }
 
@@ -418,8 +429,7 @@ int pk_bin_spectrum(hgpm_ctx* c, int fold, double* k, double* pk, int64_t* count
     }
     // sums and counts are one allocation: one copy
     std::vector<double> sums(2 * (size_t)nb);
-    HIPCHK(c, hipMemcpyAsync(sums.data(), c->pk_sums, 2 * sizeof(double) * nb, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
+    if (int rc = to_host(c, {{sums.data(), c->pk_sums, 2 * sizeof(double) * nb}})) return rc;
     std::vector<long long> cnt(nb);
     memcpy(cnt.data(), sums.data() + nb, sizeof(long long) * nb);
     for (int i = 0; i < nb; i++) {
@@ -471,6 +481,7 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
         return fail(nullptr, HGPM_ERR_HIP, "no HIP device available");
     }
     hgpm_ctx* c = new hgpm_ctx();
+    host_copy_add_owner();
     c->p = *p;
     c->ng = p->ng;
     c->np = p->np;
@@ -619,6 +630,7 @@ int hgpm_destroy(hgpm_ctx* c) {
     for (auto& pe : c->pending) { (void)hipEventDestroy(pe.a); (void)hipEventDestroy(pe.b); }
     for (auto e : c->evpool) (void)hipEventDestroy(e);
     if (c->st) (void)hipStreamDestroy(c->st);
+    host_copy_release_owner();
     delete c;
     return HGPM_OK;
 }
@@ -641,21 +653,22 @@ int hgpm_set_particles(hgpm_ctx* c, const float* pos, const float* vel) {
     const size_t n3 = 3 * (size_t)c->N;
     c->boxes_valid = false;
     if (c->prec == HGPM_FP32) {
-        // the device conversion to fixed point takes rint(x 2^22) as a 64-bit integer:
-        // reject what it cannot hold, and NaN / Inf, before anything reaches the device
-        for (size_t i = 0; i < n3; i++)
-            if (!(std::fabs(pos[i]) < 1073741824.0f) || !std::isfinite(vel[i]))
-                return fail(c, HGPM_ERR_ARG, "non-finite particle (or |x| >= 2^30) at index " + std::to_string(i / 3));
-        float* tmp = nullptr;
-        int rc = dalloc(c, &tmp, sizeof(float) * 2 * n3, "staging");
+        // staged in the arena, which holds nothing between deposits (24 bytes per grid cell).
+        // The device conversion to fixed point takes rint(x 2^22) as a 64-bit integer:
+        // what it cannot hold, and NaN / Inf, is found on the way and rejected before it
+        float* tmp = (float*)c->arena;
+        int bad = -1;
+        int rc = to_device(c, {{(void*)pos, tmp, sizeof(float) * n3, 2}, {(void*)vel, tmp + n3, sizeof(float) * n3, 1}},
+                           &bad);
         if (rc) return rc;
-        c->bytes -= sizeof(float) * 2 * n3;
-        HIPCHK(c, hipMemcpyAsync(tmp, pos, sizeof(float) * n3, hipMemcpyHostToDevice, c->st));
-        HIPCHK(c, hipMemcpyAsync(tmp + n3, vel, sizeof(float) * n3, hipMemcpyHostToDevice, c->st));
+        if (bad >= 0)
+            for (size_t i = 0; i < n3; i++)
+                if (!(std::fabs(pos[i]) < 1073741824.0f) || !std::isfinite(vel[i]))
+                    return fail(c, HGPM_ERR_ARG,
+                                "non-finite particle (or |x| >= 2^30) at index " + std::to_string(i / 3));
         launch_split_from_float3(tmp, tmp + n3, c->pos, c->vel, c->N, c->np, c->ng, c->st);
         LAUNCHCHK(c);
         HIPCHK(c, hipStreamSynchronize(c->st));
-        (void)hipFree(tmp);
     } else {
         std::vector<double> p(n3), v(n3);
         for (size_t i = 0; i < n3; i++) {
@@ -667,9 +680,8 @@ int hgpm_set_particles(hgpm_ctx* c, const float* pos, const float* vel) {
             p[i] = x;
             v[i] = vel[i];
         }
-        HIPCHK(c, hipMemcpyAsync(c->pos64, p.data(), sizeof(double) * n3, hipMemcpyHostToDevice, c->st));
-        HIPCHK(c, hipMemcpyAsync(c->vel64, v.data(), sizeof(double) * n3, hipMemcpyHostToDevice, c->st));
-        HIPCHK(c, hipStreamSynchronize(c->st));
+        if (int rc = to_device(c, {{p.data(), c->pos64, sizeof(double) * n3}, {v.data(), c->vel64, sizeof(double) * n3}}))
+            return rc;
     }
     c->have_particles = true;
     c->have_density = c->have_force = false;
@@ -682,21 +694,14 @@ int hgpm_get_particles(hgpm_ctx* c, float* pos, float* vel) {
     if (rc) return rc;
     const size_t n3 = 3 * (size_t)c->N;
     if (c->prec == HGPM_FP32) {
-        float* tmp = nullptr;
-        rc = dalloc(c, &tmp, sizeof(float) * 2 * n3, "staging");
-        if (rc) return rc;
-        c->bytes -= sizeof(float) * 2 * n3;
+        float* tmp = (float*)c->arena; // as in hgpm_set_particles
         launch_split_to_float3(c->pos, c->vel, tmp, tmp + n3, c->N, c->np, c->st);
         LAUNCHCHK(c);
-        HIPCHK(c, hipMemcpyAsync(pos, tmp, sizeof(float) * n3, hipMemcpyDeviceToHost, c->st));
-        HIPCHK(c, hipMemcpyAsync(vel, tmp + n3, sizeof(float) * n3, hipMemcpyDeviceToHost, c->st));
-        HIPCHK(c, hipStreamSynchronize(c->st));
-        (void)hipFree(tmp);
+        return to_host(c, {{pos, tmp, sizeof(float) * n3}, {vel, tmp + n3, sizeof(float) * n3}});
     } else {
         std::vector<double> p(n3), v(n3);
-        HIPCHK(c, hipMemcpyAsync(p.data(), c->pos64, sizeof(double) * n3, hipMemcpyDeviceToHost, c->st));
-        HIPCHK(c, hipMemcpyAsync(v.data(), c->vel64, sizeof(double) * n3, hipMemcpyDeviceToHost, c->st));
-        HIPCHK(c, hipStreamSynchronize(c->st));
+        if ((rc = to_host(c, {{p.data(), c->pos64, sizeof(double) * n3}, {v.data(), c->vel64, sizeof(double) * n3}})))
+            return rc;
         for (size_t i = 0; i < n3; i++) { pos[i] = (float)p[i]; vel[i] = (float)v[i]; }
     }
     return HGPM_OK;
@@ -749,20 +754,12 @@ int hgpm_set_particles_split(hgpm_ctx* c, const int32_t* cell, const float* off,
         }
         h[i] = PosPackH{X[0], X[1], X[2]};
     }
-    PosPackH* sp = nullptr;
-    float* sv = nullptr;
-    int rc = dalloc(c, &sp, sizeof(PosPackH) * n, "staging");
-    if (rc) return rc;
-    rc = dalloc(c, &sv, sizeof(float) * 3 * n, "staging");
-    if (rc) { (void)hipFree(sp); return rc; }
-    c->bytes -= sizeof(PosPackH) * n + sizeof(float) * 3 * n;
-    HIPCHK(c, hipMemcpyAsync(sp, h.data(), sizeof(PosPackH) * n, hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(sv, vel, sizeof(float) * 3 * n, hipMemcpyHostToDevice, c->st));
+    PosPackH* sp = (PosPackH*)c->arena; // as in hgpm_set_particles
+    float* sv = (float*)(sp + n);
+    if (int rc = to_device(c, {{h.data(), sp, sizeof(PosPackH) * n}, {(void*)vel, sv, sizeof(float) * 3 * n}})) return rc;
     launch_to_internal(sp, sv, c->pos, c->vel, c->N, c->np, c->st);
     LAUNCHCHK(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
-    (void)hipFree(sp);
-    (void)hipFree(sv);
     c->have_particles = true;
     c->have_density = c->have_force = false;
     return HGPM_OK;
@@ -775,20 +772,11 @@ int hgpm_get_particles_split(hgpm_ctx* c, int32_t* cell, float* off, float* vel)
     if (rc) return rc;
     const size_t n = (size_t)c->N;
     std::vector<PosPackH> h(n);
-    PosPackH* sp = nullptr;
-    float* sv = nullptr;
-    rc = dalloc(c, &sp, sizeof(PosPackH) * n, "staging");
-    if (rc) return rc;
-    rc = dalloc(c, &sv, sizeof(float) * 3 * n, "staging");
-    if (rc) { (void)hipFree(sp); return rc; }
-    c->bytes -= sizeof(PosPackH) * n + sizeof(float) * 3 * n;
+    PosPackH* sp = (PosPackH*)c->arena; // as in hgpm_set_particles
+    float* sv = (float*)(sp + n);
     launch_to_reference(c->pos, c->vel, sp, sv, c->N, c->np, c->st);
     LAUNCHCHK(c);
-    HIPCHK(c, hipMemcpyAsync(h.data(), sp, sizeof(PosPackH) * n, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipMemcpyAsync(vel, sv, sizeof(float) * 3 * n, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    (void)hipFree(sp);
-    (void)hipFree(sv);
+    if ((rc = to_host(c, {{h.data(), sp, sizeof(PosPackH) * n}, {vel, sv, sizeof(float) * 3 * n}}))) return rc;
     for (size_t i = 0; i < n; i++) {
         constexpr unsigned M = (1u << HGPM_FRAC_BITS_H) - 1u;
         const unsigned X[3] = {h[i].x, h[i].y, h[i].z};
@@ -807,9 +795,8 @@ int hgpm_set_particles_f64(hgpm_ctx* c, const double* pos, const double* vel) {
     for (size_t i = 0; i < n3; i++)
         if (!(pos[i] >= 0.0 && pos[i] < (double)c->ng) || !std::isfinite(vel[i]))
             return fail(c, HGPM_ERR_ARG, "FP64 particle out of [0, ng) or non-finite at index " + std::to_string(i / 3));
-    HIPCHK(c, hipMemcpyAsync(c->pos64, pos, sizeof(double) * n3, hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->vel64, vel, sizeof(double) * n3, hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
+    if (int rc = to_device(c, {{(void*)pos, c->pos64, sizeof(double) * n3}, {(void*)vel, c->vel64, sizeof(double) * n3}}))
+        return rc;
     c->have_particles = true;
     c->have_density = c->have_force = false;
     return HGPM_OK;
@@ -821,10 +808,7 @@ int hgpm_get_particles_f64(hgpm_ctx* c, double* pos, double* vel) {
     int rc = need_particles(c);
     if (rc) return rc;
     const size_t n3 = 3 * (size_t)c->N;
-    HIPCHK(c, hipMemcpyAsync(pos, c->pos64, sizeof(double) * n3, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipMemcpyAsync(vel, c->vel64, sizeof(double) * n3, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    return HGPM_OK;
+    return to_host(c, {{pos, c->pos64, sizeof(double) * n3}, {vel, c->vel64, sizeof(double) * n3}});
 }
 
 // ------------------------------------------- particle state between contexts ----
@@ -994,14 +978,21 @@ int hgpm_generate_ic(hgpm_ctx* c, const double* ipk, int ipk_bins, double ipk_k_
                      double delta, double dot_delta, double fscal, double deltaT) {
     int rc = ic_check(c, ipk, ipk_bins, ipk_k_delta, ipk_k_max, "hgpm_generate_ic");
     if (rc) return rc;
-    double* d_ipk = nullptr;
-    if ((rc = dalloc(c, &d_ipk, sizeof(double) * ipk_bins, "ipk"))) return rc;
-    c->bytes -= sizeof(double) * ipk_bins;
-    hipError_t e = hipMemcpyAsync(d_ipk, ipk, sizeof(double) * ipk_bins, hipMemcpyHostToDevice, c->st);
-    if (e == hipSuccess) rc = generate_ic_from(c, d_ipk, ipk_bins, ipk_k_delta, delta, dot_delta, fscal, deltaT);
-    else rc = fail(c, HGPM_ERR_HIP, std::string("hgpm_generate_ic: ") + hipGetErrorString(e));
-    (void)hipStreamSynchronize(c->st);
-    (void)hipFree(d_ipk);
+    // the table goes to the arena where the first n3 * 8 bytes hold it (free until the y
+    // pass of the displacements), else to a buffer of its own
+    const size_t bytes = sizeof(double) * ipk_bins, n3 = (size_t)c->np * c->np * c->np;
+    const bool own = c->prec != HGPM_FP32 || bytes > 8 * n3;
+    double* d_ipk = (double*)c->arena;
+    if (own) {
+        if ((rc = dalloc(c, &d_ipk, bytes, "ipk"))) return rc;
+        c->bytes -= bytes;
+    }
+    rc = to_device(c, {{(void*)ipk, d_ipk, bytes}});
+    if (!rc) rc = generate_ic_from(c, d_ipk, ipk_bins, ipk_k_delta, delta, dot_delta, fscal, deltaT);
+    if (own) {
+        (void)hipStreamSynchronize(c->st);
+        (void)hipFree(d_ipk);
+    }
     return rc;
 }
 
@@ -1059,9 +1050,7 @@ int hgpm_get_density(hgpm_ctx* c, int64_t* rho) {
     if (!c || !rho) return fail(c, HGPM_ERR_ARG, "hgpm_get_density: null argument");
     if (c->prec != HGPM_FP32) return fail(c, HGPM_ERR_UNSUPPORTED, "int64 density needs an FP32 context");
     if (!c->have_density) return fail(c, HGPM_ERR_STATE, "no density: call hgpm_cic first");
-    HIPCHK(c, hipMemcpyAsync(rho, c->B, sizeof(int64_t) * c->G, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    return HGPM_OK;
+    return to_host(c, {{rho, c->B, sizeof(int64_t) * c->G}});
 }
 
 int hgpm_get_density_f64(hgpm_ctx* c, double* rho) {
@@ -1069,15 +1058,13 @@ int hgpm_get_density_f64(hgpm_ctx* c, double* rho) {
     if (!c->have_density) return fail(c, HGPM_ERR_STATE, "no density: call hgpm_cic first");
     if (c->prec == HGPM_FP32) {
         std::vector<int64_t> q(c->G);
-        HIPCHK(c, hipMemcpyAsync(q.data(), c->B, sizeof(int64_t) * c->G, hipMemcpyDeviceToHost, c->st));
-        HIPCHK(c, hipStreamSynchronize(c->st));
+        if (int rc = to_host(c, {{q.data(), c->B, sizeof(int64_t) * c->G}})) return rc;
         for (int64_t i = 0; i < c->G; i++) rho[i] = (double)q[i] * (1.0 / 16777216.0);
     } else {
         double* tmp = (double*)c->grad64; // scratch
         launch_f64_density_to_real(c->grid64, tmp, c->G, c->st);
         LAUNCHCHK(c);
-        HIPCHK(c, hipMemcpyAsync(rho, tmp, sizeof(double) * c->G, hipMemcpyDeviceToHost, c->st));
-        HIPCHK(c, hipStreamSynchronize(c->st));
+        return to_host(c, {{rho, tmp, sizeof(double) * c->G}});
     }
     return HGPM_OK;
 }
@@ -1088,9 +1075,7 @@ int hgpm_set_density(hgpm_ctx* c, const int64_t* rho) {
     long long tot = 0;
     for (int64_t i = 0; i < c->G; i++) tot += rho[i];
     unsigned long long ut = (unsigned long long)tot;
-    HIPCHK(c, hipMemcpyAsync(c->B, rho, sizeof(int64_t) * c->G, hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipMemcpyAsync(c->total, &ut, sizeof(ut), hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
+    if (int rc = to_device(c, {{(void*)rho, c->B, sizeof(int64_t) * c->G}, {&ut, c->total, sizeof(ut)}})) return rc;
     c->have_density = true;
     c->dens_f32 = false;
     c->have_force = false;
@@ -1102,8 +1087,7 @@ int hgpm_set_density_f64(hgpm_ctx* c, const double* rho) {
     if (c->prec != HGPM_FP64) return fail(c, HGPM_ERR_UNSUPPORTED, "FP64 density needs an FP64 context");
     std::vector<double> g(2 * (size_t)c->G, 0.0);
     for (int64_t i = 0; i < c->G; i++) g[2 * i] = rho[i];
-    HIPCHK(c, hipMemcpyAsync(c->grid64, g.data(), sizeof(double) * 2 * c->G, hipMemcpyHostToDevice, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
+    if (int rc = to_device(c, {{g.data(), c->grid64, sizeof(double) * 2 * c->G}})) return rc;
     c->have_density = true;
     c->have_force = false;
     return HGPM_OK;
@@ -1123,16 +1107,10 @@ int hgpm_get_force(hgpm_ctx* c, float* f) {
     if (!c || !f) return fail(c, HGPM_ERR_ARG, "hgpm_get_force: null argument");
     if (c->prec != HGPM_FP32) return fail(c, HGPM_ERR_UNSUPPORTED, "use hgpm_get_force_f64 on an FP64 context");
     if (!c->have_force) return fail(c, HGPM_ERR_STATE, "no force: call hgpm_solve_gradient first");
-    float* tmp = nullptr;
-    int rc = dalloc(c, &tmp, sizeof(float) * 3 * c->G, "staging");
-    if (rc) return rc;
-    c->bytes -= sizeof(float) * 3 * c->G;
+    float* tmp = (float*)c->arena; // 24 bytes per grid cell, free between deposits
     launch_force_from_psi(c->psi, tmp, c->ng, c->st);
     LAUNCHCHK(c);
-    HIPCHK(c, hipMemcpyAsync(f, tmp, sizeof(float) * 3 * c->G, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
-    (void)hipFree(tmp);
-    return HGPM_OK;
+    return to_host(c, {{f, tmp, sizeof(float) * 3 * c->G}});
 }
 
 int hgpm_get_force_f64(hgpm_ctx* c, double* f) {
@@ -1151,10 +1129,9 @@ int hgpm_get_force_f64(hgpm_ctx* c, double* f) {
     c->bytes -= sizeof(double) * 3 * c->G;
     launch_f64_grad_to_force(c->grad64, tmp, c->G, c->st);
     LAUNCHCHK(c);
-    HIPCHK(c, hipMemcpyAsync(f, tmp, sizeof(double) * 3 * c->G, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
+    rc = to_host(c, {{f, tmp, sizeof(double) * 3 * c->G}});
     (void)hipFree(tmp);
-    return HGPM_OK;
+    return rc;
 }
 
 int hgpm_update_velocities(hgpm_ctx* c, double deltaT, double fscal) {
@@ -1246,11 +1223,8 @@ int hgpm_fft_host(hgpm_ctx* c, void* grid, int direction) {
     if (!c || !grid || (direction != -1 && direction != 1)) return fail(c, HGPM_ERR_ARG, "hgpm_fft_host: bad arguments");
     size_t bytes = (c->prec == HGPM_FP32 ? sizeof(float2) : sizeof(double2)) * (size_t)c->G;
     void* d = c->prec == HGPM_FP32 ? (void*)c->A : (void*)c->grid64;
-    HIPCHK(c, hipMemcpyAsync(d, grid, bytes, hipMemcpyHostToDevice, c->st));
-    int rc = hgpm_fft_device(c, d, direction);
-    if (rc) return rc;
-    HIPCHK(c, hipMemcpyAsync(grid, d, bytes, hipMemcpyDeviceToHost, c->st));
-    HIPCHK(c, hipStreamSynchronize(c->st));
+    int rc = to_device(c, {{grid, d, bytes}});
+    if (rc || (rc = hgpm_fft_device(c, d, direction)) || (rc = to_host(c, {{grid, d, bytes}}))) return rc;
     c->have_density = c->have_force = false;
     return HGPM_OK;
 }

@@ -972,6 +972,46 @@ def test_driver_analysis_hook(hg, tmp_path):
     assert np.array_equal(ana[:, 4:7], snap[3 * n:].reshape(n, 3))
 
 
+# ---------------------------------------------------------- host transfers ----
+@pytest.mark.parametrize("n", [32, 64, 128])
+def test_host_transfers(hg, n):
+    """Particles through the pinned ring: one slot, a few and several rounds of it (1 MB
+    slots, 8 of them), bit for bit, from two host threads with a context each; a value out
+    of range anywhere is refused with its index and leaves the state as it was."""
+    import threading
+    case(f"host transfers {n}^3")
+    rng = np.random.default_rng(n)
+    got = {}
+
+    def trip(who, seed):
+        r = np.random.default_rng(seed)
+        # multiples of 2^-12: exact in the fixed-point positions and in float32
+        pos = (r.integers(0, n << 12, (n ** 3, 3)) * 2.0 ** -12).astype(np.float32)
+        vel = r.normal(0, 1, (n ** 3, 3)).astype(np.float32)
+        with mk(hg, n) as m:
+            for _ in range(3):
+                m.set_particles(pos, vel)
+                p, v = m.get_particles()
+                got[who] = got.get(who, True) and np.array_equal(p, pos) and np.array_equal(v, vel)
+            for where, bad in ((0, np.nan), (3 * n ** 3 - 1, 2.0 ** 30), (int(rng.integers(3 * n ** 3)), -np.inf)):
+                for a in (0, 1):
+                    if a and abs(bad) == 2.0 ** 30:
+                        continue
+                    q = [pos.copy(), vel.copy()]
+                    q[a].reshape(-1)[where] = bad
+                    with pytest.raises(hg.HgpmError, match=f"index {where // 3}"):
+                        m.set_particles(*q)
+            p, v = m.get_particles()
+            got[who] = got[who] and np.array_equal(p, pos) and np.array_equal(v, vel)
+
+    th = [threading.Thread(target=trip, args=(i, 10 * n + i)) for i in range(2)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert got == {0: True, 1: True}
+
+
 # -------------------------------------------------------------- ensemble ----
 def _ic_inputs(hg, p):
     import tempfile
