@@ -53,9 +53,11 @@ struct hgpm_ctx {
     float2* A = nullptr;             // spectrum (8 B per cell) / half spectra of the solve
     float2* B = nullptr;             // int64 density (8 B per cell)
     float* psi = nullptr;            // half the potential of the solve (4 B per cell); F = its differences
-    unsigned long long* ctl = nullptr;    // deposit control words (shared by the boxes)
-    unsigned long long* totals = nullptr; // deposited mass per box
-    unsigned long long* total = nullptr;  // = totals (of the viewed box, see BoxView)
+    unsigned long long* ctl = nullptr; // two sets of deposit control words, used in turn
+    int set_words = 0;                 // words of a set: control words, mass partial sums per box
+    int set_next = 0;                  // the set of the next deposit; the other is the last one's
+    unsigned long long* last_ctl() const { return ctl + (size_t)(set_next ^ 1) * set_words; }
+    unsigned long long* last_mass() const { return last_ctl() + HGPM_DEP_CTL + 1; }
     // deposit arena route (k_particles.hip): window arena, per-owner-block chunk slots
     unsigned* arena = nullptr; // 32-bit window cells
     unsigned long long arena_alloc = 0, arena_cap = 0; // cells allocated / usable
@@ -65,7 +67,6 @@ struct hgpm_ctx {
     unsigned* deferred = nullptr;
     unsigned* wide = nullptr;
     unsigned short* wide_slots = nullptr;
-    unsigned long long* tile_total = nullptr;
     void* boxes = nullptr;   // half-tile cell boxes of the last windows pass
     bool boxes_valid = false; // ... and the positions have not changed since
     int nslots = HGPM_DEP_SLOTS;
@@ -281,11 +282,11 @@ DepositBuffers dep_buffers(hgpm_ctx* c, int fold) {
     b.deferred = c->deferred;
     b.wide = c->wide;
     b.wide_slots = c->wide_slots;
-    b.ctl = c->ctl;
-    b.tile_total = c->tile_total;
+    b.ctl = c->ctl + (size_t)c->set_next * c->set_words;
+    b.next = c->ctl + (size_t)(c->set_next ^ 1) * c->set_words;
+    b.set_words = c->set_words;
     b.boxes = c->boxes;
     b.nbox = c->nbox;
-    b.totals = c->total;
     b.ppt = fold ? 8 : c->dep_ppt;
     b.fold = fold;
     // about 256 tiles per sub-arena, at most HGPM_DEP_NSUB sub-arenas
@@ -302,7 +303,6 @@ DepositBuffers dep_buffers(hgpm_ctx* c, int fold) {
 int f32_deposit(hgpm_ctx* c, bool fused = false, int fold = 0) {
     const DepositBuffers b = dep_buffers(c, fold);
     Timed t(c, "deposit");
-    launch_deposit_begin(c->ctl, (unsigned long long)(c->ng / 16) * (c->ng / 16) * (c->ng / 16) * c->nbox, c->st);
     if (fold) {
         Timed t1(c, "deposit_binned");
         launch_deposit_binned(c->pos, c->N, c->ng, ref_mass(c), (long long*)c->B, fused ? c->psi : nullptr, b, c->st);
@@ -313,10 +313,6 @@ int f32_deposit(hgpm_ctx* c, bool fused = false, int fold = 0) {
             launch_deposit_windows(c->pos, c->N * c->nbox, c->ng, ref_mass(c), b, c->st);
             c->boxes_valid = true;
         }
-        if (fused) {
-            Timed t2(c, "deposit_totals");
-            launch_deposit_totals(c->N * c->nbox, b, c->st);
-        }
         Timed t2(c, "deposit_owner");
         launch_deposit_owner(c->ng, (long long*)c->B, fused ? c->psi : nullptr, b, c->st);
     }
@@ -324,6 +320,7 @@ int f32_deposit(hgpm_ctx* c, bool fused = false, int fold = 0) {
         Timed t3(c, "deposit_deferred");
         launch_deposit_deferred(c->pos, c->N * c->nbox, c->ng, ref_mass(c), (long long*)c->B, b, c->st);
     }
+    c->set_next ^= 1;
     c->dens_f32 = fused;
     LAUNCHCHK(c);
     return HGPM_OK;
@@ -337,7 +334,7 @@ int f32_solve(hgpm_ctx* c) {
     const FftOps* f = c->fft;
     {
         Timed t(c, "fft_fwd_z_r2c");
-        f->fwd_z_r2c((const long long*)c->B, c->dens_f32 ? c->psi : nullptr, c->ctl, c->total, c->A, c->twf,
+        f->fwd_z_r2c((const long long*)c->B, c->dens_f32 ? c->psi : nullptr, c->last_ctl(), c->last_mass(), c->A, c->twf,
                      c->nbox, c->st);
     }
     {
@@ -524,10 +521,10 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
             (rc = dalloc(c, &c->A, sizeof(float2) * GB, "grid A")) ||
             (rc = dalloc(c, &c->B, sizeof(float2) * GB, "grid B")) ||
             (rc = dalloc(c, &c->psi, sizeof(float) * GB, "potential")) ||
-            (rc = dalloc(c, &c->ctl, (HGPM_DEP_CTL + 1) * sizeof(unsigned long long), "deposit control")) ||
-            (rc = dalloc(c, &c->totals, sizeof(unsigned long long) * nbox, "deposit totals")))
+            (rc = dalloc(c, &c->ctl,
+                         2 * sizeof(unsigned long long) * (c->set_words = HGPM_DEP_CTL + 1 + HGPM_DEP_MASS * nbox),
+                         "deposit control")))
             return bail(rc);
-        c->total = c->totals;
         {
             // window arena: 6 cells (32-bit) per grid cell holds every tile window of the
             // runs measured here through z = 0 (the windows' total grows from ~1.4 G to
@@ -543,13 +540,12 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
                 (rc = dalloc(c, &c->wide, sizeof(unsigned) * ntiles, "deposit 64-bit list")) ||
                 (rc = dalloc(c, &c->wide_slots, sizeof(unsigned short) * HGPM_DEP_WKEEP * ntiles,
                              "deposit 64-bit slots")) ||
-                (rc = dalloc(c, &c->tile_total, sizeof(unsigned long long) * ntiles, "deposit tile totals")) ||
                 (rc = dalloc(c, (char**)&c->boxes, 32 * ntiles, "gather boxes")))
                 return bail(rc);
             c->dwide = (unsigned char*)(c->dcount + nblk);
             // particles start at cell 0, offset 0 (valid if never set; a step refuses them)
             if (hipMemset(c->dcount, 0, (sizeof(unsigned) + 1) * nblk) != hipSuccess ||
-                hipMemset(c->ctl, 0, (HGPM_DEP_CTL + 1) * sizeof(unsigned long long)) != hipSuccess ||
+                hipMemset(c->ctl, 0, 2 * sizeof(unsigned long long) * c->set_words) != hipSuccess ||
                 hipMemset(c->pos, 0, sizeof(PosPackH) * NB) != hipSuccess ||
                 hipMemset(c->vel, 0, sizeof(float) * 3 * NB) != hipSuccess) {
                 c->err = "hipMemset failed";
@@ -619,7 +615,7 @@ int hgpm_create(const hgpm_params* p, hgpm_ctx** out) { return ctx_create(p, 1, 
 int hgpm_destroy(hgpm_ctx* c) {
     if (!c) return HGPM_OK;
     if (c->st) (void)hipStreamSynchronize(c->st);
-    void* ptrs[] = {c->pos, c->vel, c->A, c->B, c->psi, c->ctl, c->totals, c->arena, c->dslots, c->dcount, c->deferred, c->wide, c->wide_slots, c->tile_total, c->boxes, c->twf, c->twr, c->hs,
+    void* ptrs[] = {c->pos, c->vel, c->A, c->B, c->psi, c->ctl, c->arena, c->dslots, c->dcount, c->deferred, c->wide, c->wide_slots, c->boxes, c->twf, c->twr, c->hs,
                     c->pos64, c->vel64, c->grid64, c->grad64, c->tw64, c->pk_partial, c->pk_sums,
                     c->pk_win, c->flag};
     for (void* q : ptrs)
@@ -1074,8 +1070,8 @@ int hgpm_set_density(hgpm_ctx* c, const int64_t* rho) {
     if (c->prec != HGPM_FP32) return fail(c, HGPM_ERR_UNSUPPORTED, "int64 density needs an FP32 context");
     long long tot = 0;
     for (int64_t i = 0; i < c->G; i++) tot += rho[i];
-    unsigned long long ut = (unsigned long long)tot;
-    if (int rc = to_device(c, {{(void*)rho, c->B, sizeof(int64_t) * c->G}, {&ut, c->total, sizeof(ut)}})) return rc;
+    unsigned long long ut[HGPM_DEP_MASS] = {(unsigned long long)tot};
+    if (int rc = to_device(c, {{(void*)rho, c->B, sizeof(int64_t) * c->G}, {ut, c->last_mass(), sizeof(ut)}})) return rc;
     c->have_density = true;
     c->dens_f32 = false;
     c->have_force = false;
@@ -1239,7 +1235,7 @@ int hgpm_power_spectrum_grid(hgpm_ctx* c, int fold, double* k, double* pk, int64
         {
             // half spectra, as the solve's: the density is real
             Timed t(c, "pk_fwd_z_density");
-            c->fft->fwd_z_r2c((const long long*)c->B, c->dens_f32 ? c->psi : nullptr, c->ctl, c->total, c->A, c->twf, 1,
+            c->fft->fwd_z_r2c((const long long*)c->B, c->dens_f32 ? c->psi : nullptr, c->last_ctl(), c->last_mass(), c->A, c->twf, 1,
                               c->st);
         }
         {
@@ -1410,7 +1406,7 @@ int hgpm_get_tunable(hgpm_ctx* c, const char* key, int* value) {
         // of the 64-bit pass (an upper bound of the window volume, not the volume)
         if (c->prec != HGPM_FP32) { *value = 0; return HGPM_OK; }
         std::vector<unsigned long long> v(HGPM_DEP_CTL);
-        HIPCHK(c, hipMemcpyAsync(v.data(), c->ctl, sizeof(unsigned long long) * HGPM_DEP_CTL, hipMemcpyDeviceToHost,
+        HIPCHK(c, hipMemcpyAsync(v.data(), c->last_ctl(), sizeof(unsigned long long) * HGPM_DEP_CTL, hipMemcpyDeviceToHost,
                                  c->st));
         HIPCHK(c, hipStreamSynchronize(c->st));
         unsigned long long t = 0;
@@ -1426,7 +1422,7 @@ int hgpm_get_tunable(hgpm_ctx* c, const char* key, int* value) {
         if (!strcmp(key, dkeys[i])) {
             if (c->prec != HGPM_FP32) { *value = 0; return HGPM_OK; }
             unsigned long long v[4];
-            HIPCHK(c, hipMemcpyAsync(v, c->ctl, sizeof(v), hipMemcpyDeviceToHost, c->st));
+            HIPCHK(c, hipMemcpyAsync(v, c->last_ctl(), sizeof(v), hipMemcpyDeviceToHost, c->st));
             HIPCHK(c, hipStreamSynchronize(c->st));
             *value = (int)v[i];
             return HGPM_OK;
@@ -1667,7 +1663,8 @@ size_t batch_bytes(const hgpm_params& p, int nstore, int nwave) {
     b += (2 * sizeof(float2) + sizeof(float)) * G * nwave;              // A, B, psi
     b += 6 * sizeof(unsigned) * G * nwave;                              // arena
     b += (16 * HGPM_DEP_SLOTS + sizeof(unsigned) + 1) * nblk;           // slots, counts, marks
-    b += (2 * sizeof(unsigned) + sizeof(unsigned long long) + 32 + 2 * HGPM_DEP_WKEEP) * ntiles; // tile buffers
+    b += (2 * sizeof(unsigned) + 32 + 2 * HGPM_DEP_WKEEP) * ntiles;    // tile buffers
+    b += 2 * sizeof(unsigned long long) * HGPM_DEP_MASS * nwave;        // mass partial sums
     b += 64ull << 20;                                                   // tables, P(k), slack
     return b;
 }
@@ -1909,7 +1906,8 @@ int hgpm_ensemble_run(hgpm_ensemble* e, int nsteps, const hgpm_step_coeffs* coef
         if (hipEventRecord(e->ev[g], e->batch[g]->st) != hipSuccess || hipStreamWaitEvent(s0, e->ev[g], 0) != hipSuccess)
             return efail(e, HGPM_ERR_HIP, "hgpm_ensemble_run: stream ordering failed");
     }
-    std::vector<int> timing(ng);
+    std::vector<int> timing(ng), set(ng);
+    for (size_t g = 0; g < ng; g++) set[g] = e->batch[g]->set_next;
     for (size_t g = 0; g < ng; g++) { timing[g] = e->batch[g]->timing; e->batch[g]->timing = false; }
     std::string what;
     int rc = HGPM_OK;
@@ -1940,16 +1938,22 @@ int hgpm_ensemble_run(hgpm_ensemble* e, int nsteps, const hgpm_step_coeffs* coef
         rc = HGPM_ERR_HIP;
     }
     if (graph) (void)hipGraphDestroy(graph);
+    // the captured deposits did not run: the control sets stand as before
+    auto rewind = [&] { for (size_t g = 0; g < ng; g++) e->batch[g]->set_next = set[g]; };
     if (rc) {
         if (exec) (void)hipGraphExecDestroy(exec);
+        rewind();
         return efail(e, rc, "hgpm_ensemble_run: " + what);
     }
     hipEvent_t done;
     if (hipEventCreateWithFlags(&done, hipEventDisableTiming) != hipSuccess) {
+        rewind();
         (void)hipGraphExecDestroy(exec);
         return efail(e, HGPM_ERR_HIP, "hgpm_ensemble_run: hipEventCreate failed");
     }
-    if (hipGraphLaunch(exec, s0) != hipSuccess || hipEventRecord(done, s0) != hipSuccess) {
+    const hipError_t launched = hipGraphLaunch(exec, s0);
+    if (launched != hipSuccess) rewind();
+    if (launched != hipSuccess || hipEventRecord(done, s0) != hipSuccess) {
         (void)hipStreamSynchronize(s0);
         (void)hipGraphExecDestroy(exec);
         (void)hipEventDestroy(done);

@@ -28,14 +28,15 @@ struct FftOps {
     void (*pass_f32)(float2* d, int axis, int dir, const float2* tw, int variant, hipStream_t s);
     void (*pass_f64)(double2* d, int axis, int dir, const double2* tw, hipStream_t s);
     // half-spectrum solve (rows of hz = n/2 + 16 complex, k_z = 0..n/2) on nbox grids of
-    // the same shape stored back to back; totals[b] is box b's deposited mass
+    // the same shape stored back to back; mass: HGPM_DEP_MASS partial sums of the deposited
+    // mass per box
     int hz;
     size_t plane; // elements from one x plane of half spectra to the next
     void (*pass_half)(float2* d, int axis, int dir, const float2* tw, int variant, int nbox, hipStream_t s);
     // rhof non-null: the density is the FP32 grid rhof when ctl[1] == 0 (no deferred
     // tiles, see launch_deposit_owner), else the int64 grid rho
     void (*fwd_z_r2c)(const long long* rho, const float* rhof, const unsigned long long* ctl,
-                      const unsigned long long* totals, float2* out, const float2* tw, int nbox, hipStream_t s);
+                      const unsigned long long* mass, float2* out, const float2* tw, int nbox, hipStream_t s);
     // forward x, psi^ = g rho^, inverse x, in place (the potential's half spectrum)
     void (*x_psi)(float2* h1, const float2* twf, const float2* twr, const float* hs, int variant, int nbox,
                   hipStream_t s);
@@ -90,21 +91,22 @@ void launch_drift(PosPackH* pos, const float* vel, int64_t np3, int ng, float pf
 //              64-bit chunk, or a cell sum of 2^32 units or more), bit 0 = summed by
 //              the 64-bit pass before (later deposits send it there at once);
 //   deferred : one entry per tile;
-//   ctl      : HGPM_DEP_CTL + 1 words.  [0 .. HGPM_DEP_CTL) are cleared at the start of
-//              each deposit (launch_deposit_begin): [0] blocks that went to the 64-bit
-//              owner pass (handed over, or all of them that needed it in the all-64-bit
-//              route), [1] deferred tiles, of
+//   ctl      : a set of control words, HGPM_DEP_CTL + 1 words followed by HGPM_DEP_MASS per
+//              box.  Two sets are used in turn (zero at creation): a deposit finds its own
+//              cleared and leaves the other (next, set_words words) cleared at its end.
+//              [0] blocks that went to the 64-bit owner pass (handed over, or all of them
+//              that needed it in the all-64-bit route), [1] deferred tiles, of
 //              them [3] for a full slot list or sub-arena (the others had too many
 //              chunks); [2] tiles stored with 64-bit cells; [4 + s] cells reserved in
-//              sub-arena s; [HGPM_DEP_CTL], kept across deposits (zero at creation):
-//              the owner pass's route, 1 = every block in 64-bit sums;
-//   tile_total: deposited mass per tile.
+//              sub-arena s; [HGPM_DEP_CTL]: the owner pass's route, 1 = every block in
+//              64-bit sums; then the partial sums of the deposited mass.
 // A deposit tile is DEP_NT * ppt consecutive particles: a whole 16^3 Lagrangian tile
 // (ppt 8) or half of one (ppt 4); per-tile buffers are sized for half tiles.
 #define HGPM_DEP_SLOTS 64
 #define HGPM_DEP_WKEEP 32
 #define HGPM_DEP_NSUB 64
 #define HGPM_DEP_CTL (4 + HGPM_DEP_NSUB)
+#define HGPM_DEP_MASS 64
 struct DepositBuffers {
     unsigned* arena; // 32-bit window cells
     unsigned long long cap;
@@ -116,11 +118,11 @@ struct DepositBuffers {
     unsigned* wide; // tiles stored again with 64-bit cells: one entry per tile
     unsigned short* wide_slots; // HGPM_DEP_WKEEP slot indices per entry of wide
     unsigned long long* ctl;
-    unsigned long long* tile_total;
+    unsigned long long* next;
+    int set_words;
     int nsub; // sub-arenas in use, 1..HGPM_DEP_NSUB
     void* boxes; // 32 B per half tile: the cell box the gather stages (written by the windows pass)
     int nbox;    // boxes of the same shape stored back to back (particles, grids, owner blocks)
-    unsigned long long* totals; // deposited mass per box
     int ppt;                    // particles per thread of a deposit tile: 8 or 4 (8 when folded)
     int fold;                   // folds of the positions (P(k)), 0 = none
 };
@@ -128,22 +130,17 @@ struct DepositBuffers {
 // cell over 2^32 - 1 mass units).  ctl must be cleared and the chunk counts zero.
 void launch_deposit_windows(const PosPackH* pos, int64_t np3, int ng, float mass, const DepositBuffers& b,
                             hipStream_t s);
-// Start of a deposit: the owner pass's route from the previous deposit's ctl[0] (every
-// block in 64-bit sums when more than 1/8 of the nall owner blocks needed them, back to
-// the 32-bit pass below 1/16), then the per-deposit control words cleared.
-void launch_deposit_begin(unsigned long long* ctl, unsigned long long nall, hipStream_t s);
 // rhof non-null: if no tile was deferred, write the FP32 density (q - mean) * 2^-24 to
-// rhof instead of the int64 density to rho (needs the totals: launch_deposit_totals first)
+// rhof instead of the int64 density to rho
 // The route in ctl[HGPM_DEP_CTL] picks, on the device, either every block in 64-bit sums
-// (one kernel; the blocks that need them counted in ctl[0]) or the 32-bit pass, which
-// hands blocks to the 64-bit one (counted); the kernels of the other route exit at once.
+// (the blocks that need them counted in ctl[0]) or the 32-bit pass, which hands blocks to
+// the 64-bit one (counted).
 void launch_deposit_owner(int ng, long long* rho, float* rhof, const DepositBuffers& b, hipStream_t s);
-// totals[box] = sum of the box's tile totals
-void launch_deposit_totals(int64_t np3, const DepositBuffers& b, hipStream_t s);
+// the tiles listed as deferred, and the other set of control words made ready
 void launch_deposit_deferred(const PosPackH* pos, int64_t np3, int ng, float mass, long long* rho,
                              const DepositBuffers& b, hipStream_t s);
-// The deposit of one box's folded positions (b.fold > 0), between launch_deposit_begin and
-// launch_deposit_deferred in place of the windows, totals and owner passes: rho / rhof as
+// The deposit of one box's folded positions (b.fold > 0), before launch_deposit_deferred in
+// place of the windows and owner passes: rho / rhof as
 // launch_deposit_owner writes them.
 void launch_deposit_binned(const PosPackH* pos, int64_t np3, int ng, float mass, long long* rho, float* rhof,
                            const DepositBuffers& b, hipStream_t s);

@@ -98,15 +98,21 @@ template <int RC, bool REAL>
 __global__ __launch_bounds__(NT) void k_rows_r2c_density(const long long* __restrict rho,
                                                          const float* __restrict rhof,
                                                          const unsigned long long* __restrict ctl,
-                                                         const unsigned long long* __restrict total,
+                                                         const unsigned long long* __restrict mass,
                                                          float2* __restrict out, const float2* __restrict tw) {
     constexpr int PC = RC / 2;
     __shared__ float2 lds[lds_elems<N, PC>()];
     float2* spec = lds; // the last stage has read all its inputs before the first output
     const size_t row0 = (size_t)blockIdx.x * RC;
     const bool f32 = REAL || (rhof != nullptr && ctl[1] == 0ull);
-    // total of this row's box: a batch holds several boxes of the same shape
-    const double mean = REAL ? 0.0 : (double)(long long)total[row0 / ((size_t)N * N)] / ((double)N * N * N);
+    // mass of this row's box (a batch holds several boxes of the same shape), from its
+    // partial sums
+    double mean = 0.0;
+    if (!f32) {
+        unsigned long long t = mass[row0 / ((size_t)N * N) * HGPM_DEP_MASS + (threadIdx.x & 63)];
+        for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+        mean = (double)(long long)t / ((double)N * N * N);
+    }
     fft_tile<float2, N, PC, NT, -1, false, true>(
         [&](int, int, int n, int c) {
             if (f32) return make_float2(rhof[(row0 + 2 * c) * N + n], rhof[(row0 + 2 * c + 1) * N + n]);
@@ -373,10 +379,10 @@ void pass_f64(double2* d, int axis, int dir, const double2* tw, hipStream_t s) {
 }
 // nbox grids of the same shape back to back (rows of every box in one launch)
 void fwd_z_r2c(const long long* rho, const float* rhof, const unsigned long long* ctl,
-               const unsigned long long* totals, float2* out, const float2* tw, int nbox, hipStream_t s) {
+               const unsigned long long* mass, float2* out, const float2* tw, int nbox, hipStream_t s) {
     constexpr int RC = 2 * rc32();
     unsigned nb = (unsigned)((size_t)nbox * N * N / RC);
-    k_rows_r2c_density<RC, false><<<nb, NT, 0, s>>>(rho, rhof, ctl, totals, out, tw);
+    k_rows_r2c_density<RC, false><<<nb, NT, 0, s>>>(rho, rhof, ctl, mass, out, tw);
 }
 void fwd_z_r2c_real(const float* in, float2* out, const float2* tw, hipStream_t s) {
     constexpr int RC = 2 * rc32();

@@ -454,16 +454,23 @@ __device__ __forceinline__ long long dep_window_atomic(unsigned long long* win, 
     return (long long)dep;
 }
 
-// Workgroup sum of the threads' deposited mass, stored by thread 0 as the tile's total
-// (a plain store: one word per tile, summed by k_deposit_total).
-__device__ __forceinline__ void dep_tile_total(long long local, long long* s_tot, unsigned long long* out) {
+// A box's deposited mass is kept as HGPM_DEP_MASS partial sums (whole numbers: the order
+// of the additions does not matter), one addition per tile spread over them, and added up
+// by whoever needs the mean: no kernel of its own between the windows and the owner pass,
+// and no single address that every tile adds to.
+static_assert(HGPM_DEP_MASS == 64, "one lane per partial sum");
+__device__ __forceinline__ unsigned long long* dep_mass_slot(unsigned long long* mass, int tile, int ntb) {
+    return mass + (tile / ntb) * HGPM_DEP_MASS + tile % ntb % HGPM_DEP_MASS;
+}
+// Workgroup sum of the threads' deposited mass, added by thread 0.
+__device__ __forceinline__ void dep_tile_total(long long local, long long* s_tot, unsigned long long* slot) {
     for (int off = 32; off > 0; off >>= 1) local += __shfl_down(local, off, 64);
     if ((threadIdx.x & 63) == 0) s_tot[threadIdx.x >> 6] = local;
     __syncthreads();
     if (threadIdx.x == 0) {
         long long t = 0;
         for (int w = 0; w < DEP_NT / 64; w++) t += s_tot[w];
-        *out = (unsigned long long)t;
+        atomicAdd(slot, (unsigned long long)t);
     }
 }
 
@@ -509,7 +516,7 @@ struct DepWindowArgs {
     // 32-bit pass), taken again by the 64-bit pass
     unsigned short* __restrict wide_slots;
     unsigned long long* __restrict ctl;
-    unsigned long long* __restrict tile_total;
+    unsigned long long* __restrict mass_sum; // HGPM_DEP_MASS partial sums per box
     int nsub;
     int4* __restrict boxes;
     int ntb;  // tiles per box
@@ -643,7 +650,7 @@ __device__ __forceinline__ void dep_windows_tile(int tile, unsigned q, const Dep
         if (tid == 0) {
             g.deferred[atomicAdd(&g.ctl[1], 1ull)] = (unsigned)tile;
             if (state == 2) atomicAdd(&g.ctl[3], 1ull);
-            g.tile_total[tile] = 0ull; // written by k_deposit_deferred
+            // (its mass is added by k_deposit_deferred)
         }
         return;
     }
@@ -661,7 +668,7 @@ __device__ __forceinline__ void dep_windows_tile(int tile, unsigned q, const Dep
         unsigned long long t = 0, d = 0;
         for (int w = 0; w < DEP_NT / 64; w++) { t += sh.tot[w]; d += sh.dif[w]; }
         sh.over = d != 0ull;
-        if (!d) g.tile_total[tile] = t;
+        if (!d) atomicAdd(dep_mass_slot(g.mass_sum, tile, g.ntb), t);
     }
     __syncthreads();
     if (!WIDE && sh.over) {
@@ -705,20 +712,26 @@ __global__ __launch_bounds__(DEP_NT) void k_deposit_wide(DepWindowArgs g) {
 // for its arena address and one for its LDS address; U planes are loaded before the
 // first LDS add so that their loads are in flight together.
 // Two kernels: k_deposit_owner sums in uint32 LDS cells (16 KB a block, few registers:
-// eight waves per SIMD) and hands a block to k_deposit_owner64 (int64 LDS cells) when
+// eight waves per SIMD) and hands a block to k_deposit_owner64 (int64 LDS cells, one
+// workgroup per block, those of blocks not handed over exit at once) when
 // one of its chunks has 64-bit cells or a cell's sum reached 2^32 (its stored cells
 // then sum to less than the values added).  A handed-over block writes nothing and
 // keeps its count.  wide_blk (one byte per block, kept across deposits): bit 1 = handed
 // over in this deposit (ctl[0] counts them), bit 0 = found to need 64-bit sums by an
 // earlier deposit, which sends the block to the 64-bit pass at once (a dense block
 // stays dense).  When many blocks needed 64-bit sums in the previous deposit, the route
-// word ctl[HGPM_DEP_CTL] (set by k_deposit_begin) sends every block to
-// k_deposit_owner64_all instead (the ones that need it counted in ctl[0]), and the
-// 32-bit kernels exit at once.  The marks and the route only route blocks (every kernel
-// gives the same bits): a stale one costs time, never results.
+// word ctl[HGPM_DEP_CTL] (set at the end of that deposit) sends every block to
+// k_deposit_owner64 (the ones that need it counted in ctl[0]), and the 32-bit kernel exits
+// at once.  The marks and the route only route blocks (both kernels give the same bits): a
+// stale one costs time, never results.
 // rhof (may be null): when no tile was deferred (ctl[1] == 0) the block is written as
 // FP32 (q - mean) * 2^-24 to rhof, the form the forward z transform takes, instead of
-// int64 q to rho; mean = totals[box] / ng^3 (the totals of every tile are final).
+// int64 q to rho; mean = the box's mass / ng^3 (that of every tile is final).
+// WG threads: 256, or 1024 where the grid has so few blocks that they leave the chip
+// mostly idle and a block's time is a chain of memory latencies: four waves then share a
+// chunk, one plane group each.  Measured, 256 against 1024 threads: 22.5 / 16.9 us with 8
+// blocks (32^3), 15.9 / 13.5 with 216, 16.8 / 16.0 with 512, 28.3 / 48.6 with 1728 (192^3):
+// hence OWN_FEW.
 struct OwnerArgs {
     const unsigned* __restrict arena;
     const uint4* __restrict slots;
@@ -729,20 +742,26 @@ struct OwnerArgs {
     float* __restrict rhof;
     const unsigned long long* __restrict ctl;
     unsigned long long* __restrict nredo; // = ctl[0]
-    const unsigned long long* __restrict totals;
+    const unsigned long long* __restrict mass;
     int nblk;
-    int nall; // owner blocks of every box
-    int count_need; // k_deposit_owner64_all: count the blocks that need 64-bit sums in ctl[0]
     int64_t gcells;
 };
+// The mass of box b, in every lane (a whole wave).
+__device__ __forceinline__ long long box_mass(const unsigned long long* __restrict mass, int b) {
+    unsigned long long t = mass[b * HGPM_DEP_MASS + (threadIdx.x & 63)];
+    for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
+    return (long long)t;
+}
 constexpr int OWN_U32 = 8;  // arena loads in flight per lane, 32-bit pass
 constexpr int OWN_U64 = 16; // 64-bit pass
+constexpr unsigned OWN_FEW = 512; // owner blocks up to which 1024 threads take one
 // Returns false when the block needs the 64-bit pass (ACC = unsigned only).
-template <typename ACC, int U>
+template <typename ACC, int U, int WG>
 __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* acc, uint4* desc, int* s_n, int* s_redo,
                                             unsigned long long* s_dif) {
     constexpr bool A64 = sizeof(ACC) == 8;
     constexpr int OWN_J = OB * OB / 64; // plane slots per lane (a plane holds <= OB^2 cells)
+    constexpr int JW = WG == 1024 ? OWN_J : 1; // waves that share a chunk
     const int nb = g.ng / OB;
     const int box = blk / g.nblk, lb = blk - box * g.nblk;
     const bool f32 = g.rhof != nullptr && g.ctl[1] == 0ull;
@@ -768,12 +787,12 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
         *s_dif = 0ull;
     }
     if (tid < g.nslots) desc[tid] = dl;
-    for (int i = tid; i < OB * OB * OB; i += OWN_NT) acc[i] = (ACC)0;
+    for (int i = tid; i < OB * OB * OB; i += WG) acc[i] = (ACC)0;
     __syncthreads();
     const int nd = *s_n;
     bool wrap = false;             // a chunk with 64-bit cells
     unsigned long long added = 0;  // this lane's sum of the values added (32-bit pass)
-    for (int d = wv; d < nd; d += OWN_NT / 64) {
+    for (int d = wv / JW; d < nd; d += WG / 64 / JW) {
         // one descriptor per wave: its words are uniform (scalar registers)
         uint4 de = desc[d];
         de.x = __builtin_amdgcn_readfirstlane(de.x);
@@ -794,7 +813,7 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
         // p -> (ly, lz) by multiplication with a rounded reciprocal: exact here because
         // p < 256 keeps the rounding error below the 0.5/mz margin of (p + 0.5)
         const float rmz = 1.0f / (float)mz;
-        for (int j = 0; j < OWN_J && j * 64 < myz; j++) {
+        for (int j = JW > 1 ? wv % JW : 0; j < OWN_J && j * 64 < myz; j += JW) {
             const int pl = lane + 64 * j;
             const bool pv = pl < myz;
             const int ly = (int)(((float)pl + 0.5f) * rmz), lz = pl - ly * mz;
@@ -855,8 +874,8 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
     __syncthreads();
     // thread tid writes (x, y, z) = (k, t / OB, t % OB), t = tid % OB^2, of the block for
     // k = tid / OB^2, tid / OB^2 + KS, ...
-    constexpr int KS = OWN_NT / (OB * OB);
-    static_assert(OWN_NT % (OB * OB) == 0 && OB % KS == 0, "whole (y, z) planes per pass");
+    constexpr int KS = WG / (OB * OB);
+    static_assert(WG % (OB * OB) == 0 && OB % KS == 0, "whole (y, z) planes per pass");
     const int t = tid % (OB * OB), k0 = tid / (OB * OB);
     if constexpr (!A64) {
         // a cell whose sum reached 2^32 wrapped: the stored cells then sum to less than
@@ -882,7 +901,7 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
     const int64_t plane = (int64_t)g.ng * g.ng;
     unsigned long long hi = 0; // a cell of 2^32 units or more (64-bit pass)
     if (f32) {
-        const double mean = (double)(long long)g.totals[box] / (double)g.gcells;
+        const double mean = (double)box_mass(g.mass, box) / (double)g.gcells;
         float* __restrict rf = g.rhof + (int64_t)box * g.gcells;
 #pragma unroll 4
         for (int k = k0; k < OB; k += KS) {
@@ -901,74 +920,58 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
     }
     if constexpr (A64) {
         // mark the block for later deposits: it needs 64-bit sums (a 64-bit chunk or a
-        // cell of 2^32 units or more); with every block in this pass (count_need), count it
+        // cell of 2^32 units or more); with every block in this pass, count it
         if (__builtin_amdgcn_ballot_w64(hi != 0ull) && lane == 0) *s_redo = 1;
         __syncthreads();
         if (tid == 0) {
             g.wide_blk[blk] = *s_redo ? 1 : 0;
-            if (g.count_need && *s_redo) atomicAdd(g.nredo, 1ull);
+            if (g.ctl[HGPM_DEP_CTL] && *s_redo) atomicAdd(g.nredo, 1ull);
         }
     } else {
         if (tid == 0) g.count[blk] = 0u;
     }
     return true;
 }
-// ctl[0] of the previous deposit -> the route; then the control words of this one cleared
-__global__ __launch_bounds__(64) void k_deposit_begin(unsigned long long* __restrict ctl, unsigned long long nall) {
-    if (threadIdx.x == 0) {
-        const unsigned long long need = ctl[0];
-        unsigned long long r = ctl[HGPM_DEP_CTL];
-        if (!r && need * 8 > nall) r = 1;
-        else if (r && need * 16 < nall) r = 0;
-        ctl[HGPM_DEP_CTL] = r;
-    }
-    __syncthreads();
-    for (int i = threadIdx.x; i < HGPM_DEP_CTL; i += blockDim.x) ctl[i] = 0ull;
-}
-__global__ __launch_bounds__(OWN_NT) void k_deposit_owner(OwnerArgs g) {
-    if (g.ctl[HGPM_DEP_CTL]) return; // every block in k_deposit_owner64_all
+template <int WG> __global__ __launch_bounds__(WG) void k_deposit_owner(OwnerArgs g) {
+    if (g.ctl[HGPM_DEP_CTL]) return; // every block in k_deposit_owner64
     __shared__ unsigned acc[OB * OB * OB];
     __shared__ uint4 desc[HGPM_DEP_SLOTS];
     __shared__ int s_n, s_redo;
     __shared__ unsigned long long s_dif;
-    owner_block<unsigned, OWN_U32>(g, (int)xcd_remap(blockIdx.x, gridDim.x), acc, desc, &s_n, &s_redo, &s_dif);
+    owner_block<unsigned, OWN_U32, WG>(g, (int)xcd_remap(blockIdx.x, gridDim.x), acc, desc, &s_n, &s_redo, &s_dif);
 }
-// Every block in 64-bit cells, one workgroup per block (a deposit with many dense
-// blocks, late in a run: the 32-bit attempt would be wasted on them).
-__global__ __launch_bounds__(OWN_NT) void k_deposit_owner64_all(OwnerArgs g) {
-    if (!g.ctl[HGPM_DEP_CTL]) return; // the 32-bit route
-    __shared__ unsigned long long acc[OB * OB * OB];
-    __shared__ uint4 desc[HGPM_DEP_SLOTS];
-    __shared__ int s_n, s_redo;
-    __shared__ unsigned long long s_dif;
-    owner_block<unsigned long long, OWN_U64>(g, (int)xcd_remap(blockIdx.x, gridDim.x), acc, desc, &s_n, &s_redo, &s_dif);
-}
+// In 64-bit cells: the blocks handed over, or every block on that route (a deposit with
+// many dense blocks, late in a run: the 32-bit attempt would be wasted on them).  A
+// workgroup per block: the empty ones cost 56 us at 1024^3 (262144 of them), and dense
+// blocks, which lie together, spread over the chip (one workgroup scanning 256 blocks'
+// marks and summing the marked ones in turn took 0.3 ms a step late in a 512^3 run).
 __global__ __launch_bounds__(OWN_NT) void k_deposit_owner64(OwnerArgs g) {
+    const int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
+    if (!g.ctl[HGPM_DEP_CTL] && !(g.wide_blk[blk] & 2)) return;
     __shared__ unsigned long long acc[OB * OB * OB];
     __shared__ uint4 desc[HGPM_DEP_SLOTS];
     __shared__ int s_n, s_redo;
     __shared__ unsigned long long s_dif;
-    __shared__ unsigned long long s_mask[OWN_NT / 64];
-    if (g.ctl[HGPM_DEP_CTL]) return; // every block in k_deposit_owner64_all
-    // a workgroup scans OWN_NT consecutive blocks (one mark per thread) and sums the
-    // handed-over ones in turn: neighbouring blocks, which share the arena lines of
-    // their tiles' windows, stay on one XCD, and a deposit with none handed over costs
-    // one mark load per block
-    const int base = (int)xcd_remap(blockIdx.x, gridDim.x) * OWN_NT;
-    const int tid = threadIdx.x;
-    const bool f = base + tid < g.nall && (g.wide_blk[base + tid] & 2);
-    const unsigned long long m = __builtin_amdgcn_ballot_w64(f);
-    if ((tid & 63) == 0) s_mask[tid >> 6] = m;
-    __syncthreads();
-#pragma unroll 1
-    for (int w = 0; w < OWN_NT / 64; w++) {
-        unsigned long long mm = s_mask[w];
-        while (mm) {
-            const int bit = __builtin_ctzll(mm);
-            mm &= mm - 1;
-            owner_block<unsigned long long, OWN_U64>(g, base + 64 * w + bit, acc, desc, &s_n, &s_redo, &s_dif);
-            __syncthreads();
-        }
+    owner_block<unsigned long long, OWN_U64, OWN_NT>(g, blk, acc, desc, &s_n, &s_redo, &s_dif);
+}
+
+// The end of a deposit: the control words of the next one (the other of two sets, used in
+// turn) cleared, and its owner route set from the blocks that needed 64-bit sums in this
+// one (more than 1/8 of them: every block in 64-bit sums; below 1/16: back).
+struct DepNext {
+    unsigned long long* __restrict set; // ctl, then the mass partial sums
+    int words;
+    unsigned long long nall; // owner blocks; 0: the route stays
+};
+__device__ __forceinline__ void dep_next(const unsigned long long* __restrict ctl, const DepNext& n) {
+    for (int i = threadIdx.x; i < n.words; i += DEP_NT)
+        if (i != HGPM_DEP_CTL) n.set[i] = 0ull;
+    if (threadIdx.x == 0) {
+        const unsigned long long need = ctl[0];
+        unsigned long long r = ctl[HGPM_DEP_CTL];
+        if (n.nall && !r && need * 8 > n.nall) r = 1;
+        else if (n.nall && r && need * 16 < n.nall) r = 0;
+        n.set[HGPM_DEP_CTL] = r;
     }
 }
 
@@ -978,11 +981,12 @@ __global__ __launch_bounds__(DEP_NT) void k_deposit_deferred(POS pos, int64_t n,
                                                              float mass, unsigned long long* __restrict rho,
                                                              const unsigned long long* __restrict ctl,
                                                              const unsigned* __restrict deferred,
-                                                             unsigned long long* __restrict tile_total, int ntb,
-                                                             int64_t gcells) {
+                                                             unsigned long long* __restrict mass_sum, int ntb,
+                                                             int64_t gcells, DepNext next) {
     __shared__ unsigned long long win[DEP_LDS / 8];
     __shared__ int red[12][DEP_NT / 64];
     __shared__ long long s_tot[DEP_NT / 64];
+    if (blockIdx.x == 0) dep_next(ctl, next);
     const unsigned long long nd = ctl[1];
     for (unsigned long long q = blockIdx.x; q < nd; q += gridDim.x) {
         const unsigned tile = deferred[q];
@@ -993,25 +997,9 @@ __global__ __launch_bounds__(DEP_NT) void k_deposit_deferred(POS pos, int64_t n,
         dep_load_box(pos, p0, ng, r0, R, red, lo, e);
         unsigned long long* box_rho = rho + (int64_t)(tile / ntb) * gcells;
         const long long local = dep_window_atomic<SMALL>(win, R, lo, e, r0, ng, mass, box_rho);
-        dep_tile_total(local, s_tot, &tile_total[tile]);
+        dep_tile_total(local, s_tot, dep_mass_slot(mass_sum, (int)tile, ntb));
         __syncthreads();
     }
-}
-
-// totals[b] = sum of the totals of box b's tiles: DEP_TOT_WG workgroups per box each
-// add their share (integer sums, order-free) to a zeroed totals[b].
-constexpr int DEP_TOT_WG = 32;
-__global__ __launch_bounds__(256) void k_deposit_total(const unsigned long long* __restrict tile_total,
-                                                       int64_t ntb, unsigned long long* __restrict totals) {
-    __shared__ unsigned long long s[256 / 64];
-    const int box = blockIdx.x / DEP_TOT_WG, part = blockIdx.x % DEP_TOT_WG;
-    unsigned long long t = 0;
-    tile_total += (int64_t)box * ntb;
-    for (int64_t i = (int64_t)part * 256 + threadIdx.x; i < ntb; i += (int64_t)DEP_TOT_WG * 256) t += tile_total[i];
-    for (int off = 32; off > 0; off >>= 1) t += __shfl_down(t, off, 64);
-    if ((threadIdx.x & 63) == 0) s[threadIdx.x >> 6] = t;
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(&totals[box], s[0] + s[1] + s[2] + s[3]);
 }
 
 // ----------------------------------------------------------------------------------
@@ -1047,10 +1035,9 @@ struct BinArgs {
     unsigned* __restrict cursor; // ... and the next free one (k_bin_pass<true>)
     unsigned long long* __restrict ctl;
     unsigned* __restrict deferred;
-    unsigned long long* __restrict tile_total;
+    unsigned long long* __restrict mass_sum;
     unsigned long long* __restrict rho;
     float* __restrict rhof; // see OwnerArgs
-    const unsigned long long* __restrict totals;
     int nblk, nt;
     int64_t gcells;
 };
@@ -1131,7 +1118,7 @@ template <bool SMALL, bool FILL> __global__ __launch_bounds__(DEP_NT) void k_bin
             });
         }
     } else {
-        dep_tile_total(dep, s_tot, &g.tile_total[tile]);
+        dep_tile_total(dep, s_tot, dep_mass_slot(g.mass_sum, tile, g.nt));
     }
 }
 constexpr int BIN_SCAN = 1024;
@@ -1153,6 +1140,7 @@ __global__ __launch_bounds__(BIN_SCAN) void k_bin_scan(BinArgs g) {
     if (all > g.cap) { // no entries: every block is written empty, every tile is deferred
         for (int b = b0; b < b1; b++) g.count[b] = 0u;
         for (int i = tid; i < g.nt; i += BIN_SCAN) g.deferred[i] = (unsigned)i;
+        if (tid < HGPM_DEP_MASS) g.mass_sum[tid] = 0ull; // added again with the tiles
         if (tid == 0) g.ctl[1] = (unsigned long long)g.nt;
         return;
     }
@@ -1201,7 +1189,7 @@ template <bool SMALL> __global__ __launch_bounds__(OWN_NT) void k_bin_owner(BinA
     }
     __syncthreads();
     const bool f32 = g.rhof != nullptr && g.ctl[1] == 0ull;
-    const double mean = (double)(long long)g.totals[0] / (double)g.gcells;
+    const double mean = (double)box_mass(g.mass_sum, 0) / (double)g.gcells;
     for (int i = tid; i < OB * OB * OB; i += OWN_NT) {
         const int64_t at = gidx(ng, b[0] + i / (OB * OB), b[1] + i / OB % OB, b[2] + i % OB);
         if (f32) g.rhof[at] = (float)(((double)(long long)acc[i] - mean) * (1.0 / 16777216.0));
@@ -1743,7 +1731,7 @@ DepWindowArgs window_args(const PosPackH* pos, int64_t n, int ng, float mass, co
     g.wide = b.wide;
     g.wide_slots = b.wide_slots;
     g.ctl = b.ctl;
-    g.tile_total = b.tile_total;
+    g.mass_sum = b.ctl + HGPM_DEP_CTL + 1;
     g.nsub = b.nsub;
     g.boxes = (int4*)b.boxes;
     g.ntb = (int)(n / b.nbox / (DEP_NT * b.ppt));
@@ -1775,9 +1763,6 @@ void launch_deposit_windows(const PosPackH* pos, int64_t n, int ng, float mass, 
     if (b.ppt == 4) run(std::integral_constant<int, 4>{});
     else run(std::integral_constant<int, 8>{});
 }
-void launch_deposit_begin(unsigned long long* ctl, unsigned long long nall, hipStream_t s) {
-    k_deposit_begin<<<1, 64, 0, s>>>(ctl, nall);
-}
 void launch_deposit_owner(int ng, long long* rho, float* rhof, const DepositBuffers& b, hipStream_t s) {
     const unsigned nb = (unsigned)(ng / OB);
     const int nblk = (int)(nb * nb * nb);
@@ -1792,23 +1777,13 @@ void launch_deposit_owner(int ng, long long* rho, float* rhof, const DepositBuff
     g.rhof = rhof;
     g.ctl = b.ctl;
     g.nredo = b.ctl; // ctl[0]
-    g.totals = b.totals;
+    g.mass = b.ctl + HGPM_DEP_CTL + 1;
     g.nblk = nblk;
     g.gcells = (int64_t)ng * ng * ng;
     const unsigned nall = (unsigned)nblk * (unsigned)b.nbox;
-    g.nall = (int)nall;
-    g.count_need = 0;
-    k_deposit_owner<<<nall, OWN_NT, 0, s>>>(g);
-    // the blocks handed over (none, mostly), OWN_NT blocks' marks per workgroup
-    k_deposit_owner64<<<(nall + OWN_NT - 1) / OWN_NT, OWN_NT, 0, s>>>(g);
-    g.count_need = 1;
-    k_deposit_owner64_all<<<nall, OWN_NT, 0, s>>>(g);
-}
-void launch_deposit_totals(int64_t n, const DepositBuffers& b, hipStream_t s) {
-    if (!n) return;
-    const int ntb = (int)(n / (DEP_NT * b.ppt) / b.nbox);
-    k_zero_u64<<<1, 64, 0, s>>>(b.totals, (size_t)b.nbox);
-    k_deposit_total<<<b.nbox * DEP_TOT_WG, 256, 0, s>>>(b.tile_total, ntb, b.totals);
+    if (nall <= OWN_FEW) k_deposit_owner<1024><<<nall, 1024, 0, s>>>(g);
+    else k_deposit_owner<OWN_NT><<<nall, OWN_NT, 0, s>>>(g);
+    k_deposit_owner64<<<nall, OWN_NT, 0, s>>>(g);
 }
 void launch_deposit_deferred(const PosPackH* pos, int64_t n, int ng, float mass, long long* rho,
                              const DepositBuffers& b, hipStream_t s) {
@@ -1817,20 +1792,22 @@ void launch_deposit_deferred(const PosPackH* pos, int64_t n, int ng, float mass,
     const int ntb = (int)(nt / b.nbox);
     const int64_t gc = (int64_t)ng * ng * ng;
     const unsigned grid = (unsigned)(nt < 512 ? nt : 512);
+    unsigned long long* mass_sum = b.ctl + HGPM_DEP_CTL + 1;
+    const unsigned long long nall = (unsigned long long)(ng / OB) * (ng / OB) * (ng / OB) * b.nbox;
+    const DepNext next{b.next, b.set_words, b.fold ? 0ull : nall};
     auto run = [&](auto pc, auto p) {
         constexpr int PPT = decltype(pc)::value;
         if (mass < 128.0f)
             k_deposit_deferred<true, PPT><<<grid, DEP_NT, 0, s>>>(p, n, ng, mass, (unsigned long long*)rho, b.ctl,
-                                                                  b.deferred, b.tile_total, ntb, gc);
+                                                                  b.deferred, mass_sum, ntb, gc, next);
         else
             k_deposit_deferred<false, PPT><<<grid, DEP_NT, 0, s>>>(p, n, ng, mass, (unsigned long long*)rho, b.ctl,
-                                                                   b.deferred, b.tile_total, ntb, gc);
+                                                                   b.deferred, mass_sum, ntb, gc, next);
     };
     const StoredPos sp{(const PosPack*)pos};
     if (b.fold) run(std::integral_constant<int, 8>{}, FoldedPos{(const PosPack*)pos, b.fold, ng});
     else if (b.ppt == 4) run(std::integral_constant<int, 4>{}, sp);
     else run(std::integral_constant<int, 8>{}, sp);
-    launch_deposit_totals(n, b, s);
 }
 void launch_deposit_binned(const PosPackH* pos, int64_t n, int ng, float mass, long long* rho, float* rhof,
                            const DepositBuffers& b, hipStream_t s) {
@@ -1848,17 +1825,15 @@ void launch_deposit_binned(const PosPackH* pos, int64_t n, int ng, float mass, l
     g.cursor = g.start + g.nblk;
     g.ctl = b.ctl;
     g.deferred = b.deferred;
-    g.tile_total = b.tile_total;
+    g.mass_sum = b.ctl + HGPM_DEP_CTL + 1;
     g.rho = (unsigned long long*)rho;
     g.rhof = rhof;
-    g.totals = b.totals;
     g.nt = (int)(n / DEP_TILE);
     g.gcells = (int64_t)ng * ng * ng;
     auto run = [&](auto sc) {
         constexpr bool SMALL = decltype(sc)::value;
         k_bin_pass<SMALL, false><<<(unsigned)g.nt, DEP_NT, 0, s>>>(g);
         k_bin_scan<<<1, BIN_SCAN, 0, s>>>(g);
-        launch_deposit_totals(n, b, s);
         k_bin_pass<SMALL, true><<<(unsigned)g.nt, DEP_NT, 0, s>>>(g);
         k_bin_owner<SMALL><<<(unsigned)g.nblk, OWN_NT, 0, s>>>(g);
     };
