@@ -93,7 +93,7 @@ struct hgpm_ctx {
     std::vector<hipEvent_t> evpool;
     // tunables: column-pass and x-pass variants of the FFT (see k_fft.hip), set by
     // hgpm_set_tunable or hgpm_autotune
-    int var_cols = 2, var_xs = 2;
+    int var_cols = 0, var_xs = 0; // FftOps::variant at creation
     int fft_plan = 0; // radix order of the FFT passes: 0 = fft_ops(ng), 1 = fft_ops_alt(ng) (tunable "fft_plan")
     int var_gather = 0; // gather workgroup shape (k_particles.hip), tunable "gather_tile"
     int dep_ppt = 8;    // deposit tile: a whole 16^3 Lagrangian tile (8) or half (4), tunable "deposit_tile"
@@ -249,7 +249,7 @@ int set_fft_plan(hgpm_ctx* c, int plan) {
 // 3-D transform of an n^3 grid through the generic passes (z, y, x).
 int fft3d_f32(hgpm_ctx* c, const FftOps* ops, float2* d, const float2* tw, int dir) {
     Timed t(c, "fft3d_f32");
-    const int v = ops == c->fft ? c->var_cols : 2;
+    const int v = ops == c->fft ? c->var_cols : ops->variant;
     ops->pass_f32(d, 2, dir, tw, v, c->st);
     ops->pass_f32(d, 1, dir, tw, v, c->st);
     ops->pass_f32(d, 0, dir, tw, v, c->st);
@@ -492,6 +492,7 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
     c->nbox = nwave;
     c->fft = fft_ops(p->ng);
     c->fftic = fft_ops(p->np);
+    c->var_cols = c->var_xs = c->fft->variant;
     (void)hipGetDevice(&c->device);
     int rc = HGPM_OK;
     auto bail = [&](int code) {
@@ -915,7 +916,7 @@ int generate_ic_from(hgpm_ctx* c, const double* d_ipk, int ipk_bins, double ipk_
         float2* h3 = (float2*)c->arena;
         float* real = (float*)(c->arena + 2 * n3);
         float *sx = real, *sy = real + n3, *sz = real + 2 * n3;
-        const int v = f == c->fft ? c->var_cols : 2;
+        const int v = f == c->fft ? c->var_cols : f->variant;
         IcSpectrum sp;
         sp.tab = d_ipk;
         sp.nbins = ipk_bins;
@@ -1459,14 +1460,14 @@ int hgpm_autotune(hgpm_ctx* c, int reps, double* ms_cols, double* ms_xsolve) {
     // then the whole solve with them; the order with the fastest solve is kept
     const int nplans = fft_ops_alt(c->ng) ? 2 : 1;
     double best_solve = 1e30;
-    int best_plan = 0, best_vc = 2, best_vx = 2;
+    int best_plan = 0, best_vc = c->fft->variant, best_vx = best_vc;
     std::vector<double> pc((size_t)nplans * NVAR_MAX, -1.0), px((size_t)nplans * NVAR_MAX, -1.0);
     int rc = HGPM_OK;
     for (int plan = 0; plan < nplans && !rc; plan++) {
         if ((rc = set_fft_plan(c, plan))) break;
         const FftOps* f = c->fft;
         double best_c = 1e30, best_x = 1e30;
-        int vc = 2, vx = 2;
+        int vc = f->variant, vx = vc;
         for (int v = 0; v < f->n_variants && v < NVAR_MAX && !rc; v++) {
             if (!((f->valid_mask >> v) & 1u)) continue;
             double per = 0.0;

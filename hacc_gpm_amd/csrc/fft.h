@@ -218,11 +218,35 @@ template <int N, bool REV> __host__ __device__ constexpr int stage_L(int s) {
 // st(b, r, n, c, v) consumes transformed element n of column c.  Stage 0 calls ld,
 // the last stage calls st; the stages in between exchange through lds.  With
 // REV = true the radices run in reverse order, so that ld of a REV transform can
-// take the register slots st of a forward transform produced.
-template <typename V, int N, int COLS, int NT, int DIR, bool REV, bool ROW, typename LD, typename ST>
-__device__ __forceinline__ void fft_tile(LD&& ld, ST&& st, V* lds, const V* tw) {
+// take the register slots st of a forward transform produced.  after0() runs once stage
+// 0's outputs are in LDS and its registers are free: loads it issues for the next tile are
+// in flight while the other stages work.
+struct Nothing { __device__ __forceinline__ void operator()() const {} };
+// The twiddles a plan's stages read (apply_twiddles: powers 1, 2 and 4 where the others are
+// composed), packed for LDS: stage s at tw_at(s), entry r L + k.
+constexpr int tw_powers(int R) { return R >= 8 ? 5 : (R == 4 ? 3 : R); }
+template <int N, bool REV> __host__ __device__ constexpr int tw_at(int s) {
+    int n = 0;
+    for (int i = 1; i < s; i++) n += tw_powers(stage_R<N, REV>(i)) * stage_L<N, REV>(i);
+    return n;
+}
+template <int N, bool REV> constexpr int tw_packed() { return tw_at<N, REV>(Plan<N>::S); }
+template <typename V, int N, bool REV, int NT> __device__ __forceinline__ void tw_pack(V* to, const V* __restrict tw) {
+    auto one = [&](auto sc) {
+        constexpr int s = decltype(sc)::value;
+        if constexpr (s > 0) {
+            constexpr int n = tw_powers(stage_R<N, REV>(s)) * stage_L<N, REV>(s);
+            for (int i = threadIdx.x; i < n; i += NT) to[tw_at<N, REV>(s) + i] = tw[s * N + i];
+        }
+    };
+    static_for<Plan<N>::S>(one);
+}
+// PACKED: tw is such an LDS table.
+template <typename V, int N, int COLS, int NT, int DIR, bool REV, bool ROW, bool PACKED = false, typename LD,
+          typename ST, typename A0 = Nothing>
+__device__ __forceinline__ void fft_tile(LD&& ld, ST&& st, V* lds, const V* tw, A0&& after0 = A0(),
+                                         const int tid = (int)threadIdx.x) {
     constexpr int S = Plan<N>::S;
-    const int tid = threadIdx.x;
     auto body = [&](auto sc) {
         constexpr int s = decltype(sc)::value;
         constexpr int R = stage_R<N, REV>(s);
@@ -251,7 +275,7 @@ __device__ __forceinline__ void fft_tile(LD&& ld, ST&& st, V* lds, const V* tw) 
                 int c = ROW ? w / SS::NBF : w % COLS;
                 int j = ROW ? w % SS::NBF : w / COLS;
                 int k = j % L;
-                if constexpr (L > 1) apply_twiddles<R, DIR>(x[b], tw + s * N + k, L);
+                if constexpr (L > 1) apply_twiddles<R, DIR>(x[b], tw + (PACKED ? tw_at<N, REV>(s) : s * N) + k, L);
                 DFT<R, DIR, V>::run(x[b]);
                 if constexpr (s == S - 1) {
 #pragma unroll
@@ -263,6 +287,7 @@ __device__ __forceinline__ void fft_tile(LD&& ld, ST&& st, V* lds, const V* tw) 
                 }
             }
         }
+        if constexpr (s == 0) after0();
         if constexpr (s < S - 1) __syncthreads();
     };
     static_for<S>(body);

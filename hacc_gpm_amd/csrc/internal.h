@@ -22,6 +22,7 @@ struct FftOps {
     int n;
     int stages;
     int n_variants;      // column-pass / x-pass variant ids 0..n_variants-1
+    int variant;         // the one a context starts with
     unsigned valid_mask; // bit v set: variant v usable for this length
     void (*twiddles)(double* fwd, double* rev); // stages*n complex each
     // axis 2 = rows (z), 1 = y, 0 = x; variant selects the column-pass shape

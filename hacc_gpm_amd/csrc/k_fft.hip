@@ -68,25 +68,77 @@ __global__ __launch_bounds__(NT) void k_rows_c2c(V* __restrict d, const V* __res
 // ------------------------------------------------------------- cols ----
 // axis 1 (y): tile = (x, z-chunk), element (n=y, c) at x N^2 + n N + z0 + c
 // axis 0 (x): tile = (y, z-chunk), element (n=x, c) at n N^2 + y N + z0 + c
+// First element of column tile t: outer runs over (box, x) for the y pass and (box, y) for
+// the x pass (a batch holds several grids of the same shape back to back).  NP: x-plane
+// pitch (N pz for full grids, NPH for half spectra).
+template <int CC> __device__ __forceinline__ size_t col_base(int t, int axis, int pz, size_t NP) {
+    const int nzc = pz / CC, outer = t / nzc, zc = t % nzc;
+    return axis == 1 ? (size_t)outer * NP + (size_t)zc * CC
+                     : (size_t)(outer / N) * N * NP + (size_t)(outer % N) * pz + (size_t)zc * CC;
+}
 template <typename V, int CC, int NTC, int DIR>
 __global__ __launch_bounds__(NTC) void k_cols_c2c(V* __restrict d, const V* __restrict tw, int axis, int pz,
                                                   size_t plane) {
     __shared__ V lds[lds_elems<N, CC>()];
     // adjacent z-chunks of one row share 128-byte lines: keep them on one XCD's L2
-    const int tile = (int)xcd_remap(blockIdx.x, gridDim.x);
-    const int nzc = pz / CC;
-    // outer runs over (box, x) for the y pass and (box, y) for the x pass: a batch holds
-    // several grids of the same shape back to back
-    const int outer = tile / nzc, zc = tile % nzc;
-    const size_t NP = plane; // x-plane pitch (N pz for full grids, NPH for half spectra)
-    const size_t base = axis == 1 ? (size_t)outer * NP + (size_t)zc * CC
-                                  : (size_t)(outer / N) * N * NP + (size_t)(outer % N) * pz + (size_t)zc * CC;
-    const size_t stride = axis == 1 ? (size_t)pz : NP;
+    const size_t base = col_base<CC>((int)xcd_remap(blockIdx.x, gridDim.x), axis, pz, plane);
+    const size_t stride = axis == 1 ? (size_t)pz : plane;
     fft_tile<V, N, CC, NTC, DIR, false, false>(
         [&](int, int, int n, int c) { return d[base + n * stride + c]; },
         [&](int, int, int n, int c, V v) { d[base + n * stride + c] = v; }, lds, tw);
 }
 
+// Streaming: where one workgroup fills a CU (large tiles: its LDS or its registers leave no
+// room for a second one) its loads, transforms and stores would follow one another.  The
+// x pass of the solve, which transforms twice per tile, is then one workgroup per CU that
+// walks the tiles of its XCD's contiguous range (neighbouring z-chunks at the same time
+// on one L2); the next tile is loaded into registers while the current one is
+// transformed, and the stores drain behind it.
+constexpr int NCU = 256, NXCD = 8;
+struct TileWalk {
+    int t, end;
+    static constexpr int step = NCU / NXCD;
+    __device__ __forceinline__ TileWalk(int nt) {
+        const int x = blockIdx.x % NXCD, per = nt / NXCD, rem = nt % NXCD;
+        const int first = x * per + min(x, rem);
+        t = first + (int)blockIdx.x / NXCD;
+        end = first + per + (x < rem ? 1 : 0);
+    }
+};
+// Opaque copy for one tile: the indices derived from it are the same for every tile, and
+// kept across them they would take the registers of the next tile's elements.  (The
+// twiddles lie in LDS: a global load issued behind the next tile's would wait for it, the
+// vector memory counter being in order.)
+__device__ __forceinline__ int opaque(int tid) {
+    asm volatile("" : "+v"(tid));
+    return tid;
+}
+// A thread's elements of a tile's stage 0.
+template <int CC, int NTC> struct TileRegs {
+    static constexpr int R = Plan<N>::R(0);
+    typedef StageShape<N, CC, NTC, R> SS;
+    static_assert(SS::TOT % NTC == 0, "whole tiles");
+    float2 x[SS::NB][R];
+};
+// Element j + r * NBF of column c of the tile at d (uniform): a scalar base per r and one
+// 32-bit byte offset per lane (j * stride * 8 < 2^32 for every plan), so an address costs
+// one register.
+__device__ __forceinline__ float2* tile_at(float2* d, int nbf, int r, int j, int c, size_t stride) {
+    return (float2*)((char*)(d + (size_t)(r * nbf) * stride) + ((unsigned)j * (unsigned)stride + (unsigned)c) * 8u);
+}
+template <int CC, int NTC>
+__device__ __forceinline__ void load_tile(TileRegs<CC, NTC>& X, float2* d, size_t stride, int tid) {
+    typedef TileRegs<CC, NTC> T;
+#pragma unroll
+    for (int b = 0; b < T::SS::NB; b++) {
+        const int w = tid + b * NTC, c = w % CC, j = w / CC;
+#pragma unroll
+        for (int r = 0; r < T::R; r++) X.x[b][r] = *tile_at(d, T::SS::NBF, r, j, c, stride);
+    }
+}
+// The first tile's loads are waited for before the loop, so that inside it the wait for a
+// tile counts the stores issued behind its loads and leaves them in flight.
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); } // vmcnt(0)
 // ------------------------------------------------- half-spectrum solve ----
 // Forward z transform of the int64 density, mean removed in FP64 (the k = 0 normalisation)
 // before the FP32 rounding, for RC real rows: rows 2c and 2c+1 form the complex column c = a + i b, transformed
@@ -263,6 +315,59 @@ __global__ __launch_bounds__(NTC) void k_y_ic(float2* __restrict h2, float2* __r
         [&](int, int, int n, int c, float2 v) { h3[base + (size_t)n * HZ + c] = v; }, lds, tw);
 }
 
+// k_x_psi as a streaming pass: the next tile is loaded once the inverse transform's first
+// stage has freed the spectrum's registers.  Measured in a run, against the same shape (16
+// columns x 1024 threads) with a workgroup per tile: 2.54 -> 2.24 ms at 1024, 1.15 -> 0.86
+// at 768; at 512, where a tile takes half the LDS, 0.267 -> 0.25-0.31 with one or two
+// workgroups per CU, so the plain form stays there.  The y passes, one transform per tile,
+// gained nothing from the same treatment (1.80 / 1.67 -> 1.93 / 1.72 ms at 1024).
+constexpr bool STREAM_X = N > 512;
+template <int CC, int NTC>
+__global__ __launch_bounds__(NTC) void k_x_psi_stream(float2* h1, const float2* __restrict twf,
+                                                      const float2* __restrict twr, const float* __restrict hs,
+                                                      float gcoef, int nt) {
+    __shared__ float2 lds[lds_elems<N, CC>()];
+    __shared__ float2 tf[tw_packed<N, false>()], tr[tw_packed<N, true>()];
+    __shared__ float hl[N];
+    TileWalk w(nt);
+    if (w.t >= w.end) return;
+    tw_pack<float2, N, false, NTC>(tf, twf);
+    tw_pack<float2, N, true, NTC>(tr, twr);
+    for (int i = threadIdx.x; i < N; i += NTC) hl[i] = hs[i];
+    __syncthreads();
+    typedef LastShape<N, CC, NTC> LS;
+    constexpr int NBL = N / RevPlan<N>::R(RevPlan<N>::S - 1);
+    TileRegs<CC, NTC> X;
+    float2 R[LS::NB][LS::R];
+    float2* at = h1 + col_base<CC>(w.t, 0, HZ, NPH);
+    load_tile(X, at, NPH, (int)threadIdx.x);
+    wait_loads();
+    for (;;) {
+        const int tid = opaque((int)threadIdx.x);
+        const int tn = w.t + TileWalk::step < w.end ? w.t + TileWalk::step : w.t;
+        float2* next = h1 + col_base<CC>(tn, 0, HZ, NPH);
+        const int y = w.t / (HZ / CC) % N, z = w.t % (HZ / CC) * CC + tid % CC;
+        const float hyz = hl[y] + hl[z];
+        fft_tile<float2, N, CC, NTC, -1, false, false, true>(
+            [&](int b, int r, int, int) { return X.x[b][r]; },
+            [&](int b, int r, int, int, float2 v) { R[b][r] = v; }, lds, tf, Nothing(), tid);
+        const int tid2 = opaque((int)threadIdx.x);
+        fft_tile<float2, N, CC, NTC, +1, true, false, true>(
+            [&](int b, int r, int n, int) {
+                float q = hl[n] + hyz; // see k_x_psi
+                asm volatile("" : "+v"(q)); // (no branch around the quotient)
+                const float gq = gcoef * __builtin_amdgcn_rcpf(q);
+                const float g = (n | y | z) == 0 ? 0.0f : gq;
+                return make_float2(g * R[b][r].x, g * R[b][r].y);
+            },
+            [&](int, int r, int n, int c, float2 v) { *tile_at(at, NBL, r, n - r * NBL, c, NPH) = v; }, lds, tr,
+            [&] { load_tile(X, next, NPH, tid2); }, tid2);
+        if (tn == w.t) return;
+        w.t = tn;
+        at = next;
+    }
+}
+
 // Element n of the Hermitian extension of a half-spectrum row: h[n] for n <= N/2,
 // conj h[N-n] above.
 __device__ __forceinline__ float2 herm(const float2* __restrict row, int n) {
@@ -320,7 +425,7 @@ __global__ __launch_bounds__(NT) void k_rows_c2r_real(const float2* __restrict h
 // --------------------------------------------------------- launchers ----
 // Column-pass / x-pass variants (columns per tile, threads per workgroup):
 //   0: (4, 256)  1: (4, 512)  2: (8, 512)  3: (16, 512)  4: (8, 1024)  5: (16, 1024)
-// chosen per transform length by the autotuner (default 2).  More threads per tile
+// chosen per transform length by the autotuner (default VDEF).  More threads per tile
 // means fewer elements, and registers, per thread: the fused x pass holds the
 // spectrum between its two transforms.
 template <typename V, int CC, int NTC>
@@ -345,9 +450,15 @@ constexpr unsigned variant_mask() {
         if (variant_ok(v)) m |= 1u << v;
     return m;
 }
-static_assert(variant_ok(2), "default variant");
+// The shape a context starts with (hgpm_autotune may pick another): 16 columns, whole
+// 128-byte lines, with 1024 threads from 512 on, where fewer leave too few waves per CU.
+// Measured against 8 columns x 512 threads (forward y, inverse y, x pass, us): 256: 30 28 33
+// against 37 29 42; 384: 92 75 99 / 118 74 100; 512: 212 216 267 / 228 226 287; 768: 802
+// 761 857 / 821 775 1132; 1024: 1795 1669 2243 / 1928 1861 2832.
+constexpr int VDEF = N >= 512 ? 5 : 3;
+static_assert(variant_ok(VDEF), "default variant");
 
-// Calls f(IntC<v>) for the runtime variant v when it is valid for N, else variant 2.
+// Calls f(IntC<v>) for the runtime variant v when it is valid for N, else the default.
 template <typename F> void with_variant(int variant, F&& f) {
     bool done = false;
     auto one = [&](auto vc) {
@@ -357,7 +468,7 @@ template <typename F> void with_variant(int variant, F&& f) {
         }
     };
     one(IntC<0>{}); one(IntC<1>{}); one(IntC<2>{}); one(IntC<3>{}); one(IntC<4>{}); one(IntC<5>{});
-    if (!done) f(IntC<2>{});
+    if (!done) f(IntC<VDEF>{});
 }
 void pass_f32(float2* d, int axis, int dir, const float2* tw, int variant, hipStream_t s) {
     if (axis == 2) { rows_launch<float2, rc32()>(d, dir, tw, s); return; }
@@ -411,7 +522,9 @@ template <int CC, int NTC>
 void x_psi_launch(float2* h1, const float2* twf, const float2* twr, const float* hs, int nbox, hipStream_t s) {
     unsigned nb = (unsigned)((size_t)nbox * N * (HZ / CC));
     const float gcoef = (float)(0.125 / ((double)N * N * N)); // g / 2: the stored field is psi / 2
-    k_x_psi<CC, NTC><<<nb, NTC, 0, s>>>(h1, twf, twr, hs, gcoef);
+    if constexpr (STREAM_X && NTC == 1024 && CC == 16)
+        k_x_psi_stream<CC, NTC><<<NCU, NTC, 0, s>>>(h1, twf, twr, hs, gcoef, (int)nb);
+    else k_x_psi<CC, NTC><<<nb, NTC, 0, s>>>(h1, twf, twr, hs, gcoef);
 }
 void x_psi(float2* h1, const float2* twf, const float2* twr, const float* hs, int variant, int nbox, hipStream_t s) {
     with_variant(variant, [&](auto vc) {
@@ -435,7 +548,7 @@ extern const FftOps HGPM_CAT(HGPM_CAT(fft_ops_, HGPM_FFT_N), _alt) = {
 #else
 extern const FftOps HGPM_CAT(fft_ops_, HGPM_FFT_N) = {
 #endif
-    N, Plan<N>::S, NVAR, variant_mask(), twiddles, pass_f32, pass_f64,
+    N, Plan<N>::S, NVAR, VDEF, variant_mask(), twiddles, pass_f32, pass_f64,
     HZ, NPH, pass_half, fwd_z_r2c, x_psi, inv_z_c2r_real, fwd_z_r2c_real, ic_x, ic_y, ic_z,
 };
 } // namespace hgpm
