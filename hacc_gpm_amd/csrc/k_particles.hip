@@ -1009,21 +1009,24 @@ __global__ __launch_bounds__(DEP_NT) void k_deposit_deferred(POS pos, int64_t n,
 // sorted to the owner blocks whose cells they touch (one block, or two per axis where the
 // upper CIC corner lies in the next one: 1.2 entries per particle on average):
 //   k_bin_pass<false> : entries per block, counted per workgroup of 4096 particles in an
-//                       LDS hash table, one global atomic per block it touches; the
-//                       tiles' deposited mass;
+//                       LDS table of the BIN_W^3 blocks around its first particle (every
+//                       block of a grid of up to BIN_W blocks a side), one global atomic
+//                       per block it touches; the tiles' deposited mass;
 //   k_bin_scan        : where each block's entries start in the arena;
 //   k_bin_pass<true>  : the folded positions written there;
 //   k_bin_owner       : a workgroup per block adds its entries' weights in int64 LDS cells
 //                       and writes every cell once.
 // The sums are whole numbers, so the bits are those of every other route.  Entries beyond
 // the arena send the deposit to the atomic route (all tiles listed as deferred).  Bound by
-// the LDS table (an insertion or lookup per entry in both passes) more than by the 60
-// bytes a particle it moves.  Measured on evolved boxes with one fold: 0.66 ms at 256^3,
-// 4.9 ms at 512^3, 35 ms at 1024^3; through windows, nearly all of them deferred, a
-// fold's deposit took 5 ms at 256^3.
-constexpr int BIN_HASH = 8192;  // blocks a workgroup can count in LDS (64 KB with the keys)
-constexpr int BIN_PROBES = 64;  // slots tried before a block is counted in memory directly
-constexpr unsigned BIN_EMPTY = 0xFFFFFFFFu;
+// the scattered writes, the LDS atomics and the memory it moves (about 60 bytes a
+// particle).  Evolved boxes, np = ng, one fold: 0.39 ms at 256^3 (count 0.106, write 0.127,
+// owner blocks 0.142), 2.65 ms at 512^3, 18.8 ms at 1024^3; with the blocks in an LDS hash
+// table, probed for every entry, 0.66, 4.95 and 35.4 ms; through windows, nearly all of
+// them deferred, 5 ms at 256^3.
+// The box is 20 blocks wide: a tile of 16 particles a side covers 2 * 16 / 16 + 1 blocks at
+// fold 1 where np = ng, twice that with each fold until it is the grid's width.
+constexpr int BIN_W = 20;
+constexpr int BIN_SLOTS = BIN_W * BIN_W * BIN_W; // 32 KB of counters
 struct BinArgs {
     const PosPack* __restrict pos;
     int ng, fold;
@@ -1041,80 +1044,102 @@ struct BinArgs {
     int nblk, nt;
     int64_t gcells;
 };
-__device__ __forceinline__ unsigned bin_slot(unsigned* key, unsigned blk) {
-    unsigned h = (blk * 2654435761u) >> 19;
-    static_assert(BIN_HASH == 1 << 13, "13 hash bits");
-    for (int i = 0; i < BIN_PROBES; i++) {
-        const unsigned old = atomicCAS(&key[h], BIN_EMPTY, blk);
-        if (old == BIN_EMPTY || old == blk) return h;
-        h = (h + 1) & (BIN_HASH - 1);
+// The blocks a workgroup counts in LDS: the whole grid (w = nb), or the w = BIN_W blocks per
+// axis from `first` on (periodic).
+struct BinBox {
+    int nb, w, first[3];
+    __device__ __forceinline__ BinBox(const PosPack& q, int ng) : nb(ng / OB), w(min(ng / OB, BIN_W)) {
+        const unsigned X[3] = {q.x, q.y, q.z};
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            const int b = fx_cell(X[d]) / OB - BIN_W / 2;
+            first[d] = nb <= BIN_W ? 0 : (b < 0 ? b + nb : b);
+        }
     }
-    return BIN_EMPTY;
-}
-// body(block) for every owner block the particle's corners lie in.
-template <typename F> __device__ __forceinline__ void bin_blocks(const PosPack& q, int ng, F&& body) {
-    const int nb = ng / OB;
+    __device__ __forceinline__ int rel(int b, int d) const {
+        const int r = b - first[d];
+        return r < 0 ? r + nb : r;
+    }
+    __device__ __forceinline__ unsigned block(int slot) const {
+        int b[3] = {slot / (w * w), slot / w % w, slot % w};
+#pragma unroll
+        for (int d = 0; d < 3; d++) {
+            b[d] += first[d];
+            b[d] -= b[d] >= nb ? nb : 0;
+        }
+        return (unsigned)((b[0] * nb + b[1]) * nb + b[2]);
+    }
+};
+// body(slot, block) for every owner block the particle's corners lie in; slot -1: outside
+// the box.
+template <typename F>
+__device__ __forceinline__ void bin_blocks(const PosPack& q, int ng, const BinBox& box, F&& body) {
     const unsigned X[3] = {q.x, q.y, q.z};
-    int b[3][2];
+    int b[3][2], r[3][2];
     bool two[3];
 #pragma unroll
     for (int d = 0; d < 3; d++) {
         const int c = fx_cell(X[d]);
-        b[d][0] = c / OB;
         two[d] = c % OB == OB - 1;
+        b[d][0] = c / OB;
         b[d][1] = c + 1 == ng ? 0 : c / OB + 1;
+        r[d][0] = box.rel(b[d][0], d);
+        r[d][1] = box.rel(b[d][1], d);
     }
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const int ix = i >> 2, iy = (i >> 1) & 1, iz = i & 1;
-        if ((ix && !two[0]) || (iy && !two[1]) || (iz && !two[2])) continue;
-        body((unsigned)((b[0][ix] * nb + b[1][iy]) * nb + b[2][iz]));
+        const int x = i >> 2, y = (i >> 1) & 1, z = i & 1;
+        if ((x && !two[0]) || (y && !two[1]) || (z && !two[2])) continue;
+        const bool in = r[0][x] < box.w && r[1][y] < box.w && r[2][z] < box.w;
+        body(in ? (r[0][x] * box.w + r[1][y]) * box.w + r[2][z] : -1,
+             (unsigned)((b[0][x] * box.nb + b[1][y]) * box.nb + b[2][z]));
     }
 }
 template <bool SMALL, bool FILL> __global__ __launch_bounds__(DEP_NT) void k_bin_pass(BinArgs g) {
-    __shared__ unsigned key[BIN_HASH], num[BIN_HASH];
+    __shared__ unsigned num[BIN_SLOTS];
     __shared__ long long s_tot[DEP_NT / 64];
     if (FILL && g.ctl[1]) return; // the entries do not fit: the atomic route
     const int tid = threadIdx.x;
     const int tile = (int)xcd_remap(blockIdx.x, gridDim.x);
-    for (int i = tid; i < BIN_HASH; i += DEP_NT) {
-        key[i] = BIN_EMPTY;
-        num[i] = 0u;
-    }
-    const PosPack* __restrict at = g.pos + (int64_t)tile * DEP_TILE + tid; // tiles are full
+    const PosPack* __restrict at = g.pos + (int64_t)tile * DEP_TILE; // tiles are full
+    PosPack P[DEP_PPT];
+#pragma unroll
+    for (int k = 0; k < DEP_PPT; k++) P[k] = at[tid + k * DEP_NT];
+    const BinBox box(fold_pos(at[0], g.fold, g.ng), g.ng);
+    const int slots = box.w * box.w * box.w;
+    for (int i = tid; i < slots; i += DEP_NT) num[i] = 0u;
     __syncthreads();
     long long dep = 0;
-#pragma unroll 1
+#pragma unroll
     for (int k = 0; k < DEP_PPT; k++) {
-        const PosPack q = fold_pos(at[k * DEP_NT], g.fold, g.ng);
-        bin_blocks(q, g.ng, [&](unsigned blk) {
-            const unsigned s = bin_slot(key, blk);
-            if (s != BIN_EMPTY) atomicAdd(&num[s], 1u);
+        P[k] = fold_pos(P[k], g.fold, g.ng);
+        bin_blocks(P[k], g.ng, box, [&](int slot, unsigned blk) {
+            if (slot >= 0) atomicAdd(&num[slot], 1u);
             else if (!FILL) atomicAdd(&g.count[blk], 1u);
         });
         if constexpr (!FILL) {
             constexpr float ONE = (float)(1u << HGPM_FRAC_BITS);
-            const float fx = fx_off_units(q.x), fy = fx_off_units(q.y), fz = fx_off_units(q.z);
+            const float fx = fx_off_units(P[k].x), fy = fx_off_units(P[k].y), fz = fx_off_units(P[k].z);
 #pragma unroll
             for (int i = 0; i < 8; i++)
                 dep += fixed_weight<SMALL>(i & 4 ? fx : ONE - fx, i & 2 ? fy : ONE - fy, i & 1 ? fz : ONE - fz, g.mass);
         }
     }
     __syncthreads();
-    for (int i = tid; i < BIN_HASH; i += DEP_NT) {
-        const unsigned blk = key[i];
-        if (blk == BIN_EMPTY) continue;
-        if constexpr (FILL) num[i] = atomicAdd(&g.cursor[blk], num[i]);
-        else atomicAdd(&g.count[blk], num[i]);
+    for (int i = tid; i < slots; i += DEP_NT) {
+        const unsigned n = num[i];
+        if (n == 0u) continue;
+        if constexpr (FILL) num[i] = atomicAdd(&g.cursor[box.block(i)], n);
+        else atomicAdd(&g.count[box.block(i)], n);
     }
     if constexpr (FILL) {
         __syncthreads();
-#pragma unroll 1
+#pragma unroll
         for (int k = 0; k < DEP_PPT; k++) {
-            const PosPack q = fold_pos(at[k * DEP_NT], g.fold, g.ng);
-            bin_blocks(q, g.ng, [&](unsigned blk) {
-                const unsigned s = bin_slot(key, blk);
-                g.entries[s != BIN_EMPTY ? atomicAdd(&num[s], 1u) : atomicAdd(&g.cursor[blk], 1u)] = q;
+            // computed anew: the first loop's blocks kept for this one cost 120 registers
+            asm volatile("" : "+v"(P[k].x), "+v"(P[k].y), "+v"(P[k].z));
+            bin_blocks(P[k], g.ng, box, [&](int slot, unsigned blk) {
+                g.entries[slot >= 0 ? atomicAdd(&num[slot], 1u) : atomicAdd(&g.cursor[blk], 1u)] = P[k];
             });
         }
     } else {

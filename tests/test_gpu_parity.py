@@ -685,12 +685,13 @@ def test_power_spectrum(hg, orc, ng, folds):
 
 
 @pytest.mark.parametrize("ng,np_,folds,nb,sigma", [(32, 32, 6, 64, 0.7), (96, 96, 3, 65, 3.0), (128, 64, 2, 256, 0.7),
-                                                   (192, 32, 1, 1, 0.7), (64, 64, 3, 221, 3.0)])
+                                                   (192, 32, 1, 1, 0.7), (64, 64, 3, 221, 3.0),
+                                                   (384, 32, 1, 64, 0.7)])
 def test_power_spectrum_folded_lattice(hg, orc, ng, np_, folds, nb, sigma):
     """The binned deposit of folded positions: a displaced lattice at every fold, a radix-3
     length, particle masses 8 and 216 (weights over 31 bits), both accumulator widths of the
-    bins (up to 64 and above) and their extremes: counts equal and values as in
-    test_power_spectrum.  With an arena too small for the entries the fold takes the atomic
+    bins (up to 64 and above) and their extremes, tiles wider than the 320 cells a workgroup
+    counts in LDS: counts equal and values as in test_power_spectrum.  With an arena too small for the entries the fold takes the atomic
     route, with the same bits."""
     case(f"power folded ng={ng} np={np_} folds={folds} bins={nb}")
     rng = np.random.default_rng(ng + nb)
