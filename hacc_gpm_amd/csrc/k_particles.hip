@@ -706,14 +706,19 @@ __global__ __launch_bounds__(DEP_NT) void k_deposit_wide(DepWindowArgs g) {
 
 // Owner pass: one workgroup per OB^3 owner block sums the chunks listed for it in LDS
 // and writes every cell of the block once (the grid is not cleared beforehand); the
-// block's chunk count is reset for the next deposit.  A wave takes one chunk at a
-// time: each lane holds up to OWN_J cells of one (y, z) plane of the chunk (p = lane +
-// 64 j, decoded once per chunk) and walks the chunk's x planes, so a cell costs an add
-// for its arena address and one for its LDS address; U planes are loaded before the
-// first LDS add so that their loads are in flight together.
+// block's chunk count is reset for the next deposit.  Every wave holds the block's chunk
+// descriptors in its lanes (a readlane each, no LDS, no barrier) and takes 64 cells of a
+// chunk's (y, z) plane at a time, one per lane, walking the chunk's x planes, so a cell
+// costs an add for its arena address and one for its LDS address; U planes are loaded
+// before the first LDS add so that their loads are in flight together, 2 or 4 where the
+// chunk is that thin.
+// Bound by the arena reads (1.6 times the grid's bytes at np = ng) and the grid's writes,
+// which add up: at 1024^3 2.2 ms without the writes, 1.2 ms without the reads, 2.8 ms in
+// all for 11.5 GB.  Whole chunks to waves, the descriptors in LDS and every thin chunk
+// loading 8 planes: 3.5 ms; at 256^3 52 against 60 us, at 768^3 with 384^3 particles 0.9
+// to 1.07 against 1.2 to 1.34 ms (with the memory the buffers get).
 // Two kernels: k_deposit_owner sums in uint32 LDS cells (16 KB a block, few registers:
-// eight waves per SIMD) and hands a block to k_deposit_owner64 (int64 LDS cells, one
-// workgroup per block, those of blocks not handed over exit at once) when
+// eight waves per SIMD) and hands a block to k_deposit_owner64 (int64 LDS cells) when
 // one of its chunks has 64-bit cells or a cell's sum reached 2^32 (its stored cells
 // then sum to less than the values added).  A handed-over block writes nothing and
 // keeps its count.  wide_blk (one byte per block, kept across deposits): bit 1 = handed
@@ -728,10 +733,10 @@ __global__ __launch_bounds__(DEP_NT) void k_deposit_wide(DepWindowArgs g) {
 // FP32 (q - mean) * 2^-24 to rhof, the form the forward z transform takes, instead of
 // int64 q to rho; mean = the box's mass / ng^3 (that of every tile is final).
 // WG threads: 256, or 1024 where the grid has so few blocks that they leave the chip
-// mostly idle and a block's time is a chain of memory latencies: four waves then share a
-// chunk, one plane group each.  Measured, 256 against 1024 threads: 22.5 / 16.9 us with 8
-// blocks (32^3), 15.9 / 13.5 with 216, 16.8 / 16.0 with 512, 28.3 / 48.6 with 1728 (192^3):
-// hence OWN_FEW.
+// mostly idle and a block's time is a chain of memory latencies: sixteen waves then take
+// the chunks four at a time.  Measured over a run, 256 against 1024 threads: 14.2 / 9.4 us
+// with 8 blocks (32^3), 10.2 / 7.9 with 216, 11.1 / 10.5 with 512, 20.8 / 28.1 with 1728
+// (192^3): hence OWN_FEW.
 struct OwnerArgs {
     const unsigned* __restrict arena;
     const uint4* __restrict slots;
@@ -752,21 +757,28 @@ __device__ __forceinline__ long long box_mass(const unsigned long long* __restri
     for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
     return (long long)t;
 }
-constexpr int OWN_U32 = 8;  // arena loads in flight per lane, 32-bit pass
+constexpr int OWN_U32 = 16; // arena loads in flight per lane, 32-bit pass
 constexpr int OWN_U64 = 16; // 64-bit pass
 constexpr unsigned OWN_FEW = 512; // owner blocks up to which 1024 threads take one
 // Returns false when the block needs the 64-bit pass (ACC = unsigned only).
 template <typename ACC, int U, int WG>
-__device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* acc, uint4* desc, int* s_n, int* s_redo,
+__device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* acc, int* s_redo,
                                             unsigned long long* s_dif) {
     constexpr bool A64 = sizeof(ACC) == 8;
     constexpr int OWN_J = OB * OB / 64; // plane slots per lane (a plane holds <= OB^2 cells)
-    constexpr int JW = WG == 1024 ? OWN_J : 1; // waves that share a chunk
+    constexpr int DW = WG / 64 / OWN_J; // chunks in work at a time, OWN_J waves each
+    static_assert(WG % (64 * OWN_J) == 0 && HGPM_DEP_SLOTS <= 64, "whole groups of waves, a descriptor per lane");
     const int nb = g.ng / OB;
     const int box = blk / g.nblk, lb = blk - box * g.nblk;
     const bool f32 = g.rhof != nullptr && g.ctl[1] == 0ull;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    if (!A64 && g.wide_blk[blk]) {
+    // the mark, the count and every slot descriptor (one per lane, in every wave; the unused
+    // ones are ignored) are loaded together: one memory latency
+    const unsigned char mark = A64 ? (unsigned char)0 : g.wide_blk[blk];
+    const unsigned cnt = g.count[blk];
+    uint4 dl = make_uint4(0u, 0u, 0x80000000u, 0u);
+    if (lane < g.nslots) dl = g.slots[(size_t)blk * g.nslots + lane];
+    if (!A64 && mark) {
         // summed in 64 bits by an earlier deposit (a dense block stays dense): straight
         // to the 64-bit pass, without a 32-bit attempt
         if (tid == 0) {
@@ -775,99 +787,101 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
         }
         return false;
     }
-    // every slot descriptor is loaded together with the count (the unused ones are
-    // ignored), so the two loads cost one memory latency
-    uint4 dl = make_uint4(0u, 0u, 0x80000000u, 0u);
-    if (tid < g.nslots) dl = g.slots[(size_t)blk * g.nslots + tid];
     if (tid == 0) {
-        const unsigned c = g.count[blk];
-        if (A64) g.count[blk] = 0u;
-        *s_n = (int)min(c, (unsigned)g.nslots);
         *s_redo = 0;
         *s_dif = 0ull;
     }
-    if (tid < g.nslots) desc[tid] = dl;
     for (int i = tid; i < OB * OB * OB; i += WG) acc[i] = (ACC)0;
     __syncthreads();
-    const int nd = *s_n;
+    if (A64 && tid == 0) g.count[blk] = 0u;
+    const bool live = lane < (int)min(cnt, (unsigned)g.nslots) && !(dl.z >> 31);
     bool wrap = false;             // a chunk with 64-bit cells
     unsigned long long added = 0;  // this lane's sum of the values added (32-bit pass)
-    for (int d = wv / JW; d < nd; d += WG / 64 / JW) {
-        // one descriptor per wave: its words are uniform (scalar registers)
-        uint4 de = desc[d];
-        de.x = __builtin_amdgcn_readfirstlane(de.x);
-        de.y = __builtin_amdgcn_readfirstlane(de.y);
-        de.z = __builtin_amdgcn_readfirstlane(de.z);
-        de.w = __builtin_amdgcn_readfirstlane(de.w);
-        if (de.z >> 31) continue;
-        if (!A64 && (de.z & 0x40000000u)) { // 64-bit cells: the 64-bit pass
-            wrap = true;
-            break;
-        }
+    // The wave's share of chunk d: cells j * 64 .. j * 64 + 63 of its (y, z) planes, another
+    // j with each chunk, so that the chunks of a block (one large, the others slivers of
+    // neighbouring tiles' windows) spread evenly over the waves.
+    const int lj = (wv + lane / DW) % OWN_J;
+    unsigned long long todo = __builtin_amdgcn_ballot_w64(
+        live && lane % DW == wv / OWN_J && lj * 64 < (int)((((dl.z >> 16) & 15u) + 1u) * (((dl.z >> 20) & 15u) + 1u)));
+    if (!A64 && __builtin_amdgcn_ballot_w64(live && (dl.z & 0x40000000u))) { // 64-bit cells: the 64-bit pass
+        wrap = true;
+        todo = 0ull;
+    }
+    for (; todo; todo &= todo - 1ull) {
+        const int d = __builtin_ctzll(todo);
+        const uint4 de = make_uint4(__builtin_amdgcn_readlane(dl.x, d), __builtin_amdgcn_readlane(dl.y, d),
+                                    __builtin_amdgcn_readlane(dl.z, d), __builtin_amdgcn_readlane(dl.w, d));
         const unsigned* __restrict ch = g.arena + ((unsigned long long)de.x | ((unsigned long long)de.y << 32));
         const int ox = de.z & 15, oy = (de.z >> 4) & 15, oz = (de.z >> 8) & 15;
         const int mx = ((de.z >> 12) & 15) + 1, my = ((de.z >> 16) & 15) + 1, mz = ((de.z >> 20) & 15) + 1;
         const int e2 = (int)(de.w >> 16);
         const unsigned e12 = (de.w & 0xFFFFu) * (unsigned)e2; // arena stride of an x plane
         const int myz = my * mz;
+        const int j = (wv + d / DW) % OWN_J;
         // p -> (ly, lz) by multiplication with a rounded reciprocal: exact here because
         // p < 256 keeps the rounding error below the 0.5/mz margin of (p + 0.5)
         const float rmz = 1.0f / (float)mz;
-        for (int j = JW > 1 ? wv % JW : 0; j < OWN_J && j * 64 < myz; j += JW) {
-            const int pl = lane + 64 * j;
-            const bool pv = pl < myz;
-            const int ly = (int)(((float)pl + 0.5f) * rmz), lz = pl - ly * mz;
-            unsigned po = pv ? (unsigned)(ly * e2 + lz) : 0u; // arena offset in the plane
-            // (opaque: the address of plane x stays x * e12 + po, a scalar product and one
-            // add, instead of being refactored into a multiply per load)
-            asm volatile("" : "+v"(po));
-            const int la = ox * OB * OB + (oy + ly) * OB + oz + lz; // LDS cell of x plane 0
-            // lanes past the plane sit the chunk out; inside, every condition is uniform
-            // (scalar branches): the values are added unconditionally (zeros included),
-            // which costs less than masking each add
-            if (!pv) continue;
-            if (A64 && (de.z & 0x40000000u)) {
-                // a window of 64-bit cells (two arena words per cell)
-                wrap = true;
-                for (int x0 = 0; x0 < mx; x0 += U) {
-                    unsigned long long v[U];
-#pragma unroll
-                    for (int u = 0; u < U; u++) {
-                        const unsigned xu = (unsigned)min(x0 + u, mx - 1);
-                        v[u] = *(const unsigned long long*)((const char*)ch + (xu * e12 + po) * 8u);
-                    }
-#pragma unroll
-                    for (int u = 0; u < U; u++)
-                        if (x0 + u < mx) atomicAdd(&acc[la + (x0 + u) * OB * OB], (ACC)v[u]);
-                }
-                continue;
-            }
+        const int pl = lane + 64 * j;
+        const bool pv = pl < myz;
+        const int ly = (int)(((float)pl + 0.5f) * rmz), lz = pl - ly * mz;
+        unsigned po = pv ? (unsigned)(ly * e2 + lz) : 0u; // arena offset in the plane
+        // (opaque: the address of plane x stays x * e12 + po, a scalar product and one
+        // add, instead of being refactored into a multiply per load)
+        asm volatile("" : "+v"(po));
+        const int la = ox * OB * OB + (oy + ly) * OB + oz + lz; // LDS cell of x plane 0
+        // lanes past the plane sit the chunk out; inside, every condition is uniform
+        // (scalar branches): the values are added unconditionally (zeros included),
+        // which costs less than masking each add
+        if (!pv) continue;
+        if (A64 && (de.z & 0x40000000u)) {
+            // a window of 64-bit cells (two arena words per cell)
+            wrap = true;
             for (int x0 = 0; x0 < mx; x0 += U) {
-                unsigned v[U];
+                unsigned long long v[U];
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    // every slot loads (planes past the chunk's last load that one again)
-                    // so that the U loads issue together.  A chunk lies in a window of at
-                    // most DEP_MAXCH owner blocks: byte offsets from its first cell fit 32
-                    // bits (also for 64-bit cells)
                     const unsigned xu = (unsigned)min(x0 + u, mx - 1);
-                    v[u] = *(const unsigned*)((const char*)ch + (xu * e12 + po) * 4u);
+                    v[u] = *(const unsigned long long*)((const char*)ch + (xu * e12 + po) * 8u);
                 }
-                if (x0 + U <= mx) {
 #pragma unroll
-                    for (int u = 0; u < U; u++) {
+                for (int u = 0; u < U; u++)
+                    if (x0 + u < mx) atomicAdd(&acc[la + (x0 + u) * OB * OB], (ACC)v[u]);
+            }
+            continue;
+        }
+        // NU planes from x0 on.  Every slot loads (planes past the chunk's last load that
+        // one again) so that the loads issue together.  A chunk lies in a window of at
+        // most DEP_MAXCH owner blocks: byte offsets from its first cell fit 32 bits (also
+        // for 64-bit cells)
+        auto planes = [&](auto nu, int x0) {
+            constexpr int NU = decltype(nu)::value;
+            unsigned v[NU];
+#pragma unroll
+            for (int u = 0; u < NU; u++) {
+                const unsigned xu = (unsigned)min(x0 + u, mx - 1);
+                v[u] = *(const unsigned*)((const char*)ch + (xu * e12 + po) * 4u);
+            }
+            if (x0 + NU <= mx) {
+#pragma unroll
+                for (int u = 0; u < NU; u++) {
+                    atomicAdd(&acc[la + (x0 + u) * OB * OB], (ACC)v[u]);
+                    if constexpr (!A64) added += v[u];
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < NU; u++)
+                    if (x0 + u < mx) {
                         atomicAdd(&acc[la + (x0 + u) * OB * OB], (ACC)v[u]);
                         if constexpr (!A64) added += v[u];
                     }
-                } else {
-#pragma unroll
-                    for (int u = 0; u < U; u++)
-                        if (x0 + u < mx) {
-                            atomicAdd(&acc[la + (x0 + u) * OB * OB], (ACC)v[u]);
-                            if constexpr (!A64) added += v[u];
-                        }
-                }
             }
+        };
+        if (mx <= 2) {
+            planes(std::integral_constant<int, 2>{}, 0);
+        } else if (mx <= 4) {
+            planes(std::integral_constant<int, 4>{}, 0);
+        } else {
+            for (int x0 = 0; x0 < mx; x0 += U) planes(std::integral_constant<int, U>{}, x0);
         }
     }
     if (wrap) *s_redo = 1;
@@ -935,24 +949,29 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
 template <int WG> __global__ __launch_bounds__(WG) void k_deposit_owner(OwnerArgs g) {
     if (g.ctl[HGPM_DEP_CTL]) return; // every block in k_deposit_owner64
     __shared__ unsigned acc[OB * OB * OB];
-    __shared__ uint4 desc[HGPM_DEP_SLOTS];
-    __shared__ int s_n, s_redo;
+    __shared__ int s_redo;
     __shared__ unsigned long long s_dif;
-    owner_block<unsigned, OWN_U32, WG>(g, (int)xcd_remap(blockIdx.x, gridDim.x), acc, desc, &s_n, &s_redo, &s_dif);
+    owner_block<unsigned, OWN_U32, WG>(g, (int)xcd_remap(blockIdx.x, gridDim.x), acc, &s_redo, &s_dif);
 }
 // In 64-bit cells: the blocks handed over, or every block on that route (a deposit with
 // many dense blocks, late in a run: the 32-bit attempt would be wasted on them).  A
-// workgroup per block: the empty ones cost 56 us at 1024^3 (262144 of them), and dense
-// blocks, which lie together, spread over the chip (one workgroup scanning 256 blocks'
-// marks and summing the marked ones in turn took 0.3 ms a step late in a 512^3 run).
-__global__ __launch_bounds__(OWN_NT) void k_deposit_owner64(OwnerArgs g) {
-    const int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
-    if (!g.ctl[HGPM_DEP_CTL] && !(g.wide_blk[blk] & 2)) return;
+// workgroup takes up to OWN_64B blocks, one in gridDim.x: mostly none is marked, and a
+// workgroup per block then cost 144 us at 1024^3 (262144 of them; now 20 us).  Dense blocks
+// lie together and so fall to different workgroups (one workgroup taking 256 neighbouring
+// blocks took 0.3 ms a step late in a 512^3 run, against 0.06).
+constexpr int OWN_64B = 8;
+__global__ __launch_bounds__(OWN_NT) void k_deposit_owner64(OwnerArgs g, int nall) {
     __shared__ unsigned long long acc[OB * OB * OB];
-    __shared__ uint4 desc[HGPM_DEP_SLOTS];
-    __shared__ int s_n, s_redo;
+    __shared__ int s_redo;
     __shared__ unsigned long long s_dif;
-    owner_block<unsigned long long, OWN_U64, OWN_NT>(g, blk, acc, desc, &s_n, &s_redo, &s_dif);
+    const int first = (int)xcd_remap(blockIdx.x, gridDim.x);
+    const int mine = first + (int)(threadIdx.x & 63) * (int)gridDim.x; // of the lane
+    const bool has = (threadIdx.x & 63) < OWN_64B && mine < nall;
+    unsigned long long todo =
+        __builtin_amdgcn_ballot_w64(has && (g.ctl[HGPM_DEP_CTL] || (g.wide_blk[mine] & 2)));
+    for (; todo; todo &= todo - 1ull) // the same blocks in every wave; ends at a barrier
+        owner_block<unsigned long long, OWN_U64, OWN_NT>(g, first + __builtin_ctzll(todo) * (int)gridDim.x, acc, &s_redo,
+                                                         &s_dif);
 }
 
 // The end of a deposit: the control words of the next one (the other of two sets, used in
@@ -1808,7 +1827,7 @@ void launch_deposit_owner(int ng, long long* rho, float* rhof, const DepositBuff
     const unsigned nall = (unsigned)nblk * (unsigned)b.nbox;
     if (nall <= OWN_FEW) k_deposit_owner<1024><<<nall, 1024, 0, s>>>(g);
     else k_deposit_owner<OWN_NT><<<nall, OWN_NT, 0, s>>>(g);
-    k_deposit_owner64<<<nall, OWN_NT, 0, s>>>(g);
+    k_deposit_owner64<<<(nall + OWN_64B - 1) / OWN_64B, OWN_NT, 0, s>>>(g, (int)nall);
 }
 void launch_deposit_deferred(const PosPackH* pos, int64_t n, int ng, float mass, long long* rho,
                              const DepositBuffers& b, hipStream_t s) {

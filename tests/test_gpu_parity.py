@@ -152,6 +152,31 @@ def test_deposit_dense_cells_take_the_wide_route(hg, orc, np_):
                 assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("ng,dense", [(32, 3), (64, 13), (64, 64), (96, 29), (96, 2)])
+def test_deposit_dense_blocks_spread(hg, orc, ng, dense):
+    """A workgroup of the 64-bit owner pass takes up to eight owner blocks, the marked ones
+    of every gridDim-th: none, several or all of its blocks dense (512 particles on one
+    lattice point inside the block), in three deposits in turn (marks kept, the route of a
+    mostly dense grid), bit-exact against the oracle."""
+    case(f"deposit dense blocks ng={ng} dense={dense}")
+    rng = np.random.default_rng(ng + dense)
+    nb = ng // 16
+    with mk(hg, ng) as m:
+        cell, off = lattice_split(rng, ng, ng, 0.0)
+        for b in rng.choice(nb ** 3, dense, replace=False):
+            org = 16 * np.array([b // (nb * nb), b // nb % nb, b % nb])
+            inside = ((cell >= org + 4) & (cell < org + 12)).all(axis=1)  # 8^3 lattice particles
+            cell[inside] = org + 7
+            off[inside] = 0.0
+        m.set_particles_split(cell, off, np.zeros((m.N, 3), np.float32))
+        ref = orc.cic_split(ng, cell, off)
+        for _ in range(3):
+            m.cic()
+            assert np.array_equal(m.get_density(), ref)
+            # a tile's 64-bit window marks every block that it touches
+            assert dense <= m.get_tunable("deposit_owner_redo") <= min(27 * dense, nb ** 3)
+
+
 def test_deposit_owner_sum_wraps_32_bits(hg, orc):
     """The owner pass sums chunks in 32-bit LDS cells and hands a block to the 64-bit
     owner pass when a cell's sum reaches 2^32 units.  Eight Lagrangian tiles each pile
