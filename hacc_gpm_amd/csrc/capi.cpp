@@ -56,6 +56,11 @@ struct hgpm_ctx {
     unsigned long long* ctl = nullptr; // two sets of deposit control words, used in turn
     int set_words = 0;                 // words of a set: control words, mass partial sums per box
     int set_next = 0;                  // the set of the next deposit; the other is the last one's
+    // the force components' grids (FP64)
+    ForceF64 force64() const {
+        const double* g = (const double*)grad64;
+        return {{g + 2 * G, g + 3 * G, g}};
+    }
     unsigned long long* last_ctl() const { return ctl + (size_t)(set_next ^ 1) * set_words; }
     unsigned long long* last_mass() const { return last_ctl() + HGPM_DEP_CTL + 1; }
     // deposit arena route (k_particles.hip): window arena, per-owner-block chunk slots
@@ -73,8 +78,9 @@ struct hgpm_ctx {
     float2 *twf = nullptr, *twr = nullptr, *twf_ic = nullptr, *twr_ic = nullptr; // _ic: length np, shared when np = ng
     float* hs = nullptr; // sin^2(pi m/ng), the Green's function's per-axis terms
     // FP64 plain path
-    double *pos64 = nullptr, *vel64 = nullptr, *grad64 = nullptr;
-    double2* grid64 = nullptr;
+    double *pos64 = nullptr, *vel64 = nullptr;
+    double2 *grid64 = nullptr, *grad64 = nullptr; // grad64: a work grid, then F_x and F_y; F_z over the work grid
+    double2* modes64 = nullptr;                   // cos, sin of the grid's wavenumbers
     double2 *tw64 = nullptr, *tw64_ic = nullptr;
     // P(k)
     double *pk_partial = nullptr, *pk_sums = nullptr, *pk_win = nullptr;
@@ -367,22 +373,11 @@ int f64_deposit(hgpm_ctx* c, const double* pos) {
 int f64_solve(hgpm_ctx* c) {
     int rc = fft3d_f64(c, c->fft, c->grid64, c->tw64, -1);
     if (rc) return rc;
-    {
-        Timed t(c, "f64_copy_to_grad");
-        launch_f64_copy_to_grad(c->grid64, c->grad64, c->G, c->st);
-    }
-    for (int d = 0; d < 3; d++) {
-        {
-            Timed t(c, "f64_kspace");
-            launch_f64_kspace(c->grid64, c->grad64, c->ng, d, c->st);
-        }
-        rc = fft3d_f64(c, c->fft, c->grid64, c->tw64, +1);
-        if (rc) return rc;
-        {
-            Timed t(c, "f64_real_to_grad");
-            launch_f64_real_to_grad(c->grid64, c->grad64, c->G, d, c->st);
-        }
-    }
+    Timed t(c, "f64_force");
+    const ForceF64 F = c->force64();
+    for (int d = 0; d < 3; d++) // z last: over the density's modes
+        c->fft->force_f64(c->grid64, d < 2 ? c->grad64 : c->grid64, const_cast<double*>(F.f[d]), c->tw64, c->modes64, d,
+                          c->st);
     LAUNCHCHK(c);
     return HGPM_OK;
 }
@@ -577,8 +572,16 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
         if ((rc = dalloc(c, &c->pos64, sizeof(double) * 3 * N, "pos64")) ||
             (rc = dalloc(c, &c->vel64, sizeof(double) * 3 * N, "vel64")) ||
             (rc = dalloc(c, &c->grid64, sizeof(double2) * G, "grid64")) ||
-            (rc = dalloc(c, &c->grad64, grad_bytes, "grad64")))
+            (rc = dalloc(c, &c->grad64, grad_bytes, "grad64")) ||
+            (rc = dalloc(c, &c->modes64, sizeof(double2) * p->ng, "modes64")))
             return bail(rc);
+        std::vector<double2> modes(p->ng);
+        const double d = (2 * HGPM_PI_D) / (double)p->ng;
+        for (int i = 0; i < p->ng; i++) modes[i] = make_double2(cos(d * i), sin(d * (i > p->ng / 2 - 1 ? i - p->ng : i)));
+        if (hipMemcpy(c->modes64, modes.data(), sizeof(double2) * p->ng, hipMemcpyHostToDevice) != hipSuccess) {
+            c->err = "table upload failed";
+            return bail(HGPM_ERR_HIP);
+        }
         if ((rc = upload_twiddles<double2>(c, c->fft, &c->tw64, nullptr))) return bail(rc);
         if (c->np != c->ng) {
             if ((rc = upload_twiddles<double2>(c, c->fftic, &c->tw64_ic, nullptr))) return bail(rc);
@@ -617,7 +620,7 @@ int hgpm_destroy(hgpm_ctx* c) {
     if (!c) return HGPM_OK;
     if (c->st) (void)hipStreamSynchronize(c->st);
     void* ptrs[] = {c->pos, c->vel, c->A, c->B, c->psi, c->ctl, c->arena, c->dslots, c->dcount, c->deferred, c->wide, c->wide_slots, c->boxes, c->twf, c->twr, c->hs,
-                    c->pos64, c->vel64, c->grid64, c->grad64, c->tw64, c->pk_partial, c->pk_sums,
+                    c->pos64, c->vel64, c->grid64, c->grad64, c->modes64, c->tw64, c->pk_partial, c->pk_sums,
                     c->pk_win, c->flag};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
@@ -953,7 +956,7 @@ int generate_ic_from(hgpm_ctx* c, const double* d_ipk, int ipk_bins, double ipk_
     } else {
         double velA = a - deltaT * 0.5;
         double velMul = velA * velA * dot_delta * fscal;
-        double2* amp = (double2*)c->grad64;
+        double2* amp = c->grad64;
         launch_ic_noise_f64(amp, np, seed, c->st);
         if ((rc = fft3d_f64(c, c->fftic, amp, c->tw64_ic, -1))) return rc;
         launch_ic_scale_f64(amp, np, d_ipk, ipk_bins, ipk_k_delta, c->p.rl, c->st);
@@ -1124,7 +1127,7 @@ int hgpm_get_force_f64(hgpm_ctx* c, double* f) {
     int rc = dalloc(c, &tmp, sizeof(double) * 3 * c->G, "staging");
     if (rc) return rc;
     c->bytes -= sizeof(double) * 3 * c->G;
-    launch_f64_grad_to_force(c->grad64, tmp, c->G, c->st);
+    launch_f64_force_out(c->force64(), tmp, c->G, c->st);
     LAUNCHCHK(c);
     rc = to_host(c, {{f, tmp, sizeof(double) * 3 * c->G}});
     (void)hipFree(tmp);
@@ -1142,7 +1145,7 @@ int hgpm_update_velocities(hgpm_ctx* c, double deltaT, double fscal) {
                            c->boxes_valid ? c->boxes : nullptr, c->nbox, c->st);
     } else {
         Timed t(c, "f64_icic");
-        launch_f64_icic(c->pos64, c->vel64, c->grad64, c->N, c->ng, deltaT, fscal, c->st);
+        launch_f64_icic(c->pos64, c->vel64, c->force64(), c->N, c->ng, deltaT, fscal, c->st);
     }
     LAUNCHCHK(c);
     return HGPM_OK;

@@ -88,6 +88,39 @@ __global__ __launch_bounds__(NTC) void k_cols_c2c(V* __restrict d, const V* __re
         [&](int, int, int n, int c, V v) { d[base + n * stride + c] = v; }, lds, tw);
 }
 
+// FP64 force of one component, from the density's modes: the reference multiplies rho^ by
+// the component's factor in a pass of its own and takes the real part of the inverse
+// transform in another (kspace_solve_gradient, getRealGrid); here the z pass multiplies as
+// it loads (rho^ stays for the next component; w may be rho^ itself for the last one: a
+// workgroup has loaded its rows before it stores them) and the x pass stores the real
+// part only.  All three passes are bound by memory.
+template <int RC>
+__global__ __launch_bounds__(NT) void k_rows_force(const double2* rho, double2* w, const double2* __restrict tw,
+                                                   const double2* __restrict modes, int dim) {
+    __shared__ double2 lds[lds_elems<N, RC>()];
+    const size_t row0 = (size_t)blockIdx.x * RC;
+    fft_tile<double2, N, RC, NT, +1, false, true>(
+        [&](int, int, int n, int c) {
+            const size_t row = row0 + c;
+            const double2 q = rho[row * N + n], X = modes[row / N], Y = modes[row % N], Z = modes[n];
+            // Green's function; the mean's mode (where it is infinite) is dropped
+            const double G = (0.5 / ((double)N * N * N)) / (X.x + Y.x + Z.x - 3.0);
+            const double f = row + n == 0 ? 0.0 : -(dim == 0 ? X.y : dim == 1 ? Y.y : Z.y) * G;
+            return row + n == 0 ? make_double2(0.0, 0.0) : make_double2(-f * q.y, f * q.x);
+        },
+        [&](int, int, int n, int c, double2 v) { w[(row0 + c) * N + n] = v; }, lds, tw);
+}
+template <int CC, int NTC>
+__global__ __launch_bounds__(NTC) void k_cols_force(const double2* __restrict w, double* __restrict out,
+                                                    const double2* __restrict tw) {
+    __shared__ double2 lds[lds_elems<N, CC>()];
+    const size_t plane = (size_t)N * N;
+    const size_t base = col_base<CC>((int)xcd_remap(blockIdx.x, gridDim.x), 0, N, plane);
+    fft_tile<double2, N, CC, NTC, +1, false, false>(
+        [&](int, int, int n, int c) { return w[base + n * plane + c]; },
+        [&](int, int, int n, int c, double2 v) { out[base + n * plane + c] = v.x; }, lds, tw);
+}
+
 // Streaming: where one workgroup fills a CU (large tiles: its LDS or its registers leave no
 // room for a second one) its loads, transforms and stores would follow one another.  The
 // x pass of the solve, which transforms twice per tile, is then one workgroup per CU that
@@ -478,6 +511,12 @@ void pass_f32(float2* d, int axis, int dir, const float2* tw, int variant, hipSt
     });
 }
 // Column pass over nbox half-spectrum grids N x N x HZ.
+void force_f64(const double2* rho, double2* w, double* out, const double2* tw, const double2* modes, int dim,
+               hipStream_t s) {
+    k_rows_force<rc64()><<<(unsigned)((size_t)N * N / rc64()), NT, 0, s>>>(rho, w, tw, modes, dim);
+    cols_launch<double2, cc64(), 512>(w, 1, +1, tw, N, (size_t)N * N, s);
+    k_cols_force<cc64(), 512><<<(unsigned)((size_t)N * N / cc64()), 512, 0, s>>>(w, out, tw);
+}
 void pass_half(float2* d, int axis, int dir, const float2* tw, int variant, int nbox, hipStream_t s) {
     with_variant(variant, [&](auto vc) {
         constexpr int v = decltype(vc)::value;
@@ -548,7 +587,7 @@ extern const FftOps HGPM_CAT(HGPM_CAT(fft_ops_, HGPM_FFT_N), _alt) = {
 #else
 extern const FftOps HGPM_CAT(fft_ops_, HGPM_FFT_N) = {
 #endif
-    N, Plan<N>::S, NVAR, VDEF, variant_mask(), twiddles, pass_f32, pass_f64,
+    N, Plan<N>::S, NVAR, VDEF, variant_mask(), twiddles, pass_f32, pass_f64, force_f64,
     HZ, NPH, pass_half, fwd_z_r2c, x_psi, inv_z_c2r_real, fwd_z_r2c_real, ic_x, ic_y, ic_z,
 };
 } // namespace hgpm

@@ -1,14 +1,17 @@
-// k_fp64.hip — the plain FP64 path: one kernel per reference kernel of the serial
-// step, every quantity in FP64 (double3 positions and velocities, complex128 grid,
-// double4 gradient grid).  It is the "FP64 plain GPU path" the FP32 engine is
-// measured against, structured as the reference's default build
+// k_fp64.hip — the plain FP64 path: every quantity in FP64 (double3 positions and
+// velocities, complex128 grids).  It is the "FP64 plain GPU path" the FP32 engine is
+// measured against, the serial step of the reference's default build
 // (src/haccgpm.hpp:67-72) with grid_t = complex128:
-//   UpdatePosKernel            src/pm_actions/cuda/update_positions_pm.cu:3-20
-//   memset + CICKernel         src/pm_actions/cuda/cic_pm.cu:46-87,142-147
-//   copyGridToFloat4           src/pm_solver/cuda/combine.cu:21-34
-//   kspace_solve_gradient      src/pm_solver/cuda/kspace_solver.cu:55-90 (+ calcGreens)
-//   getRealGrid                src/initial_conditions/cuda/transform_density_field_initializer.cu:14-28
-//   ICICKernel                 src/pm_actions/cuda/icic_pm.cu:72-127
+//   k_drift   UpdatePosKernel       src/pm_actions/cuda/update_positions_pm.cu:3-20
+//   k_cic     memset + CICKernel    src/pm_actions/cuda/cic_pm.cu:46-87,142-147
+//   FftOps.force_f64 (k_rows_force, k_cols_force) kspace_solve_gradient,
+//             src/pm_solver/cuda/kspace_solver.cu:55-90 (+ calcGreens), and its real part,
+//             getRealGrid, src/initial_conditions/cuda/transform_density_field_initializer.cu:14-28
+//   k_icic    ICICKernel            src/pm_actions/cuda/icic_pm.cu:72-127
+// The gather reads the three force components from grids of their own (copyGridToFloat4,
+// src/pm_solver/cuda/combine.cu:21-34, joins them).  A step of 128^3 went from 0.62 ms
+// (a pass for each component's modes, one for its real part, eight atomics per particle)
+// to 0.33 ms.
 #include "common.h"
 #include "internal.h"
 
@@ -36,77 +39,64 @@ __global__ void k_zero(double* __restrict p, size_t n) {
     for (; i < n; i += st) p[i] = 0.0;
 }
 
-__global__ void k_cic(const double* __restrict pos, int64_t n, int ng, double mass, double2* __restrict grid) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double X = pos[3 * i], Y = pos[3 * i + 1], Z = pos[3 * i + 2];
-    int ci = (int)X, cj = (int)Y, ck = (int)Z;
-    double fx = X - ci, fy = Y - cj, fz = Z - ck;
-    // positions are wrapped into [0, ng); keep the cell index in range for any input
-    ci = ((ci % ng) + ng) % ng;
-    cj = ((cj % ng) + ng) % ng;
-    ck = ((ck % ng) + ng) % ng;
+// cells per axis of the 8 corners: c[d][0] the particle's (kept in range for any input;
+// positions are wrapped into [0, ng)), c[d][1] the next one, periodic
+__device__ __forceinline__ void corners(double X, double Y, double Z, int ng, int c[3][2], double f[3]) {
+    const double x[3] = {X, Y, Z};
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        int i = (int)x[d];
+        f[d] = x[d] - i;
+        if ((unsigned)i >= (unsigned)ng) i = ((i % ng) + ng) % ng;
+        c[d][0] = i;
+        c[d][1] = i + 1 == ng ? 0 : i + 1;
+    }
+}
+
+// Bound by the FP64 atomics on L2 (88 G/s).  Particles are in lattice order, z fastest:
+// where the next lane's particle lies in the next cell of the same row, this lane's four
+// upper corners are that lane's lower ones and are added by it, four atomics per particle
+// instead of eight: 0.194 -> 0.098 ms at 128^3.
+__global__ __launch_bounds__(BS) void k_cic(const double* __restrict pos, int64_t n, int ng, double mass,
+                                            double2* __restrict grid) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const bool valid = i < n;
+    const int64_t j = valid ? i : 0;
+    int c[3][2];
+    double f[3];
+    corners(pos[3 * j], pos[3 * j + 1], pos[3 * j + 2], ng, c, f);
+    // row (x, y) of the cell, < 2^20, -1 for no particle
+    const int row = valid ? c[0][0] * ng + c[1][0] : -1;
+    const int prow = __shfl_up(row, 1, 64), pz = __shfl_up(c[2][1], 1, 64);
+    const int nrow = __shfl_down(row, 1, 64), nz = __shfl_down(c[2][0], 1, 64);
+    const bool take = lane > 0 && valid && prow == row && pz == c[2][0]; // the previous lane's upper corners
+    const bool give = lane < 63 && valid && nrow == row && nz == c[2][1];
 #pragma unroll
     for (int x = 0; x < 2; x++)
 #pragma unroll
-        for (int y = 0; y < 2; y++)
-#pragma unroll
-            for (int z = 0; z < 2; z++) {
-                double dx = x ? fx : 1.0 - fx;
-                double dy = y ? fy : 1.0 - fy;
-                double dz = z ? fz : 1.0 - fz;
-                int64_t id = gidx(ng, (ci + x) % ng, (cj + y) % ng, (ck + z) % ng);
-                unsafeAtomicAdd(&grid[id].x, dx * dy * dz * mass);
+        for (int y = 0; y < 2; y++) {
+            const double dx = x ? f[0] : 1.0 - f[0];
+            const double dy = y ? f[1] : 1.0 - f[1];
+            double lo = dx * dy * (1.0 - f[2]) * mass;
+            const double up = dx * dy * f[2] * mass;
+            const double prev = __shfl_up(up, 1, 64);
+            if (take) lo += prev;
+            if (valid) {
+                const int64_t r = gidx(ng, c[0][x], c[1][y], 0);
+                unsafeAtomicAdd(&grid[r + c[2][0]].x, lo);
+                if (!give) unsafeAtomicAdd(&grid[r + c[2][1]].x, up);
             }
+        }
 }
 
-__global__ void k_copy_to_grad(const double2* __restrict grid, double4* __restrict grad, int64_t g3) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g3) return;
-    double2 c = grid[i];
-    grad[i] = make_double4(0.0, 0.0, c.x, c.y);
-}
-
-__global__ void k_kspace(double2* __restrict grid, const double4* __restrict grad, int ng, int dim) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t g3 = (int64_t)ng * ng * ng;
-    if (i >= g3) return;
-    int ix = (int)(i / ((int64_t)ng * ng)), iy = (int)((i / ng) % ng), iz = (int)(i % ng);
-    double2 out = make_double2(0.0, 0.0);
-    if ((ix | iy | iz) != 0) {
-        const double d = (2 * HGPM_PI) / (double)ng;
-        double G = (0.5 / ((double)ng * ng * ng)) / (cos(d * ix) + cos(d * iy) + cos(d * iz) - 3.0);
-        int m = dim == 0 ? ix : (dim == 1 ? iy : iz);
-        if (m > ng / 2 - 1) m -= ng;
-        double c = -sin(d * m) * G;
-        double4 a = grad[i];
-        out = make_double2(-c * a.w, c * a.z);
-    }
-    grid[i] = out;
-}
-
-__global__ void k_real_to_grad(const double2* __restrict grid, double4* __restrict grad, int64_t g3, int dim) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g3) return;
-    double4 a = grad[i];
-    double v = grid[i].x;
-    if (dim == 0) a.x = v;
-    else if (dim == 1) a.y = v;
-    else a.z = v;
-    grad[i] = a;
-}
-
-__global__ void k_icic(const double* __restrict pos, double* __restrict vel, const double4* __restrict grad,
-                       int64_t n, int ng, double deltaT, double fscal) {
+__global__ void k_icic(const double* __restrict pos, double* __restrict vel, const hgpm::ForceF64 F, int64_t n, int ng,
+                       double deltaT, double fscal) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
-    double X = pos[3 * i], Y = pos[3 * i + 1], Z = pos[3 * i + 2];
-    int ci = (int)X, cj = (int)Y, ck = (int)Z;
-    double fx = X - ci, fy = Y - cj, fz = Z - ck;
-    // positions are wrapped into [0, ng); keep the cell index in range for any input
-    ci = ((ci % ng) + ng) % ng;
-    cj = ((cj % ng) + ng) % ng;
-    ck = ((ck % ng) + ng) % ng;
+    int c[3][2];
+    double f[3];
+    corners(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], ng, c, f);
     double dv0 = 0, dv1 = 0, dv2 = 0;
 #pragma unroll
     for (int x = 0; x < 2; x++)
@@ -114,14 +104,14 @@ __global__ void k_icic(const double* __restrict pos, double* __restrict vel, con
         for (int y = 0; y < 2; y++)
 #pragma unroll
             for (int z = 0; z < 2; z++) {
-                double dx = x ? fx : 1.0 - fx;
-                double dy = y ? fy : 1.0 - fy;
-                double dz = z ? fz : 1.0 - fz;
-                double4 g = grad[gidx(ng, (ci + x) % ng, (cj + y) % ng, (ck + z) % ng)];
+                double dx = x ? f[0] : 1.0 - f[0];
+                double dy = y ? f[1] : 1.0 - f[1];
+                double dz = z ? f[2] : 1.0 - f[2];
+                const int64_t at = gidx(ng, c[0][x], c[1][y], c[2][z]);
                 double mul = dx * dy * dz * deltaT * fscal;
-                dv0 += mul * g.x;
-                dv1 += mul * g.y;
-                dv2 += mul * g.z;
+                dv0 += mul * F.f[0][at];
+                dv1 += mul * F.f[1][at];
+                dv2 += mul * F.f[2][at];
             }
     vel[3 * i] += dv0;
     vel[3 * i + 1] += dv1;
@@ -140,13 +130,11 @@ __global__ void k_density_to_real(const double2* __restrict g, double* __restric
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < g3) out[i] = g[i].x;
 }
-__global__ void k_grad_to_force(const double4* __restrict g, double* __restrict out, int64_t g3) {
+__global__ void k_force_out(const hgpm::ForceF64 F, double* __restrict out, int64_t g3) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= g3) return;
-    double4 a = g[i];
-    out[3 * i] = a.x;
-    out[3 * i + 1] = a.y;
-    out[3 * i + 2] = a.z;
+#pragma unroll
+    for (int d = 0; d < 3; d++) out[3 * i + d] = F.f[d][i];
 }
 } // namespace
 
@@ -163,18 +151,9 @@ void launch_f64_cic(const double* pos, int64_t n, int ng, double mass, double2* 
     launch_f64_zero((double*)grid, (size_t)2 * ng * ng * ng, s);
     if (n) k_cic<<<nblk(n), BS, 0, s>>>(pos, n, ng, mass, grid);
 }
-void launch_f64_copy_to_grad(const double2* grid, double* grad4, int64_t g3, hipStream_t s) {
-    k_copy_to_grad<<<nblk(g3), BS, 0, s>>>(grid, (double4*)grad4, g3);
-}
-void launch_f64_kspace(double2* grid, const double* grad4, int ng, int dim, hipStream_t s) {
-    k_kspace<<<nblk((int64_t)ng * ng * ng), BS, 0, s>>>(grid, (const double4*)grad4, ng, dim);
-}
-void launch_f64_real_to_grad(const double2* grid, double* grad4, int64_t g3, int dim, hipStream_t s) {
-    k_real_to_grad<<<nblk(g3), BS, 0, s>>>(grid, (double4*)grad4, g3, dim);
-}
-void launch_f64_icic(const double* pos, double* vel, const double* grad4, int64_t n, int ng, double deltaT,
+void launch_f64_icic(const double* pos, double* vel, const ForceF64& f, int64_t n, int ng, double deltaT,
                      double fscal, hipStream_t s) {
-    if (n) k_icic<<<nblk(n), BS, 0, s>>>(pos, vel, (const double4*)grad4, n, ng, deltaT, fscal);
+    if (n) k_icic<<<nblk(n), BS, 0, s>>>(pos, vel, f, n, ng, deltaT, fscal);
 }
 void launch_f64_fold(double* pos, int64_t n, int ng, hipStream_t s) {
     if (n) k_fold<<<nblk(3 * n), BS, 0, s>>>(pos, 3 * n, ng);
@@ -182,7 +161,7 @@ void launch_f64_fold(double* pos, int64_t n, int ng, hipStream_t s) {
 void launch_f64_density_to_real(const double2* grid, double* out, int64_t g3, hipStream_t s) {
     k_density_to_real<<<nblk(g3), BS, 0, s>>>(grid, out, g3);
 }
-void launch_f64_grad_to_force(const double* grad4, double* out, int64_t g3, hipStream_t s) {
-    k_grad_to_force<<<nblk(g3), BS, 0, s>>>((const double4*)grad4, out, g3);
+void launch_f64_force_out(const ForceF64& f, double* out, int64_t g3, hipStream_t s) {
+    k_force_out<<<nblk(g3), BS, 0, s>>>(f, out, g3);
 }
 } // namespace hgpm

@@ -624,6 +624,40 @@ def test_fused_drift_large_moves(hg, orc, ng, np_, dist):
         assert np.array_equal(c2, cref) and np.array_equal(o2, oref)
 
 
+@pytest.mark.parametrize("ng,np_,kind", [(32, 32, "lattice"), (96, 32, "lattice"), (64, 32, "rows"), (32, 32, "shuffled"),
+                                         (128, 64, "lattice"), (64, 64, "one cell")])
+def test_deposit_fp64_neighbours(hg, orc, ng, np_, kind):
+    """The FP64 deposit adds a lane's upper corners in the next lane where that particle lies
+    in the next cell of the row: lattices where all, some or no lanes do (rows that end on
+    the seam or in the middle of a wave), every particle in the next cell of the one before
+    (63 of 64 lanes, over the seam), any order, one cell.  A cell is a sum of M terms of one
+    sign in any order, here and in the oracle: within 2 M roundings (2^-53) of each other,
+    and 8 for the weights."""
+    case(f"deposit fp64 ng={ng} np={np_} {kind}")
+    rng = np.random.default_rng(ng + np_)
+    n = np_ ** 3
+    i = np.arange(n)
+    x = np.stack([i // (np_ * np_), i // np_ % np_, i % np_], 1) * (ng / np_) + rng.normal(0.3, 0.15, (n, 3))
+    if kind == "rows":
+        x = np.stack([i // ng // ng, i // ng % ng, i % ng], 1) + rng.random((n, 3))
+    elif kind == "shuffled":
+        rng.shuffle(x)
+    elif kind == "one cell":
+        x = 17.0 + rng.random((n, 3))
+    x %= ng
+    with mk(hg, ng, np_, prec=1) as m:
+        m.set_particles_f64(x, np.zeros_like(x))
+        m.cic()
+        got = m.get_density_f64()
+    ref = orc.cic_f64(ng, x, (ng / np_) ** 3)
+    cells = np.floor(x).astype(np.int64)
+    near = np.zeros((ng,) * 3, np.int64)
+    for c in range(8):
+        d = (cells + np.array([c >> 2, c >> 1 & 1, c & 1])) % ng
+        np.add.at(near, tuple(d.T), 1)
+    assert (np.abs(got.reshape(near.shape) - ref) <= (near + 4) * 2.0 ** -52 * ref).all()
+
+
 def test_fp64_kick_drift(hg, orc):
     case("kick/drift fp64 ng=32")
     ng = 32
