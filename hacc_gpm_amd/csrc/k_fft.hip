@@ -179,8 +179,8 @@ __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70
 // half spectra, k = 0..N/2, written with pitch HZ (padding written as zero).
 // rhof: see fwd_z_r2c (the owner pass wrote the same FP32 values when no tile was deferred).
 // REAL: the rows are those of the FP32 grid rhof (initial conditions' noise).
-template <int RC, bool REAL>
-__global__ __launch_bounds__(NT) void k_rows_r2c_density(const long long* __restrict rho,
+template <int RC, bool REAL, int NTX>
+__global__ __launch_bounds__(NTX) void k_rows_r2c_density(const long long* __restrict rho,
                                                          const float* __restrict rhof,
                                                          const unsigned long long* __restrict ctl,
                                                          const unsigned long long* __restrict mass,
@@ -198,7 +198,7 @@ __global__ __launch_bounds__(NT) void k_rows_r2c_density(const long long* __rest
         for (int off = 32; off > 0; off >>= 1) t += __shfl_xor(t, off, 64);
         mean = (double)(long long)t / ((double)N * N * N);
     }
-    fft_tile<float2, N, PC, NT, -1, false, true>(
+    fft_tile<float2, N, PC, NTX, -1, false, true>(
         [&](int, int, int n, int c) {
             if (f32) return make_float2(rhof[(row0 + 2 * c) * N + n], rhof[(row0 + 2 * c + 1) * N + n]);
             const double qa = (double)rho[(row0 + 2 * c) * N + n];
@@ -207,7 +207,7 @@ __global__ __launch_bounds__(NT) void k_rows_r2c_density(const long long* __rest
         },
         [&](int, int, int n, int c, float2 v) { spec[lds_slot<N, PC, true>(n, c)] = v; }, lds, tw);
     __syncthreads();
-    for (int i = threadIdx.x; i < PC * HZ; i += NT) {
+    for (int i = threadIdx.x; i < PC * HZ; i += NTX) {
         const int c = i / HZ, k = i % HZ;
         float2 a = make_float2(0.0f, 0.0f), b = make_float2(0.0f, 0.0f);
         if (k <= N / 2) {
@@ -416,8 +416,8 @@ __device__ __forceinline__ float2 herm(const float2* __restrict row, int n) {
 // N <= 256) its direct stores would scatter each wave over several rows in short
 // pieces; the rows then go through LDS and are stored whole, lane after lane.
 // KZ: the half spectra are multiplied by -i k_z first (k_z = m dk; zero at N/2, see k_x_ic).
-template <int RC, bool KZ>
-__global__ __launch_bounds__(NT) void k_rows_c2r_real(const float2* __restrict hz, float* __restrict out,
+template <int RC, bool KZ, int NTX>
+__global__ __launch_bounds__(NTX) void k_rows_c2r_real(const float2* __restrict hz, float* __restrict out,
                                                       const float2* __restrict tw, double dk) {
     constexpr int PC = RC / 2;
     constexpr bool STAGED = N / Plan<N>::R(Plan<N>::S - 1) < 64;
@@ -434,7 +434,7 @@ __global__ __launch_bounds__(NT) void k_rows_c2r_real(const float2* __restrict h
         return make_float2(a.x - b.y, a.y + b.x);
     };
     if constexpr (!STAGED) {
-        fft_tile<float2, N, PC, NT, +1, false, true>(
+        fft_tile<float2, N, PC, NTX, +1, false, true>(
             ld,
             [&](int, int, int n, int c, float2 v) {
                 out[(row0 + 2 * c) * N + n] = v.x;
@@ -443,10 +443,10 @@ __global__ __launch_bounds__(NT) void k_rows_c2r_real(const float2* __restrict h
             lds, tw);
     } else {
         // the last stage has read all its inputs before the first output
-        fft_tile<float2, N, PC, NT, +1, false, true>(
+        fft_tile<float2, N, PC, NTX, +1, false, true>(
             ld, [&](int, int, int n, int c, float2 v) { lds[lds_slot<N, PC, true>(n, c)] = v; }, lds, tw);
         __syncthreads();
-        for (int i = threadIdx.x; i < PC * N; i += NT) {
+        for (int i = threadIdx.x; i < PC * N; i += NTX) {
             const int c = i / N, n = i - c * N;
             const float2 v = lds[lds_slot<N, PC, true>(n, c)];
             out[(row0 + 2 * c) * N + n] = v.x;
@@ -510,13 +510,13 @@ void pass_f32(float2* d, int axis, int dir, const float2* tw, int variant, hipSt
         cols_launch<float2, cc_of(v), nt_of(v)>(d, axis, dir, tw, N, (size_t)N * N, s);
     });
 }
-// Column pass over nbox half-spectrum grids N x N x HZ.
 void force_f64(const double2* rho, double2* w, double* out, const double2* tw, const double2* modes, int dim,
                hipStream_t s) {
     k_rows_force<rc64()><<<(unsigned)((size_t)N * N / rc64()), NT, 0, s>>>(rho, w, tw, modes, dim);
     cols_launch<double2, cc64(), 512>(w, 1, +1, tw, N, (size_t)N * N, s);
     k_cols_force<cc64(), 512><<<(unsigned)((size_t)N * N / cc64()), 512, 0, s>>>(w, out, tw);
 }
+// Column pass over nbox half-spectrum grids N x N x HZ.
 void pass_half(float2* d, int axis, int dir, const float2* tw, int variant, int nbox, hipStream_t s) {
     with_variant(variant, [&](auto vc) {
         constexpr int v = decltype(vc)::value;
@@ -527,21 +527,26 @@ void pass_f64(double2* d, int axis, int dir, const double2* tw, hipStream_t s) {
     if (axis == 2) rows_launch<double2, rc64()>(d, dir, tw, s);
     else cols_launch<double2, cc64(), 512>(d, axis, dir, tw, N, (size_t)N * N, s);
 }
+// Real rows: eight (four complex columns) to a workgroup of 128 threads, 256 for the
+// lengths 384 and 768 (with 128: 384 c2r 115 against 107 us, 768 c2r 980 / 850, r2c 716 /
+// 660).  Small workgroups fill the chip where a grid has few rows and give up their place
+// sooner where it has many.  Against 8 to 128 rows (16 to 32 KB) and 256 threads, r2c and
+// c2r in us: 32: 3.9 3.7 (4.5 4.3), 64: 4.2 4.2 (6.9 6.5), 96: 5.3 5.5 (6.8 8.7), 128: 6.6
+// 6.2 (8.2 7.6), 192: 15.4 16.4 (16.7 17.6), 256: 29.1 28.0 (28.1 29.1), 384: 83 107 (83
+// 115), 512: 192 246 (192 248), 1024: 1508 1671 (1593 1721).
+constexpr int RR = 8, NTR = N % 3 == 0 && N >= 384 ? 256 : 128;
 // nbox grids of the same shape back to back (rows of every box in one launch)
 void fwd_z_r2c(const long long* rho, const float* rhof, const unsigned long long* ctl,
                const unsigned long long* mass, float2* out, const float2* tw, int nbox, hipStream_t s) {
-    constexpr int RC = 2 * rc32();
-    unsigned nb = (unsigned)((size_t)nbox * N * N / RC);
-    k_rows_r2c_density<RC, false><<<nb, NT, 0, s>>>(rho, rhof, ctl, mass, out, tw);
+    unsigned nb = (unsigned)((size_t)nbox * N * N / RR);
+    k_rows_r2c_density<RR, false, NTR><<<nb, NTR, 0, s>>>(rho, rhof, ctl, mass, out, tw);
 }
 void fwd_z_r2c_real(const float* in, float2* out, const float2* tw, hipStream_t s) {
-    constexpr int RC = 2 * rc32();
-    k_rows_r2c_density<RC, true><<<(unsigned)((size_t)N * N / RC), NT, 0, s>>>(nullptr, in, nullptr, nullptr, out, tw);
+    k_rows_r2c_density<RR, true, NTR><<<(unsigned)((size_t)N * N / RR), NTR, 0, s>>>(nullptr, in, nullptr, nullptr, out, tw);
 }
 void inv_z_c2r_real(const float2* hz, float* out, const float2* tw, int nbox, hipStream_t s) {
-    constexpr int RC = 2 * rc32();
-    unsigned nb = (unsigned)((size_t)nbox * N * N / RC);
-    k_rows_c2r_real<RC, false><<<nb, NT, 0, s>>>(hz, out, tw, 0.0);
+    unsigned nb = (unsigned)((size_t)nbox * N * N / RR);
+    k_rows_c2r_real<RR, false, NTR><<<nb, NTR, 0, s>>>(hz, out, tw, 0.0);
 }
 // The initial conditions' passes, one box: 16 columns (128-byte rows), 1024 threads where
 // such a tile leaves one workgroup per CU; the x pass then 8 columns (k_x_ic).
@@ -554,8 +559,7 @@ void ic_y(float2* h2, float2* h3, const float2* tw, double dk, hipStream_t s) {
     k_y_ic<16, NT_IC><<<N * (HZ / 16), NT_IC, 0, s>>>(h2, h3, tw, dk);
 }
 void ic_z(const float2* hz, float* out, const float2* tw, double dk, hipStream_t s) {
-    constexpr int RC = 2 * rc32();
-    k_rows_c2r_real<RC, true><<<(unsigned)((size_t)N * N / RC), NT, 0, s>>>(hz, out, tw, dk);
+    k_rows_c2r_real<RR, true, NTR><<<(unsigned)((size_t)N * N / RR), NTR, 0, s>>>(hz, out, tw, dk);
 }
 template <int CC, int NTC>
 void x_psi_launch(float2* h1, const float2* twf, const float2* twr, const float* hs, int nbox, hipStream_t s) {
