@@ -46,8 +46,8 @@ extern "C" {
 #define HGPM_FP32 0  /* build layout: integer cell + FP32 offset (stored as one 32-bit
                         cell index with 10 bits per axis, so NG <= 1024), int64
                         fixed-point deposit, complex64 Stockham FFT, fused kernels     */
-#define HGPM_FP64 1  /* plain reference-structured path in FP64: double3 positions,
-                        FP64 atomics, complex128 FFT, one kernel per reference kernel  */
+#define HGPM_FP64 1  /* plain path in FP64: double3 positions, FP64 atomics, complex128
+                        FFT, the three force components transformed                    */
 
 /* Mass unit of the int64 fixed-point density: one particle of mass (ng/np)^3 deposits
    round(w * 2^24) per cell, w the FP32 CIC weight times the mass. */

@@ -152,6 +152,22 @@ def test_deposit_dense_cells_take_the_wide_route(hg, orc, np_):
                 assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("ng,np_,sigma", [(64, 32, 0.4), (64, 32, 2.0), (96, 32, 0.4), (64, 64, 4.0), (192, 32, 1.0)])
+def test_deposit_window_slabs(hg, orc, ng, np_, sigma):
+    """Windows over one LDS pass, in slabs of whole (y, z) planes that start 0 to 3 cells past
+    a 16-byte line of the arena (extents that differ by tile and seed), and (192 / 32: planes
+    of 98 x 98 cells and more) also with the smallest slabs: bit-exact against the oracle."""
+    case(f"deposit slabs ng={ng} np={np_} sigma={sigma}")
+    with mk(hg, ng, np_) as m:
+        for seed in range(4):
+            rng = np.random.default_rng(1000 * ng + seed)
+            cell, off = lattice_split(rng, np_, ng, sigma)
+            m.set_particles_split(cell, off, np.zeros((m.N, 3), np.float32))
+            m.cic()
+            assert np.array_equal(m.get_density(), orc.cic_split(ng, cell, off, (ng / np_) ** 3)), seed
+            assert m.get_tunable("deposit_deferred") < m.N // 4096  # a sub-arena may be full
+
+
 @pytest.mark.parametrize("ng,dense", [(32, 3), (64, 13), (64, 64), (96, 29), (96, 2)])
 def test_deposit_dense_blocks_spread(hg, orc, ng, dense):
     """A workgroup of the 64-bit owner pass takes up to eight owner blocks, the marked ones
