@@ -790,11 +790,11 @@ __device__ __forceinline__ long long box_mass(const unsigned long long* __restri
 constexpr int OWN_U32 = 16; // arena loads in flight per lane, 32-bit pass
 constexpr int OWN_U64 = 16; // 64-bit pass
 constexpr unsigned OWN_FEW = 512; // owner blocks up to which 1024 threads take one
-// Returns false when the block needs the 64-bit pass (ACC = unsigned only).
-template <typename ACC, int U, int WG>
-__device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* acc, int* s_redo,
+// Hands the block to the 64-bit pass when it needs 64-bit sums.
+template <int WG>
+__device__ __forceinline__ void owner_block(const OwnerArgs& g, int blk, unsigned* acc, int* s_redo,
                                             unsigned long long* s_dif) {
-    constexpr bool A64 = sizeof(ACC) == 8;
+    constexpr int U = OWN_U32;
     constexpr int OWN_J = OB * OB / 64; // plane slots per lane (a plane holds <= OB^2 cells)
     constexpr int DW = WG / 64 / OWN_J; // chunks in work at a time, OWN_J waves each
     static_assert(WG % (64 * OWN_J) == 0 && HGPM_DEP_SLOTS <= 64, "whole groups of waves, a descriptor per lane");
@@ -804,36 +804,35 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     // the mark, the count and every slot descriptor (one per lane, in every wave; the unused
     // ones are ignored) are loaded together: one memory latency
-    const unsigned char mark = A64 ? (unsigned char)0 : g.wide_blk[blk];
+    const unsigned char mark = g.wide_blk[blk];
     const unsigned cnt = g.count[blk];
     uint4 dl = make_uint4(0u, 0u, 0x80000000u, 0u);
     if (lane < g.nslots) dl = g.slots[(size_t)blk * g.nslots + lane];
-    if (!A64 && mark) {
+    if (mark) {
         // summed in 64 bits by an earlier deposit (a dense block stays dense): straight
         // to the 64-bit pass, without a 32-bit attempt
         if (tid == 0) {
             g.wide_blk[blk] = 3;
             atomicAdd(g.nredo, 1ull);
         }
-        return false;
+        return;
     }
     if (tid == 0) {
         *s_redo = 0;
         *s_dif = 0ull;
     }
-    for (int i = tid; i < OB * OB * OB; i += WG) acc[i] = (ACC)0;
+    for (int i = tid; i < OB * OB * OB; i += WG) acc[i] = 0u;
     __syncthreads();
-    if (A64 && tid == 0) g.count[blk] = 0u;
     const bool live = lane < (int)min(cnt, (unsigned)g.nslots) && !(dl.z >> 31);
     bool wrap = false;             // a chunk with 64-bit cells
-    unsigned long long added = 0;  // this lane's sum of the values added (32-bit pass)
+    unsigned long long added = 0;  // this lane's sum of the values added
     // The wave's share of chunk d: cells j * 64 .. j * 64 + 63 of its (y, z) planes, another
     // j with each chunk, so that the chunks of a block (one large, the others slivers of
     // neighbouring tiles' windows) spread evenly over the waves.
     const int lj = (wv + lane / DW) % OWN_J;
     unsigned long long todo = __builtin_amdgcn_ballot_w64(
         live && lane % DW == wv / OWN_J && lj * 64 < (int)((((dl.z >> 16) & 15u) + 1u) * (((dl.z >> 20) & 15u) + 1u)));
-    if (!A64 && __builtin_amdgcn_ballot_w64(live && (dl.z & 0x40000000u))) { // 64-bit cells: the 64-bit pass
+    if (__builtin_amdgcn_ballot_w64(live && (dl.z & 0x40000000u))) { // 64-bit cells: the 64-bit pass
         wrap = true;
         todo = 0ull;
     }
@@ -863,26 +862,9 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
         // (scalar branches): the values are added unconditionally (zeros included),
         // which costs less than masking each add
         if (!pv) continue;
-        if (A64 && (de.z & 0x40000000u)) {
-            // a window of 64-bit cells (two arena words per cell)
-            wrap = true;
-            for (int x0 = 0; x0 < mx; x0 += U) {
-                unsigned long long v[U];
-#pragma unroll
-                for (int u = 0; u < U; u++) {
-                    const unsigned xu = (unsigned)min(x0 + u, mx - 1);
-                    v[u] = *(const unsigned long long*)((const char*)ch + (xu * e12 + po) * 8u);
-                }
-#pragma unroll
-                for (int u = 0; u < U; u++)
-                    if (x0 + u < mx) atomicAdd(&acc[la + (x0 + u) * OB * OB], (ACC)v[u]);
-            }
-            continue;
-        }
         // NU planes from x0 on.  Every slot loads (planes past the chunk's last load that
         // one again) so that the loads issue together.  A chunk lies in a window of at
-        // most DEP_MAXCH owner blocks: byte offsets from its first cell fit 32 bits (also
-        // for 64-bit cells)
+        // most DEP_MAXCH owner blocks: byte offsets from its first cell fit 32 bits
         auto planes = [&](auto nu, int x0) {
             constexpr int NU = decltype(nu)::value;
             unsigned v[NU];
@@ -894,15 +876,15 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
             if (x0 + NU <= mx) {
 #pragma unroll
                 for (int u = 0; u < NU; u++) {
-                    atomicAdd(&acc[la + (x0 + u) * OB * OB], (ACC)v[u]);
-                    if constexpr (!A64) added += v[u];
+                    atomicAdd(&acc[la + (x0 + u) * OB * OB], v[u]);
+                    added += v[u];
                 }
             } else {
 #pragma unroll
                 for (int u = 0; u < NU; u++)
                     if (x0 + u < mx) {
-                        atomicAdd(&acc[la + (x0 + u) * OB * OB], (ACC)v[u]);
-                        if constexpr (!A64) added += v[u];
+                        atomicAdd(&acc[la + (x0 + u) * OB * OB], v[u]);
+                        added += v[u];
                     }
             }
         };
@@ -921,25 +903,146 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
     constexpr int KS = WG / (OB * OB);
     static_assert(WG % (OB * OB) == 0 && OB % KS == 0, "whole (y, z) planes per pass");
     const int t = tid % (OB * OB), k0 = tid / (OB * OB);
-    if constexpr (!A64) {
-        // a cell whose sum reached 2^32 wrapped: the stored cells then sum to less than
-        // the values added (an exact test, one add per cell); the block goes to the
-        // 64-bit pass
-        unsigned long long stored = 0;
-        for (int k = k0; k < OB; k += KS) stored += acc[k * OB * OB + t];
-        // the block's sum of (added - stored), modulo 2^64: k wraps leave k 2^32 < 2^64
-        unsigned long long dif = added - stored;
-        for (int off = 32; off > 0; off >>= 1) dif += __shfl_xor(dif, off, 64);
-        if (lane == 0) atomicAdd(s_dif, dif);
-        __syncthreads();
-        if (*s_redo || *s_dif) {
-            if (tid == 0) {
-                g.wide_blk[blk] = 2;
-                atomicAdd(g.nredo, 1ull);
-            }
-            return false;
+    // a cell whose sum reached 2^32 wrapped: the stored cells then sum to less than
+    // the values added (an exact test, one add per cell); the block goes to the
+    // 64-bit pass
+    unsigned long long stored = 0;
+    for (int k = k0; k < OB; k += KS) stored += acc[k * OB * OB + t];
+    // the block's sum of (added - stored), modulo 2^64: k wraps leave k 2^32 < 2^64
+    unsigned long long dif = added - stored;
+    for (int off = 32; off > 0; off >>= 1) dif += __shfl_xor(dif, off, 64);
+    if (lane == 0) atomicAdd(s_dif, dif);
+    __syncthreads();
+    if (*s_redo || *s_dif) {
+        if (tid == 0) {
+            g.wide_blk[blk] = 2;
+            atomicAdd(g.nredo, 1ull);
+        }
+        return;
+    }
+    const int bx = lb / (nb * nb), by = (lb / nb) % nb, bz = lb % nb;
+    const int64_t at = gidx(g.ng, bx * OB, by * OB + (t >> 4), bz * OB + (t & 15));
+    const int64_t plane = (int64_t)g.ng * g.ng;
+    if (f32) {
+        const double mean = (double)box_mass(g.mass, box) / (double)g.gcells;
+        float* __restrict rf = g.rhof + (int64_t)box * g.gcells;
+#pragma unroll 4
+        for (int k = k0; k < OB; k += KS) {
+            rf[at + k * plane] = (float)(((double)acc[k * OB * OB + t] - mean) * (1.0 / 16777216.0));
+        }
+    } else {
+        unsigned long long* __restrict r = g.rho + (int64_t)box * g.gcells;
+#pragma unroll 4
+        for (int k = k0; k < OB; k += KS) {
+            r[at + k * plane] = acc[k * OB * OB + t];
         }
     }
+    if (tid == 0) g.count[blk] = 0u;
+}
+// The same in int64 cells, a chunk to a wave at a time, its descriptor from LDS (5.7 ms for
+// every block at the end of a 1024^3 run).
+__device__ __forceinline__ void owner_block64(const OwnerArgs& g, int blk, unsigned long long* acc, uint4* desc,
+                                              int* s_n, int* s_redo) {
+    constexpr int U = OWN_U64, WG = OWN_NT;
+    constexpr int OWN_J = OB * OB / 64; // plane slots per lane (a plane holds <= OB^2 cells)
+    const int nb = g.ng / OB;
+    const int box = blk / g.nblk, lb = blk - box * g.nblk;
+    const bool f32 = g.rhof != nullptr && g.ctl[1] == 0ull;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    // every slot descriptor is loaded together with the count (the unused ones are
+    // ignored), so the two loads cost one memory latency
+    uint4 dl = make_uint4(0u, 0u, 0x80000000u, 0u);
+    if (tid < g.nslots) dl = g.slots[(size_t)blk * g.nslots + tid];
+    if (tid == 0) {
+        const unsigned c = g.count[blk];
+        g.count[blk] = 0u;
+        *s_n = (int)min(c, (unsigned)g.nslots);
+        *s_redo = 0;
+    }
+    if (tid < g.nslots) desc[tid] = dl;
+    for (int i = tid; i < OB * OB * OB; i += WG) acc[i] = 0ull;
+    __syncthreads();
+    const int nd = *s_n;
+    bool wrap = false;             // a chunk with 64-bit cells
+    for (int d = wv; d < nd; d += WG / 64) {
+        // one descriptor per wave: its words are uniform (scalar registers)
+        uint4 de = desc[d];
+        de.x = __builtin_amdgcn_readfirstlane(de.x);
+        de.y = __builtin_amdgcn_readfirstlane(de.y);
+        de.z = __builtin_amdgcn_readfirstlane(de.z);
+        de.w = __builtin_amdgcn_readfirstlane(de.w);
+        if (de.z >> 31) continue;
+        const unsigned* __restrict ch = g.arena + ((unsigned long long)de.x | ((unsigned long long)de.y << 32));
+        const int ox = de.z & 15, oy = (de.z >> 4) & 15, oz = (de.z >> 8) & 15;
+        const int mx = ((de.z >> 12) & 15) + 1, my = ((de.z >> 16) & 15) + 1, mz = ((de.z >> 20) & 15) + 1;
+        const int e2 = (int)(de.w >> 16);
+        const unsigned e12 = (de.w & 0xFFFFu) * (unsigned)e2; // arena stride of an x plane
+        const int myz = my * mz;
+        // p -> (ly, lz) by multiplication with a rounded reciprocal: exact here because
+        // p < 256 keeps the rounding error below the 0.5/mz margin of (p + 0.5)
+        const float rmz = 1.0f / (float)mz;
+        for (int j = 0; j < OWN_J && j * 64 < myz; j++) {
+            const int pl = lane + 64 * j;
+            const bool pv = pl < myz;
+            const int ly = (int)(((float)pl + 0.5f) * rmz), lz = pl - ly * mz;
+            unsigned po = pv ? (unsigned)(ly * e2 + lz) : 0u; // arena offset in the plane
+            // (opaque: the address of plane x stays x * e12 + po, a scalar product and one
+            // add, instead of being refactored into a multiply per load)
+            asm volatile("" : "+v"(po));
+            const int la = ox * OB * OB + (oy + ly) * OB + oz + lz; // LDS cell of x plane 0
+            // lanes past the plane sit the chunk out; inside, every condition is uniform
+            // (scalar branches): the values are added unconditionally (zeros included),
+            // which costs less than masking each add
+            if (!pv) continue;
+            if (de.z & 0x40000000u) {
+                // a window of 64-bit cells (two arena words per cell)
+                wrap = true;
+                for (int x0 = 0; x0 < mx; x0 += U) {
+                    unsigned long long v[U];
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        const unsigned xu = (unsigned)min(x0 + u, mx - 1);
+                        v[u] = *(const unsigned long long*)((const char*)ch + (xu * e12 + po) * 8u);
+                    }
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        if (x0 + u < mx) atomicAdd(&acc[la + (x0 + u) * OB * OB], (unsigned long long)v[u]);
+                }
+                continue;
+            }
+            for (int x0 = 0; x0 < mx; x0 += U) {
+                unsigned v[U];
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    // every slot loads (planes past the chunk's last load that one again)
+                    // so that the U loads issue together.  A chunk lies in a window of at
+                    // most DEP_MAXCH owner blocks: byte offsets from its first cell fit 32
+                    // bits (also for 64-bit cells)
+                    const unsigned xu = (unsigned)min(x0 + u, mx - 1);
+                    v[u] = *(const unsigned*)((const char*)ch + (xu * e12 + po) * 4u);
+                }
+                if (x0 + U <= mx) {
+#pragma unroll
+                    for (int u = 0; u < U; u++) {
+                        atomicAdd(&acc[la + (x0 + u) * OB * OB], (unsigned long long)v[u]);
+                    }
+                } else {
+#pragma unroll
+                    for (int u = 0; u < U; u++)
+                        if (x0 + u < mx) {
+                            atomicAdd(&acc[la + (x0 + u) * OB * OB], (unsigned long long)v[u]);
+                            }
+                }
+            }
+        }
+    }
+    if (wrap) *s_redo = 1;
+    __syncthreads();
+    // thread tid writes (x, y, z) = (k, t / OB, t % OB), t = tid % OB^2, of the block for
+    // k = tid / OB^2, tid / OB^2 + KS, ...
+    constexpr int KS = WG / (OB * OB);
+    static_assert(WG % (OB * OB) == 0 && OB % KS == 0, "whole (y, z) planes per pass");
+    const int t = tid % (OB * OB), k0 = tid / (OB * OB);
     const int bx = lb / (nb * nb), by = (lb / nb) % nb, bz = lb % nb;
     const int64_t at = gidx(g.ng, bx * OB, by * OB + (t >> 4), bz * OB + (t & 15));
     const int64_t plane = (int64_t)g.ng * g.ng;
@@ -949,7 +1052,7 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
         float* __restrict rf = g.rhof + (int64_t)box * g.gcells;
 #pragma unroll 4
         for (int k = k0; k < OB; k += KS) {
-            const unsigned long long q64 = (unsigned long long)acc[k * OB * OB + t];
+            const unsigned long long q64 = acc[k * OB * OB + t];
             hi |= q64 >> 32;
             rf[at + k * plane] = (float)(((double)(long long)q64 - mean) * (1.0 / 16777216.0));
         }
@@ -957,51 +1060,39 @@ __device__ __forceinline__ bool owner_block(const OwnerArgs& g, int blk, ACC* ac
         unsigned long long* __restrict r = g.rho + (int64_t)box * g.gcells;
 #pragma unroll 4
         for (int k = k0; k < OB; k += KS) {
-            const unsigned long long q64 = (unsigned long long)acc[k * OB * OB + t];
+            const unsigned long long q64 = acc[k * OB * OB + t];
             hi |= q64 >> 32;
             r[at + k * plane] = q64;
         }
     }
-    if constexpr (A64) {
-        // mark the block for later deposits: it needs 64-bit sums (a 64-bit chunk or a
-        // cell of 2^32 units or more); with every block in this pass, count it
-        if (__builtin_amdgcn_ballot_w64(hi != 0ull) && lane == 0) *s_redo = 1;
-        __syncthreads();
-        if (tid == 0) {
-            g.wide_blk[blk] = *s_redo ? 1 : 0;
-            if (g.ctl[HGPM_DEP_CTL] && *s_redo) atomicAdd(g.nredo, 1ull);
-        }
-    } else {
-        if (tid == 0) g.count[blk] = 0u;
+    // mark the block for later deposits: it needs 64-bit sums (a 64-bit chunk or a cell of
+    // 2^32 units or more); with every block in this pass, count it
+    if (__builtin_amdgcn_ballot_w64(hi != 0ull) && lane == 0) *s_redo = 1;
+    __syncthreads();
+    if (tid == 0) {
+        g.wide_blk[blk] = *s_redo ? 1 : 0;
+        if (g.ctl[HGPM_DEP_CTL] && *s_redo) atomicAdd(g.nredo, 1ull);
     }
-    return true;
 }
 template <int WG> __global__ __launch_bounds__(WG) void k_deposit_owner(OwnerArgs g) {
     if (g.ctl[HGPM_DEP_CTL]) return; // every block in k_deposit_owner64
     __shared__ unsigned acc[OB * OB * OB];
     __shared__ int s_redo;
     __shared__ unsigned long long s_dif;
-    owner_block<unsigned, OWN_U32, WG>(g, (int)xcd_remap(blockIdx.x, gridDim.x), acc, &s_redo, &s_dif);
+    owner_block<WG>(g, (int)xcd_remap(blockIdx.x, gridDim.x), acc, &s_redo, &s_dif);
 }
 // In 64-bit cells: the blocks handed over, or every block on that route (a deposit with
 // many dense blocks, late in a run: the 32-bit attempt would be wasted on them).  A
-// workgroup takes up to OWN_64B blocks, one in gridDim.x: mostly none is marked, and a
-// workgroup per block then cost 144 us at 1024^3 (262144 of them; now 20 us).  Dense blocks
-// lie together and so fall to different workgroups (one workgroup taking 256 neighbouring
-// blocks took 0.3 ms a step late in a 512^3 run, against 0.06).
-constexpr int OWN_64B = 8;
-__global__ __launch_bounds__(OWN_NT) void k_deposit_owner64(OwnerArgs g, int nall) {
+// workgroup per block: the empty ones cost 145 us at 1024^3 (262144 of them).  Workgroups
+// that look at eight blocks each take 23 us there when none is dense, but 11.1 against
+// 5.7 ms a step at the end of that run, when every block comes here.
+__global__ __launch_bounds__(OWN_NT) void k_deposit_owner64(OwnerArgs g) {
+    const int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
+    if (!g.ctl[HGPM_DEP_CTL] && !(g.wide_blk[blk] & 2)) return;
     __shared__ unsigned long long acc[OB * OB * OB];
-    __shared__ int s_redo;
-    __shared__ unsigned long long s_dif;
-    const int first = (int)xcd_remap(blockIdx.x, gridDim.x);
-    const int mine = first + (int)(threadIdx.x & 63) * (int)gridDim.x; // of the lane
-    const bool has = (threadIdx.x & 63) < OWN_64B && mine < nall;
-    unsigned long long todo =
-        __builtin_amdgcn_ballot_w64(has && (g.ctl[HGPM_DEP_CTL] || (g.wide_blk[mine] & 2)));
-    for (; todo; todo &= todo - 1ull) // the same blocks in every wave; ends at a barrier
-        owner_block<unsigned long long, OWN_U64, OWN_NT>(g, first + __builtin_ctzll(todo) * (int)gridDim.x, acc, &s_redo,
-                                                         &s_dif);
+    __shared__ uint4 desc[HGPM_DEP_SLOTS];
+    __shared__ int s_n, s_redo;
+    owner_block64(g, blk, acc, desc, &s_n, &s_redo);
 }
 
 // The end of a deposit: the control words of the next one (the other of two sets, used in
@@ -1857,7 +1948,7 @@ void launch_deposit_owner(int ng, long long* rho, float* rhof, const DepositBuff
     const unsigned nall = (unsigned)nblk * (unsigned)b.nbox;
     if (nall <= OWN_FEW) k_deposit_owner<1024><<<nall, 1024, 0, s>>>(g);
     else k_deposit_owner<OWN_NT><<<nall, OWN_NT, 0, s>>>(g);
-    k_deposit_owner64<<<(nall + OWN_64B - 1) / OWN_64B, OWN_NT, 0, s>>>(g, (int)nall);
+    k_deposit_owner64<<<nall, OWN_NT, 0, s>>>(g);
 }
 void launch_deposit_deferred(const PosPackH* pos, int64_t n, int ng, float mass, long long* rho,
                              const DepositBuffers& b, hipStream_t s) {

@@ -170,10 +170,9 @@ def test_deposit_window_slabs(hg, orc, ng, np_, sigma):
 
 @pytest.mark.parametrize("ng,dense", [(32, 3), (64, 13), (64, 64), (96, 29), (96, 2)])
 def test_deposit_dense_blocks_spread(hg, orc, ng, dense):
-    """A workgroup of the 64-bit owner pass takes up to eight owner blocks, the marked ones
-    of every gridDim-th: none, several or all of its blocks dense (512 particles on one
-    lattice point inside the block), in three deposits in turn (marks kept, the route of a
-    mostly dense grid), bit-exact against the oracle."""
+    """The 64-bit owner pass over few, several or all blocks of a grid (512 particles on one
+    lattice point inside each dense block), in three deposits in turn (marks kept, the route
+    of a mostly dense grid), bit-exact against the oracle."""
     case(f"deposit dense blocks ng={ng} dense={dense}")
     rng = np.random.default_rng(ng + dense)
     nb = ng // 16
@@ -1051,7 +1050,7 @@ def test_driver_analysis_hook(hg, tmp_path):
 # ---------------------------------------------------------- host transfers ----
 @pytest.mark.parametrize("n", [32, 64, 128])
 def test_host_transfers(hg, n):
-    """Particles through the pinned ring: one slot, a few and several rounds of it (1 MB
+    """Particles through the pinned ring: one slot, a few and several rounds of it (2 MB
     slots, 8 of them), bit for bit, from two host threads with a context each; a value out
     of range anywhere is refused with its index and leaves the state as it was."""
     import threading
