@@ -56,6 +56,7 @@ struct hgpm_ctx {
     unsigned long long* ctl = nullptr; // two sets of deposit control words, used in turn
     int set_words = 0;                 // words of a set: control words, mass partial sums per box
     int set_next = 0;                  // the set of the next deposit; the other is the last one's
+    bool dep_dirty = false;            // a deposit's launches failed: its words, sums and counts may be anything
     // the force components' grids (FP64)
     ForceF64 force64() const {
         const double* g = (const double*)grad64;
@@ -306,9 +307,18 @@ DepositBuffers dep_buffers(hgpm_ctx* c, int fold) {
 // (a step whose solve follows at once) the owner pass writes it as the FP32 grid the
 // forward z transform takes, into psi's buffer, when no tile was deferred (decided on
 // the device).  fold: the positions folded that many times (P(k) of one box).
+// A deposit starts from its set of control words cleared and no chunk listed, as the one
+// before it leaves them; after one whose launches failed they are cleared here.
 int f32_deposit(hgpm_ctx* c, bool fused = false, int fold = 0) {
     const DepositBuffers b = dep_buffers(c, fold);
     Timed t(c, "deposit");
+    if (c->dep_dirty) {
+        // (the owner blocks' counts and marks: 5 bytes a block, a multiple of 8 blocks)
+        const size_t nb = c->ng / 16, nblk = nb * nb * nb * c->nwave;
+        launch_zero_u64(c->ctl, 2 * (size_t)c->set_words, c->st);
+        launch_zero_u64((unsigned long long*)c->dcount, nblk * 5 / 8, c->st);
+    }
+    c->dep_dirty = true; // until its launches are known to have succeeded
     if (fold) {
         Timed t1(c, "deposit_binned");
         launch_deposit_binned(c->pos, c->N, c->ng, ref_mass(c), (long long*)c->B, fused ? c->psi : nullptr, b, c->st);
@@ -326,9 +336,10 @@ int f32_deposit(hgpm_ctx* c, bool fused = false, int fold = 0) {
         Timed t3(c, "deposit_deferred");
         launch_deposit_deferred(c->pos, c->N * c->nbox, c->ng, ref_mass(c), (long long*)c->B, b, c->st);
     }
+    LAUNCHCHK(c);
+    c->dep_dirty = false;
     c->set_next ^= 1;
     c->dens_f32 = fused;
-    LAUNCHCHK(c);
     return HGPM_OK;
 }
 
@@ -1942,8 +1953,13 @@ int hgpm_ensemble_run(hgpm_ensemble* e, int nsteps, const hgpm_step_coeffs* coef
         rc = HGPM_ERR_HIP;
     }
     if (graph) (void)hipGraphDestroy(graph);
-    // the captured deposits did not run: the control sets stand as before
-    auto rewind = [&] { for (size_t g = 0; g < ng; g++) e->batch[g]->set_next = set[g]; };
+    // the captured deposits did not run, nor a clearing before them: the next one clears
+    auto rewind = [&] {
+        for (size_t g = 0; g < ng; g++) {
+            e->batch[g]->set_next = set[g];
+            e->batch[g]->dep_dirty = true;
+        }
+    };
     if (rc) {
         if (exec) (void)hipGraphExecDestroy(exec);
         rewind();

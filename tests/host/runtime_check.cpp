@@ -1,0 +1,292 @@
+// Host-side check of the engine's control code (capi.cpp, hostcopy.cpp, host.cpp, compiled
+// for the host) against a HIP runtime of its own: device memory is host memory, streams run
+// at once, kernels are replaced by what they leave in the buffers that the control code
+// relies on, and calls fail where a scenario says so.  Error paths that no call sequence
+// brings about on a healthy GPU run here, without one.  runtime_check <scenario> prints
+// "<cases> <bad>" after a line for each bad one.
+#include "../../include/hgpm.h"
+#include "hostcopy.h"
+#include "internal.h"
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <mutex>
+#include <string>
+#include <vector>
+
+// ---------------------------------------------------------------- the runtime ----
+namespace fake {
+std::mutex mu;
+thread_local hipError_t last = hipSuccess;
+bool capturing = false;     // launches are recorded, not run
+bool graph_fails = false;   // hipGraphLaunch
+int launch_no = 0;          // launches since the last reset ...
+int launch_fails = -1;      // ... the one that fails (< 0: none)
+void clear() {
+    launch_no = 0;
+    launch_fails = -1;
+}
+hipError_t err(hipError_t e) { return e == hipSuccess ? e : last = e; }
+// One launch: true when its effects happen.
+bool launch() {
+    const bool bad = launch_no++ == launch_fails;
+    if (bad) last = hipErrorOutOfMemory;
+    return !bad && !capturing;
+}
+} // namespace fake
+using fake::err;
+
+extern "C" {
+hipError_t hipGetLastError() {
+    const hipError_t e = fake::last;
+    fake::last = hipSuccess;
+    return e;
+}
+const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "error"; }
+hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipMemGetInfo(size_t* f, size_t* t) { return *f = *t = (size_t)4 << 30, hipSuccess; }
+hipError_t hipMalloc(void** p, size_t n) { return *p = calloc(1, n), hipSuccess; }
+hipError_t hipFree(void* p) { return free(p), hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return *p = malloc(n), hipSuccess; }
+hipError_t hipHostFree(void* p) { return free(p), hipSuccess; }
+hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return memcpy(d, s, n), hipSuccess; }
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+    if (!fake::capturing) memcpy(d, s, n);
+    return hipSuccess;
+}
+hipError_t hipMemset(void* d, int v, size_t n) { return memset(d, v, n), hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = (hipStream_t) new int(0), hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) { return delete (int*)s, hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return *e = (hipEvent_t) new int(0), hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
+hipError_t hipEventDestroy(hipEvent_t e) { return delete (int*)e, hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.0f, hipSuccess; }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) { return fake::capturing = true, hipSuccess; }
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t* g) { return fake::capturing = false, *g = nullptr, hipSuccess; }
+hipError_t hipGraphInstantiate(hipGraphExec_t* e, hipGraph_t, hipGraphNode_t*, char*, size_t) {
+    return *e = nullptr, hipSuccess;
+}
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return err(fake::graph_fails ? hipErrorOutOfMemory : hipSuccess); }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+}
+
+// ---------------------------------------------------------------- the kernels ----
+namespace hgpm {
+// What the deposit's kernels rely on and leave behind: the control words and mass sums of
+// their set cleared, no chunk listed; cursors, lists and sums used; the other set cleared.
+int dep_stale = 0; // deposits that started from anything else
+void launch_deposit_windows(const PosPackH*, int64_t, int ng, float, const DepositBuffers& b, hipStream_t) {
+    if (!fake::launch()) return;
+    const int nblk = (ng / 16) * (ng / 16) * (ng / 16) * b.nbox;
+    bool clean = true;
+    for (int i = 0; i < b.set_words; i++) clean = clean && (i == HGPM_DEP_CTL || b.ctl[i] == 0);
+    for (int i = 0; i < nblk; i++) clean = clean && b.count[i] == 0;
+    dep_stale += !clean;
+    b.ctl[1] += 2;
+    b.ctl[4] += 100;
+    for (int i = 0; i < HGPM_DEP_MASS * b.nbox; i++) b.ctl[HGPM_DEP_CTL + 1 + i] += 7;
+    for (int i = 0; i < nblk; i++) b.count[i] += 3;
+}
+void launch_deposit_binned(const PosPackH* p, int64_t n, int ng, float m, long long*, float*, const DepositBuffers& b,
+                           hipStream_t s) {
+    launch_deposit_windows(p, n, ng, m, b, s);
+    memset(b.count, 0, sizeof(unsigned) * (ng / 16) * (ng / 16) * (ng / 16) * b.nbox);
+}
+void launch_deposit_owner(int ng, long long*, float*, const DepositBuffers& b, hipStream_t) {
+    if (fake::launch()) memset(b.count, 0, sizeof(unsigned) * (ng / 16) * (ng / 16) * (ng / 16) * b.nbox);
+}
+void launch_deposit_deferred(const PosPackH*, int64_t, int, float, long long*, const DepositBuffers& b, hipStream_t) {
+    if (fake::launch()) memset(b.next, 0, sizeof(unsigned long long) * b.set_words);
+}
+void launch_zero_u64(unsigned long long* p, size_t n, hipStream_t) {
+    if (fake::launch()) memset(p, 0, sizeof(*p) * n);
+}
+#define STUB(name, ...) \
+    void name(__VA_ARGS__) { (void)fake::launch(); }
+STUB(launch_drift, PosPackH*, const float*, int64_t, int, float, hipStream_t)
+STUB(launch_compare, const PosPackH*, const float*, const double*, const double*, const PosPackH*, const float*,
+     const double*, const double*, int64_t, int, int, double*, hipStream_t)
+STUB(launch_f64_cic, const double*, int64_t, int, double, double2*, hipStream_t)
+STUB(launch_f64_fold, double*, int64_t, int, hipStream_t)
+STUB(launch_f64_icic, const double*, double*, const ForceF64&, int64_t, int, double, double, hipStream_t)
+STUB(launch_f64_drift, double*, const double*, int64_t, int, double, hipStream_t)
+STUB(launch_f64_force_out, const ForceF64&, double*, int64_t, hipStream_t)
+STUB(launch_f64_density_to_real, const double2*, double*, int64_t, hipStream_t)
+STUB(launch_ic_lines, const double*, int, double, double, double2*, int, hipStream_t)
+STUB(launch_ic_noise_f32, float*, int, uint32_t, hipStream_t)
+STUB(launch_ic_noise_f64, double2*, int, uint32_t, hipStream_t)
+STUB(launch_ic_place_split, const float*, const float*, const float*, PosPackH*, float*, int, int, double, float, hipStream_t)
+STUB(launch_ic_place_f64, const double2*, double*, double*, int, int, int, double, double, hipStream_t)
+STUB(launch_ic_scale_f64, double2*, int, const double*, int, double, double, hipStream_t)
+STUB(launch_ic_displacement_f64, const double2*, double2*, int, int, double, double, hipStream_t)
+STUB(launch_gather_kick, PosPackH*, float*, int64_t, int, const float*, double, double, int, float, int, const void*, int, hipStream_t)
+STUB(launch_to_internal, const PosPackH*, const float*, PosPackH*, float*, int64_t, int, hipStream_t)
+STUB(launch_to_reference, const PosPackH*, const float*, PosPackH*, float*, int64_t, int, hipStream_t)
+STUB(launch_split_to_f64, const PosPackH*, const float*, double*, double*, int64_t, int, hipStream_t)
+STUB(launch_split_from_f64, const double*, const double*, PosPackH*, float*, int64_t, int, int, hipStream_t)
+STUB(launch_split_to_float3, const PosPackH*, const float*, float*, float*, int64_t, int, hipStream_t)
+STUB(launch_split_from_float3, const float*, const float*, PosPackH*, float*, int64_t, int, int, hipStream_t)
+STUB(launch_force_from_psi, const float*, float*, int, hipStream_t)
+int compare_partials() { return 1; }
+int power_partial_blocks(int) { return 1; }
+int ic_static_table(int, double** p) {
+    static double t[HGPM_IC_STATIC_BINS];
+    return *p = t, 0;
+}
+template <typename V, bool H>
+void launch_power_bins(const V*, int, int, size_t, double, double, double, int, const double*, double, double*, int,
+                       double*, long long*, hipStream_t) {
+    (void)fake::launch();
+}
+template void launch_power_bins<float2, true>(const float2*, int, int, size_t, double, double, double, int,
+                                              const double*, double, double*, int, double*, long long*, hipStream_t);
+template void launch_power_bins<double2, false>(const double2*, int, int, size_t, double, double, double, int,
+                                                const double*, double, double*, int, double*, long long*, hipStream_t);
+
+FftOps table(int n) {
+    FftOps f{};
+    f.n = n;
+    f.stages = 1;
+    f.n_variants = f.valid_mask = 1;
+    f.hz = n / 2 + 16;
+    f.plane = (size_t)n * f.hz;
+    f.twiddles = [](double*, double*) {};
+    f.pass_f32 = [](float2*, int, int, const float2*, int, hipStream_t) { (void)fake::launch(); };
+    f.pass_f64 = [](double2*, int, int, const double2*, hipStream_t) { (void)fake::launch(); };
+    f.force_f64 = [](const double2*, double2*, double*, const double2*, const double2*, int, hipStream_t) { (void)fake::launch(); };
+    f.pass_half = [](float2*, int, int, const float2*, int, int, hipStream_t) { (void)fake::launch(); };
+    f.fwd_z_r2c = [](const long long*, const float*, const unsigned long long*, const unsigned long long*, float2*,
+                     const float2*, int, hipStream_t) { (void)fake::launch(); };
+    f.x_psi = [](float2*, const float2*, const float2*, const float*, int, int, hipStream_t) { (void)fake::launch(); };
+    f.inv_z_c2r_real = [](const float2*, float*, const float2*, int, hipStream_t) { (void)fake::launch(); };
+    return f;
+}
+#define TABLE(n) extern const FftOps fft_ops_##n; const FftOps fft_ops_##n = table(n);
+HGPM_FFT_SIZES(TABLE)
+extern const FftOps fft_ops_1024_alt;
+const FftOps fft_ops_1024_alt = table(1024);
+} // namespace hgpm
+
+// -------------------------------------------------------------- the scenarios ----
+namespace {
+int cases = 0, bad = 0;
+void check(bool ok, const std::string& what) {
+    cases++;
+    if (!ok) {
+        bad++;
+        printf("bad: %s\n", what.c_str());
+    }
+}
+hgpm_params params(int ng, int precision = HGPM_FP32) {
+    hgpm_params p{};
+    p.ng = p.np = ng;
+    p.rl = 2.0 * ng;
+    p.nsteps = 10;
+    p.z_ini = 50.0;
+    p.hubble = 0.7;
+    p.omega_cdm = 0.25;
+    p.omega_matter = p.omega_cb = 0.3;
+    p.ss8 = 0.8;
+    p.ns = 0.96;
+    p.t_cmb = 2.7;
+    p.pk_folds = 1;
+    p.pk_bins = 16;
+    p.precision = precision;
+    return p;
+}
+hgpm_ctx* box(int ng, int precision = HGPM_FP32) {
+    const hgpm_params p = params(ng, precision);
+    hgpm_ctx* c = nullptr;
+    if (hgpm_create(&p, &c)) {
+        printf("hgpm_create: %s\n", hgpm_last_error(nullptr));
+        exit(2);
+    }
+    std::vector<float> x(3 * (size_t)ng * ng * ng, 1.0f);
+    if (hgpm_set_particles(c, x.data(), x.data())) exit(2);
+    fake::clear();
+    return c;
+}
+struct Spectrum {
+    double k[16], pk[16];
+    int64_t n[16];
+    int of(hgpm_ctx* c, int fold) { return hgpm_power_spectrum(c, fold, k, pk, n); }
+};
+
+// A deposit whose launches failed, in whatever call made it: the next one starts from
+// cleared control words and mass sums, and no chunk listed.
+void deposit() {
+    const hgpm_step_coeffs co{};
+    Spectrum sp;
+    const std::function<int(hgpm_ctx*)> calls[] = {
+        [](hgpm_ctx* c) { return hgpm_cic(c); }, [&](hgpm_ctx* c) { return hgpm_step(c, &co); },
+        [&](hgpm_ctx* c) { return sp.of(c, 0); }, [&](hgpm_ctx* c) { return sp.of(c, 1); }};
+    for (int call = 0; call < 4; call++)
+        for (int before = 0; before < 2; before++)  // either set of control words
+            for (int at = 0; at < 4; at++)          // the launch that fails
+                for (int twice = 0; twice < 2; twice++) { // and the one after it
+                    hgpm_ctx* c = box(32);
+                    for (int i = 0; i < before; i++) (void)hgpm_cic(c);
+                    const std::string what = "call " + std::to_string(call) + " before " + std::to_string(before) +
+                                             " launch " + std::to_string(at) + " twice " + std::to_string(twice);
+                    hgpm::dep_stale = 0;
+                    for (int i = 0; i <= twice; i++) {
+                        fake::clear();
+                        fake::launch_fails = at;
+                        const int rc = calls[call](c);
+                        check(rc == (fake::launch_no > at ? HGPM_ERR_HIP : HGPM_OK), what + ": the failure is reported");
+                    }
+                    fake::clear();
+                    hgpm::dep_stale = 0; // (a deposit that fails may start from anything)
+                    for (int i = 0; i < 3; i++) check(hgpm_cic(c) == HGPM_OK, what + ": the deposit after it");
+                    check(hgpm::dep_stale == 0, what + ": stale control words");
+                    int deferred = -1;
+                    check(hgpm_get_tunable(c, "deposit_deferred", &deferred) == HGPM_OK && deferred == 2,
+                          what + ": the last deposit's words");
+                    hgpm_destroy(c);
+                }
+    // a graph run whose capture or launch fails, then steps one by one
+    for (int how = 0; how < 2; how++)
+        for (int before = 0; before < 2; before++) {
+            const hgpm_params p[2] = {params(32), params(64)};
+            hgpm_ensemble* e = nullptr;
+            check(hgpm_ensemble_create(2, p, &e) == HGPM_OK, "ensemble");
+            for (int b = 0; b < 2; b++) {
+                std::vector<float> x(3 * (size_t)p[b].np * p[b].np * p[b].np, 1.0f);
+                check(hgpm_ensemble_set_particles(e, b, x.data(), x.data()) == HGPM_OK, "ensemble particles");
+            }
+            const hgpm_step_coeffs co3[6] = {};
+            fake::clear();
+            for (int i = 0; i < before; i++) check(hgpm_ensemble_step(e, co3) == HGPM_OK, "ensemble step");
+            fake::clear();
+            if (how == 0) fake::launch_fails = 12;
+            else fake::graph_fails = true;
+            const std::string what = "ensemble run " + std::to_string(how) + " before " + std::to_string(before);
+            check(hgpm_ensemble_run(e, 3, co3) == HGPM_ERR_HIP, what + ": the failure is reported");
+            fake::clear();
+            fake::graph_fails = false;
+            (void)hipGetLastError();
+            hgpm::dep_stale = 0;
+            for (int i = 0; i < 3; i++) check(hgpm_ensemble_step(e, co3) == HGPM_OK, what + ": the steps after it");
+            check(hgpm::dep_stale == 0, what + ": stale control words");
+            hgpm_ensemble_destroy(e);
+        }
+}
+} // namespace
+
+int main(int argc, char** argv) {
+    const std::string s = argc > 1 ? argv[1] : "";
+    if (s == "deposit") deposit();
+    else return 3;
+    printf("%d %d\n", cases, bad);
+    return 0;
+}
