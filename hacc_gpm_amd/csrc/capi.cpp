@@ -319,6 +319,8 @@ int f32_deposit(hgpm_ctx* c, bool fused = false, int fold = 0) {
         launch_zero_u64((unsigned long long*)c->dcount, nblk * 5 / 8, c->st);
     }
     c->dep_dirty = true; // until its launches are known to have succeeded
+    c->have_density = false;
+    if (fused) c->have_force = false; // psi's buffer holds the density from here on
     if (fold) {
         Timed t1(c, "deposit_binned");
         launch_deposit_binned(c->pos, c->N, c->ng, ref_mass(c), (long long*)c->B, fused ? c->psi : nullptr, b, c->st);
@@ -342,6 +344,10 @@ int f32_deposit(hgpm_ctx* c, bool fused = false, int fold = 0) {
     c->dens_f32 = fused;
     return HGPM_OK;
 }
+
+// The transforms of a solve or a P(k) only read the int64 density, so it outlives one that
+// fails; FP64 transforms in place, and after a fused deposit there is no int64 density.
+bool keeps_density(const hgpm_ctx* c) { return c->prec == HGPM_FP32 && !c->dens_f32; }
 
 // Poisson solve on half spectra: density (B, int64, or FP32 in psi's buffer) -> rho^ (A,
 // pitch hz) -> (g/2) rho^ -> half the potential, psi (real, 4 B per cell).  The forces
@@ -376,6 +382,7 @@ int f32_solve(hgpm_ctx* c) {
 
 // ------------------------------------------------------------ FP64 ops ----
 int f64_deposit(hgpm_ctx* c, const double* pos) {
+    c->have_density = false;
     Timed t(c, "f64_cic");
     launch_f64_cic(pos, c->N, c->ng, pow((double)c->ng / (double)c->np, 3.0), c->grid64, c->st);
     LAUNCHCHK(c);
@@ -1107,6 +1114,7 @@ int hgpm_set_density_f64(hgpm_ctx* c, const double* rho) {
 int hgpm_solve_gradient(hgpm_ctx* c) {
     if (!c) return HGPM_ERR_ARG;
     if (!c->have_density) return fail(c, HGPM_ERR_STATE, "no density: call hgpm_cic first");
+    c->have_density = keeps_density(c);
     int rc = c->prec == HGPM_FP32 ? f32_solve(c) : f64_solve(c);
     if (rc) return rc;
     c->have_density = false;
@@ -1234,10 +1242,10 @@ int hgpm_fft_host(hgpm_ctx* c, void* grid, int direction) {
     if (!c || !grid || (direction != -1 && direction != 1)) return fail(c, HGPM_ERR_ARG, "hgpm_fft_host: bad arguments");
     size_t bytes = (c->prec == HGPM_FP32 ? sizeof(float2) : sizeof(double2)) * (size_t)c->G;
     void* d = c->prec == HGPM_FP32 ? (void*)c->A : (void*)c->grid64;
-    int rc = to_device(c, {{grid, d, bytes}});
-    if (rc || (rc = hgpm_fft_device(c, d, direction)) || (rc = to_host(c, {{grid, d, bytes}}))) return rc;
     c->have_density = c->have_force = false;
-    return HGPM_OK;
+    int rc = to_device(c, {{grid, d, bytes}});
+    if (rc || (rc = hgpm_fft_device(c, d, direction))) return rc;
+    return to_host(c, {{grid, d, bytes}});
 }
 
 // ------------------------------------------------------------------- P(k) ----
@@ -1245,6 +1253,7 @@ int hgpm_power_spectrum_grid(hgpm_ctx* c, int fold, double* k, double* pk, int64
     if (!c) return HGPM_ERR_ARG;
     if (fold < 0 || fold > c->p.pk_folds) return fail(c, HGPM_ERR_ARG, "fold out of range");
     if (!c->have_density) return fail(c, HGPM_ERR_STATE, "no density: call hgpm_cic or hgpm_set_density first");
+    c->have_density = keeps_density(c);
     int rc;
     if (c->prec == HGPM_FP32) {
         {

@@ -85,6 +85,8 @@ namespace hgpm {
 // What the deposit's kernels rely on and leave behind: the control words and mass sums of
 // their set cleared, no chunk listed; cursors, lists and sums used; the other set cleared.
 int dep_stale = 0; // deposits that started from anything else
+// What the grids hold: the density as its reader takes it, the potential (FP32).
+bool holds_density = false, holds_potential = false;
 void launch_deposit_windows(const PosPackH*, int64_t, int ng, float, const DepositBuffers& b, hipStream_t) {
     if (!fake::launch()) return;
     const int nblk = (ng / 16) * (ng / 16) * (ng / 16) * b.nbox;
@@ -97,16 +99,22 @@ void launch_deposit_windows(const PosPackH*, int64_t, int ng, float, const Depos
     for (int i = 0; i < HGPM_DEP_MASS * b.nbox; i++) b.ctl[HGPM_DEP_CTL + 1 + i] += 7;
     for (int i = 0; i < nblk; i++) b.count[i] += 3;
 }
-void launch_deposit_binned(const PosPackH* p, int64_t n, int ng, float m, long long*, float*, const DepositBuffers& b,
-                           hipStream_t s) {
+void launch_deposit_binned(const PosPackH* p, int64_t n, int ng, float m, long long*, float* rhof,
+                           const DepositBuffers& b, hipStream_t s) {
+    holds_density = !rhof;
+    holds_potential = holds_potential && !rhof;
     launch_deposit_windows(p, n, ng, m, b, s);
     memset(b.count, 0, sizeof(unsigned) * (ng / 16) * (ng / 16) * (ng / 16) * b.nbox);
 }
-void launch_deposit_owner(int ng, long long*, float*, const DepositBuffers& b, hipStream_t) {
+void launch_deposit_owner(int ng, long long*, float* rhof, const DepositBuffers& b, hipStream_t) {
+    holds_potential = holds_potential && !rhof; // whether it runs or not
+    holds_density = false;
     if (fake::launch()) memset(b.count, 0, sizeof(unsigned) * (ng / 16) * (ng / 16) * (ng / 16) * b.nbox);
+    holds_density = !rhof;
 }
 void launch_deposit_deferred(const PosPackH*, int64_t, int, float, long long*, const DepositBuffers& b, hipStream_t) {
     if (fake::launch()) memset(b.next, 0, sizeof(unsigned long long) * b.set_words);
+    else holds_density = false;
 }
 void launch_zero_u64(unsigned long long* p, size_t n, hipStream_t) {
     if (fake::launch()) memset(p, 0, sizeof(*p) * n);
@@ -116,7 +124,7 @@ void launch_zero_u64(unsigned long long* p, size_t n, hipStream_t) {
 STUB(launch_drift, PosPackH*, const float*, int64_t, int, float, hipStream_t)
 STUB(launch_compare, const PosPackH*, const float*, const double*, const double*, const PosPackH*, const float*,
      const double*, const double*, int64_t, int, int, double*, hipStream_t)
-STUB(launch_f64_cic, const double*, int64_t, int, double, double2*, hipStream_t)
+void launch_f64_cic(const double*, int64_t, int, double, double2*, hipStream_t) { holds_density = fake::launch(); }
 STUB(launch_f64_fold, double*, int64_t, int, hipStream_t)
 STUB(launch_f64_icic, const double*, double*, const ForceF64&, int64_t, int, double, double, hipStream_t)
 STUB(launch_f64_drift, double*, const double*, int64_t, int, double, hipStream_t)
@@ -162,13 +170,13 @@ FftOps table(int n) {
     f.plane = (size_t)n * f.hz;
     f.twiddles = [](double*, double*) {};
     f.pass_f32 = [](float2*, int, int, const float2*, int, hipStream_t) { (void)fake::launch(); };
-    f.pass_f64 = [](double2*, int, int, const double2*, hipStream_t) { (void)fake::launch(); };
+    f.pass_f64 = [](double2*, int, int, const double2*, hipStream_t) { holds_density = fake::launch() && false; };
     f.force_f64 = [](const double2*, double2*, double*, const double2*, const double2*, int, hipStream_t) { (void)fake::launch(); };
     f.pass_half = [](float2*, int, int, const float2*, int, int, hipStream_t) { (void)fake::launch(); };
     f.fwd_z_r2c = [](const long long*, const float*, const unsigned long long*, const unsigned long long*, float2*,
                      const float2*, int, hipStream_t) { (void)fake::launch(); };
     f.x_psi = [](float2*, const float2*, const float2*, const float*, int, int, hipStream_t) { (void)fake::launch(); };
-    f.inv_z_c2r_real = [](const float2*, float*, const float2*, int, hipStream_t) { (void)fake::launch(); };
+    f.inv_z_c2r_real = [](const float2*, float*, const float2*, int, hipStream_t) { holds_potential = fake::launch(); };
     return f;
 }
 #define TABLE(n) extern const FftOps fft_ops_##n; const FftOps fft_ops_##n = table(n);
@@ -281,11 +289,71 @@ void deposit() {
             hgpm_ensemble_destroy(e);
         }
 }
+
+// A call whose launches fail: what it has overwritten is refused afterwards, what it has
+// not is still there.
+void state() {
+    const hgpm_step_coeffs co{};
+    Spectrum sp;
+    for (int prec : {HGPM_FP32, HGPM_FP64}) {
+        const bool f32 = prec == HGPM_FP32;
+        const size_t n = 32 * 32 * 32;
+        std::vector<double> buf(3 * n);
+        auto density = [&](hgpm_ctx* c) {
+            return f32 ? hgpm_get_density(c, (int64_t*)buf.data()) : hgpm_get_density_f64(c, buf.data());
+        };
+        auto force = [&](hgpm_ctx* c) { return f32 ? hgpm_get_force(c, (float*)buf.data()) : hgpm_get_force_f64(c, buf.data()); };
+        struct Call {
+            const char* name;
+            bool solved; // starts from a force, else from a density
+            std::function<int(hgpm_ctx*)> run;
+        };
+        const Call calls[] = {{"P(k)", true, [&](hgpm_ctx* c) { return sp.of(c, 0); }},
+                              {"folded P(k)", true, [&](hgpm_ctx* c) { return sp.of(c, 1); }},
+                              {"P(k), density", false, [&](hgpm_ctx* c) { return sp.of(c, 0); }},
+                              {"step", true, [&](hgpm_ctx* c) { return hgpm_step(c, &co); }},
+                              {"step, density", false, [&](hgpm_ctx* c) { return hgpm_step(c, &co); }},
+                              {"cic", true, [](hgpm_ctx* c) { return hgpm_cic(c); }},
+                              {"fft", false, [&](hgpm_ctx* c) { return hgpm_fft_host(c, buf.data(), -1); }},
+                              {"solve", false, [](hgpm_ctx* c) { return hgpm_solve_gradient(c); }},
+                              {"grid P(k)", false, [&](hgpm_ctx* c) {
+                                   return hgpm_power_spectrum_grid(c, 0, sp.k, sp.pk, sp.n);
+                               }}};
+        for (const Call& call : calls)
+            for (int at = 0;; at++) {
+                hgpm_ctx* c = box(32, prec);
+                (void)hgpm_cic(c);
+                if (call.solved) (void)hgpm_solve_gradient(c);
+                fake::clear();
+                fake::launch_fails = at;
+                const int rc = call.run(c);
+                const bool failed = fake::launch_no > at;
+                const std::string name = call.name, what = std::string(f32 ? "FP32 " : "FP64 ") + name + " launch " + std::to_string(at);
+                check(rc == (failed ? HGPM_ERR_HIP : HGPM_OK), what + ": reported");
+                fake::clear();
+                const bool has_density = hgpm::holds_density, has_force = !f32 || hgpm::holds_potential;
+                const int d = density(c), f = force(c);
+                check(d == HGPM_ERR_STATE || (d == HGPM_OK && has_density), what + ": density");
+                check(f == HGPM_ERR_STATE || (f == HGPM_OK && has_force), what + ": force");
+                check(hgpm_update_velocities(c, 0.0, 1.0) == f, what + ": kick");
+                check(hgpm_kick_drift(c, 0.0, 1.0, 0.0) == f, what + ": kick and drift");
+                // the transforms of these only read the int64 density
+                if (failed && f32 && (name == "solve" || name == "grid P(k)") && at < 3)
+                    check(d == HGPM_OK, what + ": the density is still there");
+                // P(k) of FP64 leaves the force grids alone until it has its spectrum
+                if (failed && !f32 && call.solved && name == "P(k)" && at == 0)
+                    check(f == HGPM_OK, what + ": the force is still there");
+                hgpm_destroy(c);
+                if (!failed) break;
+            }
+    }
+}
 } // namespace
 
 int main(int argc, char** argv) {
     const std::string s = argc > 1 ? argv[1] : "";
     if (s == "deposit") deposit();
+    else if (s == "state") state();
     else return 3;
     printf("%d %d\n", cases, bad);
     return 0;
