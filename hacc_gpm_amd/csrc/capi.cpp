@@ -138,11 +138,11 @@ template <typename T> int dalloc(hgpm_ctx* c, T** p, size_t bytes, const char* w
 
 // Host arrays to and from the device on the context's stream; both wait for the data.
 int to_host(hgpm_ctx* c, std::initializer_list<HostSeg> s) {
-    HIPCHK(c, copy_to_host(s.begin(), (int)s.size(), c->st));
+    HIPCHK(c, copy_to_host(s.begin(), (int)s.size(), c->device, c->st));
     return HGPM_OK;
 }
 int to_device(hgpm_ctx* c, std::initializer_list<HostSeg> s, int* bad = nullptr) {
-    HIPCHK(c, copy_to_device(s.begin(), (int)s.size(), c->st, bad));
+    HIPCHK(c, copy_to_device(s.begin(), (int)s.size(), c->device, c->st, bad));
     return HGPM_OK;
 }
 

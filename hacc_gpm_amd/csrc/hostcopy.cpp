@@ -68,13 +68,26 @@ std::mutex g_mu;
 std::vector<std::unique_ptr<Ring>>& g_idle = *new std::vector<std::unique_ptr<Ring>>;
 int g_owners = 0;
 
-// A ring on the current device for one transfer; put back by its destructor.
+// The device current for a scope: a ring's events belong to the device that they are made
+// on, and a context may be used from a thread whose current device is another one.
+class OnDevice {
+public:
+    explicit OnDevice(int device) {
+        if (hipGetDevice(&was_) != hipSuccess || was_ == device) was_ = -1;
+        else (void)hipSetDevice(device);
+    }
+    ~OnDevice() {
+        if (was_ >= 0) (void)hipSetDevice(was_);
+    }
+
+private:
+    int was_ = -1;
+};
+
+// A ring on a device, the current one, for one transfer; put back by its destructor.
 class Lease {
 public:
-    hipError_t take() {
-        int dev = 0;
-        hipError_t e = hipGetDevice(&dev);
-        if (e != hipSuccess) return e;
+    hipError_t take(int dev) {
         {
             std::lock_guard<std::mutex> lock(g_mu);
             for (auto& r : g_idle)
@@ -87,7 +100,7 @@ public:
         }
         ring_.reset(new Ring);
         ring_->device = dev;
-        e = hipHostMalloc((void**)&ring_->pin, SLOTS * SLOT, hipHostMallocDefault);
+        hipError_t e = hipHostMalloc((void**)&ring_->pin, SLOTS * SLOT, hipHostMallocDefault);
         if (e != hipSuccess) ring_->pin = nullptr;
         for (int i = 0; i < SLOTS && e == hipSuccess; i++) {
             e = hipEventCreateWithFlags(&ring_->ev[i], hipEventDisableTiming);
@@ -107,13 +120,14 @@ private:
     std::unique_ptr<Ring> ring_;
 };
 
-hipError_t move(const HostSeg* seg, int n, hipStream_t st, bool up, int* bad) {
+hipError_t move(const HostSeg* seg, int n, int device, hipStream_t st, bool up, int* bad) {
     if (bad) *bad = -1;
     size_t total = 0;
     for (int s = 0; s < n; s++) total += seg[s].bytes;
     if (!total) return hipSuccess;
+    OnDevice on(device);
     Lease lease;
-    hipError_t e = lease.take();
+    hipError_t e = lease.take(device);
     if (e != hipSuccess) return e;
     Ring& r = *lease;
     auto slot = [&](int i) { return r.pin + (size_t)(i % SLOTS) * SLOT; };
@@ -200,8 +214,12 @@ hipError_t move(const HostSeg* seg, int n, hipStream_t st, bool up, int* bad) {
 }
 } // namespace
 
-hipError_t copy_to_host(const HostSeg* seg, int n, hipStream_t st) { return move(seg, n, st, false, nullptr); }
-hipError_t copy_to_device(const HostSeg* seg, int n, hipStream_t st, int* bad) { return move(seg, n, st, true, bad); }
+hipError_t copy_to_host(const HostSeg* seg, int n, int device, hipStream_t st) {
+    return move(seg, n, device, st, false, nullptr);
+}
+hipError_t copy_to_device(const HostSeg* seg, int n, int device, hipStream_t st, int* bad) {
+    return move(seg, n, device, st, true, bad);
+}
 
 void host_copy_add_owner() {
     std::lock_guard<std::mutex> lock(g_mu);

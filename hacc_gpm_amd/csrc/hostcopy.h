@@ -21,8 +21,9 @@ struct HostSeg {
 // 1.4-1.7 ms; 32^3 particles (0.8 MB): 0.37 ms, now 0.08 ms.
 // bad: the first segment with a value that fails its check, or -1; every segment is
 // transferred all the same.
-hipError_t copy_to_host(const HostSeg* seg, int n, hipStream_t st);
-hipError_t copy_to_device(const HostSeg* seg, int n, hipStream_t st, int* bad);
+// st is a stream of `device`, which need not be the calling thread's current device.
+hipError_t copy_to_host(const HostSeg* seg, int n, int device, hipStream_t st);
+hipError_t copy_to_device(const HostSeg* seg, int n, int device, hipStream_t st, int* bad);
 
 // Rings are 16 MB, one per transfer under way; up to two idle ones are kept between
 // transfers, while any context lives (add and release one owner each).

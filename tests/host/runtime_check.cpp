@@ -14,12 +14,17 @@
 #include <functional>
 #include <mutex>
 #include <string>
+#include <thread>
 #include <vector>
 
 // ---------------------------------------------------------------- the runtime ----
 namespace fake {
 std::mutex mu;
 thread_local hipError_t last = hipSuccess;
+constexpr int NDEV = 2;
+thread_local int device = 0;
+struct Handle { int device; }; // a stream or an event
+hipError_t make(Handle** h) { return *h = new Handle{device}, hipSuccess; }
 bool capturing = false;     // launches are recorded, not run
 bool graph_fails = false;   // hipGraphLaunch
 int launch_no = 0;          // launches since the last reset ...
@@ -45,9 +50,12 @@ hipError_t hipGetLastError() {
     return e;
 }
 const char* hipGetErrorString(hipError_t e) { return e == hipSuccess ? "no error" : "error"; }
-hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
-hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceCount(int* n) { return *n = fake::NDEV, hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = fake::device, hipSuccess; }
+hipError_t hipSetDevice(int d) {
+    if (d < 0 || d >= fake::NDEV) return err(hipErrorInvalidDevice);
+    return fake::device = d, hipSuccess;
+}
 hipError_t hipMemGetInfo(size_t* f, size_t* t) { return *f = *t = (size_t)4 << 30, hipSuccess; }
 hipError_t hipMalloc(void** p, size_t n) { return *p = calloc(1, n), hipSuccess; }
 hipError_t hipFree(void* p) { return free(p), hipSuccess; }
@@ -59,14 +67,16 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipSt
     return hipSuccess;
 }
 hipError_t hipMemset(void* d, int v, size_t n) { return memset(d, v, n), hipSuccess; }
-hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = (hipStream_t) new int(0), hipSuccess; }
-hipError_t hipStreamDestroy(hipStream_t s) { return delete (int*)s, hipSuccess; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return fake::make((fake::Handle**)s); }
+hipError_t hipStreamDestroy(hipStream_t s) { return delete (fake::Handle*)s, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return *e = (hipEvent_t) new int(0), hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return fake::make((fake::Handle**)e); }
 hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
-hipError_t hipEventDestroy(hipEvent_t e) { return delete (int*)e, hipSuccess; }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { return delete (fake::Handle*)e, hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { // an event belongs to its stream's device
+    return err(((fake::Handle*)e)->device == ((fake::Handle*)s)->device ? hipSuccess : hipErrorInvalidHandle);
+}
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventQuery(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventElapsedTime(float* ms, hipEvent_t, hipEvent_t) { return *ms = 1.0f, hipSuccess; }
@@ -348,12 +358,68 @@ void state() {
             }
     }
 }
+
+// Every host array to and from the device and back, from the calling thread.
+void round_trips(int ng, hgpm_ctx* f32, hgpm_ctx* f64, const std::string& what) {
+    const size_t n = (size_t)ng * ng * ng;
+    std::vector<double> x(3 * n), v(3 * n), a(3 * n), b(3 * n);
+    for (size_t i = 0; i < 3 * n; i++) {
+        x[i] = (double)(i % (16 * ng)) / 16.0;
+        v[i] = (double)i;
+    }
+    check(hgpm_set_particles_f64(f64, x.data(), v.data()) == HGPM_OK, what + ": set FP64 particles");
+    check(hgpm_get_particles_f64(f64, a.data(), b.data()) == HGPM_OK, what + ": get FP64 particles");
+    check(a == x && b == v, what + ": FP64 particles");
+    std::vector<int64_t> q(n), r(n);
+    for (size_t i = 0; i < n; i++) q[i] = (int64_t)i * 3 - 7;
+    check(hgpm_set_density(f32, q.data()) == HGPM_OK, what + ": set density");
+    check(hgpm_get_density(f32, r.data()) == HGPM_OK, what + ": get density");
+    check(q == r, what + ": density");
+    std::vector<float> p(3 * n, 0.5f), w(3 * n, 0.25f);
+    check(hgpm_set_particles(f32, p.data(), w.data()) == HGPM_OK, what + ": set particles");
+    check(hgpm_get_particles(f32, p.data(), w.data()) == HGPM_OK, what + ": get particles");
+    std::vector<float> g(2 * n);
+    for (size_t i = 0; i < 2 * n; i++) g[i] = (float)(i % 1000);
+    const std::vector<float> g0 = g;
+    check(hgpm_fft_host(f32, g.data(), -1) == HGPM_OK, what + ": host FFT");
+    check(g == g0, what + ": host FFT's grid"); // (the passes here leave it as it is)
+}
+
+// Contexts of two devices, used from threads whose current device is either.
+void device() {
+    for (int ng : {32, 64, 96}) {
+        hgpm_ctx *f32[2], *f64[2];
+        for (int d = 0; d < 2; d++) {
+            (void)hipSetDevice(d);
+            f32[d] = box(ng);
+            f64[d] = box(ng, HGPM_FP64);
+        }
+        auto use = [&](int current) {
+            for (int i = 0; i < 4; i++) {
+                (void)hipSetDevice(current);
+                const std::string what = std::to_string(ng) + "^3 device " + std::to_string(i % 2) + " from " + std::to_string(current);
+                round_trips(ng, f32[i % 2], f64[i % 2], what);
+                check(fake::device == current, what + ": the current device is left alone");
+            }
+        };
+        use(0);
+        use(1);
+        std::thread other([&] { use(1); });
+        other.join();
+        for (int d = 0; d < 2; d++) {
+            hgpm_destroy(f32[d]);
+            hgpm_destroy(f64[d]);
+        }
+        (void)hipSetDevice(0);
+    }
+}
 } // namespace
 
 int main(int argc, char** argv) {
     const std::string s = argc > 1 ? argv[1] : "";
     if (s == "deposit") deposit();
     else if (s == "state") state();
+    else if (s == "device") device();
     else return 3;
     printf("%d %d\n", cases, bad);
     return 0;
