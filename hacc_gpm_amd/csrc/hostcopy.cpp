@@ -8,6 +8,7 @@
 #include <exception>
 #include <memory>
 #include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -18,11 +19,11 @@ struct Piece {
     size_t bytes;
     int seg;
 };
-// Copies n bytes of floats and tells whether all of them pass the check (no early exit:
-// the loop vectorises).
-bool copy_checked(char* to, const char* from, size_t n, int check) {
+// Whether all of n bytes of floats pass the check, copied on the way with COPY (no early
+// exit: the loop vectorises).
+template <bool COPY> bool checked(char* to, const char* from, size_t n, int check) {
     if (check == 0) {
-        memcpy(to, from, n);
+        if (COPY) memcpy(to, from, n);
         return true;
     }
     const size_t m = n / sizeof(float);
@@ -31,12 +32,12 @@ bool copy_checked(char* to, const char* from, size_t n, int check) {
     int bad = 0;
     if (check == 1)
         for (size_t i = 0; i < m; i++) {
-            t[i] = f[i];
+            if (COPY) t[i] = f[i];
             bad |= !(std::fabs(f[i]) <= 3.402823466e38f);
         }
     else
         for (size_t i = 0; i < m; i++) {
-            t[i] = f[i];
+            if (COPY) t[i] = f[i];
             bad |= !(std::fabs(f[i]) < 1073741824.0f);
         }
     return !bad;
@@ -65,7 +66,11 @@ struct Ring {
 };
 std::mutex g_mu;
 // never destroyed: a process may end with contexts alive, after the runtime's own end
-std::vector<std::unique_ptr<Ring>>& g_idle = *new std::vector<std::unique_ptr<Ring>>;
+std::vector<std::unique_ptr<Ring>>& g_idle = []() -> std::vector<std::unique_ptr<Ring>>& {
+    auto* v = new std::vector<std::unique_ptr<Ring>>;
+    v->reserve(KEPT); // a ring is put back without an allocation
+    return *v;
+}();
 int g_owners = 0;
 
 // The device current for a scope: a ring's events belong to the device that they are made
@@ -98,7 +103,8 @@ public:
                     return hipSuccess;
                 }
         }
-        ring_.reset(new Ring);
+        ring_.reset(new (std::nothrow) Ring);
+        if (!ring_) return hipErrorOutOfMemory;
         ring_->device = dev;
         hipError_t e = hipHostMalloc((void**)&ring_->pin, SLOTS * SLOT, hipHostMallocDefault);
         if (e != hipSuccess) ring_->pin = nullptr;
@@ -120,6 +126,19 @@ private:
     std::unique_ptr<Ring> ring_;
 };
 
+// The segments one after the other through the runtime's own copy.
+hipError_t move_plain(const HostSeg* seg, int n, hipStream_t st, bool up, int* bad) {
+    hipError_t e = hipSuccess;
+    for (int k = 0; k < n && e == hipSuccess; k++) {
+        if (up && bad && *bad < 0 && !checked<false>(nullptr, (const char*)seg[k].host, seg[k].bytes, seg[k].check))
+            *bad = k;
+        e = up ? hipMemcpyAsync(seg[k].dev, seg[k].host, seg[k].bytes, hipMemcpyHostToDevice, st)
+               : hipMemcpyAsync(seg[k].host, seg[k].dev, seg[k].bytes, hipMemcpyDeviceToHost, st);
+    }
+    const hipError_t w = hipStreamSynchronize(st);
+    return e == hipSuccess ? w : e;
+}
+
 hipError_t move(const HostSeg* seg, int n, int device, hipStream_t st, bool up, int* bad) {
     if (bad) *bad = -1;
     size_t total = 0;
@@ -128,7 +147,10 @@ hipError_t move(const HostSeg* seg, int n, int device, hipStream_t st, bool up, 
     OnDevice on(device);
     Lease lease;
     hipError_t e = lease.take(device);
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) { // no ring to be had (a limit on pinned memory): without one
+        (void)hipGetLastError();
+        return move_plain(seg, n, st, up, bad);
+    }
     Ring& r = *lease;
     auto slot = [&](int i) { return r.pin + (size_t)(i % SLOTS) * SLOT; };
     if (total <= SLOT) {
@@ -137,7 +159,7 @@ hipError_t move(const HostSeg* seg, int n, int device, hipStream_t st, bool up, 
         size_t o = 0;
         for (int k = 0; k < n && e == hipSuccess; o += seg[k++].bytes) {
             char* at = r.pin + o;
-            if (up && !copy_checked(at, (const char*)seg[k].host, seg[k].bytes, seg[k].check) && bad && *bad < 0) *bad = k;
+            if (up && !checked<true>(at, (const char*)seg[k].host, seg[k].bytes, seg[k].check) && bad && *bad < 0) *bad = k;
             e = up ? hipMemcpyAsync(seg[k].dev, at, seg[k].bytes, kind, st)
                    : hipMemcpyAsync(at, seg[k].dev, seg[k].bytes, kind, st);
         }
@@ -173,7 +195,7 @@ hipError_t move(const HostSeg* seg, int n, int device, hipStream_t st, bool up, 
             if (hipEventSynchronize(r.ev[i % SLOTS]) != hipSuccess) failed.store(1);
         }
         if (up) {
-            if (!copy_checked(slot(i), p[i].host, p[i].bytes, seg[p[i].seg].check)) {
+            if (!checked<true>(slot(i), p[i].host, p[i].bytes, seg[p[i].seg].check)) {
                 int b = first_bad.load();
                 while (p[i].seg < b && !first_bad.compare_exchange_weak(b, p[i].seg)) {}
             }

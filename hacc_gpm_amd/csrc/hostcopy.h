@@ -26,7 +26,8 @@ hipError_t copy_to_host(const HostSeg* seg, int n, int device, hipStream_t st);
 hipError_t copy_to_device(const HostSeg* seg, int n, int device, hipStream_t st, int* bad);
 
 // Rings are 16 MB, one per transfer under way; up to two idle ones are kept between
-// transfers, while any context lives (add and release one owner each).
+// transfers, while any context lives (add and release one owner each).  Where the host
+// cannot pin one the segments take the runtime's own copy.
 void host_copy_add_owner();
 void host_copy_release_owner();
 

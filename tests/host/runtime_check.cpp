@@ -8,6 +8,7 @@
 #include "hostcopy.h"
 #include "internal.h"
 
+#include <cmath>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -27,6 +28,8 @@ struct Handle { int device; }; // a stream or an event
 hipError_t make(Handle** h) { return *h = new Handle{device}, hipSuccess; }
 bool capturing = false;     // launches are recorded, not run
 bool graph_fails = false;   // hipGraphLaunch
+bool no_pinned = false;     // hipHostMalloc fails ...
+int events_left = -1;       // ... events do, after so many (< 0: they do not)
 int launch_no = 0;          // launches since the last reset ...
 int launch_fails = -1;      // ... the one that fails (< 0: none)
 void clear() {
@@ -59,7 +62,10 @@ hipError_t hipSetDevice(int d) {
 hipError_t hipMemGetInfo(size_t* f, size_t* t) { return *f = *t = (size_t)4 << 30, hipSuccess; }
 hipError_t hipMalloc(void** p, size_t n) { return *p = calloc(1, n), hipSuccess; }
 hipError_t hipFree(void* p) { return free(p), hipSuccess; }
-hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return *p = malloc(n), hipSuccess; }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+    if (fake::no_pinned) return err(hipErrorOutOfMemory);
+    return *p = malloc(n), hipSuccess;
+}
 hipError_t hipHostFree(void* p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
@@ -71,7 +77,10 @@ hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return fake::mak
 hipError_t hipStreamDestroy(hipStream_t s) { return delete (fake::Handle*)s, hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
-hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return fake::make((fake::Handle**)e); }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+    if (fake::events_left == 0) return err(hipErrorOutOfMemory);
+    if (fake::events_left > 0) fake::events_left--;
+    return fake::make((fake::Handle**)e); }
 hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
 hipError_t hipEventDestroy(hipEvent_t e) { return delete (fake::Handle*)e, hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { // an event belongs to its stream's device
@@ -413,6 +422,40 @@ void device() {
         (void)hipSetDevice(0);
     }
 }
+
+// A host that cannot pin memory, or make events: transfers take the runtime's own copy,
+// and values out of range are refused all the same.
+void unpinned() {
+    for (int ng : {32, 64})
+        for (int how = 0; how < 3; how++) {
+            hgpm_ctx *f32 = box(ng), *f64 = box(ng, HGPM_FP64);
+            const hgpm_params p = params(ng);
+            hgpm_destroy(f32); // (and with the last context its idle rings)
+            hgpm_destroy(f64);
+            fake::no_pinned = how == 0;
+            fake::events_left = how == 0 ? -1 : how == 1 ? 0 : 3;
+            check(hgpm_create(&p, &f32) == HGPM_OK, "create");
+            const hgpm_params p64 = params(ng, HGPM_FP64);
+            check(hgpm_create(&p64, &f64) == HGPM_OK, "create FP64");
+            const std::string what = std::to_string(ng) + "^3, way " + std::to_string(how);
+            round_trips(ng, f32, f64, what);
+            check(hipGetLastError() == hipSuccess, what + ": no error left for the next launch");
+            check(hgpm_cic(f32) == HGPM_OK, what + ": a deposit after it");
+            const size_t n3 = 3 * (size_t)ng * ng * ng;
+            for (size_t at : {(size_t)0, n3 / 2, n3 - 1})
+                for (int velocity = 0; velocity < 2; velocity++) {
+                    std::vector<float> x(n3, 1.0f), v(n3, 1.0f);
+                    (velocity ? v : x)[at] = velocity ? INFINITY : 1073741824.0f;
+                    check(hgpm_set_particles(f32, x.data(), v.data()) == HGPM_ERR_ARG, what + ": refused");
+                    check(strstr(hgpm_last_error(f32), ("index " + std::to_string(at / 3)).c_str()) != nullptr,
+                          what + ": its index");
+                }
+            hgpm_destroy(f32);
+            hgpm_destroy(f64);
+            fake::no_pinned = false;
+            fake::events_left = -1;
+        }
+}
 } // namespace
 
 int main(int argc, char** argv) {
@@ -420,6 +463,7 @@ int main(int argc, char** argv) {
     if (s == "deposit") deposit();
     else if (s == "state") state();
     else if (s == "device") device();
+    else if (s == "unpinned") unpinned();
     else return 3;
     printf("%d %d\n", cases, bad);
     return 0;
