@@ -36,6 +36,13 @@ void clear() {
     launch_no = 0;
     launch_fails = -1;
 }
+const char *lo = nullptr, *hi = nullptr; // a caller's buffer ...
+int direct = 0, copies = 0;              // ... and the copies made from or to it, and in all
+void moved(const void* d, const void* s) {
+    std::lock_guard<std::mutex> lock(mu);
+    copies++;
+    for (const void* p : {d, s}) direct += p >= lo && p < hi;
+}
 hipError_t err(hipError_t e) { return e == hipSuccess ? e : last = e; }
 // One launch: true when its effects happen.
 bool launch() {
@@ -69,6 +76,7 @@ hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
 hipError_t hipHostFree(void* p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return memcpy(d, s, n), hipSuccess; }
 hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
+    fake::moved(d, s);
     if (!fake::capturing) memcpy(d, s, n);
     return hipSuccess;
 }
@@ -84,6 +92,7 @@ hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
 hipError_t hipEventCreate(hipEvent_t* e) { return hipEventCreateWithFlags(e, 0); }
 hipError_t hipEventDestroy(hipEvent_t e) { return delete (fake::Handle*)e, hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) { // an event belongs to its stream's device
+    if (!s) return hipSuccess;
     return err(((fake::Handle*)e)->device == ((fake::Handle*)s)->device ? hipSuccess : hipErrorInvalidHandle);
 }
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
@@ -456,6 +465,54 @@ void unpinned() {
             fake::events_left = -1;
         }
 }
+
+// Transfers of every size at which the route changes, in one segment and in three, with
+// and without a check: the bytes arrive, the route is the one of the size.
+void sizes() {
+    const size_t MB = (size_t)1 << 20;
+    hgpm_ctx* keep = box(32);
+    std::vector<size_t> list = {4, 1000, MB - 4, MB, MB + 4, 2 * MB - 4, 2 * MB, 2 * MB + 4, 4 * MB,
+                                16 * MB + 8, 32 * MB - 4, 32 * MB, 32 * MB + 4, 40 * MB + 12};
+    for (size_t bytes : list)
+        for (int parts : {1, 3})
+            for (int rule = 0; rule < 3; rule++) {
+                std::vector<float> a(bytes / 4), b(bytes / 4), dev(bytes / 4);
+                for (size_t i = 0; i < a.size(); i++) a[i] = (float)(i % 65521);
+                hgpm::HostSeg up[3], down[3];
+                size_t o = 0;
+                for (int k = 0; k < parts; k++) { // uneven parts, none where there are no more bytes
+                    const size_t m = k == parts - 1 ? a.size() - o : a.size() / (k + 3);
+                    up[k] = {a.data() + o, dev.data() + o, 4 * m, rule};
+                    down[k] = {b.data() + o, dev.data() + o, 4 * m};
+                    o += m;
+                }
+                const std::string what = std::to_string(bytes) + " bytes in " + std::to_string(parts) + " check " + std::to_string(rule);
+                int out = -2;
+                fake::lo = (const char*)a.data();
+                fake::hi = fake::lo + bytes;
+                fake::direct = fake::copies = 0;
+                check(hgpm::copy_to_device(up, parts, 0, nullptr, &out) == hipSuccess && out == -1, what + ": up");
+                check(dev == a, what + ": on the device");
+                const bool plain = rule == 0 && bytes > MB && bytes <= 32 * MB;
+                check(plain ? fake::direct == fake::copies : fake::direct == 0, what + ": route up");
+                fake::lo = (const char*)b.data();
+                fake::hi = fake::lo + bytes;
+                fake::direct = 0;
+                check(hgpm::copy_to_host(down, parts, 0, nullptr) == hipSuccess, what + ": down");
+                check(b == a && fake::direct == 0, what + ": back, through the ring");
+                if (rule) { // a bad value anywhere names its segment
+                    for (size_t at : {(size_t)0, a.size() / 2, a.size() - 1}) {
+                        const float was = a[at];
+                        a[at] = rule == 1 ? NAN : -1073741824.0f;
+                        int seg = 0;
+                        while ((char*)&a[at] >= (char*)up[seg].host + up[seg].bytes) seg++;
+                        check(hgpm::copy_to_device(up, parts, 0, nullptr, &out) == hipSuccess && out == seg, what + ": bad value");
+                        a[at] = was;
+                    }
+                }
+            }
+    hgpm_destroy(keep);
+}
 } // namespace
 
 int main(int argc, char** argv) {
@@ -464,6 +521,7 @@ int main(int argc, char** argv) {
     else if (s == "state") state();
     else if (s == "device") device();
     else if (s == "unpinned") unpinned();
+    else if (s == "sizes") sizes();
     else return 3;
     printf("%d %d\n", cases, bad);
     return 0;

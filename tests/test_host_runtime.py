@@ -27,7 +27,7 @@ def exe(tmp_path_factory):
     return str(out)
 
 
-@pytest.mark.parametrize("scenario", ["deposit", "state", "device", "unpinned"])
+@pytest.mark.parametrize("scenario", ["deposit", "state", "device", "unpinned", "sizes"])
 def test_control_code(exe, scenario):
     r = subprocess.run([exe, scenario], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout + r.stderr
