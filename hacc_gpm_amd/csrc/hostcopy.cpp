@@ -146,14 +146,27 @@ hipError_t move_plain(const HostSeg* seg, int n, hipStream_t st, bool up, int* b
     return e == hipSuccess ? w : e;
 }
 
+// Memory the device reads and writes by itself: page-locked, managed or its own.
+bool reachable(const void* p) {
+    hipPointerAttribute_t a;
+    if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+        (void)hipGetLastError(); // pageable, to some versions of the runtime
+        return false;
+    }
+    return a.type != hipMemoryTypeUnregistered;
+}
+
 hipError_t move(const HostSeg* seg, int n, int device, hipStream_t st, bool up, int* bad) {
     if (bad) *bad = -1;
     size_t total = 0;
     for (int s = 0; s < n; s++) total += seg[s].bytes;
     if (!total) return hipSuccess;
-    bool check = false;
+    bool check = false, direct = true;
     for (int s = 0; s < n; s++) check = check || seg[s].check;
-    if (up && !check && total > PLAIN_MIN && total <= PLAIN_MAX) return move_plain(seg, n, st, up, bad);
+    for (int s = 0; s < n && direct; s++) direct = !seg[s].bytes || reachable(seg[s].host);
+    // a checked upload keeps the ring, whose threads check: 128^3 particles from page-locked
+    // memory 1.4 against 2.8 ms
+    if (!check && (direct || (up && total > PLAIN_MIN && total <= PLAIN_MAX))) return move_plain(seg, n, st, up, bad);
     OnDevice on(device);
     Lease lease;
     hipError_t e = lease.take(device);

@@ -20,6 +20,8 @@ struct HostSeg {
 // copy from or to pageable memory pins the caller's pages on each call, on one thread.
 // Measured, reading back 128^3 particles (50 MB, fresh memory): 5.5 ms, through the ring
 // 1.4-1.7 ms; 32^3 particles (0.8 MB): 0.37 ms, now 0.08 ms.
+// Page-locked memory of the caller's is left to the copy engine (57 GB/s; through the ring
+// 2 MB come back in 121 us instead of 45, 128 MB in 3.5 ms instead of 2.4).
 // bad: the first segment with a value that fails its check, or -1; every segment is
 // transferred all the same.
 // st is a stream of `device`, which need not be the calling thread's current device.

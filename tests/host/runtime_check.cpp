@@ -36,6 +36,7 @@ void clear() {
     launch_no = 0;
     launch_fails = -1;
 }
+int memory = 0; // what a caller's buffers are: 0 unknown to the runtime, 1 unregistered, 2 page-locked
 const char *lo = nullptr, *hi = nullptr; // a caller's buffer ...
 int direct = 0, copies = 0;              // ... and the copies made from or to it, and in all
 void moved(const void* d, const void* s) {
@@ -72,6 +73,11 @@ hipError_t hipFree(void* p) { return free(p), hipSuccess; }
 hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
     if (fake::no_pinned) return err(hipErrorOutOfMemory);
     return *p = malloc(n), hipSuccess;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) {
+    if (fake::memory == 0) return err(hipErrorInvalidValue);
+    a->type = fake::memory == 1 ? hipMemoryTypeUnregistered : hipMemoryTypeHost;
+    return hipSuccess;
 }
 hipError_t hipHostFree(void* p) { return free(p), hipSuccess; }
 hipError_t hipMemcpy(void* d, const void* s, size_t n, hipMemcpyKind) { return memcpy(d, s, n), hipSuccess; }
@@ -467,7 +473,7 @@ void unpinned() {
 }
 
 // Transfers of every size at which the route changes, in one segment and in three, with
-// and without a check: the bytes arrive, the route is the one of the size.
+// and without a check, memory of each kind: the bytes arrive, the route is the one of the size.
 void sizes() {
     const size_t MB = (size_t)1 << 20;
     hgpm_ctx* keep = box(32);
@@ -475,14 +481,15 @@ void sizes() {
                                 16 * MB + 8, 32 * MB - 4, 32 * MB, 32 * MB + 4, 40 * MB + 12};
     for (size_t bytes : list)
         for (int parts : {1, 3})
-            for (int rule = 0; rule < 3; rule++) {
+            for (int rule = 0; rule < 9; rule++) {
+                const int memory = fake::memory = rule / 3; // rule % 3: the check
                 std::vector<float> a(bytes / 4), b(bytes / 4), dev(bytes / 4);
                 for (size_t i = 0; i < a.size(); i++) a[i] = (float)(i % 65521);
                 hgpm::HostSeg up[3], down[3];
                 size_t o = 0;
                 for (int k = 0; k < parts; k++) { // uneven parts, none where there are no more bytes
                     const size_t m = k == parts - 1 ? a.size() - o : a.size() / (k + 3);
-                    up[k] = {a.data() + o, dev.data() + o, 4 * m, rule};
+                    up[k] = {a.data() + o, dev.data() + o, 4 * m, rule % 3};
                     down[k] = {b.data() + o, dev.data() + o, 4 * m};
                     o += m;
                 }
@@ -493,17 +500,18 @@ void sizes() {
                 fake::direct = fake::copies = 0;
                 check(hgpm::copy_to_device(up, parts, 0, nullptr, &out) == hipSuccess && out == -1, what + ": up");
                 check(dev == a, what + ": on the device");
-                const bool plain = rule == 0 && bytes > MB && bytes <= 32 * MB;
+                const bool plain = rule % 3 == 0 && (memory == 2 || (bytes > MB && bytes <= 32 * MB));
                 check(plain ? fake::direct == fake::copies : fake::direct == 0, what + ": route up");
                 fake::lo = (const char*)b.data();
                 fake::hi = fake::lo + bytes;
-                fake::direct = 0;
+                fake::direct = fake::copies = 0;
                 check(hgpm::copy_to_host(down, parts, 0, nullptr) == hipSuccess, what + ": down");
-                check(b == a && fake::direct == 0, what + ": back, through the ring");
-                if (rule) { // a bad value anywhere names its segment
+                check(b == a && fake::direct == (memory == 2 ? fake::copies : 0), what + ": back, and its route");
+                check(hipGetLastError() == hipSuccess, what + ": no error left for the next launch");
+                if (rule % 3) { // a bad value anywhere names its segment
                     for (size_t at : {(size_t)0, a.size() / 2, a.size() - 1}) {
                         const float was = a[at];
-                        a[at] = rule == 1 ? NAN : -1073741824.0f;
+                        a[at] = rule % 3 == 1 ? NAN : -1073741824.0f;
                         int seg = 0;
                         while ((char*)&a[at] >= (char*)up[seg].host + up[seg].bytes) seg++;
                         check(hgpm::copy_to_device(up, parts, 0, nullptr, &out) == hipSuccess && out == seg, what + ": bad value");
@@ -511,6 +519,7 @@ void sizes() {
                     }
                 }
             }
+    fake::memory = 0;
     hgpm_destroy(keep);
 }
 } // namespace
