@@ -331,10 +331,10 @@ int f32_deposit(hgpm_ctx* c, bool fused = false, int fold = 0) {
             launch_deposit_windows(c->pos, c->N * c->nbox, c->ng, ref_mass(c), b, c->st);
             c->boxes_valid = true;
         }
-        Timed t2(c, "deposit_owner");
-        launch_deposit_owner(c->ng, (long long*)c->B, fused ? c->psi : nullptr, b, c->st);
-    }
-    {
+        {
+            Timed t2(c, "deposit_owner");
+            launch_deposit_owner(c->ng, (long long*)c->B, fused ? c->psi : nullptr, b, c->st);
+        }
         Timed t3(c, "deposit_deferred");
         launch_deposit_deferred(c->pos, c->N * c->nbox, c->ng, ref_mass(c), (long long*)c->B, b, c->st);
     }

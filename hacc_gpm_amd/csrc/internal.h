@@ -145,9 +145,10 @@ void launch_deposit_owner(int ng, long long* rho, float* rhof, const DepositBuff
 // the tiles listed as deferred, and the other set of control words made ready
 void launch_deposit_deferred(const PosPackH* pos, int64_t np3, int ng, float mass, long long* rho,
                              const DepositBuffers& b, hipStream_t s);
-// The deposit of one box's folded positions (b.fold > 0), before launch_deposit_deferred in
-// place of the windows and owner passes: rho / rhof as
-// launch_deposit_owner writes them.
+// The deposit of one box's folded positions (b.fold > 0), in place of the windows, owner and
+// deferred passes: rho / rhof as launch_deposit_owner writes them, the other set of control
+// words made ready.  ctl[1] counts the tiles that took the atomic route, or the pieces of
+// crowded owner blocks that were added to the grid by it.
 void launch_deposit_binned(const PosPackH* pos, int64_t np3, int ng, float mass, long long* rho, float* rhof,
                            const DepositBuffers& b, hipStream_t s);
 // variant 0: 512-thread workgroups on half tiles; 1: 256-thread workgroups on quarter tiles

@@ -1115,23 +1115,12 @@ __device__ __forceinline__ void dep_next(const unsigned long long* __restrict ct
     }
 }
 
-// Tiles listed by k_deposit_windows as deferred, after k_deposit_owner: int64 atomics.
-// Bound by the slabs of wide tiles, each a barrier apart: two workgroups a CU (80 KB of LDS
-// each, four waves per SIMD) cover for one another where their registers allow it, 128 for
-// 32-bit weights without a spill.  With 131, one workgroup a CU: 16.8 M particles in any
-// order on 256^3 109 ms a deposit against 68 (all tiles deferred).
+// The nd tiles listed in deferred: int64 atomics.
 template <bool SMALL, int PPT, typename POS>
-__global__ __launch_bounds__(DEP_NT, SMALL ? 4 : 1) void k_deposit_deferred(POS pos, int64_t n, int ng,
-                                                             float mass, unsigned long long* __restrict rho,
-                                                             const unsigned long long* __restrict ctl,
-                                                             const unsigned* __restrict deferred,
-                                                             unsigned long long* __restrict mass_sum, int ntb,
-                                                             int64_t gcells, DepNext next) {
-    __shared__ unsigned long long win[DEP_LDS / 8];
-    __shared__ int red[12][DEP_NT / 64];
-    __shared__ long long s_tot[DEP_NT / 64];
-    if (blockIdx.x == 0) dep_next(ctl, next);
-    const unsigned long long nd = ctl[1];
+__device__ __forceinline__ void dep_deferred_tiles(const POS& pos, int ng, float mass, unsigned long long* __restrict rho,
+                                                   unsigned long long nd, const unsigned* __restrict deferred,
+                                                   unsigned long long* __restrict mass_sum, int ntb, int64_t gcells,
+                                                   unsigned long long* win, int (*red)[DEP_NT / 64], long long* s_tot) {
     for (unsigned long long q = blockIdx.x; q < nd; q += gridDim.x) {
         const unsigned tile = deferred[q];
         const int64_t p0 = (int64_t)tile * (DEP_NT * PPT);
@@ -1144,6 +1133,25 @@ __global__ __launch_bounds__(DEP_NT, SMALL ? 4 : 1) void k_deposit_deferred(POS 
         dep_tile_total(local, s_tot, dep_mass_slot(mass_sum, (int)tile, ntb));
         __syncthreads();
     }
+}
+// Tiles listed by k_deposit_windows as deferred, after k_deposit_owner.
+// Bound by the slabs of wide tiles, each a barrier apart: two workgroups a CU (80 KB of LDS
+// each, four waves per SIMD) cover for one another where their registers allow it, 128 for
+// 32-bit weights without a spill.  With 131, one workgroup a CU: 16.8 M particles in any
+// order on 256^3 109 ms a deposit against 68 (all tiles deferred).
+template <bool SMALL, int PPT>
+__global__ __launch_bounds__(DEP_NT, SMALL ? 4 : 1) void k_deposit_deferred(const PosPack* __restrict pos, int ng,
+                                                             float mass, unsigned long long* __restrict rho,
+                                                             const unsigned long long* __restrict ctl,
+                                                             const unsigned* __restrict deferred,
+                                                             unsigned long long* __restrict mass_sum, int ntb,
+                                                             int64_t gcells, DepNext next) {
+    __shared__ unsigned long long win[DEP_LDS / 8];
+    __shared__ int red[12][DEP_NT / 64];
+    __shared__ long long s_tot[DEP_NT / 64];
+    if (blockIdx.x == 0) dep_next(ctl, next);
+    dep_deferred_tiles<SMALL, PPT>(StoredPos{pos}, ng, mass, rho, ctl[1], deferred, mass_sum, ntb, gcells, win, red,
+                                   s_tot);
 }
 
 // ----------------------------------------------------------------------------------
@@ -1159,8 +1167,14 @@ __global__ __launch_bounds__(DEP_NT, SMALL ? 4 : 1) void k_deposit_deferred(POS 
 //   k_bin_scan        : where each block's entries start in the arena;
 //   k_bin_pass<true>  : the folded positions written there;
 //   k_bin_owner       : a workgroup per block adds its entries' weights in int64 LDS cells
-//                       and writes every cell once.
-// The sums are whole numbers, so the bits are those of every other route.  Entries beyond
+//                       and writes every cell once;
+//   k_bin_rest        : the entries of a block past the first BIN_PIECE, a workgroup per
+//                       piece, added to the grid with atomics (the density is then the
+//                       int64 one, as after deferred tiles).
+// A block is one workgroup's serial work, so without the pieces a box whose particles
+// crowd into few blocks took as long as one workgroup needs for most of them: a fold's P(k)
+// of 16.8 M in one cell of 256^3 52 to 112 ms (now 0.7), in a clump of two cells' width 11
+// (0.7).  The sums are whole numbers, so the bits are those of every other route.  Entries beyond
 // the arena send the deposit to the atomic route (all tiles listed as deferred).  Bound by
 // the scattered writes, the LDS atomics and the memory it moves (about 60 bytes a
 // particle).  Evolved boxes, np = ng, one fold: 0.39 ms at 256^3 (count 0.106, write 0.127,
@@ -1171,6 +1185,9 @@ __global__ __launch_bounds__(DEP_NT, SMALL ? 4 : 1) void k_deposit_deferred(POS 
 // fold 1 where np = ng, twice that with each fold until it is the grid's width.
 constexpr int BIN_W = 20;
 constexpr int BIN_SLOTS = BIN_W * BIN_W * BIN_W; // 32 KB of counters
+// 6 times the mean of a block at np = ng: evolved boxes of ordinary runs stay below it
+constexpr unsigned BIN_PIECE = 32768;
+constexpr int BIN_CTL_PIECES = DEP_CTL_SUB; // ctl word (no sub-arenas here): deferred lists pieces, not tiles
 struct BinArgs {
     const PosPack* __restrict pos;
     int ng, fold;
@@ -1181,7 +1198,8 @@ struct BinArgs {
     unsigned* __restrict start;  // per block: first entry ...
     unsigned* __restrict cursor; // ... and the next free one (k_bin_pass<true>)
     unsigned long long* __restrict ctl;
-    unsigned* __restrict deferred;
+    unsigned* __restrict deferred; // tiles, or blocks of pieces: at most 8 n / BIN_PIECE ...
+    unsigned* __restrict piece;    // ... and their first entries (both hold n / 2048)
     unsigned long long* __restrict mass_sum;
     unsigned long long* __restrict rho;
     float* __restrict rhof; // see OwnerArgs
@@ -1242,7 +1260,7 @@ __device__ __forceinline__ void bin_blocks(const PosPack& q, int ng, const BinBo
 template <bool SMALL, bool FILL> __global__ __launch_bounds__(DEP_NT) void k_bin_pass(BinArgs g) {
     __shared__ unsigned num[BIN_SLOTS];
     __shared__ long long s_tot[DEP_NT / 64];
-    if (FILL && g.ctl[1]) return; // the entries do not fit: the atomic route
+    if (FILL && g.ctl[1] && !g.ctl[BIN_CTL_PIECES]) return; // the entries do not fit: the atomic route
     const int tid = threadIdx.x;
     const int tile = (int)xcd_remap(blockIdx.x, gridDim.x);
     const PosPack* __restrict at = g.pos + (int64_t)tile * DEP_TILE; // tiles are full
@@ -1293,7 +1311,9 @@ template <bool SMALL, bool FILL> __global__ __launch_bounds__(DEP_NT) void k_bin
 constexpr int BIN_SCAN = 1024;
 __global__ __launch_bounds__(BIN_SCAN) void k_bin_scan(BinArgs g) {
     __shared__ unsigned long long s[BIN_SCAN];
+    __shared__ unsigned s_pieces;
     const int tid = threadIdx.x;
+    if (tid == 0) s_pieces = 0u; // ordered by the barriers of the scan
     const int per = (g.nblk + BIN_SCAN - 1) / BIN_SCAN, b0 = min(tid * per, g.nblk), b1 = min(b0 + per, g.nblk);
     unsigned long long t = 0;
     for (int b = b0; b < b1; b++) t += g.count[b];
@@ -1318,25 +1338,26 @@ __global__ __launch_bounds__(BIN_SCAN) void k_bin_scan(BinArgs g) {
         const unsigned n = g.count[b];
         g.start[b] = (unsigned)t;
         g.cursor[b] = (unsigned)t;
+        if (n > BIN_PIECE) {
+            unsigned q = atomicAdd(&s_pieces, (n - 1u) / BIN_PIECE);
+            for (unsigned o = BIN_PIECE; o < n; o += BIN_PIECE, q++) {
+                g.deferred[q] = (unsigned)b;
+                g.piece[q] = (unsigned)t + o;
+            }
+        }
         t += n;
     }
-}
-template <bool SMALL> __global__ __launch_bounds__(OWN_NT) void k_bin_owner(BinArgs g) {
-    __shared__ unsigned long long acc[OB * OB * OB];
-    __shared__ unsigned s_n, s_at;
-    const int tid = threadIdx.x, ng = g.ng, nb = ng / OB;
-    const int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
-    const int b[3] = {blk / (nb * nb) * OB, blk / nb % nb * OB, blk % nb * OB};
-    if (tid == 0) {
-        s_n = g.count[blk];
-        s_at = g.start[blk]; // not read when the block has no entries
-        g.count[blk] = 0u;
-    }
-    for (int i = tid; i < OB * OB * OB; i += OWN_NT) acc[i] = 0ull;
     __syncthreads();
-    const unsigned n = s_n;
-    const PosPack* __restrict e = g.entries + s_at;
-    for (unsigned i = tid; i < n; i += OWN_NT) {
+    if (tid == 0 && s_pieces) {
+        g.ctl[1] = s_pieces;
+        g.ctl[BIN_CTL_PIECES] = 1ull;
+    }
+}
+// Adds the weights of n entries to the LDS cells of the block with first cell b.
+template <bool SMALL, int WG>
+__device__ __forceinline__ void bin_add(unsigned long long* acc, const PosPack* __restrict e, unsigned n, const int b[3],
+                                        int ng, float mass) {
+    for (unsigned i = threadIdx.x; i < n; i += WG) {
         const PosPack q = e[i];
         const unsigned X[3] = {q.x, q.y, q.z};
         int c[3];
@@ -1353,9 +1374,24 @@ template <bool SMALL> __global__ __launch_bounds__(OWN_NT) void k_bin_owner(BinA
             const int x = c[0] + (k >> 2), y = c[1] + ((k >> 1) & 1), z = c[2] + (k & 1);
             if ((unsigned)x < (unsigned)OB && (unsigned)y < (unsigned)OB && (unsigned)z < (unsigned)OB)
                 atomicAdd(&acc[(x * OB + y) * OB + z], (unsigned long long)fixed_weight<SMALL>(
-                                                           w[0][k >> 2], w[1][(k >> 1) & 1], w[2][k & 1], g.mass));
+                                                           w[0][k >> 2], w[1][(k >> 1) & 1], w[2][k & 1], mass));
         }
     }
+}
+template <bool SMALL> __global__ __launch_bounds__(OWN_NT) void k_bin_owner(BinArgs g) {
+    __shared__ unsigned long long acc[OB * OB * OB];
+    __shared__ unsigned s_n, s_at;
+    const int tid = threadIdx.x, ng = g.ng, nb = ng / OB;
+    const int blk = (int)xcd_remap(blockIdx.x, gridDim.x);
+    const int b[3] = {blk / (nb * nb) * OB, blk / nb % nb * OB, blk % nb * OB};
+    if (tid == 0) {
+        s_n = g.count[blk];
+        s_at = g.start[blk]; // not read when the block has no entries
+        g.count[blk] = 0u;
+    }
+    for (int i = tid; i < OB * OB * OB; i += OWN_NT) acc[i] = 0ull;
+    __syncthreads();
+    bin_add<SMALL, OWN_NT>(acc, g.entries + s_at, min(s_n, BIN_PIECE), b, ng, g.mass);
     __syncthreads();
     const bool f32 = g.rhof != nullptr && g.ctl[1] == 0ull;
     const double mean = (double)box_mass(g.mass_sum, 0) / (double)g.gcells;
@@ -1363,6 +1399,35 @@ template <bool SMALL> __global__ __launch_bounds__(OWN_NT) void k_bin_owner(BinA
         const int64_t at = gidx(ng, b[0] + i / (OB * OB), b[1] + i / OB % OB, b[2] + i % OB);
         if (f32) g.rhof[at] = (float)(((double)(long long)acc[i] - mean) * (1.0 / 16777216.0));
         else g.rho[at] = acc[i];
+    }
+}
+// What k_bin_owner left: the pieces of crowded blocks, or every tile where the entries did
+// not fit.
+template <bool SMALL>
+__global__ __launch_bounds__(DEP_NT, SMALL ? 4 : 1) void k_bin_rest(BinArgs g, DepNext next) {
+    __shared__ unsigned long long win[DEP_LDS / 8];
+    __shared__ int red[12][DEP_NT / 64];
+    __shared__ long long s_tot[DEP_NT / 64];
+    static_assert(OB * OB * OB <= DEP_LDS / 8, "a block's cells");
+    if (blockIdx.x == 0) dep_next(g.ctl, next);
+    const unsigned long long nd = g.ctl[1];
+    if (!g.ctl[BIN_CTL_PIECES]) {
+        dep_deferred_tiles<SMALL, DEP_PPT>(FoldedPos{g.pos, g.fold, g.ng}, g.ng, g.mass, g.rho, nd, g.deferred,
+                                           g.mass_sum, g.nt, g.gcells, win, red, s_tot);
+        return;
+    }
+    const int nb = g.ng / OB;
+    for (unsigned long long q = blockIdx.x; q < nd; q += gridDim.x) {
+        const int blk = (int)g.deferred[q];
+        const unsigned at = g.piece[q], n = min(g.cursor[blk] - at, BIN_PIECE); // (the cursor is past the last entry)
+        const int b[3] = {blk / (nb * nb) * OB, blk / nb % nb * OB, blk % nb * OB};
+        for (int i = threadIdx.x; i < OB * OB * OB; i += DEP_NT) win[i] = 0ull;
+        __syncthreads();
+        bin_add<SMALL, DEP_NT>(win, g.entries + at, n, b, g.ng, g.mass);
+        __syncthreads();
+        for (int i = threadIdx.x; i < OB * OB * OB; i += DEP_NT)
+            if (win[i]) atomicAdd(&g.rho[gidx(g.ng, b[0] + i / (OB * OB), b[1] + i / OB % OB, b[2] + i % OB)], win[i]);
+        __syncthreads();
     }
 }
 
@@ -1962,21 +2027,20 @@ void launch_deposit_deferred(const PosPackH* pos, int64_t n, int ng, float mass,
     const int64_t gc = (int64_t)ng * ng * ng;
     const unsigned grid = (unsigned)(nt < 512 ? nt : 512);
     unsigned long long* mass_sum = b.ctl + HGPM_DEP_CTL + 1;
-    const unsigned long long nall = (unsigned long long)(ng / OB) * (ng / OB) * (ng / OB) * b.nbox;
-    const DepNext next{b.next, b.set_words, b.fold ? 0ull : nall};
-    auto run = [&](auto pc, auto p) {
+    const DepNext next{b.next, b.set_words, (unsigned long long)(ng / OB) * (ng / OB) * (ng / OB) * b.nbox};
+    auto run = [&](auto pc) {
         constexpr int PPT = decltype(pc)::value;
         if (mass < 128.0f)
-            k_deposit_deferred<true, PPT><<<grid, DEP_NT, 0, s>>>(p, n, ng, mass, (unsigned long long*)rho, b.ctl,
-                                                                  b.deferred, mass_sum, ntb, gc, next);
+            k_deposit_deferred<true, PPT><<<grid, DEP_NT, 0, s>>>((const PosPack*)pos, ng, mass,
+                                                                  (unsigned long long*)rho, b.ctl, b.deferred,
+                                                                  mass_sum, ntb, gc, next);
         else
-            k_deposit_deferred<false, PPT><<<grid, DEP_NT, 0, s>>>(p, n, ng, mass, (unsigned long long*)rho, b.ctl,
-                                                                   b.deferred, mass_sum, ntb, gc, next);
+            k_deposit_deferred<false, PPT><<<grid, DEP_NT, 0, s>>>((const PosPack*)pos, ng, mass,
+                                                                   (unsigned long long*)rho, b.ctl, b.deferred,
+                                                                   mass_sum, ntb, gc, next);
     };
-    const StoredPos sp{(const PosPack*)pos};
-    if (b.fold) run(std::integral_constant<int, 8>{}, FoldedPos{(const PosPack*)pos, b.fold, ng});
-    else if (b.ppt == 4) run(std::integral_constant<int, 4>{}, sp);
-    else run(std::integral_constant<int, 8>{}, sp);
+    if (b.ppt == 4) run(std::integral_constant<int, 4>{});
+    else run(std::integral_constant<int, 8>{});
 }
 void launch_deposit_binned(const PosPackH* pos, int64_t n, int ng, float mass, long long* rho, float* rhof,
                            const DepositBuffers& b, hipStream_t s) {
@@ -1994,17 +2058,20 @@ void launch_deposit_binned(const PosPackH* pos, int64_t n, int ng, float mass, l
     g.cursor = g.start + g.nblk;
     g.ctl = b.ctl;
     g.deferred = b.deferred;
+    g.piece = b.wide;
     g.mass_sum = b.ctl + HGPM_DEP_CTL + 1;
     g.rho = (unsigned long long*)rho;
     g.rhof = rhof;
     g.nt = (int)(n / DEP_TILE);
     g.gcells = (int64_t)ng * ng * ng;
+    const DepNext next{b.next, b.set_words, 0ull};
     auto run = [&](auto sc) {
         constexpr bool SMALL = decltype(sc)::value;
         k_bin_pass<SMALL, false><<<(unsigned)g.nt, DEP_NT, 0, s>>>(g);
         k_bin_scan<<<1, BIN_SCAN, 0, s>>>(g);
         k_bin_pass<SMALL, true><<<(unsigned)g.nt, DEP_NT, 0, s>>>(g);
         k_bin_owner<SMALL><<<(unsigned)g.nblk, OWN_NT, 0, s>>>(g);
+        k_bin_rest<SMALL><<<(unsigned)std::min(g.nt, 512), DEP_NT, 0, s>>>(g, next);
     };
     if (mass < 128.0f) run(std::true_type{});
     else run(std::false_type{});

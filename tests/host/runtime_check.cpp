@@ -139,6 +139,8 @@ void launch_deposit_binned(const PosPackH* p, int64_t n, int ng, float m, long l
     holds_potential = holds_potential && !rhof;
     launch_deposit_windows(p, n, ng, m, b, s);
     memset(b.count, 0, sizeof(unsigned) * (ng / 16) * (ng / 16) * (ng / 16) * b.nbox);
+    if (fake::launch()) memset(b.next, 0, sizeof(unsigned long long) * b.set_words);
+    else holds_density = false;
 }
 void launch_deposit_owner(int ng, long long*, float* rhof, const DepositBuffers& b, hipStream_t) {
     holds_potential = holds_potential && !rhof; // whether it runs or not

@@ -790,6 +790,39 @@ def test_power_spectrum_folded_lattice(hg, orc, ng, np_, folds, nb, sigma):
             c, o = orc.fold_split(ng, c, o)
 
 
+@pytest.mark.parametrize("ng,np_,kind,pieces", [(64, 64, "cell", 7), (64, 64, "edge", 14), (64, 64, "corner", 64),
+                                                (64, 64, "counts", 4), (128, 32, "corner", 0), (384, 64, "cell", 7),
+                                                (64, 64, "clump", None)])
+def test_power_spectrum_folded_crowded(hg, orc, ng, np_, kind, pieces):
+    """Folded positions crowded into few owner blocks, whose entries past the first 32768 are
+    added piece by piece: all in one cell; on the edge of two blocks (as many entries as the
+    arena holds) and on a corner of eight (more than that, the atomic route, and one piece
+    each); blocks of exactly one and two pieces and of one entry more; mass 216 (weights over
+    31 bits); a clump.  The bits of the oracle's density, and of the atomic route."""
+    case(f"power folded crowded ng={ng} np={np_} {kind}")
+    rng = np.random.default_rng(ng)
+    n = np_ ** 3
+    if kind == "counts":
+        org = rng.permutation(np.repeat(np.arange(6), [32768, 32769, 65536, 65537, 32767, 32767]))
+        y = 16.0 * np.stack([org % 2, org // 2 % 2, org // 4], 1) + 2.0 + 12.0 * rng.random((n, 3))
+    else:
+        y = np.array({"cell": 20.0, "edge": [15.0, 20.0, 20.0], "corner": 15.0, "clump": 0.0}[kind]) + rng.random((n, 3))
+        if kind == "clump":
+            y = (17.0 + rng.normal(0, 2.0, (n, 3))) % ng
+    cell, off = split_of(y / 2, ng)  # folded once: y
+    with mk(hg, ng, np_, pk_bins=32, pk_folds=1) as m:
+        m.set_particles_split(cell, off, np.zeros((n, 3), np.float32))
+        k, pk, cnt = m.power_spectrum(1)
+        got = m.get_tunable("deposit_deferred")
+        assert 0 < got <= n // 4096 if pieces is None else got == pieces
+        q = orc.cic_split(ng, *orc.fold_split(ng, cell, off), float((np.float32(ng) / np.float32(np_)) ** 3))
+        m.set_density(q)  # the oracle's density through the same transform and bins
+        kq, pkq, cntq = m.power_spectrum(1, from_grid=True)
+        assert np.array_equal(pk, pkq) and np.array_equal(cnt, cntq) and np.array_equal(k, kq)
+        m.set_tunable("deposit_arena", 1000)
+        assert np.array_equal(m.power_spectrum(1)[1], pk) and m.get_tunable("deposit_deferred") == n // 4096
+
+
 def test_power_spectrum_fp64(hg, orc):
     case("power fp64 ng=32")
     ng, nb = 32, 16
