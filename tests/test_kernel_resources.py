@@ -27,7 +27,8 @@ def kernels():
     return out
 
 
-@pytest.mark.parametrize("kernel,n", [("k_deposit_windowsILb1E", 4), ("k_deposit_deferredILb1E", 3)])
+@pytest.mark.parametrize("kernel,n", [("k_deposit_windowsILb1E", 4), ("k_deposit_deferredILb1E", 2),
+                                      ("k_bin_restILb1E", 1)])
 def test_two_workgroups_per_cu(kernels, kernel, n):
     """512 threads are two waves per SIMD: two workgroups need four.  32-bit weights (Lb1)."""
     found = {k: v for k, v in kernels.items() if kernel in k}
