@@ -57,11 +57,7 @@ struct hgpm_ctx {
     int set_words = 0;                 // words of a set: control words, mass partial sums per box
     int set_next = 0;                  // the set of the next deposit; the other is the last one's
     bool dep_dirty = false;            // a deposit's launches failed: its words, sums and counts may be anything
-    // the force components' grids (FP64)
-    ForceF64 force64() const {
-        const double* g = (const double*)grad64;
-        return {{g + 2 * G, g + 3 * G, g}};
-    }
+    double* force64() const { return (double*)grad64; } // FP64: three components a cell
     unsigned long long* last_ctl() const { return ctl + (size_t)(set_next ^ 1) * set_words; }
     unsigned long long* last_mass() const { return last_ctl() + HGPM_DEP_CTL + 1; }
     // deposit arena route (k_particles.hip): window arena, per-owner-block chunk slots
@@ -80,7 +76,8 @@ struct hgpm_ctx {
     float* hs = nullptr; // sin^2(pi m/ng), the Green's function's per-axis terms
     // FP64 plain path
     double *pos64 = nullptr, *vel64 = nullptr;
-    double2 *grid64 = nullptr, *grad64 = nullptr; // grad64: a work grid, then F_x and F_y; F_z over the work grid
+    // grad64 (40 bytes a cell): the force; in the solve a work grid in its place, F_x and F_y behind
+    double2 *grid64 = nullptr, *grad64 = nullptr;
     double2* modes64 = nullptr;                   // cos, sin of the grid's wavenumbers
     double2 *tw64 = nullptr, *tw64_ic = nullptr;
     // P(k)
@@ -392,10 +389,11 @@ int f64_solve(hgpm_ctx* c) {
     int rc = fft3d_f64(c, c->fft, c->grid64, c->tw64, -1);
     if (rc) return rc;
     Timed t(c, "f64_force");
-    const ForceF64 F = c->force64();
-    for (int d = 0; d < 3; d++) // z last: over the density's modes
-        c->fft->force_f64(c->grid64, d < 2 ? c->grad64 : c->grid64, const_cast<double*>(F.f[d]), c->tw64, c->modes64, d,
-                          c->st);
+    double *F = c->force64(), *fx = F + 3 * c->G, *fy = F + 4 * c->G;
+    c->fft->force_f64(c->grid64, c->grad64, fx, nullptr, nullptr, c->tw64, c->modes64, 0, c->st);
+    c->fft->force_f64(c->grid64, c->grad64, fy, nullptr, nullptr, c->tw64, c->modes64, 1, c->st);
+    // z last: over the density's modes
+    c->fft->force_f64(c->grid64, c->grid64, F, fx, fy, c->tw64, c->modes64, 2, c->st);
     LAUNCHCHK(c);
     return HGPM_OK;
 }
@@ -585,8 +583,7 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
             return bail(HGPM_ERR_HIP);
         }
     } else {
-        size_t grad_bytes = sizeof(double) * 4 * G;
-        if (grad_bytes < sizeof(double) * 3 * N) grad_bytes = sizeof(double) * 3 * N;
+        const size_t grad_bytes = sizeof(double) * 5 * G;
         if ((rc = dalloc(c, &c->pos64, sizeof(double) * 3 * N, "pos64")) ||
             (rc = dalloc(c, &c->vel64, sizeof(double) * 3 * N, "vel64")) ||
             (rc = dalloc(c, &c->grid64, sizeof(double2) * G, "grid64")) ||
@@ -1142,15 +1139,7 @@ int hgpm_get_force_f64(hgpm_ctx* c, double* f) {
         for (size_t i = 0; i < t.size(); i++) f[i] = t[i];
         return HGPM_OK;
     }
-    double* tmp = nullptr;
-    int rc = dalloc(c, &tmp, sizeof(double) * 3 * c->G, "staging");
-    if (rc) return rc;
-    c->bytes -= sizeof(double) * 3 * c->G;
-    launch_f64_force_out(c->force64(), tmp, c->G, c->st);
-    LAUNCHCHK(c);
-    rc = to_host(c, {{f, tmp, sizeof(double) * 3 * c->G}});
-    (void)hipFree(tmp);
-    return rc;
+    return to_host(c, {{f, c->force64(), sizeof(double) * 3 * c->G}});
 }
 
 int hgpm_update_velocities(hgpm_ctx* c, double deltaT, double fscal) {

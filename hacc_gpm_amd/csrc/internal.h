@@ -29,10 +29,11 @@ struct FftOps {
     void (*pass_f32)(float2* d, int axis, int dir, const float2* tw, int variant, hipStream_t s);
     void (*pass_f64)(double2* d, int axis, int dir, const double2* tw, hipStream_t s);
     // Force component dim from the density's modes: inverse transform of i c_dim rho (w:
-    // work grid, may be rho itself), its real part to out (apart from w).  modes:
-    // (cos(2 pi i / N), sin(2 pi m / N)), m = i or (above N/2 - 1) i - N.
-    void (*force_f64)(const double2* rho, double2* w, double* out, const double2* tw, const double2* modes, int dim,
-                      hipStream_t s);
+    // work grid, may be rho itself), its real part to out (apart from w), or, with the other
+    // two components fx and fy, all three to out cell by cell.  modes: (cos(2 pi i / N),
+    // sin(2 pi m / N)), m = i or (above N/2 - 1) i - N.
+    void (*force_f64)(const double2* rho, double2* w, double* out, const double* fx, const double* fy,
+                      const double2* tw, const double2* modes, int dim, hipStream_t s);
     // half-spectrum solve (rows of hz = n/2 + 16 complex, k_z = 0..n/2) on nbox grids of
     // the same shape stored back to back; mass: HGPM_DEP_MASS partial sums of the deposited
     // mass per box
@@ -218,14 +219,10 @@ int ic_static_table(int device, double** ptr);
 void launch_f64_drift(double* pos, const double* vel, int64_t np3, int ng, double pf, hipStream_t s);
 void launch_f64_zero(double* p, size_t n, hipStream_t s);
 void launch_f64_cic(const double* pos, int64_t np3, int ng, double mass, double2* grid, hipStream_t s);
-// f: the three force components' grids
-struct ForceF64 {
-    const double* f[3];
-};
-void launch_f64_icic(const double* pos, double* vel, const ForceF64& f, int64_t np3, int ng, double deltaT,
+// force: three components a cell
+void launch_f64_icic(const double* pos, double* vel, const double* force, int64_t np3, int ng, double deltaT,
                      double fscal, hipStream_t s);
 void launch_f64_fold(double* pos, int64_t np3, int ng, hipStream_t s);
 void launch_f64_density_to_real(const double2* grid, double* out, int64_t g3, hipStream_t s);
-void launch_f64_force_out(const ForceF64& f, double* out, int64_t g3, hipStream_t s);
 
 } // namespace hgpm

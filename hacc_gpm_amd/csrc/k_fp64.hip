@@ -8,10 +8,9 @@
 //             src/pm_solver/cuda/kspace_solver.cu:55-90 (+ calcGreens), and its real part,
 //             getRealGrid, src/initial_conditions/cuda/transform_density_field_initializer.cu:14-28
 //   k_icic    ICICKernel            src/pm_actions/cuda/icic_pm.cu:72-127
-// The gather reads the three force components from grids of their own (copyGridToFloat4,
-// src/pm_solver/cuda/combine.cu:21-34, joins them).  A step of 128^3 went from 0.62 ms
-// (a pass for each component's modes, one for its real part, eight atomics per particle)
-// to 0.33 ms.
+// The last component's x pass joins the three (copyGridToFloat4,
+// src/pm_solver/cuda/combine.cu:21-34).  A step of 128^3 went from 0.62 ms (a pass for each
+// component's modes, one for its real part, eight atomics per particle) to 0.33 ms.
 #include "common.h"
 #include "internal.h"
 
@@ -90,29 +89,44 @@ __global__ __launch_bounds__(BS) void k_cic(const double* __restrict pos, int64_
         }
 }
 
-__global__ void k_icic(const double* __restrict pos, double* __restrict vel, const hgpm::ForceF64 F, int64_t n, int ng,
-                       double deltaT, double fscal) {
+// Bound by the lines that the lanes' corners touch: the three components of a cell lie
+// together (24 bytes), and the two corners of a row are read as one run.  Kicks of early /
+// dispersed / randomly ordered particles at 192^3: 0.23 / 0.51 / 0.72 ms; from three grids
+// 0.30 / 1.14 / 1.75, cell by cell 0.26 / 0.55 / 0.74.
+__global__ void k_icic(const double* __restrict pos, double* __restrict vel, const double* __restrict force, int64_t n,
+                       int ng, double deltaT, double fscal) {
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     int c[3][2];
     double f[3];
     corners(pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], ng, c, f);
     double dv0 = 0, dv1 = 0, dv2 = 0;
+    const int z = min(c[2][0], ng - 2); // both corners of a row from one run of 48 bytes ...
 #pragma unroll
     for (int x = 0; x < 2; x++)
 #pragma unroll
-        for (int y = 0; y < 2; y++)
+        for (int y = 0; y < 2; y++) {
+            const double dx = x ? f[0] : 1.0 - f[0];
+            const double dy = y ? f[1] : 1.0 - f[1];
+            const double* row = force + 3 * gidx(ng, c[0][x], c[1][y], 0);
+            double F[6];
 #pragma unroll
-            for (int z = 0; z < 2; z++) {
-                double dx = x ? f[0] : 1.0 - f[0];
-                double dy = y ? f[1] : 1.0 - f[1];
-                double dz = z ? f[2] : 1.0 - f[2];
-                const int64_t at = gidx(ng, c[0][x], c[1][y], c[2][z]);
-                double mul = dx * dy * dz * deltaT * fscal;
-                dv0 += mul * F.f[0][at];
-                dv1 += mul * F.f[1][at];
-                dv2 += mul * F.f[2][at];
+            for (int k = 0; k < 6; k++) F[k] = row[3 * z + k];
+            if (c[2][1] == 0) { // ... but the row's last cell and its first one
+#pragma unroll
+                for (int d = 0; d < 3; d++) {
+                    F[d] = F[3 + d];
+                    F[3 + d] = row[d];
+                }
             }
+            const double lo = dx * dy * (1.0 - f[2]) * deltaT * fscal, up = dx * dy * f[2] * deltaT * fscal;
+            dv0 += lo * F[0];
+            dv1 += lo * F[1];
+            dv2 += lo * F[2];
+            dv0 += up * F[3];
+            dv1 += up * F[4];
+            dv2 += up * F[5];
+        }
     vel[3 * i] += dv0;
     vel[3 * i + 1] += dv1;
     vel[3 * i + 2] += dv2;
@@ -130,12 +144,6 @@ __global__ void k_density_to_real(const double2* __restrict g, double* __restric
     int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < g3) out[i] = g[i].x;
 }
-__global__ void k_force_out(const hgpm::ForceF64 F, double* __restrict out, int64_t g3) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= g3) return;
-#pragma unroll
-    for (int d = 0; d < 3; d++) out[3 * i + d] = F.f[d][i];
-}
 } // namespace
 
 namespace hgpm {
@@ -151,17 +159,14 @@ void launch_f64_cic(const double* pos, int64_t n, int ng, double mass, double2* 
     launch_f64_zero((double*)grid, (size_t)2 * ng * ng * ng, s);
     if (n) k_cic<<<nblk(n), BS, 0, s>>>(pos, n, ng, mass, grid);
 }
-void launch_f64_icic(const double* pos, double* vel, const ForceF64& f, int64_t n, int ng, double deltaT,
+void launch_f64_icic(const double* pos, double* vel, const double* force, int64_t n, int ng, double deltaT,
                      double fscal, hipStream_t s) {
-    if (n) k_icic<<<nblk(n), BS, 0, s>>>(pos, vel, f, n, ng, deltaT, fscal);
+    if (n) k_icic<<<nblk(n), BS, 0, s>>>(pos, vel, force, n, ng, deltaT, fscal);
 }
 void launch_f64_fold(double* pos, int64_t n, int ng, hipStream_t s) {
     if (n) k_fold<<<nblk(3 * n), BS, 0, s>>>(pos, 3 * n, ng);
 }
 void launch_f64_density_to_real(const double2* grid, double* out, int64_t g3, hipStream_t s) {
     k_density_to_real<<<nblk(g3), BS, 0, s>>>(grid, out, g3);
-}
-void launch_f64_force_out(const ForceF64& f, double* out, int64_t g3, hipStream_t s) {
-    k_force_out<<<nblk(g3), BS, 0, s>>>(f, out, g3);
 }
 } // namespace hgpm

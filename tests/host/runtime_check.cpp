@@ -162,9 +162,8 @@ STUB(launch_compare, const PosPackH*, const float*, const double*, const double*
      const double*, const double*, int64_t, int, int, double*, hipStream_t)
 void launch_f64_cic(const double*, int64_t, int, double, double2*, hipStream_t) { holds_density = fake::launch(); }
 STUB(launch_f64_fold, double*, int64_t, int, hipStream_t)
-STUB(launch_f64_icic, const double*, double*, const ForceF64&, int64_t, int, double, double, hipStream_t)
+STUB(launch_f64_icic, const double*, double*, const double*, int64_t, int, double, double, hipStream_t)
 STUB(launch_f64_drift, double*, const double*, int64_t, int, double, hipStream_t)
-STUB(launch_f64_force_out, const ForceF64&, double*, int64_t, hipStream_t)
 STUB(launch_f64_density_to_real, const double2*, double*, int64_t, hipStream_t)
 STUB(launch_ic_lines, const double*, int, double, double, double2*, int, hipStream_t)
 STUB(launch_ic_noise_f32, float*, int, uint32_t, hipStream_t)
@@ -207,7 +206,7 @@ FftOps table(int n) {
     f.twiddles = [](double*, double*) {};
     f.pass_f32 = [](float2*, int, int, const float2*, int, hipStream_t) { (void)fake::launch(); };
     f.pass_f64 = [](double2*, int, int, const double2*, hipStream_t) { holds_density = fake::launch() && false; };
-    f.force_f64 = [](const double2*, double2*, double*, const double2*, const double2*, int, hipStream_t) { (void)fake::launch(); };
+    f.force_f64 = [](const double2*, double2*, double*, const double*, const double*, const double2*, const double2*, int, hipStream_t) { (void)fake::launch(); };
     f.pass_half = [](float2*, int, int, const float2*, int, int, hipStream_t) { (void)fake::launch(); };
     f.fwd_z_r2c = [](const long long*, const float*, const unsigned long long*, const unsigned long long*, float2*,
                      const float2*, int, hipStream_t) { (void)fake::launch(); };
