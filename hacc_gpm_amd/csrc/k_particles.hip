@@ -1168,8 +1168,8 @@ __global__ __launch_bounds__(DEP_NT, SMALL ? 4 : 1) void k_deposit_deferred(cons
 //   k_bin_pass<true>  : the folded positions written there;
 //   k_bin_owner       : a workgroup per block adds its entries' weights in int64 LDS cells
 //                       and writes every cell once;
-//   k_bin_rest        : the entries of a block past the first BIN_PIECE, a workgroup per
-//                       piece, added to the grid with atomics (the density is then the
+//   k_bin_rest        : the entries of a crowded block past the first BIN_PIECE, a workgroup
+//                       per piece, added to the grid with atomics (the density is then the
 //                       int64 one, as after deferred tiles).
 // A block is one workgroup's serial work, so without the pieces a box whose particles
 // crowd into few blocks took as long as one workgroup needs for most of them: a fold's P(k)
@@ -1185,8 +1185,9 @@ __global__ __launch_bounds__(DEP_NT, SMALL ? 4 : 1) void k_deposit_deferred(cons
 // fold 1 where np = ng, twice that with each fold until it is the grid's width.
 constexpr int BIN_W = 20;
 constexpr int BIN_SLOTS = BIN_W * BIN_W * BIN_W; // 32 KB of counters
-// 6 times the mean of a block at np = ng: evolved boxes of ordinary runs stay below it
-constexpr unsigned BIN_PIECE = 32768;
+// A block is crowded from 6 times the mean at np = ng on (evolved boxes of ordinary runs
+// stay below, and keep the FP32 density), and then shared in pieces of half that.
+constexpr unsigned BIN_CROWD = 32768, BIN_PIECE = 16384;
 constexpr int BIN_CTL_PIECES = DEP_CTL_SUB; // ctl word (no sub-arenas here): deferred lists pieces, not tiles
 struct BinArgs {
     const PosPack* __restrict pos;
@@ -1338,7 +1339,7 @@ __global__ __launch_bounds__(BIN_SCAN) void k_bin_scan(BinArgs g) {
         const unsigned n = g.count[b];
         g.start[b] = (unsigned)t;
         g.cursor[b] = (unsigned)t;
-        if (n > BIN_PIECE) {
+        if (n > BIN_CROWD) {
             unsigned q = atomicAdd(&s_pieces, (n - 1u) / BIN_PIECE);
             for (unsigned o = BIN_PIECE; o < n; o += BIN_PIECE, q++) {
                 g.deferred[q] = (unsigned)b;
@@ -1391,7 +1392,7 @@ template <bool SMALL> __global__ __launch_bounds__(OWN_NT) void k_bin_owner(BinA
     }
     for (int i = tid; i < OB * OB * OB; i += OWN_NT) acc[i] = 0ull;
     __syncthreads();
-    bin_add<SMALL, OWN_NT>(acc, g.entries + s_at, min(s_n, BIN_PIECE), b, ng, g.mass);
+    bin_add<SMALL, OWN_NT>(acc, g.entries + s_at, s_n > BIN_CROWD ? BIN_PIECE : s_n, b, ng, g.mass);
     __syncthreads();
     const bool f32 = g.rhof != nullptr && g.ctl[1] == 0ull;
     const double mean = (double)box_mass(g.mass_sum, 0) / (double)g.gcells;

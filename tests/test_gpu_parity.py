@@ -790,20 +790,20 @@ def test_power_spectrum_folded_lattice(hg, orc, ng, np_, folds, nb, sigma):
             c, o = orc.fold_split(ng, c, o)
 
 
-@pytest.mark.parametrize("ng,np_,kind,pieces", [(64, 64, "cell", 7), (64, 64, "edge", 14), (64, 64, "corner", 64),
-                                                (64, 64, "counts", 4), (128, 32, "corner", 0), (384, 64, "cell", 7),
+@pytest.mark.parametrize("ng,np_,kind,pieces", [(64, 64, "cell", 15), (64, 64, "edge", 30), (64, 64, "corner", 64),
+                                                (64, 64, "counts", 10), (128, 32, "corner", 0), (384, 64, "cell", 15),
                                                 (64, 64, "clump", None)])
 def test_power_spectrum_folded_crowded(hg, orc, ng, np_, kind, pieces):
-    """Folded positions crowded into few owner blocks, whose entries past the first 32768 are
-    added piece by piece: all in one cell; on the edge of two blocks (as many entries as the
+    """Folded positions crowded into few owner blocks, shared in pieces of 16384 entries from
+    32769 on: all in one cell; on the edge of two blocks (as many entries as the
     arena holds) and on a corner of eight (more than that, the atomic route, and one piece
-    each); blocks of exactly one and two pieces and of one entry more; mass 216 (weights over
+    each); blocks of three and four pieces, whole ones and one entry more; mass 216 (weights over
     31 bits); a clump.  The bits of the oracle's density, and of the atomic route."""
     case(f"power folded crowded ng={ng} np={np_} {kind}")
     rng = np.random.default_rng(ng)
     n = np_ ** 3
     if kind == "counts":
-        org = rng.permutation(np.repeat(np.arange(6), [32768, 32769, 65536, 65537, 32767, 32767]))
+        org = rng.permutation(np.repeat(np.arange(6), [32768, 32769, 49152, 49153, 65536, 32766]))
         y = 16.0 * np.stack([org % 2, org // 2 % 2, org // 4], 1) + 2.0 + 12.0 * rng.random((n, 3))
     else:
         y = np.array({"cell": 20.0, "edge": [15.0, 20.0, 20.0], "corner": 15.0, "clump": 0.0}[kind]) + rng.random((n, 3))
