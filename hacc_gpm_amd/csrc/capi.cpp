@@ -695,7 +695,7 @@ int hgpm_set_particles(hgpm_ctx* c, const float* pos, const float* vel) {
             p[i] = x;
             v[i] = vel[i];
         }
-        if (int rc = to_device(c, {{p.data(), c->pos64, sizeof(double) * n3}, {v.data(), c->vel64, sizeof(double) * n3}}))
+        if (int rc = to_device(c, {{p.data(), c->pos64, sizeof(double) * n3, 0, true}, {v.data(), c->vel64, sizeof(double) * n3, 0, true}}))
             return rc;
     }
     c->have_particles = true;
@@ -771,7 +771,7 @@ int hgpm_set_particles_split(hgpm_ctx* c, const int32_t* cell, const float* off,
     }
     PosPackH* sp = (PosPackH*)c->arena; // as in hgpm_set_particles
     float* sv = (float*)(sp + n);
-    if (int rc = to_device(c, {{h.data(), sp, sizeof(PosPackH) * n}, {(void*)vel, sv, sizeof(float) * 3 * n}})) return rc;
+    if (int rc = to_device(c, {{h.data(), sp, sizeof(PosPackH) * n, 0, true}, {(void*)vel, sv, sizeof(float) * 3 * n}})) return rc;
     launch_to_internal(sp, sv, c->pos, c->vel, c->N, c->np, c->st);
     LAUNCHCHK(c);
     HIPCHK(c, hipStreamSynchronize(c->st));
@@ -1102,7 +1102,7 @@ int hgpm_set_density_f64(hgpm_ctx* c, const double* rho) {
     if (c->prec != HGPM_FP64) return fail(c, HGPM_ERR_UNSUPPORTED, "FP64 density needs an FP64 context");
     std::vector<double> g(2 * (size_t)c->G, 0.0);
     for (int64_t i = 0; i < c->G; i++) g[2 * i] = rho[i];
-    if (int rc = to_device(c, {{g.data(), c->grid64, sizeof(double) * 2 * c->G}})) return rc;
+    if (int rc = to_device(c, {{g.data(), c->grid64, sizeof(double) * 2 * c->G, 0, true}})) return rc;
     c->have_density = true;
     c->have_force = false;
     return HGPM_OK;

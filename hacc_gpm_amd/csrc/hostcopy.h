@@ -6,12 +6,14 @@
 namespace hgpm {
 
 // One contiguous piece of a transfer.  check (to the device only): 0 = none, 1 = every
-// float finite, 2 = every float below 2^30 in magnitude (and not NaN).
+// float finite, 2 = every float below 2^30 in magnitude (and not NaN).  scratch: host memory
+// that the calling thread has just written and will write again on its next call.
 struct HostSeg {
     void* host;
     void* dev;
     size_t bytes;
     int check = 0;
+    bool scratch = false;
 };
 
 // Move the segments in order through a ring of pinned slots, the memory copies by several

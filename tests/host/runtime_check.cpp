@@ -482,15 +482,16 @@ void sizes() {
                                 16 * MB + 8, 32 * MB - 4, 32 * MB, 32 * MB + 4, 40 * MB + 12};
     for (size_t bytes : list)
         for (int parts : {1, 3})
-            for (int rule = 0; rule < 9; rule++) {
-                const int memory = fake::memory = rule / 3; // rule % 3: the check
+            for (int rule = 0; rule < 10; rule++) {
+                const int memory = fake::memory = rule / 3 % 3; // rule % 3: the check
+                const bool scratch = rule == 9;
                 std::vector<float> a(bytes / 4), b(bytes / 4), dev(bytes / 4);
                 for (size_t i = 0; i < a.size(); i++) a[i] = (float)(i % 65521);
                 hgpm::HostSeg up[3], down[3];
                 size_t o = 0;
                 for (int k = 0; k < parts; k++) { // uneven parts, none where there are no more bytes
                     const size_t m = k == parts - 1 ? a.size() - o : a.size() / (k + 3);
-                    up[k] = {a.data() + o, dev.data() + o, 4 * m, rule % 3};
+                    up[k] = {a.data() + o, dev.data() + o, 4 * m, rule % 3, scratch && k == 0};
                     down[k] = {b.data() + o, dev.data() + o, 4 * m};
                     o += m;
                 }
@@ -501,7 +502,7 @@ void sizes() {
                 fake::direct = fake::copies = 0;
                 check(hgpm::copy_to_device(up, parts, 0, nullptr, &out) == hipSuccess && out == -1, what + ": up");
                 check(dev == a, what + ": on the device");
-                const bool plain = rule % 3 == 0 && (memory == 2 || (bytes > MB && bytes <= 32 * MB));
+                const bool plain = rule % 3 == 0 && (memory == 2 || (bytes > MB && (bytes <= 32 * MB || scratch)));
                 check(plain ? fake::direct == fake::copies : fake::direct == 0, what + ": route up");
                 fake::lo = (const char*)b.data();
                 fake::hi = fake::lo + bytes;
