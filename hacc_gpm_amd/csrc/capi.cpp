@@ -993,11 +993,13 @@ int hgpm_generate_ic(hgpm_ctx* c, const double* ipk, int ipk_bins, double ipk_k_
                      double delta, double dot_delta, double fscal, double deltaT) {
     int rc = ic_check(c, ipk, ipk_bins, ipk_k_delta, ipk_k_max, "hgpm_generate_ic");
     if (rc) return rc;
-    // the table goes to the arena where the first n3 * 8 bytes hold it (free until the y
-    // pass of the displacements), else to a buffer of its own
+    // the table goes where nothing is written before its last reader: the first n3 * 8 bytes
+    // of the arena (until the y pass of the displacements), the FP64 grid (until the first
+    // displacement); one that these do not hold to a buffer of its own
     const size_t bytes = sizeof(double) * ipk_bins, n3 = (size_t)c->np * c->np * c->np;
-    const bool own = c->prec != HGPM_FP32 || bytes > 8 * n3;
-    double* d_ipk = (double*)c->arena;
+    const bool own = bytes > (c->prec == HGPM_FP32 ? 8 * n3 : sizeof(double2) * (size_t)c->G);
+    double* d_ipk = c->prec == HGPM_FP32 ? (double*)c->arena : (double*)c->grid64;
+    c->have_density = false;
     if (own) {
         if ((rc = dalloc(c, &d_ipk, bytes, "ipk"))) return rc;
         c->bytes -= bytes;
