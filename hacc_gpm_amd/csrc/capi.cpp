@@ -78,7 +78,7 @@ struct hgpm_ctx {
     double *pos64 = nullptr, *vel64 = nullptr;
     // grad64 (40 bytes a cell): the force; in the solve a work grid in its place, F_x and F_y behind
     double2 *grid64 = nullptr, *grad64 = nullptr;
-    double2* modes64 = nullptr;                   // cos, sin of the grid's wavenumbers
+    double2* modes64 = nullptr; // cos, sin of the grid's wavenumbers (behind pk_win)
     double2 *tw64 = nullptr, *tw64_ic = nullptr;
     // P(k)
     double *pk_partial = nullptr, *pk_sums = nullptr, *pk_win = nullptr;
@@ -587,24 +587,16 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
         if ((rc = dalloc(c, &c->pos64, sizeof(double) * 3 * N, "pos64")) ||
             (rc = dalloc(c, &c->vel64, sizeof(double) * 3 * N, "vel64")) ||
             (rc = dalloc(c, &c->grid64, sizeof(double2) * G, "grid64")) ||
-            (rc = dalloc(c, &c->grad64, grad_bytes, "grad64")) ||
-            (rc = dalloc(c, &c->modes64, sizeof(double2) * p->ng, "modes64")))
+            (rc = dalloc(c, &c->grad64, grad_bytes, "grad64")))
             return bail(rc);
-        std::vector<double2> modes(p->ng);
-        const double d = (2 * HGPM_PI_D) / (double)p->ng;
-        for (int i = 0; i < p->ng; i++) modes[i] = make_double2(cos(d * i), sin(d * (i > p->ng / 2 - 1 ? i - p->ng : i)));
-        if (hipMemcpy(c->modes64, modes.data(), sizeof(double2) * p->ng, hipMemcpyHostToDevice) != hipSuccess) {
-            c->err = "table upload failed";
-            return bail(HGPM_ERR_HIP);
-        }
         if ((rc = upload_twiddles<double2>(c, c->fft, &c->tw64, nullptr))) return bail(rc);
         if (c->np != c->ng) {
             if ((rc = upload_twiddles<double2>(c, c->fftic, &c->tw64_ic, nullptr))) return bail(rc);
         } else c->tw64_ic = c->tw64;
     }
-    // P(k) scratch and CIC window table (x/sin x)^4, x = pi m_s/ng
+    // P(k) scratch and CIC window table (x/sin x)^4, x = pi m_s/ng; behind it (FP64) the modes
     c->pk_blocks = power_partial_blocks(p->ng);
-    std::vector<double> win(p->ng);
+    std::vector<double> win((c->prec == HGPM_FP64 ? 3 : 1) * (size_t)p->ng);
     for (int m = 0; m < p->ng; m++) {
         int ms = m > p->ng / 2 - 1 ? m - p->ng : m;
         if (ms == 0) win[m] = 1.0;
@@ -612,15 +604,21 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
             double x = HGPM_PI_D * ms / p->ng, r = x / sin(x);
             win[m] = r * r * r * r;
         }
+        if (c->prec == HGPM_FP64) {
+            const double d = (2 * HGPM_PI_D) / (double)p->ng;
+            win[p->ng + 2 * m] = cos(d * m);
+            win[p->ng + 2 * m + 1] = sin(d * ms);
+        }
     }
     static_assert(sizeof(long long) == sizeof(double), "counts behind the sums");
     if ((rc = dalloc(c, &c->pk_partial, 2 * sizeof(double) * (size_t)c->pk_blocks * p->pk_bins, "pk partial")) ||
         (rc = dalloc(c, &c->pk_sums, 2 * sizeof(double) * p->pk_bins, "pk sums and counts")) ||
-        (rc = dalloc(c, &c->pk_win, sizeof(double) * p->ng, "pk window")) ||
+        (rc = dalloc(c, &c->pk_win, sizeof(double) * win.size(), "pk window")) ||
         (rc = dalloc(c, &c->flag, sizeof(int), "flag")))
         return bail(rc);
     c->pk_counts = (long long*)(c->pk_sums + p->pk_bins);
-    if (hipMemcpy(c->pk_win, win.data(), sizeof(double) * p->ng, hipMemcpyHostToDevice) != hipSuccess) {
+    c->modes64 = (double2*)(c->pk_win + p->ng);
+    if (hipMemcpy(c->pk_win, win.data(), sizeof(double) * win.size(), hipMemcpyHostToDevice) != hipSuccess) {
         c->err = "window upload failed";
         return bail(HGPM_ERR_HIP);
     }
@@ -635,7 +633,7 @@ int hgpm_destroy(hgpm_ctx* c) {
     if (!c) return HGPM_OK;
     if (c->st) (void)hipStreamSynchronize(c->st);
     void* ptrs[] = {c->pos, c->vel, c->A, c->B, c->psi, c->ctl, c->arena, c->dslots, c->dcount, c->deferred, c->wide, c->wide_slots, c->boxes, c->twf, c->twr, c->hs,
-                    c->pos64, c->vel64, c->grid64, c->grad64, c->modes64, c->tw64, c->pk_partial, c->pk_sums,
+                    c->pos64, c->vel64, c->grid64, c->grad64, c->tw64, c->pk_partial, c->pk_sums,
                     c->pk_win, c->flag};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
