@@ -1120,6 +1120,35 @@ def test_host_transfers(hg, n):
     assert got == {0: True, 1: True}
 
 
+@pytest.mark.parametrize("n", [32, 64, 96])
+def test_host_transfers_refuse_bad_values(hg, n):
+    """A value out of range, first, last or anywhere, in positions or velocities (one slot,
+    several pieces), is refused with its particle's index; the particles stay as they were,
+    and the context goes on."""
+    case(f"host transfers refused {n}^3")
+    rng = np.random.default_rng(n)
+    pos = (rng.integers(0, n << 12, (n ** 3, 3)) * 2.0 ** -12).astype(np.float32)
+    vel = rng.normal(0, 1, (n ** 3, 3)).astype(np.float32)
+    last = 3 * n ** 3 - 1
+    with mk(hg, n) as m:
+        m.set_particles(pos, vel)
+        for where in (0, last, int(rng.integers(1, last)), int(rng.integers(1, last))):
+            for array, bad in ((0, np.nan), (0, 2.0 ** 30), (0, -(2.0 ** 30)), (0, np.inf), (1, np.nan), (1, -np.inf)):
+                q = [pos.copy(), vel.copy()]
+                q[array].reshape(-1)[where] = bad
+                with pytest.raises(hg.HgpmError, match=f"index {where // 3}$"):
+                    m.set_particles(*q)
+        p, v = m.get_particles()
+        assert np.array_equal(p, pos) and np.array_equal(v, vel)
+        edge = pos.copy()  # the largest that is accepted, and a whole number of boxes off
+        edge[0] = np.nextafter(np.float32(2.0 ** 30), np.float32(0))
+        edge[1] = -(2.0 ** 29)
+        m.set_particles(edge, vel)
+        p, v = m.get_particles()
+        assert np.array_equal(p[2:], pos[2:]) and np.array_equal(v, vel)
+        assert np.array_equal(p[:2], np.mod(edge[:2].astype(np.float64), n).astype(np.float32))
+
+
 # -------------------------------------------------------------- ensemble ----
 def _ic_inputs(hg, p):
     import tempfile
