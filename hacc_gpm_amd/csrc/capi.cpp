@@ -33,7 +33,7 @@ struct PendingEv {
 struct hgpm_ctx {
     hgpm_params p{};
     int ng = 0, np = 0, prec = HGPM_FP32;
-    int64_t N = 0, G = 0, Gic = 0; // per box
+    int64_t N = 0, G = 0; // per box
     int nbox = 1; // FP32 batches: boxes of the same shape stored back to back (this launch)
     // Boxes whose particles are stored (nstore) and boxes the grids, arena and tile
     // buffers hold (nwave).  nstore > nwave: a step runs the boxes in waves of nwave,
@@ -84,7 +84,6 @@ struct hgpm_ctx {
     double *pk_partial = nullptr, *pk_sums = nullptr, *pk_win = nullptr;
     long long* pk_counts = nullptr; // behind pk_sums
     int pk_blocks = 0;
-    int* flag = nullptr;
     // state
     bool have_particles = false, have_density = false, have_force = false;
     bool dens_f32 = false; // the density may be the FP32 grid in psi's buffer (f32_deposit, fused)
@@ -251,12 +250,9 @@ int set_fft_plan(hgpm_ctx* c, int plan) {
 }
 
 // 3-D transform of an n^3 grid through the generic passes (z, y, x).
-int fft3d_f32(hgpm_ctx* c, const FftOps* ops, float2* d, const float2* tw, int dir) {
+int fft3d_f32(hgpm_ctx* c, float2* d, int dir) {
     Timed t(c, "fft3d_f32");
-    const int v = ops == c->fft ? c->var_cols : ops->variant;
-    ops->pass_f32(d, 2, dir, tw, v, c->st);
-    ops->pass_f32(d, 1, dir, tw, v, c->st);
-    ops->pass_f32(d, 0, dir, tw, v, c->st);
+    for (int axis = 2; axis >= 0; axis--) c->fft->pass_f32(d, axis, dir, c->twf, c->var_cols, c->st);
     LAUNCHCHK(c);
     return HGPM_OK;
 }
@@ -496,7 +492,6 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
     c->prec = p->precision;
     c->N = (int64_t)p->np * p->np * p->np;
     c->G = (int64_t)p->ng * p->ng * p->ng;
-    c->Gic = c->G; // np <= ng
     if (nwave < 1 || nwave > nbox) nwave = nbox;
     c->nstore = nbox;
     c->nwave = nwave;
@@ -613,8 +608,7 @@ int ctx_create(const hgpm_params* p, int nbox, hgpm_ctx** out, int nwave = 0) {
     static_assert(sizeof(long long) == sizeof(double), "counts behind the sums");
     if ((rc = dalloc(c, &c->pk_partial, 2 * sizeof(double) * (size_t)c->pk_blocks * p->pk_bins, "pk partial")) ||
         (rc = dalloc(c, &c->pk_sums, 2 * sizeof(double) * p->pk_bins, "pk sums and counts")) ||
-        (rc = dalloc(c, &c->pk_win, sizeof(double) * win.size(), "pk window")) ||
-        (rc = dalloc(c, &c->flag, sizeof(int), "flag")))
+        (rc = dalloc(c, &c->pk_win, sizeof(double) * win.size(), "pk window")))
         return bail(rc);
     c->pk_counts = (long long*)(c->pk_sums + p->pk_bins);
     c->modes64 = (double2*)(c->pk_win + p->ng);
@@ -634,7 +628,7 @@ int hgpm_destroy(hgpm_ctx* c) {
     if (c->st) (void)hipStreamSynchronize(c->st);
     void* ptrs[] = {c->pos, c->vel, c->A, c->B, c->psi, c->ctl, c->arena, c->dslots, c->dcount, c->deferred, c->wide, c->wide_slots, c->boxes, c->twf, c->twr, c->hs,
                     c->pos64, c->vel64, c->grid64, c->grad64, c->tw64, c->pk_partial, c->pk_sums,
-                    c->pk_win, c->flag};
+                    c->pk_win};
     for (void* q : ptrs)
         if (q) (void)hipFree(q);
     if (c->twf_ic && c->twf_ic != c->twf) (void)hipFree(c->twf_ic);
@@ -1223,7 +1217,7 @@ int hgpm_step(hgpm_ctx* c, const hgpm_step_coeffs* k) {
 // ------------------------------------------------------------------- FFT ----
 int hgpm_fft_device(hgpm_ctx* c, void* dev, int direction) {
     if (!c || !dev || (direction != -1 && direction != 1)) return fail(c, HGPM_ERR_ARG, "hgpm_fft_device: bad arguments");
-    return c->prec == HGPM_FP32 ? fft3d_f32(c, c->fft, (float2*)dev, c->twf, direction)
+    return c->prec == HGPM_FP32 ? fft3d_f32(c, (float2*)dev, direction)
                                 : fft3d_f64(c, c->fft, (double2*)dev, c->tw64, direction);
 }
 

@@ -85,7 +85,6 @@ struct PosPackH { unsigned x, y, z; };
 constexpr int HGPM_CELL_BITS_H = 10;
 constexpr int HGPM_FRAC_BITS_H = 22;
 constexpr int HGPM_MAX_CELLS = 1 << HGPM_CELL_BITS_H; // cells per side of the FP32 engine's grid
-void launch_zero_i64(long long* p, size_t n, hipStream_t s);
 void launch_zero_u64(unsigned long long* p, size_t n, hipStream_t s);
 void launch_drift(PosPackH* pos, const float* vel, int64_t np3, int ng, float pf, hipStream_t s);
 // Deposit buffers.  np3 is a multiple of HGPM_TL^3 and ng of 16 (supported sizes).
@@ -170,7 +169,6 @@ void launch_to_reference(const PosPackH* src, const float* vsrc, PosPackH* dst, 
                          hipStream_t s);
 // forces (3 floats per cell) of one box from its potential, as the gather forms them
 void launch_force_from_psi(const float* psi, float* out, int ng, hipStream_t s);
-void launch_scan_nonfinite(const float* v, int64_t n, int* flag, hipStream_t s);
 // FP64 reference-order double3 <-> FP32 split layout in internal order (one box)
 void launch_split_from_f64(const double* p3, const double* v3, PosPackH* pos, float* vel, int64_t n, int np, int ng,
                            hipStream_t s);

@@ -1926,14 +1926,6 @@ __global__ void k_force_from_psi(const float* __restrict psi, float* __restrict 
     out[3 * i + 1] = central_diff(psi[gidx(ng, x, yp, z)], psi[gidx(ng, x, ym, z)]);
     out[3 * i + 2] = central_diff(psi[gidx(ng, x, y, zp)], psi[gidx(ng, x, y, zm)]);
 }
-
-__global__ void k_scan_nonfinite(const float* __restrict v, int64_t n, int* __restrict flag) {
-    int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t st = (int64_t)gridDim.x * blockDim.x;
-    int bad = 0;
-    for (; i < n; i += st) bad |= !isfinite(v[i]);
-    if (bad) atomicOr(flag, 1);
-}
 } // namespace
 
 namespace hgpm {
@@ -1944,9 +1936,6 @@ void launch_zero_u64(unsigned long long* p, size_t n, hipStream_t s) {
     unsigned nb = (unsigned)((n + BS - 1) / BS);
     if (nb > 65536u * 8) nb = 65536u * 8;
     k_zero_u64<<<nb, BS, 0, s>>>(p, n);
-}
-void launch_zero_i64(long long* p, size_t n, hipStream_t s) {
-    launch_zero_u64((unsigned long long*)p, n, s);
 }
 void launch_drift(PosPackH* pos, const float* vel, int64_t n, int ng, float pf, hipStream_t s) {
     if (!n) return;
@@ -2149,11 +2138,5 @@ void launch_compare(const PosPackH* pa, const float* va, const double* pa64, con
     else if (a64) k_compare<true, false><<<CMP_WG, CMP_NT, 0, s>>>(a, b, n, np, ng, partial);
     else if (b64) k_compare<false, true><<<CMP_WG, CMP_NT, 0, s>>>(a, b, n, np, ng, partial);
     else k_compare<false, false><<<CMP_WG, CMP_NT, 0, s>>>(a, b, n, np, ng, partial);
-}
-void launch_scan_nonfinite(const float* v, int64_t n, int* flag, hipStream_t s) {
-    unsigned nb = grid_blocks(n, BS);
-    if (nb > 4096) nb = 4096;
-    if (nb == 0) nb = 1;
-    k_scan_nonfinite<<<nb, BS, 0, s>>>(v, n, flag);
 }
 } // namespace hgpm
