@@ -919,8 +919,8 @@ int generate_ic_from(hgpm_ctx* c, const double* d_ipk, int ipk_bins, double ipk_
         float velMul = (float)((double)(velA * velA) * dot_delta * fscal);
         // Half spectra throughout (the noise and the displacements are real): noise ->
         // modes -> phi^ (k_x_ic) -> the three displacement components, in the arena
-        // (24 bytes per grid cell: one half spectrum and four real grids of np^3), which
-        // holds nothing between deposits.
+        // (24 bytes per grid cell: one half spectrum and three real grids of np^3 take 20),
+        // which holds nothing between deposits.
         const FftOps* f = c->fftic;
         const size_t n3 = (size_t)np * np * np;
         float2* h3 = (float2*)c->arena;

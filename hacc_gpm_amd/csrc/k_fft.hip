@@ -364,8 +364,8 @@ __global__ __launch_bounds__(NTC) void k_y_ic(float2* __restrict h2, float2* __r
 
 // k_x_psi as a streaming pass: the next tile is loaded once the inverse transform's first
 // stage has freed the spectrum's registers.  Measured in a run, against the same shape (16
-// columns x 1024 threads) with a workgroup per tile: 2.54 -> 2.24 ms at 1024, 1.15 -> 0.86
-// at 768; at 512, where a tile takes half the LDS, 0.267 -> 0.25-0.31 with one or two
+// columns x 1024 threads) with a workgroup per tile: 2.5-2.6 -> 2.25 ms at 1024, 1.12-1.15
+// -> 0.86-0.90 at 768; at 512, where a tile takes half the LDS, 0.267 -> 0.25-0.31 with one or two
 // workgroups per CU, so the plain form stays there.  The y passes, one transform per tile,
 // gained nothing from the same treatment (1.80 / 1.67 -> 1.93 / 1.72 ms at 1024).
 constexpr bool STREAM_X = N > 512;

@@ -1174,8 +1174,8 @@ __global__ __launch_bounds__(DEP_NT, SMALL ? 4 : 1) void k_deposit_deferred(cons
 // A block is one workgroup's serial work, so without the pieces a box whose particles
 // crowd into few blocks took as long as one workgroup needs for most of them: a fold's P(k)
 // of 16.8 M in one cell of 256^3 52 to 112 ms (now 0.7), in a clump of two cells' width 11
-// (0.7).  The sums are whole numbers, so the bits are those of every other route.  Entries beyond
-// the arena send the deposit to the atomic route (all tiles listed as deferred).  Bound by
+// (0.6).  The sums are whole numbers, so the bits are those of every other route.  Entries
+// beyond the arena send the deposit to the atomic route (all tiles listed as deferred).  Bound by
 // the scattered writes, the LDS atomics and the memory it moves (about 60 bytes a
 // particle).  Evolved boxes, np = ng, one fold: 0.39 ms at 256^3 (count 0.106, write 0.127,
 // owner blocks 0.142), 2.65 ms at 512^3, 18.8 ms at 1024^3; with the blocks in an LDS hash

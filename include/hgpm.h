@@ -302,7 +302,8 @@ int hgpm_reset_timings(hgpm_ctx* ctx);
    that needed 64-bit sums (a 64-bit chunk, or a cell sum of 2^32 units or more);
    "deposit_arena_mwords" (get only) = 32-bit arena words the last
    deposit reserved, in units of 2^20 (every window reservation, those of tiles then
-   found full and the doubled ones of the 64-bit pass included).  Unknown keys return HGPM_ERR_ARG. */
+   found full and the doubled ones of the 64-bit pass included; 0 after a folded
+   P(k)).  Unknown keys return HGPM_ERR_ARG. */
 int hgpm_set_tunable(hgpm_ctx* ctx, const char* key, int value);
 int hgpm_get_tunable(hgpm_ctx* ctx, const char* key, int* value);
 /* Autotuner (no reference counterpart; HACC_GPM has fixed cuFFT plans): for each radix
